@@ -3,6 +3,7 @@ measurement probes of the benchmark) in-tree for gfx950."""
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -18,6 +19,7 @@ SOURCES = {
     "w4a16_strip.hip": [],
     "w4a16_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "w4a16_prefill_wide.hip": [],
+    "w4a16_convert.hip": [],
     "f16_streamk.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -47,11 +49,11 @@ def build_library(verbose=False):
     # loop and accumulator hand-over with fixed registers) are written by a
     # generator; w4a16_prefill_wide.hip includes them from the build directory
     _run([sys.executable, os.path.join(CSRC, "gen_prefill_wide.py"), objdir], verbose)
-    objs = []
-    for src, extra in SOURCES.items():
-        obj = os.path.join(objdir, src.replace(".hip", ".o"))
-        _run([HIPCC] + FLAGS + extra + ["-c", "-o", obj, os.path.join(CSRC, src)], verbose)
-        objs.append(obj)
+    objs = [os.path.join(objdir, src.replace(".hip", ".o")) for src in SOURCES]
+    with ThreadPoolExecutor(4) as pool:
+        list(pool.map(lambda job: _run([HIPCC] + FLAGS + job[0][1] + ["-c", "-o", job[1],
+                                                                      os.path.join(CSRC, job[0][0])],
+                                       verbose), zip(SOURCES.items(), objs)))
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs, verbose)
     # the probes: a library of their own that asks the first one for its plans
     obj = os.path.join(objdir, "w4a16_probe.o")

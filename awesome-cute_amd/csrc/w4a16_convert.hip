@@ -1,0 +1,410 @@
+// Weight conversion on the GPU: fp16 weights to 4-bit integers, fake weights
+// and scales (quantise_*), and fake weights to the packed layout (pack_*), the
+// arithmetic of the reference's Layer.pack (marlin.py:92-131) and of its
+// tests' quantiser (marlin_test.py:18-40).
+//
+// Bound: memory.  As a sequence of tensor operations the two took some thirty
+// passes over the weight, half of them over 64-bit integers (n = 11008, k =
+// 4096: 1712 us for the pair).  Here each is one pass: the quantiser reads a
+// weight once (twice where a group does not fit into registers) and writes its
+// 6 bytes, the packer reads it once and writes its half byte: 97 us for the
+// pair, 70 of it the quantiser.
+//
+// Every rounding is that of the tensor operations: fp16(w / s) is the rounded
+// fp32 quotient rounded once more, the integer is rounded half to even, and
+// (q - 8) * s is rounded once.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <cstdio>
+
+#include "../../include/marlin_amd_convert.h"
+#include "w4a16_common.hpp"
+
+namespace w4a16 {
+
+namespace {
+
+typedef unsigned short us4 __attribute__((ext_vector_type(4)));
+typedef unsigned short us8 __attribute__((ext_vector_type(8)));
+
+constexpr int kQThreads = 512;
+constexpr int kPThreads = 256;
+constexpr int kKeep = 16;  // 8-byte pieces of its group a thread keeps between the two passes
+
+// Bit patterns of non-negative halves order as their values, infinity above
+// all numbers and NaN above infinity: an integer maximum hands on a NaN, as
+// the tensor operation does.
+__device__ __forceinline__ us4 abs_bits(i2 v) {
+  return __builtin_bit_cast(us4, v & (i2){0x7fff7fff, 0x7fff7fff});
+}
+__device__ __forceinline__ us4 max_of(us4 a, us4 b) { return __builtin_elementwise_max(a, b); }
+__device__ __forceinline__ us4 shfl_xor_of(us4 v, int mask) {
+  i2 x = __builtin_bit_cast(i2, v);
+  x[0] = __shfl_xor(x[0], mask);
+  x[1] = __shfl_xor(x[1], mask);
+  return __builtin_bit_cast(us4, x);
+}
+
+__device__ __forceinline__ half_t scale_of(unsigned short max_bits) {
+  return (half_t)((float)__builtin_bit_cast(half_t, max_bits) * (float)(2.0 / 15.0));
+}
+
+// round(fp16(w / s)) + 8, clamped to 0 ... 15, with r an approximation of
+// 1 / s.  The quotient of two halves is either a number of at most 12 bits or
+// at least 2^-24 of itself away from one, so a quotient within an fp32 ulp
+// that is exact where the true one has 12 bits rounds to the same half; one
+// residual step on w * r gives that.  Where the residual is not a number (a
+// zero or infinite operand, NaN) the division itself decides.
+__device__ __forceinline__ int quantised(half_t w, float s, float r) {
+  const float x = (float)w;
+  float q = x * r;
+  const float e = __builtin_fmaf(-q, s, x);
+  q = __builtin_fmaf(e, r, q);
+  if (__builtin_expect(!(__builtin_fabsf(e) < __builtin_inff()), 0)) q = x / s;
+  const float h = (float)(half_t)q;
+  // a NaN becomes 0 and an infinity the largest integer, which wraps
+  const int i = (int)((unsigned)__float2int_rn(h) + 8u);
+  return i < 0 ? 0 : i > 15 ? 15 : i;
+}
+
+template <int N>
+struct Columns {  // N columns' scales and their reciprocals
+  float s[N], r[N];
+  __device__ __forceinline__ void set(int i, half_t v) {
+    s[i] = (float)v;
+    r[i] = __builtin_amdgcn_rcpf(s[i]);
+  }
+};
+
+// Four neighbouring elements: fake weights and integers out.  Four and not
+// eight, so that the lanes of a store instruction write whole lines of both
+// (eight: two instructions that each write every other 16 bytes of the
+// integers; n = 11008, k = 4096: 101 us against 70, 5.1 TB/s).
+template <class S>
+__device__ __forceinline__ void write4(i2 v, const S& c, half_t* fake, int* q) {
+  const h4 w = __builtin_bit_cast(h4, v);
+  h4 f;
+  i4 o;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int x = quantised(w[i], c.s[i], c.r[i]);
+    f[i] = (half_t)(x - 8) * (half_t)c.s[i];
+    o[i] = x;
+  }
+  *(h4*)fake = f;
+  // (nothing reads the integers soon; the packer reads the fake weights)
+  __builtin_nontemporal_store(o, (i4*)q);
+}
+
+// (k, n), columns contiguous.  A workgroup takes one group of 4 CL columns, a
+// thread four of them and every (512 / CL)-th row.  CL = 64 for groups of up
+// to 128 rows, which then stay in registers; CL = 16 for longer ones, so that
+// one group per column still gives n / 64 workgroups (n = 11008: 172).
+template <int CL>
+__global__ __launch_bounds__(kQThreads) void quantise_rows(const half_t* w, int n, int gs,
+                                                           half_t* fake, int* q, half_t* s) {
+  constexpr int RL = kQThreads / CL;
+  constexpr bool KEEP = CL == 64;
+  __shared__ us4 part[kQThreads / kWave][CL];
+  const int cl = threadIdx.x % CL, rl = threadIdx.x / CL;
+  const int c0 = ((int)blockIdx.x * CL + cl) * 4;
+  const bool on = c0 < n;
+  const size_t base = (size_t)blockIdx.y * gs * n + c0;
+  i2 keep[KEEP ? kKeep : 1];
+  us4 top = (us4)0;
+  if (KEEP) {
+#pragma unroll
+    for (int i = 0; i < kKeep; i++) {
+      const int row = rl + i * RL;
+      keep[i] = on && row < gs ? *(const i2*)(w + base + (size_t)row * n) : (i2)0;
+    }
+#pragma unroll
+    for (int i = 0; i < kKeep; i++) top = max_of(top, abs_bits(keep[i]));
+  } else if (on) {
+#pragma unroll 8
+    for (int row = rl; row < gs; row += RL)
+      top = max_of(top, abs_bits(*(const i2*)(w + base + (size_t)row * n)));
+  }
+#pragma unroll
+  for (int m = CL; m < kWave; m *= 2) top = max_of(top, shfl_xor_of(top, m));
+  if ((threadIdx.x & 63) < CL) part[threadIdx.x / kWave][cl] = top;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kQThreads / kWave; i++) top = max_of(top, part[i][cl]);
+  if (!on) return;
+  Columns<4> col;
+  h4 sv;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    sv[i] = scale_of(top[i]);
+    col.set(i, sv[i]);
+  }
+  if (rl == 0) *(h4*)(s + (size_t)blockIdx.y * n + c0) = sv;
+  if (KEEP) {
+#pragma unroll
+    for (int i = 0; i < kKeep; i++) {
+      const int row = rl + i * RL;
+      const size_t at = base + (size_t)row * n;
+      if (row < gs) write4(keep[i], col, fake + at, q + at);
+    }
+  } else {
+#pragma unroll 4
+    for (int row = rl; row < gs; row += RL) {
+      const size_t at = base + (size_t)row * n;
+      write4(*(const i2*)(w + at), col, fake + at, q + at);
+    }
+  }
+}
+
+struct OneColumn {
+  struct Same {
+    float v;
+    __device__ __forceinline__ float operator[](int) const { return v; }
+  } s, r;
+};
+
+// The same values stored column by column, (n, k).  T neighbouring threads
+// take one group of one column, 4 T k-values at a time: 32 for groups of up to
+// 128, the whole workgroup for longer ones.
+template <int T>
+__global__ __launch_bounds__(kPThreads) void quantise_columns(const half_t* w, int n, int k, int gs,
+                                                              half_t* fake, int* q, half_t* s) {
+  __shared__ unsigned part[kPThreads / kWave];
+  const int groups = k / gs;
+  const long long team = (long long)blockIdx.x * (kPThreads / T) + threadIdx.x / T;
+  if (T < kPThreads && team >= (long long)n * groups) return;  // whole teams, no barrier below
+  const int at0 = (int)(threadIdx.x % T) * 4;
+  const size_t base = (size_t)(team / groups) * k + (size_t)(team % groups) * gs;
+  const i2 first = at0 < gs ? *(const i2*)(w + base + at0) : (i2)0;
+  us4 top = abs_bits(first);
+  for (int at = at0 + 4 * T; at < gs; at += 4 * T)
+    top = max_of(top, abs_bits(*(const i2*)(w + base + at)));
+  unsigned m = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) m = top[i] > m ? top[i] : m;
+#pragma unroll
+  for (int x = 1; x < (T < kWave ? T : kWave); x *= 2) {
+    const unsigned o = __shfl_xor(m, x);
+    m = o > m ? o : m;
+  }
+  if (T > kWave) {
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x / kWave] = m;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPThreads / kWave; i++) m = part[i] > m ? part[i] : m;
+  }
+  const half_t sv = scale_of((unsigned short)m);
+  const float sf = (float)sv;
+  const OneColumn col = {{sf}, {__builtin_amdgcn_rcpf(sf)}};
+  if (at0 == 0) s[(size_t)(team % groups) * n + team / groups] = sv;
+  if (at0 < gs) write4(first, col, fake + base + at0, q + base + at0);
+  for (int at = at0 + 4 * T; at < gs; at += 4 * T)
+    write4(*(const i2*)(w + base + at), col, fake + base + at, q + base + at);
+}
+
+// position of column c's scale in the packed order: an 8 x 8 transpose in
+// blocks of 64 columns with group scales, {2i, 2i+1} of every 8 gathered in
+// blocks of 32 with one scale per column (reference marlin.py:49-55)
+__device__ __forceinline__ int scale_slot(int c, bool grouped) {
+  if (grouped) return (c & ~63) + 8 * (c & 7) + ((c >> 3) & 7);
+  return (c & ~31) + 8 * ((c >> 1) & 3) + 2 * ((c >> 3) & 3) + (c & 1);
+}
+
+struct PackArgs {
+  const void* w;
+  const half_t* scales;
+  long long s_group, s_col;
+  int* B;
+  half_t* s_packed;
+  int k, n, gs;  // gs: k-values per scale
+  bool grouped;
+};
+
+// (k, n), columns contiguous; whole numbers (INTS) or fake weights.  Word
+// (t, c, j) of a 16 x 64 block holds rows 2t, 2t+1, 2t+8, 2t+9 of columns
+// 16j + c and 16j + c + 8 (reference marlin.py:29-48): thread (t, 8 columns)
+// reads those four rows, has one half of eight words, and exchanges four
+// halves with the thread of the other eight columns.  Four t and sixteen
+// column threads in a wave: a row is read in runs of 256 bytes, and a store
+// instruction writes runs of 64.
+template <bool INTS>
+__global__ __launch_bounds__(kPThreads) void pack_rows(PackArgs p) {
+  const int t = threadIdx.x & 3;
+  const int c0 = ((int)blockIdx.x * (kPThreads / 4) + (int)(threadIdx.x >> 2)) * 8;
+  if (c0 >= p.n) return;  // (both threads of an exchange or neither: n is a multiple of 64)
+  const int kt = blockIdx.y;
+  int half[8];
+  Columns<8> col;
+  if (!INTS) {
+    const int g = 16 * kt / p.gs;
+    half_t sv[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      sv[i] = p.scales[g * p.s_group + (c0 + i) * p.s_col];
+      col.set(i, sv[i]);
+    }
+    if (t == 0 && 16 * kt == g * p.gs) {
+      half_t* out = p.s_packed + (size_t)g * p.n;
+#pragma unroll
+      for (int i = 0; i < 8; i++) out[scale_slot(c0 + i, p.grouped)] = sv[i];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int row = 16 * kt + 2 * t + (r & 1) + 8 * (r >> 1);
+    const int shift = 16 * (r & 1) + 4 * (r >> 1);
+    const size_t at = (size_t)row * p.n + c0;
+    int v[8];
+    if (INTS) {
+      *(i4*)v = *(const i4*)((const int*)p.w + at);
+      *(i4*)(v + 4) = *(const i4*)((const int*)p.w + at + 4);
+    } else {
+      const h8 w = *(const h8*)((const half_t*)p.w + at);
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = quantised(w[i], col.s[i], col.r[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) half[i] = r == 0 ? v[i] : half[i] | (v[i] << shift);
+  }
+  const int odd = (c0 >> 3) & 1;  // columns 8 ... 15 of their sixteen
+  int* B = p.B + (size_t)kt * 2 * p.n + (c0 >> 6) * 128 + ((c0 >> 4) & 3) + 4 * t;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int got = __shfl_xor(odd ? half[i] : half[i + 4], 4);
+    // even: c = i with the partner's columns above; odd: c = i + 4
+    const int word = odd ? got | (half[i + 4] << 8) : half[i] | (got << 8);
+    B[16 * (i + 4 * odd)] = word;
+  }
+}
+
+// Fake weights stored column by column, (n, k): a thread takes 64 k-values of
+// one column (a whole cache line), a wave a 64-column block, whose four rows of
+// B it writes completely.
+__global__ __launch_bounds__(kPThreads) void pack_columns(PackArgs p) {
+  const int lane = threadIdx.x & 63;
+  const int blk = (int)blockIdx.x;
+  const int k0 = ((int)blockIdx.y * (kPThreads / kWave) + (int)(threadIdx.x >> 6)) * 64;
+  if (k0 >= p.k) return;
+  const int c = blk * 64 + lane;
+  const int g = k0 / p.gs;
+  const half_t sv = p.scales[g * p.s_group + c * p.s_col];
+  const float s = (float)sv, rs = __builtin_amdgcn_rcpf(s);
+  if (k0 == g * p.gs) p.s_packed[(size_t)g * p.n + scale_slot(c, p.grouped)] = sv;
+  const h8* src = (const h8*)((const half_t*)p.w + (size_t)c * p.k + k0);
+  const int hi = (lane >> 3) & 1;
+#pragma unroll
+  for (int kt = 0; kt < 4; kt++) {
+    const h8 a = src[2 * kt], b = src[2 * kt + 1];
+    int half[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      half[t] = quantised(a[2 * t], s, rs) | (quantised(a[2 * t + 1], s, rs) << 16) |
+                (quantised(b[2 * t], s, rs) << 4) | (quantised(b[2 * t + 1], s, rs) << 20);
+    int* B = p.B + (size_t)(k0 / 16 + kt) * 2 * p.n + blk * 128 + 16 * (lane & 7) + (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {  // columns c: words t = 0, 1; columns c + 8: t = 2, 3
+      const int got = __shfl_xor(hi ? half[i] : half[i + 2], 8);
+      B[4 * (i + 2 * hi)] = hi ? got | (half[i + 2] << 8) : half[i] | (got << 8);
+    }
+  }
+}
+
+thread_local char g_convert_error[256] = "";
+
+// `dev` current for the length of a call
+struct OnDevice {
+  int prev = -1;
+  hipError_t e;
+  explicit OnDevice(int dev) {
+    e = hipGetDevice(&prev);
+    if (e == hipSuccess && prev != dev) e = hipSetDevice(dev);
+    else prev = -1;
+    (void)hipGetLastError();  // an earlier call's error is not this launch's
+  }
+  int done() {
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) return MARLIN_OK;
+    snprintf(g_convert_error, sizeof(g_convert_error), "%s", hipGetErrorString(e));
+    return MARLIN_ERR_RUNTIME;
+  }
+  ~OnDevice() {
+    if (prev >= 0) (void)hipSetDevice(prev);
+  }
+};
+
+constexpr int kMaxGridY = 65535;
+
+bool aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+}  // namespace
+
+}  // namespace w4a16
+
+using namespace w4a16;
+
+extern "C" {
+
+int marlin_amd_quantize(const void* w, int k, int n, int groupsize, int by_column, void* fake,
+                        void* q, void* s, int dev, void* stream) {
+  const int gs = groupsize == -1 ? k : groupsize;
+  if (k <= 0 || n <= 0 || gs <= 0 || k % gs != 0 || (by_column ? gs : n) % 4 != 0 ||
+      k / gs > kMaxGridY || !aligned(w) || !aligned(fake) || !aligned(q) || !aligned(s))
+    return MARLIN_ERR_PROB_SHAPE;
+  if (by_column && (k % 4 != 0 || (long long)n * (k / gs) > 0x7fffffffLL)) return MARLIN_ERR_PROB_SHAPE;
+  OnDevice on(dev);
+  if (on.e != hipSuccess) return on.done();
+  const half_t* in = (const half_t*)w;
+  const hipStream_t st = (hipStream_t)stream;
+  if (by_column) {
+    const long long teams = (long long)n * (k / gs);
+    if (gs <= 128)
+      hipLaunchKernelGGL(quantise_columns<32>, dim3((unsigned)((teams + 7) / 8)), dim3(kPThreads), 0,
+                         st, in, n, k, gs, (half_t*)fake, (int*)q, (half_t*)s);
+    else
+      hipLaunchKernelGGL(quantise_columns<kPThreads>, dim3((unsigned)teams), dim3(kPThreads), 0, st,
+                         in, n, k, gs, (half_t*)fake, (int*)q, (half_t*)s);
+  } else if (gs <= 128) {
+    hipLaunchKernelGGL(quantise_rows<64>, dim3(ceil_div(n, 256), k / gs), dim3(kQThreads), 0, st, in,
+                       n, gs, (half_t*)fake, (int*)q, (half_t*)s);
+  } else {
+    hipLaunchKernelGGL(quantise_rows<16>, dim3(ceil_div(n, 64), k / gs), dim3(kQThreads), 0, st, in, n,
+                       gs, (half_t*)fake, (int*)q, (half_t*)s);
+  }
+  return on.done();
+}
+
+int marlin_amd_pack(const void* w, int k, int n, int groupsize, int by_column, const void* scales,
+                    long long s_group, long long s_col, void* B, void* s_packed, int dev,
+                    void* stream) {
+  const int gs = groupsize == -1 ? k : groupsize;
+  if (k <= 0 || n <= 0 || gs <= 0 || n % 64 != 0 || k % 64 != 0 || gs % 64 != 0 || k % gs != 0 ||
+      k / 16 > kMaxGridY || !aligned(w) || !aligned(B))
+    return MARLIN_ERR_PROB_SHAPE;
+  OnDevice on(dev);
+  if (on.e != hipSuccess) return on.done();
+  const PackArgs p = {w, (const half_t*)scales, s_group, s_col, (int*)B, (half_t*)s_packed,
+                      k, n, gs, groupsize != -1};
+  if (by_column)
+    hipLaunchKernelGGL(pack_columns, dim3(n / 64, ceil_div(k, 256)), dim3(kPThreads), 0,
+                       (hipStream_t)stream, p);
+  else
+    hipLaunchKernelGGL(pack_rows<false>, dim3(ceil_div(n, 2 * kPThreads), k / 16), dim3(kPThreads), 0,
+                       (hipStream_t)stream, p);
+  return on.done();
+}
+
+int marlin_amd_pack_words(const void* q, int k, int n, void* B, int dev, void* stream) {
+  if (k <= 0 || n <= 0 || n % 64 != 0 || k % 16 != 0 || k / 16 > kMaxGridY || !aligned(q) || !aligned(B))
+    return MARLIN_ERR_PROB_SHAPE;
+  OnDevice on(dev);
+  if (on.e != hipSuccess) return on.done();
+  const PackArgs p = {q, nullptr, 0, 0, (int*)B, nullptr, k, n, k, false};
+  hipLaunchKernelGGL(pack_rows<true>, dim3(ceil_div(n, 2 * kPThreads), k / 16), dim3(kPThreads), 0,
+                     (hipStream_t)stream, p);
+  return on.done();
+}
+
+const char* marlin_amd_convert_last_error(void) { return g_convert_error; }
+
+}  // extern "C"

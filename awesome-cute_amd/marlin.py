@@ -53,6 +53,14 @@ _lib.marlin_amd_force_strips.restype = None
 _lib.marlin_amd_force_strips.argtypes = [_I]
 _lib.marlin_amd_work_order.restype = None
 _lib.marlin_amd_work_order.argtypes = [_I, _P]
+_L = ctypes.c_longlong
+_lib.marlin_amd_quantize.restype = _I
+_lib.marlin_amd_quantize.argtypes = [_P, _I, _I, _I, _I, _P, _P, _P, _I, _P]
+_lib.marlin_amd_pack.restype = _I
+_lib.marlin_amd_pack.argtypes = [_P, _I, _I, _I, _I, _P, _L, _L, _P, _P, _I, _P]
+_lib.marlin_amd_pack_words.restype = _I
+_lib.marlin_amd_pack_words.argtypes = [_P, _I, _I, _P, _I, _P]
+_lib.marlin_amd_convert_last_error.restype = ctypes.c_char_p
 _lib.marlin_amd_last_error.restype = ctypes.c_char_p
 _lib.marlin_amd_version.restype = ctypes.c_char_p
 
@@ -170,11 +178,38 @@ _k_in_block, _n_in_block = _block_coords()
 _block_gather = torch.from_numpy((64 * _k_in_block + _n_in_block).reshape(-1).astype(np.int64))
 
 
+# Conversion on the GPU: one kernel each for quantising, for packing fake
+# weights and for packing integers, where the tensors are laid out as the
+# kernels read them; the tensor operations beside them serve every other device,
+# type and layout, and give the same bits.
+
+def _on_gpu(*tensors):
+    """Whether the kernels may take these tensors: plain, on one GPU, 16-byte aligned, and no
+    compiler or autograd looking on."""
+    dev = tensors[0].device
+    return (dev.type == "cuda" and not torch.compiler.is_compiling()
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            and all(t.device == dev and type(t) in (torch.Tensor, nn.Parameter)
+                    and t.data_ptr() % 16 == 0 for t in tensors))
+
+
+def _convert_check(rc):
+    if rc != 0:
+        raise RuntimeError(f"weight conversion failed with code {rc}: "
+                           f"{_lib.marlin_amd_convert_last_error().decode()}")
+
+
 def pack_weights(q):
     """(k, n) integer tensor with values in [0, 15] -> (k/16, 2n) int32 Marlin words."""
     k, n = q.shape
     if k % 16 or n % 64:
         raise ValueError("k must be divisible by 16 and n by 64")
+    if q.dtype == torch.int32 and q.numel() and q.is_contiguous() and _on_gpu(q):
+        B = torch.empty((k // 16, 2 * n), dtype=torch.int32, device=q.device)
+        dev = q.get_device()
+        _convert_check(_lib.marlin_amd_pack_words(q.data_ptr(), k, n, B.data_ptr(), dev,
+                                                  _raw_stream(dev)))
+        return B
     blocks = q.reshape(k // 16, 16, n // 64, 64).permute(0, 2, 1, 3).reshape(k // 16, n // 64, 1024)
     nib = blocks[:, :, _block_gather.to(q.device)].reshape(k // 16, n // 64, 128, 8).to(torch.int64)
     shifts = torch.arange(0, 32, 4, device=q.device, dtype=torch.int64)
@@ -186,11 +221,10 @@ def pack_weights(q):
 def pack_scales(s, groupwise):
     """(groups, n) scales -> the order the kernels read them in (marlin.py:111-118)."""
     n = s.shape[1]
-    if groupwise:
-        out = s.reshape(-1, 64)[:, _scale_perm]
-    else:
-        out = s.reshape(-1, 32)[:, _scale_perm_single]
-    return out.reshape(-1, n).contiguous()
+    # _scale_perm is an 8 x 8 transpose of every 64 columns, _scale_perm_single
+    # a 4 x 4 transpose of the pairs of every 32
+    blocks = s.reshape(-1, 8, 8) if groupwise else s.reshape(-1, 4, 4, 2)
+    return blocks.transpose(1, 2).reshape(-1, n).contiguous()
 
 
 def quantize(w, groupsize=-1):
@@ -200,6 +234,18 @@ def quantize(w, groupsize=-1):
     fake-quantised weight (k, n), q (k, n) int32 and s (groups, n)."""
     k, n = w.shape
     gs = k if groupsize == -1 else groupsize
+    if (w.dtype == torch.half and w.numel() and gs > 0 and k % gs == 0 and k // gs <= 65535
+            and _on_gpu(w)):
+        by_column = not w.is_contiguous()
+        if (w.t().is_contiguous() and gs % 4 == 0) if by_column else n % 4 == 0:
+            fake = torch.empty_like(w, memory_format=torch.preserve_format, requires_grad=False)
+            q = torch.empty_like(fake, dtype=torch.int32)
+            s = torch.empty((k // gs, n), dtype=torch.half, device=w.device)
+            dev = w.get_device()
+            _convert_check(_lib.marlin_amd_quantize(w.data_ptr(), k, n, gs, by_column,
+                                                    fake.data_ptr(), q.data_ptr(), s.data_ptr(),
+                                                    dev, _raw_stream(dev)))
+            return fake, q, s
     wg = w.reshape(k // gs, gs, n)
     s = wg.abs().amax(dim=1, keepdim=True)
     s = s * (2 / 15)
@@ -246,6 +292,16 @@ class Layer(nn.Module):
         s = scales.t()                 # (groups, n)
         w = linear.weight.data.t()     # (k, n)
         groupwise = self.groupsize != self.k
+        if (s.dtype == torch.half and s.shape == self.s.shape and w.shape == (self.k, self.n)
+                and (w.is_contiguous() or w.t().is_contiguous())
+                and self.B.is_contiguous() and self.s.is_contiguous()
+                and _on_gpu(w, self.B, self.s) and s.device == w.device and not s.requires_grad):
+            dev = w.get_device()
+            _convert_check(_lib.marlin_amd_pack(
+                w.data_ptr(), self.k, self.n, self.groupsize if groupwise else -1,
+                not w.is_contiguous(), s.data_ptr(), s.stride(0), s.stride(1), self.B.data_ptr(),
+                self.s.data_ptr(), dev, _raw_stream(dev)))
+            return
         s_full = s.repeat_interleave(self.groupsize, dim=0) if groupwise else s
         q = torch.clamp(torch.round(w / s_full).int() + 8, 0, 15)
         self.B[:, :] = pack_weights(q).to(self.B.device)

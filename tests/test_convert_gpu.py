@@ -1,0 +1,92 @@
+"""GPU tests of the weight conversion kernels (quantiser, packers) against the
+sequence of tensor operations that defines them, evaluated on the same GPU: the
+integers, the packed words and every half are the same bits."""
+import os
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "awesome-cute_amd"))
+
+
+@pytest.fixture(scope="module")
+def env():
+    import torch
+    import marlin
+    assert torch.cuda.is_available()
+    return torch, marlin
+
+
+def _weights(torch, k, n, by_column, seed):
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(seed)
+    shape = (n, k) if by_column else (k, n)
+    w = torch.randn(shape, dtype=torch.half, device="cuda:0", generator=gen)
+    w *= 2.0 ** torch.randint(-20, 12, shape, device="cuda:0", generator=gen)  # subnormals to thousands
+    w = w.t() if by_column else w
+    w[: k // 2, 0] = 0.0   # a column whose first groups are all zero
+    w[:, 1] = 7.5          # ties: w / s = 7.5 and halves of it
+    w[1::2, 1] = 1.25
+    w[0, 2] = float("inf")
+    w[k - 1, 3] = float("nan")
+    return w
+
+
+def _quantise(torch, w, gs):
+    k, n = w.shape
+    wg = w.contiguous().reshape(k // gs, gs, n)
+    s = wg.abs().amax(dim=1, keepdim=True) * (2 / 15)
+    q = torch.clamp(torch.round(wg / s).int() + 8, 0, 15)
+    return ((q - 8).to(w.dtype) * s).reshape(k, n), q.reshape(k, n), s.reshape(k // gs, n)
+
+
+def _same(torch, got, want):
+    assert got.shape == want.shape and got.dtype == want.dtype
+    if want.dtype == torch.half:  # NaN of any payload
+        assert torch.equal(got.isnan(), want.isnan())
+        got, want = (torch.nan_to_num(x.contiguous(), 0.0, posinf=float("inf"), neginf=float("-inf"))
+                     .view(torch.int16) for x in (got, want))
+    assert torch.equal(got.contiguous(), want.contiguous())
+
+
+@pytest.mark.parametrize("by_column", [False, True])
+@pytest.mark.parametrize("k,n,gs", [(4, 4, 4), (12, 260, 12), (128, 64, 128), (256, 520, 128), (384, 1096, 128), (120, 512, 40),
+                                    (136, 72, -1), (4096, 64, -1), (2304, 136, 1152), (512, 256, 256)])
+def test_quantise_is_the_tensor_sequence(env, k, n, gs, by_column):
+    torch, marlin = env
+    w = _weights(torch, k, n, by_column, seed=k + n)
+    got = marlin.quantize(w, gs)
+    for g, want in zip(got, _quantise(torch, w, k if gs == -1 else gs)):
+        _same(torch, g, want)
+    assert got[0].stride() == w.stride() and got[1].stride() == w.stride()
+
+
+@pytest.mark.parametrize("by_column", [False, True])
+@pytest.mark.parametrize("k,n,gs", [(128, 256, 128), (256, 512, 128), (384, 768, 128), (128, 256, -1), (1152, 1280, -1)])
+def test_pack_is_the_tensor_sequence(env, k, n, gs, by_column):
+    torch, marlin = env
+    fake, q, s = marlin.quantize(_weights(torch, k, n, by_column, seed=k * n), gs)
+    linear = torch.nn.Linear(k, n, bias=False, device="cuda:0", dtype=torch.half)
+    linear.weight.data = fake.t()
+    groups = s.shape[0]
+    for scales in (s.t(), s.t().contiguous()):
+        layer = marlin.Layer(k, n, gs).to("cuda:0")
+        layer.pack(linear, scales)
+        again = torch.clamp(torch.round(fake / s.repeat_interleave(k // groups, 0)).int() + 8, 0, 15)
+        assert torch.equal(layer.B.cpu(), marlin.pack_weights(again.cpu()))
+        _same(torch, layer.s, marlin.pack_scales(s, groups > 1))
+
+
+@pytest.mark.parametrize("k,n", [(16, 64), (48, 576), (256, 1088)])
+def test_packed_integers(env, k, n):
+    torch, marlin = env
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(n)
+    q = torch.randint(0, 16, (k, n), dtype=torch.int32, device="cuda:0", generator=gen)
+    want = marlin.pack_weights(q.cpu())
+    assert torch.equal(marlin.pack_weights(q).cpu(), want)
+    assert torch.equal(marlin.pack_weights(q.t().contiguous().t()).cpu(), want)  # other layouts and types
+    assert torch.equal(marlin.pack_weights(q.to(torch.int64)).cpu(), want)
