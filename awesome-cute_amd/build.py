@@ -1,13 +1,17 @@
-"""Builds libmarlin_amd.so (HIP kernels + C ABI) and libmarlin_amd_probe.so (the
-measurement probes of the benchmark) in-tree for gfx950."""
+"""Builds libmarlin_amd.so (HIP kernels + C ABI), _marlin_torch.so (the same calls on
+tensors) and libmarlin_amd_probe.so (the measurement probes of the benchmark) in-tree
+for gfx950."""
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmarlin_amd.so")
+BINDING = os.path.join(HERE, "_marlin_torch.so")
 PROBE_LIB = os.path.join(HERE, "libmarlin_amd_probe.so")
 # source -> extra flags.  The prefill kernel keeps its 128 accumulator registers
 # in ordinary VGPRs (it fits in 256), which spares the AGPR copy traffic the
@@ -31,13 +35,31 @@ FLAGS = [
 ]
 
 
+# the tensor binding is host code over torch's headers, which name the platform
+# through these two macros
+CXX = os.environ.get("CXX", "g++")
+TORCH = os.path.dirname(importlib.util.find_spec("torch").origin)
+TORCH_LIBS = os.path.join(TORCH, "lib")
+CXX_FLAGS = [
+    "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    "-I", os.path.join(TORCH, "include"), "-I", os.path.join(TORCH, "include/torch/csrc/api/include"),
+    "-I", "/opt/rocm/include", "-I", sysconfig.get_paths()["include"],
+]
+
+
+def _compile_binding(objdir, verbose):
+    obj = os.path.join(objdir, "torch_binding.o")
+    _run([CXX] + CXX_FLAGS + ["-c", "-o", obj, os.path.join(CSRC, "torch_binding.cpp")], verbose)
+    return obj
+
+
 def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     out = "\n".join(l for l in res.stdout.splitlines() if "packed-fp32-ops" not in l)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + out)
+        raise RuntimeError(f"{cmd[0]} failed:\n{out}")
     if verbose and out.strip():
         print(out)
 
@@ -51,10 +73,14 @@ def build_library(verbose=False):
     _run([sys.executable, os.path.join(CSRC, "gen_prefill_wide.py"), objdir], verbose)
     objs = [os.path.join(objdir, src.replace(".hip", ".o")) for src in SOURCES]
     with ThreadPoolExecutor(4) as pool:
+        binding = pool.submit(_compile_binding, objdir, verbose)
         list(pool.map(lambda job: _run([HIPCC] + FLAGS + job[0][1] + ["-c", "-o", job[1],
                                                                       os.path.join(CSRC, job[0][0])],
                                        verbose), zip(SOURCES.items(), objs)))
+        binding_obj = binding.result()
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs, verbose)
+    _run([CXX, "-shared", "-o", BINDING, binding_obj, "-L", HERE, "-lmarlin_amd", "-L", TORCH_LIBS,
+          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"], verbose)
     # the probes: a library of their own that asks the first one for its plans
     obj = os.path.join(objdir, "w4a16_probe.o")
     _run([HIPCC] + FLAGS + ["-c", "-o", obj, os.path.join(CSRC, "w4a16_probe.hip")], verbose)

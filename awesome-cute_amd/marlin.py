@@ -5,20 +5,14 @@ no fallback path, and a missing library is an import-time error.
 """
 import ctypes
 import os
-import threading
 
 import numpy as np
 import torch
 import torch.nn as nn
 
-_HERE = os.path.dirname(os.path.abspath(__file__))
-_LIB_PATH = os.path.join(_HERE, "libmarlin_amd.so")
+from native import lib as _lib, torch_binding as _torch_binding
 
-if not os.path.exists(_LIB_PATH):
-    raise ImportError(
-        f"{_LIB_PATH} is missing: build it first (python __graft_entry__.py build, or "
-        "python awesome-cute_amd/build.py); the W4A16 GEMM has no other implementation")
-_lib = ctypes.CDLL(_LIB_PATH)
+_HERE = os.path.dirname(os.path.abspath(__file__))
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -81,26 +75,7 @@ def mul(A, B, C, s, workspace, thread_k=-1, thread_n=-1, sms=-1, max_par=16, cut
         # workspace (the reference advertises use within torch.compile, marlin.py:12)
         return torch.ops.marlin_amd.mul(A, B, C, s, workspace, thread_k, thread_n, sms, max_par,
                                         cute_version)
-    _mul_eager(A, B, C, s, workspace, thread_k, thread_n, sms, max_par, cute_version)
-
-
-def _mul_eager(A, B, C, s, workspace, thread_k, thread_n, sms, max_par, cute_version):
-    if not (A.is_cuda and B.is_cuda and C.is_cuda and s.is_cuda and workspace.is_cuda):
-        _complain((("A", A), ("B", B), ("C", C), ("s", s), ("workspace", workspace)), "is_cuda",
-                  "must be a GPU tensor")
-    if not (A.is_contiguous() and B.is_contiguous() and C.is_contiguous() and s.is_contiguous()
-            and workspace.is_contiguous()):
-        _complain((("A", A), ("B", B), ("C", C), ("s", s), ("workspace", workspace)),
-                  "is_contiguous", "must be contiguous")
-    dev = A.get_device()
-    err = _errbuf()
-    rc = _lib.marlin_mul(A.data_ptr(), B.data_ptr(), C.data_ptr(), s.data_ptr(),
-                         A.size(0), C.size(1), A.size(1), s.size(0),
-                         workspace.data_ptr(), workspace.numel(), dev, _raw_stream(dev),
-                         thread_k, thread_n, sms, max_par, 1 if cute_version else 0,
-                         err, 512)
-    if rc != 0:
-        raise RuntimeError(err.value.decode() or f"marlin_mul failed with code {rc}")
+    _torch_binding.mul(A, B, C, s, workspace, thread_k, thread_n, sms, max_par, cute_version)
 
 
 # The same call as an operator of torch's dispatcher, for compilers that trace
@@ -111,7 +86,7 @@ def _mul_eager(A, B, C, s, workspace, thread_k, thread_n, sms, max_par, cute_ver
 def _mul_op(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor, s: torch.Tensor,
             workspace: torch.Tensor, thread_k: int, thread_n: int, sms: int, max_par: int,
             cute_version: bool) -> None:
-    _mul_eager(A, B, C, s, workspace, thread_k, thread_n, sms, max_par, cute_version)
+    _torch_binding.mul(A, B, C, s, workspace, thread_k, thread_n, sms, max_par, cute_version)
 
 
 @_mul_op.register_fake
@@ -119,26 +94,7 @@ def _mul_fake(A, B, C, s, workspace, thread_k, thread_n, sms, max_par, cute_vers
     return None
 
 
-def _complain(named, attr, what):
-    for name, t in named:
-        v = getattr(t, attr)
-        if not (v() if callable(v) else v):
-            raise RuntimeError(f"{name} {what}")
-
-
-# The host side of a call matters at one row (the kernel takes 6.5 us): the
-# error buffer is kept per thread, and the current stream is read through
-# torch's raw-handle accessor where this torch build has it.
-_tls = threading.local()
-
-
-def _errbuf():
-    buf = getattr(_tls, "err", None)
-    if buf is None:
-        buf = _tls.err = ctypes.create_string_buffer(512)
-    return buf
-
-
+# the current stream's handle, through torch's raw accessor where this torch build has it
 _get_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
@@ -279,6 +235,11 @@ class Layer(nn.Module):
                              persistent=False)
 
     def forward(self, A):
+        if not torch.compiler.is_compiling():
+            # (the buffers by name: as attributes each costs a Python call)
+            held = self._buffers
+            return _torch_binding.linear(A, held['B'], held['s'], held['workspace'],
+                                         self.cute_version)
         C = torch.empty(A.shape[:-1] + (self.s.shape[1],), dtype=A.dtype, device=A.device)
         mul(A.reshape((-1, A.shape[-1])), self.B, C.view((-1, C.shape[-1])), self.s,
             self.workspace, cute_version=self.cute_version)
