@@ -12,13 +12,16 @@ which MFMA, and every s_waitcnt is computed from the order of issue.
 The statement covers prologue, loop and the first part of the epilogue:
   prologue  requests of stages 0 and 1, slab 0 to LDS, unpack of the first k step
   loop      two 64-deep stages per turn (stage parity u is static), see stage()
-  epilogue  row blocks 4..7 of the accumulator go to LDS for the other k half,
-            row blocks 0..3 to v[0:127], which are the statement's outputs
+  epilogue  the last HB = RB/2 (rounded up) row blocks of the accumulator go to
+            LDS for the other k half, the first HB to v[0:32*HB-1], which are the
+            statement's outputs
+It is written for tiles of RB = 5 to 8 row blocks of 16; the figures in the
+comments are those of 8.
 
 Register map (v = VGPR, a = AGPR, s = SGPR):
   a[32i+4o : +3]   accumulator of row block i, operand o = 2j+h (16-column group j, half h)
   v[32b+4o : +3]   unpacked weights, buffer b (k step parity), operand o
-  v[64+4x : +3]    activation operand ring, x = row block % 4
+  v[64+4x : +3]    activation operand ring, x = row blocks since the turn began % 4
   v[80+4i : +3]    activation slab staging register i (8 per thread)
   v[112+16u+4r:+3] packed weights of stage parity u, 16-deep row r of the stage
   v[144+4u : +3]   group scales of stage parity u
@@ -44,11 +47,16 @@ import sys
 #   b0, b1   preferred MFMAs of the weight (and scale) loads of steps 0 and 1
 OPT = {"ahead": 2, "rdoff": 0, "slab0": (2, 5), "slab1": (1, 3.5), "b0": (52, 58), "b1": (52, 56, 60)}
 
-RB = 8
-PLANE = 128 * 16
-STEP_BYTES = 4 * PLANE + 128
-SLAB_BYTES = 2 * STEP_BYTES           # 16640 = 65 * 256
-assert SLAB_BYTES % 256 == 0
+
+
+def set_rows(rb):
+    """row blocks of a tile, and what follows from them"""
+    global RB, HB, MFMAS, PLANE, STEP_BYTES, SLAB_BYTES
+    RB, HB, MFMAS = rb, (rb + 1) // 2, 8 * rb
+    PLANE = 256 * rb
+    STEP_BYTES = 4 * PLANE + 128
+    SLAB_BYTES = 2 * STEP_BYTES       # 16640 = 65 * 256
+    assert SLAB_BYTES % 256 == 0
 
 
 def W(b, o): return 32 * b + 4 * o
@@ -193,8 +201,8 @@ def slab_op(e, slab, x, first_i):
     if g < 2:
         if g == 0:
             e.wait(vm_regs=[AREG(i)])
-        unit = slab * (SLAB_BYTES // 256) + 16 * g + i
-        e.lds_write2(AREG(i) + 2 * g, AREG(i) + 2 * g + 1, unit, unit + 8)
+        unit = slab * (SLAB_BYTES // 256) + 2 * RB * g + i
+        e.lds_write2(AREG(i) + 2 * g, AREG(i) + 2 * g + 1, unit, unit + RB)
     else:
         e.load(AREG(i), ALANE(i), RA, S_SOFFA)
 
@@ -205,26 +213,26 @@ def mfma(e, i, o, buf, x):
 
 
 def assign_slots(prefs):
-    """distinct MFMA slots 0..63 for operations with preferred slots `prefs`
+    """distinct MFMA slots 0..MFMAS-1 for operations with preferred slots `prefs`
     (ascending): each gets its preference or the next free slot after the one
     before it; if they run past the end, the tail is pushed back"""
     slots, last = [], -1
     for pr in prefs:
         last = max(last + 1, int(pr))
         slots.append(last)
-    over = slots[-1] - 63 if slots else 0
+    over = slots[-1] - (MFMAS - 1) if slots else 0
     if over > 0:
         for k in range(len(slots) - 1, -1, -1):
-            cap = 63 - (len(slots) - 1 - k)
+            cap = MFMAS - 1 - (len(slots) - 1 - k)
             if slots[k] <= cap:
                 break
             slots[k] = cap
-    assert len(set(slots)) == len(slots) and all(0 <= x < 64 for x in slots), slots
+    assert len(set(slots)) == len(slots) and all(0 <= x < MFMAS for x in slots), slots
     return slots
 
 
 def step(e, group, h, slab_cur, mem_ops, unpack_u, unpack_rows):
-    """64 MFMAs on buffer h and LDS step (slab_cur, h), while the next step's
+    """8 RB MFMAs on buffer h and LDS step (slab_cur, h), while the next step's
     weights (rows unpack_rows of stage parity unpack_u) are unpacked into buffer
     h^1 and the memory operations mem_ops -- (preferred slot, emit function),
     the step's operand reads are added here -- are issued.
@@ -239,18 +247,19 @@ def step(e, group, h, slab_cur, mem_ops, unpack_u, unpack_rows):
     cur = slab_cur * SLAB_BYTES + h * STEP_BYTES
     nxt = (slab_cur * SLAB_BYTES + STEP_BYTES) if h == 0 else (slab_cur ^ 1) * SLAB_BYTES
     ahead = OPT["ahead"]
+    ring = RB * (2 * slab_cur + h)   # row blocks since the turn began
     ops = list(mem_ops)
     for i in range(RB):
         tgt = i + ahead
         off = (cur + tgt * 256) if tgt < RB else (nxt + (tgt - RB) * 256)
-        ops.append((8 * i + OPT["rdoff"], lambda e, tgt=tgt, off=off: e.lds_read(AF(tgt & 3), off)))
+        ops.append((8 * i + OPT["rdoff"], lambda e, tgt=tgt, off=off: e.lds_read(AF((ring + tgt) & 3), off)))
     ops.sort(key=lambda x: x[0])
     slots = assign_slots([pr for pr, _ in ops])
     mem_at = dict(zip(slots, (fn for _, fn in ops)))
     # the unpack: 8 words x ops_per_word operations, rows in lockstep
     todo = [(t // ops_per_word, t % ops_per_word, r) for t in range(4 * ops_per_word)
             for r in (0, 1)]
-    free = [m for m in range(64) if m not in mem_at]
+    free = [m for m in range(MFMAS) if m not in mem_at]
     per = [2] * len(free)
     short = len(todo) - 2 * len(free)
     k = 0
@@ -260,10 +269,10 @@ def step(e, group, h, slab_cur, mem_ops, unpack_u, unpack_rows):
         short -= 1
     valu_at = dict(zip(free, per))
     for i in range(RB):
-        e.wait(lgkm_regs=[AF(i & 3)])
+        e.wait(lgkm_regs=[AF((ring + i) & 3)])
         for o in range(8):
             m = 8 * i + o
-            mfma(e, i, o, h, i & 3)
+            mfma(e, i, o, h, (ring + i) & 3)
             if m in mem_at:
                 mem_at[m](e)
             n = min(valu_at.get(m, 0), len(todo))
@@ -281,10 +290,10 @@ def step(e, group, h, slab_cur, mem_ops, unpack_u, unpack_rows):
 
 def stage(e, group, u):
     """One 64-deep stage cs of parity u.  Step 0: rows 2, 3 of this stage are
-    unpacked, staging registers 0..3 go to LDS slab u^1 (stage cs+1) and are
-    requested again for stage cs+2, rows 0, 1 of stage cs+2 are requested.
-    Step 1: rows 0, 1 of stage cs+1 are unpacked, staging registers 4..7 go to
-    LDS; then the one barrier of the stage -- after it nobody reads slab u
+    unpacked, the first HB staging registers go to LDS slab u^1 (stage cs+1) and
+    are requested again for stage cs+2, rows 0, 1 of stage cs+2 are requested.
+    Step 1: rows 0, 1 of stage cs+1 are unpacked, the other staging registers go
+    to LDS; then the one barrier of the stage -- after it nobody reads slab u
     again, so the next stage may overwrite it, and slab u^1 is complete --
     before the first operands of stage cs+1 are read; rows 2, 3 and the scales
     of stage cs+2 are requested."""
@@ -295,16 +304,20 @@ def stage(e, group, u):
         e.drained(lgkm=True)
         e.emit("s_barrier")
 
+    # (the preferred slots are those of 64 MFMAs and 12 slab operations)
+    f = RB / 8
     a, st = OPT["slab0"]
-    ops0 = [(a + st * x, lambda e, x=x: slab_op(e, u ^ 1, x, 0)) for x in range(12)]
-    ops0 += [(OPT["b0"][r], lambda e, r=r: load_b(e, u, r)) for r in (0, 1)]
+    st *= f * 4 / HB
+    ops0 = [(a + st * x, lambda e, x=x: slab_op(e, u ^ 1, x, 0)) for x in range(3 * HB)]
+    ops0 += [(f * OPT["b0"][r], lambda e, r=r: load_b(e, u, r)) for r in (0, 1)]
     a, st = OPT["slab1"]
+    st *= f * 4 / (RB - HB)
     bar = 8 * (RB - OPT["ahead"]) + OPT["rdoff"] - 0.5  # just before the first read of the next slab
-    ops1 = [(min(a + st * x, bar - 0.75), lambda e, x=x: slab_op(e, u ^ 1, x, 4)) for x in range(12)]
+    ops1 = [(min(a + st * x, bar - 0.75), lambda e, x=x: slab_op(e, u ^ 1, x, HB)) for x in range(3 * (RB - HB))]
     ops1 += [(bar, barrier)]
-    ops1 += [(OPT["b1"][r], lambda e, r=r: load_b(e, u, 2 + r)) for r in (0, 1)]
+    ops1 += [(f * OPT["b1"][r], lambda e, r=r: load_b(e, u, 2 + r)) for r in (0, 1)]
     if group:
-        ops1 += [(OPT["b1"][2], lambda e: e.load(SREG(u), VSOFF, RS, S_SOFFS))]
+        ops1 += [(f * OPT["b1"][2], lambda e: e.load(SREG(u), VSOFF, RS, S_SOFFS))]
     step(e, group, 0, u, ops0, u, (2, 3))
     step(e, group, 1, u, ops1, u ^ 1, (0, 1))
 
@@ -328,7 +341,7 @@ def prologue(e, group):
             for i in range(RB):
                 e.load(AREG(i), ALANE(i), RA, S_SOFFA)
             # the accumulators start at zero
-            for n in range(256):
+            for n in range(32 * RB):
                 e.emit(f"v_accvgpr_write_b32 a{n}, 0")
         else:
             # slab 0 to LDS, its registers requested again for stage 1
@@ -359,10 +372,10 @@ def epilogue(e):
     e.emit("s_nop 15")
     e.emit("s_waitcnt vmcnt(0) lgkmcnt(0)")
     e.emit("s_barrier")          # every wave is done with the slabs
-    for i in range(4, RB):
+    for i in range(RB - HB, RB):
         for o in range(8):
-            e.emit(f"ds_write_b128 v{VSWAP}, {aq(32 * i + 4 * o)} offset:{((i - 4) * 8 + o) * 1024}")
-    for n in range(128):
+            e.emit(f"ds_write_b128 v{VSWAP}, {aq(32 * i + 4 * o)} offset:{((i - RB + HB) * 8 + o) * 1024}")
+    for n in range(32 * HB):
         e.emit(f"v_accvgpr_read_b32 v{n}, a{n}")
     e.emit("s_waitcnt lgkmcnt(0)")
 
@@ -406,7 +419,7 @@ def statement(group):
     out = ["// generated by gen_prefill_wide.py -- do not edit", "asm volatile("]
     out += [f'    "{l}\\n\\t"' for l in lines]
     outs = [f'"={{v[{32 * i + 4 * o}:{32 * i + 4 * o + 3}]}}"(fin[{i}][{o}])'
-            for i in range(4) for o in range(8)]
+            for i in range(HB) for o in range(8)]
     outs.append(f'"+{{s[{RA}:{RA + 3}]}}"(ra_words)')
     out.append("    : " + ",\n      ".join(outs))
     ins = [f'"{{s[{RB_}:{RB_ + 3}]}}"(rb_words)',
@@ -417,8 +430,8 @@ def statement(group):
     ins += [f'"{{v{VBOFF}}}"(b_lane)', f'"{{v{VSOFF}}}"(s_lane)', f'"{{v{VRD}}}"(lds_rd)',
             f'"{{v{VWR}}}"(lds_wr)', f'"{{v{VSWAP}}}"(lds_swap)']
     out.append("    : " + ",\n      ".join(ins))
-    clob = [f'"v{n}"' for n in range(128, 152)] + [f'"v{n}"' for n in (164, 165, 166, 167)]
-    clob += [f'"a{n}"' for n in range(256)]
+    clob = [f'"v{n}"' for n in range(32 * HB, 152)] + [f'"v{n}"' for n in (164, 165, 166, 167)]
+    clob += [f'"a{n}"' for n in range(32 * RB)]
     clob += [f'"s{n}"' for n in range(S_CS, S_TMP + 1)] + ['"scc"', '"memory"']
     out.append("    : " + ", ".join(clob) + ");")
     return "\n".join(out) + "\n"
@@ -429,6 +442,8 @@ if __name__ == "__main__":
     for arg in sys.argv[2:]:
         key, val = arg.split("=")
         OPT[key] = tuple(float(x) for x in val.split(",")) if "," in val else int(val)
-    for group, name in ((True, "group"), (False, "chan")):
-        with open(f"{outdir}/w4a16_prefill_wide_{name}.inc", "w") as f:
-            f.write(statement(group))
+    for rows in (5, 6, 7, 8):
+        set_rows(rows)
+        for group, name in ((True, "group"), (False, "chan")):
+            with open(f"{outdir}/w4a16_prefill_wide_{name}{16 * rows}.inc", "w") as f:
+                f.write(statement(group))

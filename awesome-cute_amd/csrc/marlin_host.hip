@@ -130,16 +130,18 @@ struct Plan {
 };
 
 constexpr int kStreamMaxRows = 64;
+constexpr int kSliceCounterStride = 16;  // ints: a prefill tile's slices meet in a cache line of their own
 
 // Overrides of the planner for the calling thread (tests and tools; see
 // marlin_amd_force_*): which kernel (0 = by cost, 1 = streaming in chunks of
 // 64 rows, 2 = prefill, 3 = column strips, 4 = by cost without the column
 // strips), slices of the k range per prefill tile (0 = by cost),
-// rows of C per prefill workgroup (0 = by cost, 64 or 128).
+// rows of C per prefill workgroup (0 = by cost, 64 to 128 in steps of 16).
 struct Force {
   int kernel = 0, k_slices = 0, tile_rows = 0;
   int row_halves = 0;  // streaming kernel: 0 = by cost, 1 = never cut the rows, 2 = cut them where possible
   int strips = 0;      // column-strip kernel: 0 = by cost, or 1 to 4 strips per workgroup
+  int finish_polls = -1;  // looks at the other slices of a tile before leaving; -1 = kFinishPolls
 };
 thread_local Force t_force;
 
@@ -152,44 +154,57 @@ struct PlanCtx {
   int counters = 16;  // ints of the workspace per column tile: min(max_par, 16)
 };
 
-// Cost in us of the prefill kernel with `tiles` tiles of tile_rows rows cut into
-// s slices, fitted to measurements on MI355X.  A full-depth tile takes
-// 6 + 0.0130 k with 128 rows and 5 + 0.0080 k with 64 (every unpacked weight
-// then meets four row blocks instead of eight, so a 64-row tile costs more than
-// half of a 128-row one) when the launch fills the CUs; k slices divide that
-// and add their exchange, 3 + 2 s (128 rows: 128 KiB of partial sums per
-// workgroup) or 3 + 1.5 s (64 rows).
+// Cost in us of the prefill kernels with `tiles` tiles of tile_rows rows cut
+// into s slices, linear in what they do and fitted to 2700 launches on MI355X
+// (M = 65 ... 2100 on eleven (N, K) from 1024 x 1024 to 28672 x 8192, every
+// tile height and slice count; 4 % rms for 64 rows, 5 % for the others): a
+// launch, a round of workgroups, a 64-deep stage of each k half of a workgroup
+// (dearer the fuller the chip: the board's power), and with slices their
+// meeting, dearer with their number and with the traffic of a full chip.  R is
+// the row blocks of a tile of the four-wave kernel.
 double prefill_cost_slices(int tiles, int tile_rows, int k, int cus, int s) {
   // more workgroups than CUs run in rounds, the last of which is faster the
   // emptier it is: half way between whole rounds and the plain ratio fits
-  // (N = K = 4096, M = 3072: 384 tiles of 128 rows, 102.7 us, where one round
-  // of 256 takes 59.3)
   const double ratio = (double)tiles * s / cus;
   const double rounds = ratio <= 1.0 ? 1.0 : 0.5 * (ceil_div(tiles * s, cus) + ratio);
-  // ... and a launch that leaves CUs idle runs its tiles faster (clock, and
-  // fewer workgroups at the memory): 0.9 of the time at three quarters full
-  const double fill = ratio < 1.0 ? 0.6 + 0.4 * ratio : 1.0;
-  const double tile = (tile_rows == 64 ? 5.0 + 0.0080 * k : 6.0 + 0.0130 * k) * fill;
-  const double exchange = s > 1 ? 3.0 + (tile_rows == 64 ? 1.5 : 2.0) * s : 0.0;
-  return rounds * (tile / s + exchange);
+  const double fill = ratio < 1.0 ? ratio : 1.0;
+  const double stages = rounds * ceil_div(ceil_div(ceil_div(k, 64), s), 2);
+  if (tile_rows == 64)
+    return -2.24 + 7.07 * rounds + (0.753 + 0.256 * fill) * stages +
+           (s > 1 ? 0.86 + 0.61 * s + 1.90 * fill * rounds : 0.0);
+  const double R = tile_rows / 16.0;
+  return 5.16 - 1.97 * R + (2.63 * R - 2.42) * rounds +
+         (0.519 + (0.0586 + 0.0419 * fill) * R) * stages +
+         (s > 1 ? 2.12 + 0.302 * s + 0.625 * fill * rounds * R : 0.0);
+}
+
+// Whether a tile height is cut into s slices at all.  With 64 rows no more than
+// six (eight gain nothing where the streaming kernel does not win anyway: M =
+// 100, N = 4096, K = 11008 24.1 us with six, 25.3 with eight).  Three row
+// blocks per wave finish in six pieces, which only 2, 3 and 6 slices share
+// evenly (80 rows, M = 150, N = 4096, K = 11008: four slices 31.0 us, five
+// 28.6, six 26.4, seven 28.0, eight 27.8); eight pieces are less particular.
+bool slices_share(int tile_rows, int s) {
+  if (tile_rows == 64) return s <= 6;
+  return tile_rows > 96 || 6 % s == 0;
 }
 
 // Slices of the k range per tile: the cheapest count among those that keep
 // the launch within one workgroup per CU, slices at least 256 deep (two
 // 64-deep stages for each half of the workgroup), and the partial sums and
-// tile counters within the scratch.  Up to eight; in practice four, six where
-// k is deep (N = 4096, K = 11008, M = 128: 24.8 us with six against 26.9 with
-// four).
+// tile counters within the scratch.  Up to eight.
 int prefill_k_slices(int tiles, int tile_rows, int k, const PlanCtx& cx) {
   int most = k / 256;
-  if (most > 8) most = 8;
-  while (most > 1 && (size_t)tiles * most * tile_rows * 256 * 4 > cx.partial_limit) --most;
-  if (most < 1 || tiles > kMaxCounters) return 1;
+  if (most > kMaxSlices) most = kMaxSlices;
+  while (most > 1 && (size_t)tiles * most * ceil_div(tile_rows, 32) * 32 * 256 * 4 > cx.partial_limit)
+    --most;
+  if (most < 1 || tiles > kMaxCounters / kSliceCounterStride) return 1;
   if (cx.force.k_slices > 0) return cx.force.k_slices < most ? cx.force.k_slices : most;
   if (most > cx.cus / tiles) most = cx.cus / tiles;
   int best = 1;
   double best_cost = prefill_cost_slices(tiles, tile_rows, k, cx.cus, 1);
   for (int s = 2; s <= most; s++) {
+    if (!slices_share(tile_rows, s)) continue;
     const double c = prefill_cost_slices(tiles, tile_rows, k, cx.cus, s);
     if (c < best_cost) {
       best = s;
@@ -199,29 +214,35 @@ int prefill_k_slices(int tiles, int tile_rows, int k, const PlanCtx& cx) {
   return best;
 }
 
-// Either kernel can do any problem whose n is a multiple of 256: the prefill
-// kernel once, or the streaming kernel once per 64 rows, reading the weights
-// again every time.
 double prefill_cost_rows(int m, int n, int k, const PlanCtx& cx, int tile_rows) {
   const int tiles = ceil_div(m, tile_rows) * (n / 256);
   return prefill_cost_slices(tiles, tile_rows, k, cx.cus,
                              prefill_k_slices(tiles, tile_rows, k, cx));
 }
 
-// Rows of C per prefill workgroup.  64-row tiles are twice as many, so they
-// need fewer k slices to fill the CUs (or none), which wins while the problem
-// is small: at N = K = 4096 up to about 512 rows (M = 128: 16.0 against
-// 21.9 us), at N = 4096, K = 11008 up to 256 (27.5 against 38.9 us at M = 128).
+// Rows of C per prefill workgroup: the cheapest of 64 (eight waves) and 80 to
+// 128 in steps of 16 (four).  Heights other than 64 and 128 are there for row
+// counts that 64-row tiles would pad -- M = 150, N = 12288, K = 4096: 31.6 us
+// with 64 rows, 31.7 with 128, 26.0 with 80; M = 300, N = K = 8192 59.1, 51.2
+// and 45.4; M = 203, N = 5120, K = 13568 46.8, 42.6 and 40.1 with 112; M = 300,
+// N = 28672, K = 8192 189, 172 and 142 -- and others are left to those two.
 int prefill_tile_rows(int m, int n, int k, const PlanCtx& cx) {
-  if (cx.force.tile_rows == 64 || cx.force.tile_rows == 128) return cx.force.tile_rows;
+  if (cx.force.tile_rows != 0) return cx.force.tile_rows;
   if (m <= 64) return 64;
-  return prefill_cost_rows(m, n, k, cx, 64) < prefill_cost_rows(m, n, k, cx, 128) ? 64 : 128;
+  int best = 64;
+  double best_cost = prefill_cost_rows(m, n, k, cx, 64);
+  for (int rows = m % 64 == 0 ? 128 : 80; rows <= 128; rows += 16) {
+    const double c = prefill_cost_rows(m, n, k, cx, rows);
+    if (c < best_cost) {
+      best = rows;
+      best_cost = c;
+    }
+  }
+  return best;
 }
 
 double prefill_cost(int m, int n, int k, const PlanCtx& cx) {
-  // (the tile fits were made at K >= 4096: at K <= 1024 the prefill kernels
-  // measure a third more, 56 and 64 rows at every N from 256 to 11008)
-  return prefill_cost_rows(m, n, k, cx, prefill_tile_rows(m, n, k, cx)) * (k < 2048 ? 1.33 : 1.0);
+  return prefill_cost_rows(m, n, k, cx, prefill_tile_rows(m, n, k, cx));
 }
 
 // The streaming kernel's split of the granule sequence over the compute units
@@ -551,7 +572,7 @@ Plan make_plan(int m, int n, int k, int sms, const PlanCtx& cx) {
     pl.grid = tiles * pl.ksplit;
     pl.sp = make_stream_plan(n, k, 1);
     pl.launches = 1;
-    if (pl.ksplit > 1) pl.partial_bytes = (size_t)pl.grid * pl.tile_rows * 256 * 4;
+    if (pl.ksplit > 1) pl.partial_bytes = (size_t)pl.grid * ceil_div(pl.tile_rows, 32) * 32 * 256 * 4;
     return pl;
   }
   pl.kernel = 1;
@@ -658,16 +679,17 @@ int enqueue(const Plan& pl, const ScratchView& view, const void* A, const void* 
     a.N = n;
     a.K = k;
     a.locks = view.counters;
-    a.lock_stride = 1;
+    a.lock_stride = kSliceCounterStride;
     a.scratch = view.partials;
     a.gpb = 0;
     a.wpt = 0;
     a.row_parts = 1;
     a.part_rows = 0;
+    a.finish_polls = t_force.finish_polls < 0 ? kFinishPolls : t_force.finish_polls;
     // 128-row tiles: four waves with 128 x 128 accumulators; 64-row tiles: eight
     // waves with 64 x 64
-    rc = pl.tile_rows == 128 ? launch_prefill_wide(a, groupsize != -1, pl.ksplit, stream)
-                             : launch_prefill(a, groupsize != -1, pl.ksplit, stream);
+    rc = pl.tile_rows > 64 ? launch_prefill_wide(a, groupsize != -1, pl.tile_rows, pl.ksplit, stream)
+                           : launch_prefill(a, groupsize != -1, pl.ksplit, stream);
   } else {
     // a launch per 64 rows, or one launch over all rows cut into parts
     const int rows_per_launch = pl.launches == 1 ? m : kStreamMaxRows;
@@ -899,7 +921,13 @@ void marlin_amd_force_k_slices(int slices) { t_force.k_slices = slices > 0 ? sli
 
 void marlin_amd_force_row_halves(int mode) { t_force.row_halves = mode == 1 || mode == 2 ? mode : 0; }
 
-void marlin_amd_force_tile_rows(int rows) { t_force.tile_rows = rows == 64 || rows == 128 ? rows : 0; }
+void marlin_amd_force_tile_rows(int rows) {
+  t_force.tile_rows = rows >= 64 && rows <= 128 && rows % 16 == 0 ? rows : 0;
+}
+
+void marlin_amd_force_finish_polls(int polls) {
+  t_force.finish_polls = polls < 0 || polls > kFinishPolls ? -1 : polls;
+}
 
 void marlin_amd_work_order(int grid, int* out) {
   for (int b = 0; b < grid; b++) out[b] = xcd_work_index(b, grid);

@@ -176,10 +176,64 @@ struct GemmArgs {
                     // lock_stride >= row_parts.  Column-strip kernel: 1, or the number
                     // of 16-row parts, a workgroup per strip set and part
   int part_rows;    // rows of a part: 16 or 32
+  int finish_polls; // prefill kernels: looks at a tile's other slices before leaving them a share
 };
 
 // bytes of fp32 partial sums of mb row blocks of 16 (one slot)
 constexpr size_t stream_slot_bytes(int mb) { return (size_t)mb * 4 * 2 * 64 * 16; }
+
+// How the workgroups that hold slices of one tile finish it together.  The
+// tile is cut into as many shares as there are slices; every slice writes its
+// partial sums of the others' shares through to memory, and whoever sees all
+// slices arrived adds up its own, all slices of it in slice order.  (With the
+// last arrival adding up everything by itself, seven partial tiles of 128 KiB
+// passed through one compute unit at some 77 GB/s while the others had left.)
+//
+// `word` (zero on entry, and again when the tile's last workgroup is done with
+// it): bits 0-7 count arrivals, 8-15 workgroups that will not look at the word
+// again, bit 16 + i says that slice i left.  An arrival waits for the others
+// for some 50 us at most -- the slices of a tile are equally long and start
+// together, but nothing promises that they run at the same time -- then writes
+// its own share out too, sets its bit and leaves, and the last arrival takes
+// that share as well; or the leaver finds the count complete in the word it
+// replaced, and stays.  So every share has exactly one taker, whatever runs
+// when, and nobody waits for long.
+//
+// All three are called by thread 0, finish_arrive once the workgroup's partial
+// sums have been acknowledged: the shares to take as a bit mask, or 0 when the
+// wait ran out, and then finish_abandon once its own share is out as well: the
+// same, 0 meaning leave.  finish_leave comes last, in either case.
+constexpr int kMaxSlices = 8;
+constexpr int kFinishPolls = 64;
+__device__ __forceinline__ int finish_arrive(int* word, int slices, int mine, int max_polls) {
+  int v = __hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((v & 0xff) == slices - 1) return 1 << mine | ((v >> 16) & ((1 << slices) - 1));
+  for (int polls = 0; polls < max_polls; polls++) {
+    __builtin_amdgcn_s_sleep(2);
+    v = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((v & 0xff) == slices) return 1 << mine;
+  }
+  return 0;
+}
+__device__ __forceinline__ int finish_abandon(int* word, int slices, int mine) {
+  const int v =
+      __hip_atomic_fetch_or(word, 0x10000 << mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return (v & 0xff) == slices ? 1 << mine : 0;
+}
+__device__ __forceinline__ void finish_leave(int* word, int slices) {
+  const int v = __hip_atomic_fetch_add(word, 0x100, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (((v >> 8) & 0xff) == slices - 1)
+    __hip_atomic_store(word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// the pieces of a tile of `pieces` that make up these shares, as a bit mask
+__device__ __forceinline__ int finish_pieces(int shares, int slices, int pieces) {
+  int mask = 0;
+  for (; shares != 0; shares &= shares - 1) {
+    const int r = __builtin_ctz(shares);
+    mask |= (1 << (pieces * (r + 1) / slices)) - (1 << (pieces * r / slices));
+  }
+  return mask;
+}
 
 // Result of a kernel launch for the launch helpers below: 0, or 3 with the
 // runtime's error kept per thread for the caller's message (reading the
@@ -208,9 +262,10 @@ int launch_strip(const GemmArgs& a, bool group, int strips, hipStream_t stream);
 // counter per tile, zero again afterwards)
 // 64-row x 256-column tiles, eight waves (w4a16_prefill.hip)
 int launch_prefill(const GemmArgs& a, bool group, int ksplit, hipStream_t stream);
-// 128-row x 256-column tiles, four waves with 128 x 128 accumulators
-// (w4a16_prefill_wide.hip); same scratch layout and counters
+// tiles of 80, 96, 112 or 128 rows x 256 columns, four waves with accumulators of
+// all rows x 128 columns (w4a16_prefill_wide.hip); same counters, and the
+// scratch of a tile has its rows rounded up to 32
 int configure_prefill_wide_kernels();
-int launch_prefill_wide(const GemmArgs& a, bool group, int ksplit, hipStream_t stream);
+int launch_prefill_wide(const GemmArgs& a, bool group, int tile_rows, int ksplit, hipStream_t stream);
 
 }  // namespace w4a16

@@ -472,7 +472,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(GemmArgs p, int tiles_m, i
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): my stores have been acknowledged
     __syncthreads();
     if (threadIdx.x == 0)
-      s_ticket = __hip_atomic_fetch_add(&p.locks[tile], 1, __ATOMIC_RELAXED,
+      s_ticket = __hip_atomic_fetch_add(&p.locks[tile * p.lock_stride], 1, __ATOMIC_RELAXED,
                                         __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (s_ticket != ksplit - 1) return;  // a later slice finishes the tile
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(GemmArgs p, int tiles_m, i
 #pragma unroll
       for (int j = 0; j < 4; j++) fin[i][j] = sum[i][j];
     if (threadIdx.x == 0)  // counters are handed back zeroed
-      __hip_atomic_store(&p.locks[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&p.locks[tile * p.lock_stride], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
 

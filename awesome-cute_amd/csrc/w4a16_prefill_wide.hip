@@ -1,5 +1,10 @@
 // Prefill W4A16 kernel with one wave per SIMD: 128-row x 256-column tiles of C
-// for launches that are bound by the matrix pipe and by what competes with it.
+// for launches that are bound by the matrix pipe and by what competes with it,
+// and tiles of 112, 96 and 80 rows for row counts that would leave much of a
+// 64- or 128-row tile empty.  A step of the main loop takes a 112-row tile 0.93,
+// a 96-row tile 0.86 and an 80-row tile 0.80 of a 128-row tile's time: what is
+// spared is matrix time and power, the unpack stays (M = 300, N = 28672, K =
+// 8192: 300 rows as 3 x 128 172 us, as 4 x 80 142).
 //
 // A workgroup of four waves owns a 128 x 256 tile (and, like the other prefill
 // kernel, one of `ksplit` slices of the k range when tiles alone would leave
@@ -7,6 +12,12 @@
 // tile over the k half kh of the workgroup's range: a 128 x 128 fp32
 // accumulator, all 256 AGPRs, which is why there is one wave per SIMD.  The
 // two k halves are added through LDS at the end.
+//
+// With k slices the rest is latency: at M = 128, N = K = 4096 in eight slices
+// the loop ends at 9 us, the k halves take 0.5, the partial sums out 2.3, the
+// other slices' arrival 1.8 and adding up and writing the tile 4.  Finished by
+// the last arrival alone the launch took 26.3 us, by all slices together 18.0
+// (four slices 23.5 / 20.0; two, M = 1024, 37.8 / 35.8).
 //
 // What this shape buys over eight waves with 128 x 64 accumulators:
 //   - The packed weights never pass through LDS.  A wave's 128 columns are two
@@ -36,20 +47,26 @@ namespace w4a16 {
 
 namespace {
 
-constexpr int kWdTileM = 128;
 constexpr int kWdTileN = 256;
-constexpr int kWdRB = 8;                              // row blocks of 16
-constexpr int kWdRing = 2;                            // activation slabs in LDS per k half
-constexpr int kWdPlane = kWdTileM * 16;               // one k group of a step: rows x 16 bytes
-constexpr int kWdStepBytes = 4 * kWdPlane + 128;      // one 32-deep k step of a slab (+pad)
-constexpr int kWdSlabBytes = 2 * kWdStepBytes;        // a 64-deep stage
-constexpr int kWdRingBytes = kWdRing * kWdSlabBytes;  // per k half
-constexpr int kWdPitch = kWdTileN * 2 + 16;           // fp16 tile row in LDS on the way out
-// the epilogue reuses the rings: 4 waves x 4 row blocks x 8 KiB of fp32 to
-// swap between the k halves, then the fp16 tile with padded rows
-constexpr int kWdSwapBytes = 4 * 4 * 8 * 1024;
-constexpr int kWdLdsBytes = kWdSwapBytes > 2 * kWdRingBytes ? kWdSwapBytes : 2 * kWdRingBytes;
-static_assert(kWdTileM * kWdPitch <= kWdLdsBytes, "");
+constexpr int kWdRing = 2;                    // activation slabs in LDS per k half
+constexpr int kWdPitch = kWdTileN * 2 + 16;   // fp16 tile row in LDS on the way out
+
+// what follows from the row blocks of 16 of a tile (RB = 5 to 8)
+template <int RB>
+struct WdShape {
+  static constexpr int kTileM = 16 * RB;
+  static constexpr int kHB = (RB + 1) / 2;  // row blocks a k half finishes (the second one RB - kHB)
+  static constexpr int kPlane = kTileM * 16;               // one k group of a step: rows x 16 bytes
+  static constexpr int kStepBytes = 4 * kPlane + 128;      // one 32-deep k step of a slab (+pad)
+  static constexpr int kSlabBytes = 2 * kStepBytes;        // a 64-deep stage
+  static constexpr int kRingBytes = kWdRing * kSlabBytes;  // per k half
+  // the epilogue reuses the rings: 4 waves x kHB row blocks x 8 KiB of fp32 to
+  // swap between the k halves, then the fp16 tile with padded rows
+  static constexpr int kSwapBytes = 4 * kHB * 8 * 1024;
+  static constexpr int kLdsBytes = kSwapBytes > 2 * kRingBytes ? kSwapBytes : 2 * kRingBytes;
+  static_assert(kTileM * kWdPitch <= kLdsBytes, "");
+  static constexpr int kPartBytes = kSwapBytes;  // fp32 sums of a tile in scratch
+};
 constexpr int kOobWd = (int)0x80000000;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t wd_rsrc(const void* p, unsigned bytes) {
@@ -65,11 +82,15 @@ __device__ __forceinline__ i4 wd_rsrc_words(const void* p, unsigned bytes) {
 
 }  // namespace
 
-template <bool GROUP>
+// SLICED: with k slices of other workgroups.  Kernels of their own for whole
+// tiles: in one kernel for both, the sums of a whole tile took moves and tests
+// on the way out (M = 3614, N = 6656, K = 1280 with one scale per column 58.0
+// -> 59.3 us).
+template <bool GROUP, int RB, bool SLICED>
 __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles_m, int tiles_n,
                                                            int ksplit) {
-  extern __shared__ __attribute__((aligned(16))) char smem_all[];  // kWdLdsBytes
-  __shared__ int s_ticket;
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];  // Shape::kLdsBytes
+  __shared__ int s_shares;
   {
     // fetch every kernel argument in one round trip
     const void *a_ = p.A, *b_ = p.B, *s_ = p.S;
@@ -79,7 +100,9 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
     asm volatile("" ::"s"(a_), "s"(b_), "s"(s_), "s"(c_), "s"(l_), "s"(sc_), "s"(p.M), "s"(p.N),
                  "s"(p.K), "s"(tiles_m), "s"(tiles_n), "s"(ksplit));
   }
-  constexpr int RB = kWdRB, HB = RB / 2;
+  using Shape = WdShape<RB>;
+  constexpr int HB = Shape::kHB;
+  constexpr int kWdTileM = Shape::kTileM;
 
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int kh = wave >> 1;  // k half
@@ -88,7 +111,7 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   const int lane = threadIdx.x & 63;
   const int kg = lane >> 4;
   const int nu = lane & 15;
-  char* smem = smem_all + kh * kWdRingBytes;
+  char* smem = smem_all + kh * Shape::kRingBytes;
 
   // Same numbering of the work as the other prefill kernel: every XCD
   // (workgroup id mod 8) gets a contiguous run of tile numbers, tiles are
@@ -97,8 +120,8 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   const int total = tiles_m * tiles_n * ksplit;
   int work = (int)blockIdx.x;
   if ((total & 7) == 0) work = (work & 7) * (total >> 3) + (work >> 3);
-  const int tile = work / ksplit;
-  const int ks = work - tile * ksplit;
+  const int tile = SLICED ? work / ksplit : work;
+  const int ks = SLICED ? work - tile * ksplit : 0;
   int tm, tn;
   if ((tiles_n & 7) == 0) {
     const int per_panel = 8 * tiles_m;
@@ -127,22 +150,24 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   const int s_lane = (256 * tn + 128 * nw) * 2 + 16 * nu;
 
   // slab staging: thread (row = tid/8 + 16 i', chunk x = tid%8) moves 16 bytes,
-  // i' = (i + 4 kh) % 8: the second k half keeps its row blocks rotated by four,
-  // so that in both halves accumulator blocks 0..3 are the ones the wave
-  // finishes and 4..7 the ones it hands to the other half.  Rows past the end
-  // of A read as zeros (out-of-range buffer offset).
+  // i' = (i + HB kh) % RB: the second k half keeps its row blocks rotated by HB,
+  // so that in both halves the first accumulator blocks are the ones the wave
+  // finishes (HB of them; RB - HB in the second half) and the last HB hold the
+  // ones it hands to the other half.  Rows past the end of A read as zeros
+  // (out-of-range buffer offset).
   const int ax = tid & 7;
   int a_lane[RB];
 #pragma unroll
   for (int i = 0; i < RB; i++) {
-    const int r = (tid >> 3) + 16 * ((i + 4 * kh) & 7);
+    const int at = i + HB * kh;
+    const int r = (tid >> 3) + 16 * (at >= RB ? at - RB : at);
     a_lane[i] = r < rows ? r * p.K * 2 + 16 * ax : kOobWd;
   }
   // LDS slab: [step][k group][row][slot] dwords; chunk x -> step x/4, slot x%4
   const int lds_wr =
-      (int)(size_t)(smem + (ax >> 2) * kWdStepBytes + (tid >> 3) * 16 + (ax & 3) * 4);
-  const int lds_rd = (int)(size_t)(smem + kg * kWdPlane + nu * 16);
-  // where this wave leaves accumulator blocks 4..7 for the other k half
+      (int)(size_t)(smem + (ax >> 2) * Shape::kStepBytes + (tid >> 3) * 16 + (ax & 3) * 4);
+  const int lds_rd = (int)(size_t)(smem + kg * Shape::kPlane + nu * 16);
+  // where this wave leaves its last accumulator blocks for the other k half
   const int lds_swap = (int)(size_t)(smem_all + wave * (HB * 8 * 1024) + lane * 16);
 
   // this half's stages: [s_begin, s_end) of the K/64 stages; the loop runs the
@@ -156,12 +181,24 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   const int stages = half_stages;
   const int s_row = p.N * 2;  // bytes per row of group scales
 
-  f4 fin[HB][8];  // accumulator blocks 0..3: row blocks own .. own+3 of the tile
+  f4 fin[HB][8];  // the first accumulator blocks: row blocks own, own+1, ... of the tile
 #if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (GROUP) {
-#include "w4a16_prefill_wide_group.inc"
+  if constexpr (GROUP && RB == 8) {
+#include "w4a16_prefill_wide_group128.inc"
+  } else if constexpr (GROUP && RB == 7) {
+#include "w4a16_prefill_wide_group112.inc"
+  } else if constexpr (GROUP && RB == 6) {
+#include "w4a16_prefill_wide_group96.inc"
+  } else if constexpr (GROUP) {
+#include "w4a16_prefill_wide_group80.inc"
+  } else if constexpr (RB == 8) {
+#include "w4a16_prefill_wide_chan128.inc"
+  } else if constexpr (RB == 7) {
+#include "w4a16_prefill_wide_chan112.inc"
+  } else if constexpr (RB == 6) {
+#include "w4a16_prefill_wide_chan96.inc"
   } else {
-#include "w4a16_prefill_wide_chan.inc"
+#include "w4a16_prefill_wide_chan80.inc"
   }
 #else  // the host pass only needs the launch stub
   (void)rb_words, (void)rs_words, (void)ra_words, (void)b_row, (void)b_lane, (void)s_lane;
@@ -172,62 +209,89 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
 #endif
   // the other k half's sums of the same row blocks
   __syncthreads();
+  const int own = HB * kh;  // first row block this wave finishes
   {
-    const f4* in = (const f4*)smem_all + (size_t)(wave ^ 2) * (HB * 8 * 64);
-#pragma unroll
-    for (int i = 0; i < HB; i++)
-#pragma unroll
-      for (int o = 0; o < 8; o++) fin[i][o] += in[(i * 8 + o) * 64 + lane];
-  }
-
-  // ---- k slices of other workgroups: every slice writes its fp32 tile through
-  // to memory (whole 1 KiB lines per wave instruction), waits for the
-  // acknowledgement, takes the tile's ticket; the last arrival adds all slices
-  // in slice order (its own from registers at its place in that order) and
-  // carries on.  Nobody spins.
-  if (ksplit > 1) {
-    constexpr int part_bytes = kWdTileM * kWdTileN * 4;
-    const __amdgpu_buffer_rsrc_t rP = wd_rsrc(p.scratch, 0x7fffffffu);
-    const int at = (wave * (HB * 8) * 64 + lane) * 16;
-    const int mine = work * part_bytes;
-#pragma unroll
-    for (int i = 0; i < HB; i++)
-#pragma unroll
-      for (int o = 0; o < 8; o++)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, fin[i][o]), rP,
-                                               at + (i * 8 + o) * 1024, mine, 16 /* sc1 */);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): my stores have been acknowledged
-    __syncthreads();
-    if (threadIdx.x == 0)
-      s_ticket = __hip_atomic_fetch_add(&p.locks[tile], 1, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (s_ticket != ksplit - 1) return;  // a later slice finishes the tile
-    // one row block at a time keeps the live registers few
+    // (with an odd number of row blocks the second half's are one slot further
+    // on, and it finishes one fewer)
+    const f4* in = (const f4*)smem_all + (size_t)(wave ^ 2) * (HB * 8 * 64) +
+                   (kh ? (2 * HB - RB) * 8 * 64 : 0);
 #pragma unroll
     for (int i = 0; i < HB; i++) {
-      f4 sum[8];
-      for (int k2 = 0; k2 < ksplit; k2++) {
-        f4 v[8];
-        if (k2 != ks) {
-          const int theirs = (tile * ksplit + k2) * part_bytes;
+      if ((RB & 1) && own + i >= RB) continue;
 #pragma unroll
-          for (int o = 0; o < 8; o++)
-            v[o] = __builtin_bit_cast(
-                f4, __builtin_amdgcn_raw_buffer_load_b128(rP, at + (i * 8 + o) * 1024, theirs,
-                                                          16 /* sc1 */));
-        } else {
+      for (int o = 0; o < 8; o++) fin[i][o] += in[(i * 8 + o) * 64 + lane];
+    }
+  }
+
+  // ---- k slices of other workgroups: every slice writes the fp32 sums that
+  // others will add up through to memory (whole 1 KiB lines per wave
+  // instruction), waits for the acknowledgement and arrives; the slices then
+  // finish the tile together.  Piece e of it is half the columns (operands
+  // 4 (e%2) ... +3) of row block e/2 of every wave; all slices of it are added
+  // in slice order, this one's from registers at its place in that order.
+  constexpr int NP = 2 * HB;
+  int pieces = (1 << NP) - 1;
+  if constexpr (SLICED) {
+    constexpr int part_bytes = Shape::kPartBytes;
+    const __amdgpu_buffer_rsrc_t rP = wd_rsrc(p.scratch, 0x7fffffffu);
+    int* const word = &p.locks[tile * p.lock_stride];
+    const int at = (wave * (HB * 8) * 64 + lane) * 16;
+    auto write_out = [&](int which) {
 #pragma unroll
-          for (int o = 0; o < 8; o++) v[o] = fin[i][o];
-        }
+      for (int e = 0; e < NP; e++) {
+        if (!(which >> e & 1)) continue;
 #pragma unroll
-        for (int o = 0; o < 8; o++) sum[o] = k2 == 0 ? v[o] : sum[o] + v[o];
+        for (int o = 4 * (e & 1); o < 4 * (e & 1) + 4; o++)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, fin[e >> 1][o]), rP,
+                                                 at + ((e >> 1) * 8 + o) * 1024, work * part_bytes,
+                                                 16 /* sc1 */);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): my stores have been acknowledged
+      __syncthreads();
+    };
+    const int my_share = finish_pieces(1 << ks, ksplit, NP);
+    write_out(pieces & ~my_share);
+    if (threadIdx.x == 0) s_shares = finish_arrive(word, ksplit, ks, p.finish_polls);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_shares) == 0) {
+      write_out(my_share);
+      if (threadIdx.x == 0) s_shares = finish_abandon(word, ksplit, ks);
+      __syncthreads();
+    }
+    pieces = __builtin_amdgcn_readfirstlane(finish_pieces(s_shares, ksplit, NP));
+    // what is requested at once: a row block of up to four slices, else half of one
+    auto add_up = [&](auto SL, auto NO, int i, int o0) {
+      constexpr int sl = decltype(SL)::value, no = decltype(NO)::value;
+      f4 v[sl][no];
+#pragma unroll
+      for (int k2 = 0; k2 < sl; k2++) {
+        if (k2 >= ksplit || k2 == ks) continue;
+#pragma unroll
+        for (int o = 0; o < no; o++)
+          v[k2][o] = __builtin_bit_cast(
+              f4, __builtin_amdgcn_raw_buffer_load_b128(rP, at + (i * 8 + o0 + o) * 1024,
+                                                        (tile * ksplit + k2) * part_bytes, 16 /* sc1 */));
       }
 #pragma unroll
-      for (int o = 0; o < 8; o++) fin[i][o] = sum[o];
+      for (int o = 0; o < no; o++) {
+        f4 sum = ks == 0 ? fin[i][o0 + o] : v[0][o];
+#pragma unroll
+        for (int k2 = 1; k2 < sl; k2++)
+          if (k2 < ksplit) sum += k2 == ks ? fin[i][o0 + o] : v[k2][o];
+        fin[i][o0 + o] = sum;
+      }
+    };
+    using std::integral_constant;
+#pragma unroll
+    for (int i = 0; i < HB; i++) {
+      const int both = pieces >> (2 * i) & 3;
+      if (both == 3 && ksplit <= 4) {
+        add_up(integral_constant<int, 4>{}, integral_constant<int, 8>{}, i, 0);
+      } else {
+        if (both & 1) add_up(integral_constant<int, 8>{}, integral_constant<int, 4>{}, i, 0);
+        if (both & 2) add_up(integral_constant<int, 8>{}, integral_constant<int, 4>{}, i, 4);
+      }
     }
-    if (threadIdx.x == 0)  // counters are handed back zeroed
-      __hip_atomic_store(&p.locks[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
 
@@ -236,7 +300,6 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   // (j, h), the four consecutive columns 64(q/2) + 16j + 8h + 4(q%2) + r of its
   // wave's 128, q = lane/16.
   const int q = lane >> 4;
-  const int own = HB * kh;  // first row block this wave finishes
 #pragma unroll
   for (int o = 0; o < 8; o++) {
     const int nloc = 128 * nw + 64 * (q >> 1) + 16 * (o >> 1) + 8 * (o & 1) + 4 * (q & 1);
@@ -248,6 +311,8 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
     }
 #pragma unroll
     for (int i = 0; i < HB; i++) {
+      if ((RB & 1) && own + i >= RB) continue;
+      if (SLICED && !(pieces >> (2 * i + (o >> 2)) & 1)) continue;
       const int m = 16 * (own + i) + nu;
       h4 v = {(half_t)fin[i][o][0], (half_t)fin[i][o][1], (half_t)fin[i][o][2],
               (half_t)fin[i][o][3]};
@@ -262,34 +327,60 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
     const int piece = it * 256 + (int)threadIdx.x;  // 16-byte piece of the tile
     const int m = piece >> 5;
     const int c16 = piece & 31;
-    if (m < rows) {
+    // (row block i of either k half; columns 32 ... 63 of every 64: operands 4 to 7)
+    const int i = m >= 16 * HB ? (m >> 4) - HB : m >> 4;
+    if (m < rows && (!SLICED || (pieces >> (2 * i + ((c16 >> 2) & 1)) & 1))) {
       const i4 v = *(const i4*)(smem_all + m * kWdPitch + c16 * 16);
       // nobody reads C again in this launch: keep it out of the way of A and B in L2
       __builtin_nontemporal_store(v, (i4*)(C + (size_t)(m0 + m) * p.N + kWdTileN * tn + c16 * 8));
     }
   }
+  if (SLICED && threadIdx.x == 0) finish_leave(&p.locks[tile * p.lock_stride], ksplit);
 }
 
+template <bool GROUP, int RB>
+static int configure_wide() {
+  constexpr int lds = WdShape<RB>::kLdsBytes;
+  return hipFuncSetAttribute((const void*)prefill_wide_kernel<GROUP, RB, false>,
+                             hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
+         hipFuncSetAttribute((const void*)prefill_wide_kernel<GROUP, RB, true>,
+                             hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess;
+}
 int configure_prefill_wide_kernels() {
-  if (hipFuncSetAttribute((const void*)prefill_wide_kernel<true>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kWdLdsBytes) != hipSuccess ||
-      hipFuncSetAttribute((const void*)prefill_wide_kernel<false>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kWdLdsBytes) != hipSuccess)
-    return 3;
-  return 0;
+  return configure_wide<false, 5>() | configure_wide<false, 6>() | configure_wide<false, 7>() |
+                 configure_wide<false, 8>() | configure_wide<true, 5>() | configure_wide<true, 6>() |
+                 configure_wide<true, 7>() | configure_wide<true, 8>()
+             ? 3
+             : 0;
 }
 
-int launch_prefill_wide(const GemmArgs& a, bool group, int ksplit, hipStream_t stream) {
-  const int tiles_m = ceil_div(a.M, kWdTileM);
+template <bool GROUP, int RB>
+static int launch_wide(const GemmArgs& a, int ksplit, hipStream_t stream) {
+  constexpr int lds = WdShape<RB>::kLdsBytes;
+  const int tiles_m = ceil_div(a.M, 16 * RB);
   const int tiles_n = a.N / kWdTileN;
   const dim3 grid(tiles_m * tiles_n * ksplit);
-  if (group)
-    hipLaunchKernelGGL(prefill_wide_kernel<true>, grid, dim3(256), kWdLdsBytes, stream, a, tiles_m,
-                       tiles_n, ksplit);
-  else
-    hipLaunchKernelGGL(prefill_wide_kernel<false>, grid, dim3(256), kWdLdsBytes, stream, a,
+  if (ksplit > 1)
+    hipLaunchKernelGGL((prefill_wide_kernel<GROUP, RB, true>), grid, dim3(256), lds, stream, a,
                        tiles_m, tiles_n, ksplit);
+  else
+    hipLaunchKernelGGL((prefill_wide_kernel<GROUP, RB, false>), grid, dim3(256), lds, stream, a,
+                       tiles_m, tiles_n, 1);
   return launch_status();
+}
+
+int launch_prefill_wide(const GemmArgs& a, bool group, int tile_rows, int ksplit, hipStream_t stream) {
+  switch (tile_rows + (group ? 1 : 0)) {
+    case 80: return launch_wide<false, 5>(a, ksplit, stream);
+    case 81: return launch_wide<true, 5>(a, ksplit, stream);
+    case 96: return launch_wide<false, 6>(a, ksplit, stream);
+    case 97: return launch_wide<true, 6>(a, ksplit, stream);
+    case 112: return launch_wide<false, 7>(a, ksplit, stream);
+    case 113: return launch_wide<true, 7>(a, ksplit, stream);
+    case 128: return launch_wide<false, 8>(a, ksplit, stream);
+    case 129: return launch_wide<true, 8>(a, ksplit, stream);
+  }
+  return 2;
 }
 
 }  // namespace w4a16

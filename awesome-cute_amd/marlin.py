@@ -37,6 +37,8 @@ _lib.marlin_amd_force_k_slices.restype = None
 _lib.marlin_amd_force_k_slices.argtypes = [_I]
 _lib.marlin_amd_force_tile_rows.restype = None
 _lib.marlin_amd_force_tile_rows.argtypes = [_I]
+_lib.marlin_amd_force_finish_polls.restype = None
+_lib.marlin_amd_force_finish_polls.argtypes = [_I]
 _lib.marlin_amd_force_row_halves.restype = None
 _lib.marlin_amd_force_row_halves.argtypes = [_I]
 _lib.marlin_amd_force_kernel.restype = None
@@ -307,8 +309,15 @@ def force_k_slices(slices):
 
 
 def force_tile_rows(rows):
-    """Rows of C per prefill workgroup (64 or 128); 0 = choose by cost (calling thread only)."""
+    """Rows of C per prefill workgroup (64 to 128 in steps of 16); 0 = choose by cost (calling
+    thread only)."""
     _lib.marlin_amd_force_tile_rows(int(rows))
+
+
+def force_finish_polls(polls):
+    """How often a workgroup looks for the other k slices of its prefill tile before it leaves
+    them its share of the sums; -1 = the default (calling thread only)."""
+    _lib.marlin_amd_force_finish_polls(int(polls))
 
 
 def force_row_halves(mode):

@@ -105,9 +105,18 @@ void marlin_amd_force_row_halves(int mode);
 
 /*
  * Rows of C per workgroup of the prefill kernel, for the calling thread: 0 =
- * choose by cost (default), 64 or 128.  No reference counterpart; for tests and tools.
+ * choose by cost (default), or 64 to 128 in steps of 16.  No reference
+ * counterpart; for tests and tools.
  */
 void marlin_amd_force_tile_rows(int rows);
+
+/*
+ * How often a workgroup of the prefill kernel with 80 or more rows looks
+ * whether the other k slices of its tile have arrived before it leaves them its
+ * share of the sums, for the calling thread: -1 = the default, 0 = at once.  No
+ * reference counterpart; for tests (results do not depend on it).
+ */
+void marlin_amd_force_finish_polls(int polls);
 
 /*
  * out[0..4] = compute units, shader clock (kHz), memory clock (kHz), memory
