@@ -67,10 +67,11 @@ def _run(cmd, verbose):
 def build_library(verbose=False):
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
-    # the assembly statements of the four-wave prefill kernel (prologue, main
-    # loop and accumulator hand-over with fixed registers) are written by a
-    # generator; w4a16_prefill_wide.hip includes them from the build directory
-    _run([sys.executable, os.path.join(CSRC, "gen_prefill_wide.py"), objdir], verbose)
+    # the assembly statements of the four-wave kernels (prologue, main loop and
+    # accumulator hand-over with fixed registers) are written by generators;
+    # w4a16_prefill_wide.hip and f16_streamk.hip include them from the build directory
+    for gen in ("gen_prefill_wide.py", "gen_dense.py"):
+        _run([sys.executable, os.path.join(CSRC, gen), objdir], verbose)
     objs = [os.path.join(objdir, src.replace(".hip", ".o")) for src in SOURCES]
     with ThreadPoolExecutor(4) as pool:
         binding = pool.submit(_compile_binding, objdir, verbose)

@@ -12,32 +12,42 @@
 // to memory, takes a ticket, and the last arrival adds all slices in slice
 // order and writes C.
 //
-// Kernel: a workgroup of 8 waves (2 x 4, two per SIMD) owns a 256 x 256 tile
-// of C; a wave holds a 128 x 64 fp32 accumulator (128 registers).  Problems
-// with too few such tiles for the compute units run on 128 x 256 or 128 x 128
-// tiles (same eight waves, a wave's share 64 x 64 or 64 x 32).  With B as
-// the first MFMA operand and A as the second, v_mfma_f32_16x16x32_f16 yields
-// D[n][m]; lane l = 16kg + nu of an operand holds k = 8kg ... 8kg+7 of row nu.
-// Per 64-deep k stage (two MFMA k steps) the workgroup brings a 256 x 64 slab
-// of A and of B into a ring of LDS slabs (two; three or four for the smaller
-// tiles, whose stages are shorter than a load's latency) with buffer loads that write LDS
+// Whole tiles, 256 x 256 or (too few of them for the compute units) 128 x 256:
+// dense_kernel.  A workgroup of four waves, one per SIMD, each with a 128 x 128
+// fp32 accumulator (all 256 AGPRs): a wave per quarter of the tile, or two
+// waves per 128 columns, each taking every other k step, their sums added
+// through LDS at the end.  The main loop is one assembly statement per tile
+// shape, written by gen_dense.py, which documents the schedule and the
+// registers; the build runs it.
+//
+// 128 x 128 tiles, whole or slices: dense_small_kernel.  Eight waves of 64 x 32,
+// two per SIMD.  It computes the problems with few tiles, and the stream-K tiles
+// of the others, every 256 x 256 tile of the partial wave as four of its own.
+//
+// In both, B is the first MFMA operand and A the second, so
+// v_mfma_f32_16x16x32_f16 yields D[n][m]; lane l = 16kg + nu of an operand holds
+// k = 8kg ... 8kg+7 of row nu.  Per 64-deep stage the workgroup brings a slab of
+// A and of B rows into a ring of LDS slots with buffer loads that write LDS
 // directly (16 bytes per lane, lane l at 16*l).  Eight lanes fetch the whole
-// 128-byte k run of a row -- one cache line; with 64-byte runs every line
-// came in twice and the loads alone bounded the kernel -- so a slab is
-// row-major with 128-byte rows.  To keep the operand reads (lane (kg, nu):
-// 16 bytes at chunk 4h + kg of row nu, one ds_read_b128) free of bank
-// conflicts, the chunk stored at position c of row r is chunk c ^ (r % 8);
-// since the hardware fixes where a lane's bytes land, the swizzle is applied
-// to the address the lane fetches.  A slab is requested at least a whole stage
-// before it is needed; one barrier per stage.  The compiler cannot know which slab a
-// load in flight writes, so the LDS reads of the main loop and their waits are
-// written by hand (LDS reads return in order).
+// 128-byte k run of a row -- one cache line; with 64-byte runs every line came
+// in twice and the loads alone bounded the kernel -- so a slab is row-major with
+// 128-byte rows.  To keep the operand reads (lane (kg, nu): 16 bytes at chunk
+// 4h + kg of row nu, one ds_read_b128) free of bank conflicts, the chunk stored
+// at position c of row r is chunk c ^ (r % 8); since the hardware fixes where a
+// lane's bytes land, the swizzle is applied to the address the lane fetches.
+//
+// What bounds it: LDS and the way into it, then the board's power.  The large
+// tiles with eight waves of 128 x 64 (twelve operand reads per 32 MFMAs) kept LDS
+// as busy as the matrix pipe; 128 x 128 per wave reads 16 per 64: 4096^3 101 ->
+// 96 us, 8192 x 8192 x 2048 217 -> 208, 1152 x 4352 x 4096 (128-row tiles) 50.8 ->
+// 49.5; 8192^3, at the power limit, 1.39 PFLOP/s either way.  The small tiles
+// wait for operands: a compute unit takes in a stage's 32 KiB at 90 to 120 GB/s
+// from L2, 57 where A and B come from memory.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
 #include <mutex>
 #include <type_traits>
-#include <vector>
 
 #include "../../include/streamk_amd.h"
 #include "scratch_pool.hpp"
@@ -47,47 +57,66 @@ namespace w4a16 {
 
 namespace {
 
-constexpr int kDnTile = 256;     // columns of a tile of C, and rows of the large tile
-constexpr int kDnStageK = 64;    // k depth of a stage (two MFMA k steps)
+constexpr int kDnTile = 256;     // rows and columns of the large tile of C
+constexpr int kDnStageK = 64;    // k depth of a stage (two MFMA k steps); k is a multiple
 constexpr int kDnOob = (int)0x80000000;
 
-// LDS geometry for tiles of TM rows and TN columns (256 x 256; 128 x 256 or
-// 128 x 128 when larger tiles are too few for the compute units): a slab is
-// TM rows of A and TN rows of B
-template <int TM, int TN>
+// Tiles of dense_kernel, TM rows and 256 columns: 256 x 256 or 128 x 256
+template <int TM>
 struct DnShape {
+  static constexpr int kWK = 256 / TM;          // waves that share a 128 x 128 part's k steps
   static constexpr int kSlabA = TM * 128;
-  static constexpr int kSlab = kSlabA + TN * 128;
-  // slabs in LDS.  A stage of a small tile is shorter than a load's way from
-  // L2 (0.4 us of MFMAs for 128 x 128), so its slabs are requested further ahead.
-  static constexpr int kRing = TM * TN == 128 * 128 ? 4 : (TM * TN == 128 * 256 ? 3 : 2);
-  static constexpr int kLds = kRing * kSlab;
-  static constexpr int kRB = TM / 32;  // 16-row blocks per wave
-  static constexpr int kNJ = TN / 64;  // 16-column blocks per wave
-  static constexpr int kPartBytes = TM * TN * 4;
+  static constexpr int kSlab = kSlabA + 256 * 128;
+  static constexpr int kRing = kWK == 2 ? 3 : 2;
+  static constexpr int kSteps = 2 / kWK;        // k steps of a wave per slab
+  static constexpr int kTA = kSlabA / 4096;     // load instructions per wave and slab
+  static constexpr int kTB = 256 * 128 / 4096;
+  static constexpr int kNF = 8 / kWK;           // row blocks of 16 a wave finishes
+  static constexpr int kPitch = 256 * 2 + 16;   // bytes per row of the fp16 tile in LDS
+  static constexpr int kRingBytes = kRing * kSlab, kTileBytes = TM * kPitch;
+  static constexpr int kLds = kRingBytes > kTileBytes ? kRingBytes : kTileBytes;
+  static_assert(kWK == 1 || kLds >= 128 * 1024, "room for the sums that waves hand each other");
 };
-constexpr int kDnMaxSlots = 256;                     // slices in flight per launch
+// 128 x 128 tiles (dense_small_kernel)
+struct DnSmall {
+  static constexpr int kSlabA = 128 * 128;
+  static constexpr int kSlab = 2 * kSlabA;
+  static constexpr int kRing = 4;
+  static constexpr int kLoads = 4;              // per wave and slab
+  static constexpr int kPitch = 128 * 2 + 16;
+  static constexpr int kLds = kRing * kSlab;
+  static constexpr int kPartBytes = 128 * 128 * 4;
+};
+constexpr int kDnMaxSlots = 256;  // slices in flight per launch
 constexpr int kDnMaxSlices = 4;
+constexpr int kDnCounterStride = 16;  // ints: a tile's slices meet in a cache line of their own
 
 struct DenseArgs {
   const void* A;
   const void* B;
   void* C;
   int M, N, K;
-  int tile_rows;  // 256 or 128
-  int tile_cols;  // 256 or 128
   int tiles_m, tiles_n;
   int dp_tiles;  // tiles computed by one workgroup each
-  int sk_tiles;  // tiles (the last ones in tile order) cut into ksplit slices
+  // dense_small_kernel: tiles (the last ones in tile order) cut into ksplit
+  // slices; with quarters, the plan's tiles are 256 x 256 and those after
+  // dp_tiles are computed as four tiles each
+  int sk_tiles;
   int ksplit;
-  int* locks;      // one zeroed counter per stream-K tile, zero again afterwards
-  float* scratch;  // kDnPartBytes per slice
+  int quarters;
+  int slices_only;   // the launch has no whole tiles
+  int* locks;        // one zeroed counter per cut tile, kDnCounterStride ints apart, zero again afterwards
+  float* scratch;    // kPartBytes per slice
+  int finish_polls;  // looks at a tile's other slices before leaving them a share
 };
 
 // Tiles are numbered panel by panel: a panel is kDnPanel column tiles wide
-// (the last one narrower), and inside a panel the column tile runs fastest.
-// A run of consecutive tile numbers then covers a compact block of C, so the
-// workgroups that share an L2 read few distinct rows of A and B.
+// (the last one narrower), and inside a panel the column tile runs fastest, or
+// the row tile where there are fewer than kDnPanel of them.  A run of
+// consecutive tile numbers then covers a compact block of C, so the workgroups
+// that share an L2 read few distinct rows of A and B, and with few row tiles
+// every row of B comes from memory into one L2 only (777 x 4352 x 10240: 91.5 us,
+// with columns first 98.7).
 constexpr int kDnPanel = 8;
 __host__ __device__ __forceinline__ void dn_tile_coord(int t, int tiles_m, int tiles_n, int* tm,
                                                        int* tn) {
@@ -96,12 +125,24 @@ __host__ __device__ __forceinline__ void dn_tile_coord(int t, int tiles_m, int t
   const int first = p * kDnPanel;
   const int width = tiles_n - first < kDnPanel ? tiles_n - first : kDnPanel;
   const int o = t - p * per_panel;
-  *tm = o / width;
-  *tn = first + o - *tm * width;
+  if (tiles_m < kDnPanel) {
+    *tn = first + o / tiles_m;
+    *tm = o - (*tn - first) * tiles_m;
+  } else {
+    *tm = o / width;
+    *tn = first + o - *tm * width;
+  }
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t dn_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+
+// the four words of a raw buffer resource: 48-bit base, stride 0, size in
+// bytes, data format flags
+__device__ __forceinline__ i4 dn_rsrc_words(const void* p, unsigned bytes) {
+  const unsigned long long a = (unsigned long long)p;
+  return (i4){(int)(unsigned)a, (int)(unsigned)((a >> 32) & 0xffffu), (int)bytes, 0x00020000};
 }
 
 // 16 bytes per lane from a buffer straight into LDS: lane l's bytes land at
@@ -116,13 +157,15 @@ __device__ __forceinline__ void dn_dma16(__amdgpu_buffer_rsrc_t rsrc, char* dst,
 #endif
 }
 
-// LDS reads of the main loop, outside the compiler's dependence tracking
+// LDS reads of a main loop, outside the compiler's dependence tracking (it
+// would wait for every load in flight before each of them)
 template <int OFF>
 __device__ __forceinline__ void dn_read16(unsigned at, i4& v) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF) : "memory");
 #endif
 }
+
 // wait until at most PENDING later LDS reads are outstanding; `v` is the
 // operand the wait is for
 template <int PENDING>
@@ -140,13 +183,6 @@ __device__ __forceinline__ void drain_reads(i4 (&a)[2], i4 (&b)[2], i4 (&f)[4]) 
                  "+v"(f[3]));
 #endif
 }
-__device__ __forceinline__ void drain_reads(i4 (&a)[4], i4 (&b)[4], i4 (&f)[4]) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]),
-                 "+v"(b[3]), "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]));
-#endif
-}
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding)
 constexpr int dn_vm_lgkm0(int n) { return (n & 15) | (7 << 4) | (0 << 8) | ((n >> 4) << 14); }
 // s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
@@ -154,70 +190,230 @@ constexpr int dn_vmcnt(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 
 
 }  // namespace
 
-template <int TM, int TN>
-__global__ __launch_bounds__(512) void dense_kernel(DenseArgs p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // DnShape<TM, TN>::kLds
-  using Shape = DnShape<TM, TN>;
-  constexpr int RB = Shape::kRB;
-  constexpr int NJ = Shape::kNJ;
-  constexpr int kDnSlabA = Shape::kSlabA;
-  constexpr int kDnSlab = Shape::kSlab;
-  constexpr int kRing = Shape::kRing;
-  constexpr int kDnLds = Shape::kLds;
-  constexpr int kPart = Shape::kPartBytes;
-  __shared__ int s_ticket;
+// Pieces of an fp16 tile from LDS to C with 16-byte stores, by THREADS threads:
+// what `mine(row, operand of 16 columns)` says.
+template <int TM, int TN, int PITCH, int THREADS, class Mine>
+__device__ __forceinline__ void dense_store_tile(const char* smem, half_t* C, int N, int rows,
+                                                 Mine mine) {
+  constexpr int PR = TN / 8;  // 16-byte pieces of a row
+#pragma unroll 8
+  for (int it = 0; it < TM * PR / THREADS; it++) {
+    const int at = it * THREADS + (int)threadIdx.x;
+    const int m = at / PR, c16 = at % PR;
+    if (m < rows && mine(m, c16 / 2)) {
+      const i4 v = *(const i4*)(smem + m * PITCH + c16 * 16);
+      // nobody reads C again in this launch: keep it out of the way of A and B in L2
+      __builtin_nontemporal_store(v, (i4*)(C + (size_t)m * N + c16 * 8));
+    }
+  }
+}
+
+// A whole tile to C: the waves' row blocks (NF each, `sums(i, o)` rounded to `out`,
+// NO operands of 16 columns) through LDS in two halves, so that the second half
+// is rounded and written to LDS while the first is on its way to memory.  Rows
+// r NF 16 ... of the tile belong to one row of waves.
+template <int TM, int TN, int PITCH, int THREADS, int NF, int NO, class Sums>
+__device__ __forceinline__ void dense_write_tile(const char* smem, char* out, half_t* C, int N, int rows,
+                                                 Sums sums) {
+  constexpr int PR = TN / 8;     // 16-byte pieces of a row
+  constexpr int RUN = 8 * NF;    // rows of a wave in one half
+#pragma unroll
+  for (int half = 0; half < 2; half++) {
+#pragma unroll
+    for (int i = half * NF / 2; i < (half + 1) * NF / 2; i++)
+#pragma unroll
+      for (int o = 0; o < NO; o++) {
+        const f4 v = sums(i, o);
+        *(h4*)(out + 16 * i * PITCH + 32 * o) =
+            (h4){(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+      }
+    __syncthreads();
+#pragma unroll 8
+    for (int it = 0; it < TM / 2 * PR / THREADS; it++) {
+      const int at = it * THREADS + (int)threadIdx.x;
+      const int r = at / PR, c16 = at % PR;
+      const int m = r / RUN * (2 * RUN) + half * RUN + r % RUN;
+      if (m < rows) {
+        const i4 v = *(const i4*)(smem + m * PITCH + c16 * 16);
+        // nobody reads C again in this launch: keep it out of the way of A and B in L2
+        __builtin_nontemporal_store(v, (i4*)(C + (size_t)m * N + c16 * 8));
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ h4 dense_round(f4 v) {
+  return (h4){(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+}
+
+template <int TM>
+__global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // DnShape<TM>::kLds
+  using Shape = DnShape<TM>;
+  constexpr int WK = Shape::kWK, NF = Shape::kNF, TA = Shape::kTA, TB = Shape::kTB;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int kg = lane >> 4;
   const int nu = lane & 15;
-  const int wm = wave >> 2;  // row half of the tile
-  const int wn = wave & 3;   // column quarter of the tile
+  const int wm = WK == 1 ? wave >> 1 : 0;  // 128-row half of the tile
+  const int wn = wave & 1;                 // 128-column half
+  const int wk = WK == 1 ? 0 : wave >> 1;  // which of the k steps
 
-  // stream-K slices come first in the grid, so that they run beside the first
-  // wave of whole tiles
-  const int sk_blocks = p.sk_tiles * p.ksplit;
-  const int work = (int)blockIdx.x;
-  int tile, ks, ksplit;
-  if (work < sk_blocks) {
-    tile = p.dp_tiles + work / p.ksplit;
-    ks = work % p.ksplit;
-    ksplit = p.ksplit;
-  } else {
-    // The hardware deals workgroups to the 8 XCDs round-robin; give every XCD
-    // a contiguous run of tile numbers.  A placement hint only.
-    tile = work - sk_blocks;
-    if (((sk_blocks | p.dp_tiles) & 7) == 0) tile = (tile & 7) * (p.dp_tiles >> 3) + (tile >> 3);
-    ks = 0;
-    ksplit = 1;
-  }
+  // every XCD gets a contiguous run of tile numbers (a placement hint only)
+  const int tile = xcd_work_index((int)blockIdx.x, p.dp_tiles);
   int tm, tn;
   dn_tile_coord(tile, p.tiles_m, p.tiles_n, &tm, &tn);
   const int m0 = tm * TM;
-  const int n0 = tn * TN;
+  const int n0 = tn * 256;
   const int rows = min(TM, p.M - m0);
+
+  i4 ra_words = dn_rsrc_words((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
+  i4 rb_words = dn_rsrc_words((const char*)p.B + (size_t)n0 * p.K * 2, 256u * (unsigned)p.K * 2u);
+
+  // wave w fetches the w-th quarter of the A rows and of the B rows of a slab,
+  // eight rows per instruction: lane (r = lane/8, c = lane%8) lands at [r][c] and
+  // fetches chunk c ^ r of its row.  Rows past the end of A repeat the last row
+  // (never stored).
+  int src[TA + TB];
+  {
+    const int r8 = lane >> 3, c = (lane & 7) ^ r8;
+#pragma unroll
+    for (int t = 0; t < TA + TB; t++) {
+      int r = 8 * (t < TA ? TA * wave + t : TB * wave + t - TA) + r8;
+      if (t < TA && r >= rows) r = rows - 1;
+      src[t] = r * p.K * 2 + 16 * c;
+    }
+  }
+  const int slabs = p.K / kDnStageK;
+  int s_at = 0;  // byte offset of the next slab to request
+
+  // LDS: where this wave's loads of slot 0 go, and where its operand reads of
+  // every slot and step start
+  const int lds = (int)(size_t)smem;
+  const int lds_a = lds + wave * TA * 1024, lds_b = lds + Shape::kSlabA + wave * TB * 1024;
+  constexpr int kReads = Shape::kRing * Shape::kSteps;
+  int a_rd[kReads], b_rd[kReads];
+#pragma unroll
+  for (int j = 0; j < kReads; j++) {
+    const int c = 4 * (WK == 1 ? j % Shape::kSteps : wk) + kg;
+    const int at = lds + j / Shape::kSteps * Shape::kSlab + nu * 128 + 16 * (c ^ (nu & 7));
+    a_rd[j] = at + 128 * wm * 128;
+    b_rd[j] = at + Shape::kSlabA + 128 * wn * 128;
+  }
+
+  f4 acc[8][8];
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (WK == 1) {
+#include "f16_dense_256x256.inc"
+  } else {
+#include "f16_dense_128x256.inc"
+  }
+#else  // the host pass only needs the launch stub
+  (void)slabs, (void)s_at, (void)lds_a, (void)lds_b, (void)src;
+  (void)a_rd, (void)b_rd, (void)ra_words, (void)rb_words;
+  for (auto& r : acc)
+    for (auto& v : r) v = (f4){0.f, 0.f, 0.f, 0.f};
+#endif
+  // (nothing is on its way into LDS or registers any more)
+  __syncthreads();
+
+  // A lane holds, per (i, o), row 16i + nu and four consecutive columns.  Two
+  // waves that share k steps hand each other the four row blocks they will not
+  // finish and add; then the fp16 tile goes through LDS.
+  constexpr int kPitch = Shape::kPitch;
+  char* const out = smem + (128 * wm + 64 * wk + nu) * kPitch + (128 * wn + 4 * (lane >> 4)) * 2;
+  half_t* const C = (half_t*)p.C + (size_t)m0 * p.N + n0;
+  if constexpr (WK == 1) {
+    dense_write_tile<TM, 256, kPitch, 256, NF, 8>(smem, out, C, p.N, rows,
+                                                  [&](int i, int o) { return acc[i][o]; });
+  } else {
+    f4* const swap = (f4*)smem;
+    f4 fin[NF][8];
+    const auto add_up = [&](auto KEEP) {
+      constexpr int keep = decltype(KEEP)::value;
+#pragma unroll
+      for (int i = 0; i < NF; i++)
+#pragma unroll
+        for (int o = 0; o < 8; o++) swap[((wave * NF + i) * 8 + o) * 64 + lane] = acc[NF - keep + i][o];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < NF; i++)
+#pragma unroll
+        for (int o = 0; o < 8; o++)
+          fin[i][o] = acc[keep + i][o] + swap[(((wave ^ 2) * NF + i) * 8 + o) * 64 + lane];
+    };
+    if (wk == 0)
+      add_up(std::integral_constant<int, 0>{});
+    else
+      add_up(std::integral_constant<int, NF>{});
+    __syncthreads();
+    dense_write_tile<TM, 256, kPitch, 256, NF, 8>(smem, out, C, p.N, rows,
+                                                  [&](int i, int o) { return fin[i][o]; });
+  }
+}
+
+// CUT: some tiles are cut into slices, or are quarters of the plan's.  (One
+// kernel for both took whole tiles 0.25 us longer, 8.5 -> 8.75 us at 2048 x 2048
+// x 512.)
+template <bool CUT>
+__global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // DnSmall::kLds
+  using Sh = DnSmall;
+  __shared__ int s_shares;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int kg = lane >> 4;
+  const int nu = lane & 15;
+  const int wm = wave >> 2;  // 64-row half of the tile
+  const int wn = wave & 3;   // 32-column quarter
+
+  // Stream-K slices come first in the grid, so that they run beside the first
+  // wave of whole tiles; slices of the same k range and neighbouring tiles are
+  // neighbours in the grid.  Every XCD gets a contiguous run of slices and of
+  // tile numbers (a placement hint only).
+  int tile, ks = 0, ksplit = 1, cut = 0;
+  if constexpr (CUT) {
+    const int sk_blocks = p.sk_tiles * p.ksplit;
+    int work = (int)blockIdx.x;
+    if (p.slices_only) work = xcd_work_index(work, sk_blocks);
+    if (work < sk_blocks) {
+      ks = work / p.sk_tiles;
+      cut = work - ks * p.sk_tiles;
+      tile = p.dp_tiles + (p.quarters ? cut >> 2 : cut);
+      ksplit = p.ksplit;
+    } else {
+      tile = xcd_work_index(work - sk_blocks, p.dp_tiles);
+    }
+  } else {
+    tile = xcd_work_index((int)blockIdx.x, p.dp_tiles);
+  }
+  int tm, tn;
+  dn_tile_coord(tile, p.tiles_m, p.tiles_n, &tm, &tn);
+  int m0 = 128 * tm, n0 = 128 * tn;
+  if (CUT && p.quarters) {
+    m0 = 256 * tm + 128 * ((cut >> 1) & 1);
+    n0 = 256 * tn + 128 * (cut & 1);
+  }
+  const int rows = min(128, p.M - m0);
+  if (CUT && rows <= 0) return;  // a quarter below the last row, all its slices
 
   const __amdgpu_buffer_rsrc_t rA =
       dn_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
   const __amdgpu_buffer_rsrc_t rB =
-      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)TN * (unsigned)p.K * 2u);
+      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, 128u * (unsigned)p.K * 2u);
 
-  // wave w fetches rows (TM/8) w ... of the A slab and (TN/8) w ... of the
-  // B slab, eight rows per instruction: lane (r = lane/8, c = lane%8) lands at
-  // [r][c] and fetches chunk c ^ r of its row.  Rows past the end of A repeat
-  // the last row (never stored).
-  constexpr int TA = TM / 64;  // A instructions per wave and stage
-  constexpr int TB = TN / 64;  // B instructions per wave and stage
-  int a_src[TA], b_src[TB];
+  // wave w fetches rows 16 w ... of the A and of the B slab, as dense_kernel does
+  int a_src[2], b_src[2];
   {
     const int r8 = lane >> 3, c = (lane & 7) ^ r8;
 #pragma unroll
-    for (int t = 0; t < TA; t++) {
-      const int r = 8 * TA * wave + 8 * t + r8;
+    for (int t = 0; t < 2; t++) {
+      const int r = 16 * wave + 8 * t + r8;
       a_src[t] = (r < rows ? r : rows - 1) * p.K * 2 + 16 * c;
+      b_src[t] = r * p.K * 2 + 16 * c;
     }
-#pragma unroll
-    for (int t = 0; t < TB; t++) b_src[t] = (8 * TB * wave + 8 * t + r8) * p.K * 2 + 16 * c;
   }
   // this workgroup's stages [st0, st1) of the K/64 stages
   const int stages_all = p.K / kDnStageK;
@@ -226,50 +422,42 @@ __global__ __launch_bounds__(512) void dense_kernel(DenseArgs p) {
   const int st1 = (int)((unsigned)(ks + 1) * (unsigned)stages_all / (unsigned)ksplit);
   const int stages = st1 - st0;
 
-  auto issue_slab = [&](int s, int ring) {
+  auto issue_slab = [&](int s, int slot) {
     const int inv = s < stages ? 0 : kDnOob;  // a stage past the end fetches zeros
     const int at = (st0 + s) * (kDnStageK * 2);
-    char* base = smem + ring * kDnSlab;
+    char* base = smem + slot * Sh::kSlab + wave * 2048;
 #pragma unroll
-    for (int t = 0; t < TA; t++)
-      dn_dma16(rA, base + (8 * TA * wave + 8 * t) * 128, a_src[t] | inv, at);
+    for (int t = 0; t < 2; t++) dn_dma16(rA, base + t * 1024, a_src[t] | inv, at);
 #pragma unroll
-    for (int t = 0; t < TB; t++)
-      dn_dma16(rB, base + kDnSlabA + (8 * TB * wave + 8 * t) * 128, b_src[t] | inv, at);
+    for (int t = 0; t < 2; t++) dn_dma16(rB, base + Sh::kSlabA + t * 1024, b_src[t] | inv, at);
   };
-  constexpr int kSlabLoads = TA + TB;  // per wave
 
-  f4 acc[RB][NJ];
+  f4 acc[4][2];
 #pragma unroll
-  for (int i = 0; i < RB; i++)
+  for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int j = 0; j < NJ; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 2; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
 
-  i4 w[2][NJ];  // B operands of the two k steps of a stage
+  i4 w[2][2];  // B operands of the two k steps of a stage
   i4 af[4];    // ring of A operands, three ahead of the MFMAs
   // operand addresses in slab 0 for the two k steps
   unsigned a_rd[2], b_rd[2];
 #pragma unroll
   for (int h = 0; h < 2; h++) {
     const unsigned sw = 16 * ((4 * h + kg) ^ (nu & 7));
-    a_rd[h] = (unsigned)(size_t)smem + (16 * RB * wm + nu) * 128 + sw;
-    b_rd[h] = (unsigned)(size_t)smem + kDnSlabA + (16 * NJ * wn + nu) * 128 + sw;
+    a_rd[h] = (unsigned)(size_t)smem + (64 * wm + nu) * 128 + sw;
+    b_rd[h] = (unsigned)(size_t)smem + Sh::kSlabA + (32 * wn + nu) * 128 + sw;
   }
-  // the NJ B operands of a k step: 16 rows of the slab apart
-  auto read_b = [&](unsigned at, i4 (&dst)[NJ]) {
+  auto read_b = [&](unsigned at, i4 (&dst)[2]) {
     dn_read16<0>(at, dst[0]);
     dn_read16<2048>(at, dst[1]);
-    if constexpr (NJ == 4) {
-      dn_read16<4096>(at, dst[2]);
-      dn_read16<6144>(at, dst[3]);
-    }
   };
 
-  // prologue: slabs 0 ... kRing-1 requested; slab 0 landed (loads complete in
-  // order); its first operands read
+  // prologue: every slot requested; slab 0 landed (loads complete in order); its
+  // first operands read
 #pragma unroll
-  for (int r = 0; r < kRing; r++) issue_slab(r, r);
-  __builtin_amdgcn_s_waitcnt(dn_vmcnt((kRing - 1) * kSlabLoads));
+  for (int r = 0; r < Sh::kRing; r++) issue_slab(r, r);
+  __builtin_amdgcn_s_waitcnt(dn_vmcnt((Sh::kRing - 1) * Sh::kLoads));
   __builtin_amdgcn_s_barrier();
   read_b(b_rd[0], w[0]);
   dn_read16<0>(a_rd[0], af[0]);
@@ -277,12 +465,11 @@ __global__ __launch_bounds__(512) void dense_kernel(DenseArgs p) {
   dn_read16<4096>(a_rd[0], af[2]);
 
   // One k step (H) of the stage in slab `cur`.  LDS reads in issue order, with
-  // Ai the operand of row block i and primes the prefetches for the step after
-  // (eight row blocks per wave; with four the same three-ahead pattern):
-  //   step 0:  | B(step 1) x NJ  A3 | A4 | A5 | A6 | A7 | A0' | A1' | A2' |
-  //   step 1:  | A3 | A4 | A5 | A6 | A7 | barrier, B(next stage) x NJ  A0' | A1' | A2' |
+  // Ai the operand of row block i and primes the prefetches for the step after:
+  //   step 0:  | B(step 1) x 2  A3 | A0' | A1' | A2' |
+  //   step 1:  | A3 | barrier, B(next stage) x 2  A0' | A1' | A2' |
   // When row block i is used, the reads issued after Ai may still be pending:
-  // three A operands, plus the NJ B reads where those were issued in between
+  // three A operands, plus the two B reads where those were issued in between
   // (the three row blocks from the one that issues them).
   // The barrier of a stage sits where the first read from the next slab is
   // about to be issued: by then every wave has its own part of that slab (it
@@ -290,52 +477,41 @@ __global__ __launch_bounds__(512) void dense_kernel(DenseArgs p) {
   // the current slab, which the request for the stage after next overwrites.
   auto kstep = [&](auto H, unsigned cur, unsigned nxt, int s, int slot) {
     constexpr int h = decltype(H)::value;
-    constexpr int ib = h ? RB - 3 : 0;  // row block that issues the B reads
-    const unsigned ac = a_rd[h] + cur;                        // this step, this slab
-    const unsigned an = h ? a_rd[0] + nxt : a_rd[1] + cur;    // the step after
+    constexpr int ib = h;  // row block that issues the B reads
+    const unsigned ac = a_rd[h] + cur;                      // this step, this slab
+    const unsigned an = h ? a_rd[0] + nxt : a_rd[1] + cur;  // the step after
     const unsigned bn = h ? b_rd[0] + nxt : b_rd[1] + cur;
 #pragma unroll
-    for (int i = 0; i < RB; i++) {
+    for (int i = 0; i < 4; i++) {
       if (i == ib) {
         if (h == 1) {
           // my loads of the next slab (the slabs after it may still be on
           // their way) and my reads of this one
-          __builtin_amdgcn_s_waitcnt(dn_vm_lgkm0((kRing - 2) * kSlabLoads));
+          __builtin_amdgcn_s_waitcnt(dn_vm_lgkm0((Sh::kRing - 2) * Sh::kLoads));
           __builtin_amdgcn_s_barrier();
-          issue_slab(s + kRing, slot);
+          issue_slab(s + Sh::kRing, slot);
         }
         read_b(bn, w[h ^ 1]);
       }
       // operand of row block i + 3: of this step, or of the step after
-      auto frag = [&](auto I) {
-        constexpr int ii = decltype(I)::value;
-        if constexpr (ii < RB)
-          dn_read16<ii * 2048>(ac, af[ii & 3]);
-        else
-          dn_read16<(ii - RB) * 2048>(an, af[ii & 3]);
-      };
       switch (i) {  // i is a constant after unrolling
-        case 0: frag(std::integral_constant<int, 3>{}); break;
-        case 1: frag(std::integral_constant<int, 4>{}); break;
-        case 2: frag(std::integral_constant<int, 5>{}); break;
-        case 3: frag(std::integral_constant<int, 6>{}); break;
-        case 4: frag(std::integral_constant<int, 7>{}); break;
-        case 5: frag(std::integral_constant<int, 8>{}); break;
-        case 6: frag(std::integral_constant<int, 9>{}); break;
-        case 7: frag(std::integral_constant<int, 10>{}); break;
+        case 0: dn_read16<3 * 2048>(ac, af[3]); break;
+        case 1: dn_read16<0>(an, af[0]); break;
+        case 2: dn_read16<2048>(an, af[1]); break;
+        case 3: dn_read16<2 * 2048>(an, af[2]); break;
       }
       if (i >= ib && i <= ib + 2)
-        dn_wait<3 + NJ>(af[i & 3]);
+        dn_wait<5>(af[i]);
       else
-        dn_wait<3>(af[i & 3]);
+        dn_wait<3>(af[i]);
       if (i == 0) {
         // the B operands of this step were requested before A0 was
 #pragma unroll
-        for (int j = 0; j < NJ; j++) asm volatile("" : "+v"(w[h][j]));
+        for (int j = 0; j < 2; j++) asm volatile("" : "+v"(w[h][j]));
       }
-      const h8 a = __builtin_bit_cast(h8, af[i & 3]);
+      const h8 a = __builtin_bit_cast(h8, af[i]);
 #pragma unroll
-      for (int j = 0; j < NJ; j++)
+      for (int j = 0; j < 2; j++)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, w[h][j]), a,
                                                            acc[i][j], 0, 0, 0);
     }
@@ -343,8 +519,8 @@ __global__ __launch_bounds__(512) void dense_kernel(DenseArgs p) {
 
   int slot = 0;  // ring slot of the stage being computed
   for (int s = 0; s < stages; s++) {
-    const int slot_next = slot == kRing - 1 ? 0 : slot + 1;
-    const unsigned cur = slot * kDnSlab, nxt = slot_next * kDnSlab;
+    const int slot_next = slot == Sh::kRing - 1 ? 0 : slot + 1;
+    const unsigned cur = slot * Sh::kSlab, nxt = slot_next * Sh::kSlab;
     kstep(std::integral_constant<int, 0>{}, cur, nxt, s, slot);
     kstep(std::integral_constant<int, 1>{}, cur, nxt, s, slot);
     slot = slot_next;
@@ -360,93 +536,70 @@ __global__ __launch_bounds__(512) void dense_kernel(DenseArgs p) {
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
 
-  // ---- slices of other workgroups: every slice writes its fp32 tile through
-  // to memory (whole 1 KiB lines per wave instruction), waits for the
-  // acknowledgement and takes the tile's ticket; the last arrival adds all
-  // slices in slice order (its own from registers at its place in that order).
-  if (ksplit > 1) {
-    const __amdgpu_buffer_rsrc_t rP = dn_rsrc(p.scratch, 0x7fffffffu);
-    const int at = (wave * (RB * NJ) * 64 + lane) * 16;
-    const int mine = work * kPart;
-#pragma unroll
-    for (int i = 0; i < RB; i++)
-#pragma unroll
-      for (int j = 0; j < NJ; j++)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, acc[i][j]), rP,
-                                               at + (i * NJ + j) * 1024, mine, 16 /* sc1 */);
-    __builtin_amdgcn_s_waitcnt(dn_vmcnt(0));  // my stores have been acknowledged
-    __syncthreads();
-    const int sk_tile = tile - p.dp_tiles;
-    if (tid == 0)
-      s_ticket = __hip_atomic_fetch_add(&p.locks[sk_tile], 1, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (s_ticket != ksplit - 1) return;  // a later slice finishes the tile
-    // one row block at a time: the other slices' values are requested
-    // together, then added in slice order with my own at its place
-#pragma unroll
-    for (int i = 0; i < RB; i++) {
-      f4 v[kDnMaxSlices][NJ];
-#pragma unroll
-      for (int k2 = 0; k2 < kDnMaxSlices; k2++) {
-        const int theirs = (sk_tile * ksplit + k2) * kPart;
-        const int inv = (k2 < ksplit && k2 != ks) ? 0 : kDnOob;  // no traffic for the rest
-#pragma unroll
-        for (int j = 0; j < NJ; j++)
-          v[k2][j] = __builtin_bit_cast(
-              f4, __builtin_amdgcn_raw_buffer_load_b128(rP, (at + (i * NJ + j) * 1024) | inv,
-                                                        theirs, 16 /* sc1 */));
-      }
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        f4 sum = (ks == 0) ? acc[i][j] : v[0][j];
-#pragma unroll
-        for (int k2 = 1; k2 < kDnMaxSlices; k2++)
-          if (k2 < ksplit) sum += (k2 == ks) ? acc[i][j] : v[k2][j];
-        acc[i][j] = sum;
-      }
-    }
-    if (tid == 0)  // counters are handed back zeroed
-      __hip_atomic_store(&p.locks[sk_tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // a lane holds, per (i, j), row 16i + nu and four consecutive columns
+  char* const out = smem + (64 * wm + nu) * Sh::kPitch + (32 * wn + 4 * (lane >> 4)) * 2;
+  half_t* const C = (half_t*)p.C + (size_t)m0 * p.N + n0;
+  if (!CUT || ksplit == 1) {
+    dense_write_tile<128, 128, Sh::kPitch, 512, 4, 2>(smem, out, C, p.N, rows,
+                                                      [&](int i, int j) { return acc[i][j]; });
+    return;
   }
 
-  // ---- C: a lane holds, per (i, j), row 16i + nu and four consecutive
-  // columns.  The fp16 tile goes through LDS (the slabs are dead), one half of
-  // its rows at a time, and leaves as whole rows (512 or 256 bytes) with
-  // 16-byte stores; 8-byte stores straight from the registers cost 13 us more
-  // at 4096^3.
-  constexpr int kPitch = TN * 2 + 16;  // bytes per tile row in LDS
-  constexpr int HR = TM / 2;           // rows of a half
-  constexpr int PR = TN / 8;           // 16-byte pieces of a row
-  static_assert(HR * kPitch <= kDnLds, "");
-  half_t* C = (half_t*)p.C;
-  const int q = lane >> 4;
+  // ---- slices of other workgroups: every slice writes the fp32 sums that
+  // others will add up through to memory (whole 1 KiB lines per wave
+  // instruction), waits for the acknowledgement and arrives; the slices then
+  // finish the tile together, each its share of the tile's eight pieces (one (i,
+  // j) of every wave), all slices added in slice order.
+  const __amdgpu_buffer_rsrc_t rP = dn_rsrc(p.scratch, 0x7fffffffu);
+  int* const word = &p.locks[cut * kDnCounterStride];
+  const int at = wave * (8 * 1024) + lane * 16;
+  const auto write_out = [&](int which) {
 #pragma unroll
-  for (int hlf = 0; hlf < 2; hlf++) {
+    for (int e = 0; e < 8; e++)
+      if (which >> e & 1)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, acc[e >> 1][e & 1]), rP,
+                                               at + e * 1024, (cut * ksplit + ks) * Sh::kPartBytes,
+                                               16 /* sc1 */);
+    __builtin_amdgcn_s_waitcnt(dn_vmcnt(0));  // my stores have been acknowledged
     __syncthreads();
-    if (wm == hlf) {
-#pragma unroll
-      for (int i = 0; i < RB; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-          const h4 o = {(half_t)acc[i][j][0], (half_t)acc[i][j][1], (half_t)acc[i][j][2],
-                        (half_t)acc[i][j][3]};
-          *(h4*)(smem + (16 * i + nu) * kPitch + (16 * NJ * wn + 16 * j + 4 * q) * 2) = o;
-        }
-    }
+  };
+  const int my_share = finish_pieces(1 << ks, ksplit, 8);
+  write_out(0xff & ~my_share);
+  if (tid == 0) s_shares = finish_arrive(word, ksplit, ks, p.finish_polls);
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(s_shares) == 0) {
+    write_out(my_share);
+    if (tid == 0) s_shares = finish_abandon(word, ksplit, ks);
     __syncthreads();
-#pragma unroll
-    for (int it = 0; it < HR * PR / 512; it++) {
-      const int piece = it * 512 + tid;  // 16-byte piece of the half tile
-      const int r = piece / PR, c16 = piece % PR;
-      const int m = HR * hlf + r;
-      if (m < rows) {
-        const i4 v = *(const i4*)(smem + r * kPitch + c16 * 16);
-        // nobody reads C again in this launch: keep it out of the way of A and B in L2
-        __builtin_nontemporal_store(v, (i4*)(C + (size_t)(m0 + m) * p.N + n0 + c16 * 8));
-      }
-    }
   }
+  const int pieces = __builtin_amdgcn_readfirstlane(finish_pieces(s_shares, ksplit, 8));
+  f4 v[8][kDnMaxSlices - 1];  // all of my pieces requested at once
+#pragma unroll
+  for (int e = 0; e < 8; e++)
+    if (pieces >> e & 1)
+#pragma unroll
+      for (int x = 0; x < kDnMaxSlices - 1; x++) {
+        const int k2 = x < ks ? x : x + 1;
+        if (k2 < ksplit)
+          v[e][x] = __builtin_bit_cast(
+              f4, __builtin_amdgcn_raw_buffer_load_b128(rP, at + e * 1024,
+                                                        (cut * ksplit + k2) * Sh::kPartBytes, 16 /* sc1 */));
+      }
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    if (!(pieces >> e & 1)) continue;
+    const f4 own = acc[e >> 1][e & 1];
+    f4 sum = ks == 0 ? own : v[e][0];
+#pragma unroll
+    for (int k2 = 1; k2 < kDnMaxSlices; k2++)
+      if (k2 < ksplit) sum += k2 == ks ? own : k2 < ks ? v[e][k2 % (kDnMaxSlices - 1)] : v[e][k2 - 1];
+    *(h4*)(out + 16 * (e >> 1) * Sh::kPitch + 32 * (e & 1)) = dense_round(sum);
+  }
+  __syncthreads();
+  // (row 64 (m / 64) + 16 i + ..., operand 2 (c / 2) + j)
+  dense_store_tile<128, 128, Sh::kPitch, 512>(
+      smem, C, p.N, rows, [&](int m, int c) { return pieces >> (2 * ((m >> 4) & 3) + (c & 1)) & 1; });
+  if (tid == 0) finish_leave(word, ksplit);
 }
 
 // C = 0 for an empty k range (a kernel rather than a memset, so that the call
@@ -468,6 +621,7 @@ using namespace w4a16;
 constexpr int kDnMaxDevices = 16;
 
 thread_local char g_dn_error[256] = "";
+thread_local int t_finish_polls = -1;  // streamk_amd_force_finish_polls
 
 void dn_set_error(hipError_t e, const char* what) {
   snprintf(g_dn_error, sizeof(g_dn_error), "%s: %s", what, hipGetErrorString(e));
@@ -582,17 +736,17 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
       }
       cus = d.cus;
       if (!d.configured) {
-        e = hipFuncSetAttribute((const void*)dense_kernel<256, 256>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                DnShape<256, 256>::kLds);
+        e = hipFuncSetAttribute((const void*)dense_kernel<256>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, DnShape<256>::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_kernel<128, 256>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  DnShape<128, 256>::kLds);
+          e = hipFuncSetAttribute((const void*)dense_kernel<128>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnShape<128>::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_kernel<128, 128>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  DnShape<128, 128>::kLds);
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<false>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<true>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
         if (e != hipSuccess) {
           dn_set_error(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
           break;
@@ -601,11 +755,23 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
       }
     }
     const DnPlan pl = dn_plan(m, n, k, cus);
-    // only a launch with stream-K tiles exchanges anything
+    // The stream-K tiles of large tiles are computed as 128 x 128 quarters in a
+    // launch of their own, in slices while that leaves compute units idle: 16
+    // tiles of 256 x 256 in four slices are 64 workgroups, a quarter of the chip
+    // for a quarter of a tile's time, their quarters 256 (4096 x 4352 x 4096
+    // 142 us with one launch for both, 125 with two; 6230 x 3072 x 1280 67 and 52).
+    const bool small = pl.tile_cols == 128;
+    const bool quarters = !small && pl.sk_tiles > 0;
+    const int cut_tiles = quarters ? 4 * pl.sk_tiles : pl.sk_tiles;
+    int slices = pl.ksplit;
+    if (quarters) {
+      if (slices > cus / cut_tiles) slices = cus / cut_tiles;
+      if (slices < 1) slices = 1;
+    }
+    // only slices exchange anything
     ScratchView view = {nullptr, nullptr};
-    if (pl.sk_tiles > 0 &&
-        !scratch_acquire(dev, stream,
-                         (size_t)pl.sk_tiles * pl.ksplit * pl.tile_rows * pl.tile_cols * 4, &view,
+    if (cut_tiles > 0 && slices > 1 &&
+        !scratch_acquire(dev, stream, (size_t)cut_tiles * slices * DnSmall::kPartBytes, &view,
                          g_dn_error, sizeof(g_dn_error)))
       break;
     (void)hipGetLastError();  // an earlier call's error is not this launch's
@@ -616,23 +782,28 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     a.M = m;
     a.N = n;
     a.K = k;
-    a.tile_rows = pl.tile_rows;
-    a.tile_cols = pl.tile_cols;
     a.tiles_m = pl.tiles_m;
     a.tiles_n = pl.tiles_n;
     a.dp_tiles = pl.dp_tiles;
-    a.sk_tiles = pl.sk_tiles;
-    a.ksplit = pl.ksplit;
+    a.sk_tiles = cut_tiles;
+    a.ksplit = slices;
+    a.quarters = quarters ? 1 : 0;
+    a.slices_only = quarters || pl.dp_tiles == 0 ? 1 : 0;
     a.locks = view.counters;
     a.scratch = view.partials;
-    constexpr int lds_small = DnShape<128, 128>::kLds, lds_half = DnShape<128, 256>::kLds,
-                  lds_large = DnShape<256, 256>::kLds;
-    if (pl.tile_cols == 128)
-      hipLaunchKernelGGL((dense_kernel<128, 128>), dim3(pl.grid), dim3(512), lds_small, stream, a);
-    else if (pl.tile_rows == 128)
-      hipLaunchKernelGGL((dense_kernel<128, 256>), dim3(pl.grid), dim3(512), lds_half, stream, a);
-    else
-      hipLaunchKernelGGL((dense_kernel<256, 256>), dim3(pl.grid), dim3(512), lds_large, stream, a);
+    a.finish_polls = t_finish_polls < 0 ? kFinishPolls : t_finish_polls;
+    constexpr int lds_small = DnSmall::kLds, lds_half = DnShape<128>::kLds, lds_large = DnShape<256>::kLds;
+    if (cut_tiles > 0)
+      hipLaunchKernelGGL(dense_small_kernel<true>, dim3((small ? pl.dp_tiles : 0) + cut_tiles * slices),
+                         dim3(512), lds_small, stream, a);
+    else if (small)
+      hipLaunchKernelGGL(dense_small_kernel<false>, dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
+    if (!small && pl.dp_tiles > 0) {
+      if (pl.tile_rows == 128)
+        hipLaunchKernelGGL(dense_kernel<128>, dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
+      else
+        hipLaunchKernelGGL(dense_kernel<256>, dim3(pl.dp_tiles), dim3(256), lds_large, stream, a);
+    }
     e = hipGetLastError();
     if (e != hipSuccess) {
       dn_set_error(e, "kernel launch");
@@ -663,6 +834,10 @@ int streamk_amd_plan(int m, int n, int k, int cus, int* out) {
 
 void streamk_amd_tile_coord(int tile, int tiles_m, int tiles_n, int* out) {
   dn_tile_coord(tile, tiles_m, tiles_n, &out[0], &out[1]);
+}
+
+void streamk_amd_force_finish_polls(int polls) {
+  t_finish_polls = polls < 0 || polls > kFinishPolls ? -1 : polls;
 }
 
 long long streamk_amd_release(int dev) { return (long long)scratch_release(dev); }

@@ -13,6 +13,8 @@ _lib.streamk_amd_plan.restype = _I
 _lib.streamk_amd_plan.argtypes = [_I, _I, _I, _I, _P]
 _lib.streamk_amd_tile_coord.restype = None
 _lib.streamk_amd_tile_coord.argtypes = [_I, _I, _I, _P]
+_lib.streamk_amd_force_finish_polls.restype = None
+_lib.streamk_amd_force_finish_polls.argtypes = [_I]
 _lib.streamk_amd_last_error.restype = ctypes.c_char_p
 
 
@@ -34,6 +36,12 @@ def tile_coord(tile, tiles_m, tiles_n):
     out = (ctypes.c_int * 2)()
     _lib.streamk_amd_tile_coord(tile, tiles_m, tiles_n, out)
     return out[0], out[1]
+
+
+def force_finish_polls(polls):
+    """How often a workgroup looks for the other slices of its tile before it leaves them its
+    share of the sums; -1 = the default (calling thread only)."""
+    _lib.streamk_amd_force_finish_polls(int(polls))
 
 
 def gemm(A, B, C=None):

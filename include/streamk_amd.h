@@ -26,8 +26,8 @@ extern "C" {
  * fp32 accumulation.  m is arbitrary; n % 256 == 0 and k % 64 == 0.
  * Partial sums of the stream-K tiles live in the library-owned buffer of this
  * (device, stream) that marlin_gemm uses too (include/marlin_amd.h): sized by
- * the launch (tile rows x tile columns x 4 bytes per slice of a stream-K tile), grown on demand, none for
- * launches without stream-K tiles.  Calls on one stream may follow each other
+ * the launch (64 KiB per slice of a 128 x 128 tile), grown on demand, none for
+ * launches without slices.  Calls on one stream may follow each other
  * freely, calls that overlap must use different streams; a call that would have
  * to allocate under graph capture returns STREAMK_ERR_RUNTIME. */
 int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, int dev,
@@ -39,8 +39,10 @@ int streamk_amd_check(int m, int n, int k);
 /* the tile split for a device with `cus` compute units (counterpart of
  * SK_DP_Block_Wrapper, dp_sk_block.h:31-80): out[0..7] = tiles along m, tiles
  * along n (tiles numbered in panels of 8 column tiles), data-parallel tiles, stream-K
- * tiles (the last ones in tile order), k slices per stream-K tile, workgroups,
- * rows of a tile (256, or 128 when 256 x 256 tiles would occupy at most half
+ * tiles (the last ones in tile order), k slices per stream-K tile, (tile, slice)
+ * pairs (workgroups, except that the stream-K tiles of 256 x 256 are computed as
+ * four 128 x 128 quarters each, in as many slices as leave none without a
+ * compute unit), rows of a tile (256, or 128 when 256 x 256 tiles would occupy at most half
  * of the compute units), columns of a tile (256, or 128 when 128 x 256 tiles
  * would occupy at most half of them too) */
 int streamk_amd_plan(int m, int n, int k, int cus, int* out);
@@ -48,6 +50,11 @@ int streamk_amd_plan(int m, int n, int k, int cus, int* out);
 /* out[0], out[1] = row and column tile of tile number `tile` (0 <= tile <
  * tiles_m * tiles_n); for tests of the numbering */
 void streamk_amd_tile_coord(int tile, int tiles_m, int tiles_n, int* out);
+
+/* how often a workgroup looks whether the other slices of its tile have arrived
+ * before it leaves them its share of the sums, for the calling thread: -1 = the
+ * default, 0 = at once; for tests (results do not depend on it) */
+void streamk_amd_force_finish_polls(int polls);
 
 /* same as marlin_amd_release (include/marlin_amd.h): frees the partial-sum
  * buffers of device dev (all if dev < 0), returns the bytes freed */

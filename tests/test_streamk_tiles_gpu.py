@@ -1,0 +1,65 @@
+"""GPU tests of the dense GEMM's kernels at the edges of their tiles, stages and
+slices.  Operands are whole numbers in [-2, 2] and at most 448 deep, so every sum
+stays below 2048 in magnitude and is exact in fp16 and in any order of addition:
+the result is torch's fp32 product, bit for bit.  (Deeper sums, for slices, use
+{-1, 0, 1}.)"""
+import os
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "awesome-cute_amd"))
+
+
+@pytest.fixture(scope="module")
+def env():
+    import torch
+    import streamk
+    assert torch.cuda.is_available()
+    return torch, streamk
+
+
+def _check(env, m, n, k, top, tile):
+    torch, streamk = env
+    _, plan = streamk.plan(m, n, k)
+    assert (plan["tile_rows"], plan["tile_cols"]) == tile
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(m + n + k)
+    A, B = (torch.randint(-top, top + 1, (r, k), device="cuda:0", generator=gen).half() for r in (m, n))
+    C = torch.full((m + 1, n), 7.0, dtype=torch.half, device="cuda:0")
+    streamk.gemm(A, B, C[:m])
+    want = A.float() @ B.float().t()
+    torch.cuda.synchronize()
+    assert want.abs().max().item() < 2048
+    assert torch.equal(C[:m].float(), want)
+    assert (C[m] == 7.0).all()  # nothing past the last row
+    return plan
+
+
+# one stage to seven: every place where the loops of two and of six slabs are left
+@pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("m,n,tile", [(1281, 8192, (256, 256)), (1535, 6400, (256, 256)), (601, 8192, (128, 256)),
+                                      (767, 5632, (128, 256)), (1, 256, (128, 128)), (300, 1024, (128, 128))])
+def test_stages(env, m, n, stages, tile):
+    _check(env, m, n, 64 * stages, 2, tile)
+
+
+@pytest.mark.parametrize("polls", [-1, 0, 1])  # 0 and 1: shares left to the last arrival
+@pytest.mark.parametrize("m,n,k,tile", [
+    (2049, 8192, 1024, (256, 256)),   # 32 stream-K tiles in quarters, most of them with one row or none
+    (2100, 8192, 1088, (256, 256)),   # ... 52 rows; slices of unequal length
+    (4000, 4352, 832, (256, 256)),    # 16 tiles, 64 quarters, up to three slices
+    (129, 256, 512, (128, 128)), (300, 1280, 768, (128, 128)), (128, 512, 1216, (128, 128)),
+    (5000, 512, 576, (128, 128)),     # whole tiles only
+])
+def test_slices(env, m, n, k, tile, polls):
+    torch, streamk = env
+    streamk.force_finish_polls(polls)
+    try:
+        for _ in range(2):
+            _check(env, m, n, k, 1, tile)
+    finally:
+        streamk.force_finish_polls(-1)
