@@ -8,14 +8,16 @@
 // about 2.5: one row through the sixteen layers of four blocks of a 7B model
 // 200 -> 121 us, which is the kernels' time.
 //
-// The library is entered with the interpreter lock released, as through ctypes:
-// a launch may wait for room in the stream's queue, and a stream's first call
-// allocates.
+// Tensors are allocated and the library is entered with the interpreter lock
+// released, as torch's own calls and ctypes do: a launch may wait for room in
+// the stream's queue, a stream's first call allocates, and an allocation may
+// wait for another thread's.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
 
 #include "../../include/marlin_amd.h"
 #include "../../include/streamk_amd.h"
@@ -130,12 +132,14 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t n = s->size(1), k = A->size(-1);
   c10::SmallVector<int64_t, 6> shape(A->sizes().begin(), A->sizes().end());
   shape.back() = n;
-  at::Tensor C = at::empty(shape, A->options().requires_grad(false).memory_format(c10::nullopt));
-  at::Tensor rows;  // (a copy where the leading dimensions do not fold into one)
-  if (!A->is_contiguous() || k == 0) {
-    rows = A->reshape({-1, k});
-    A = &rows;
+  at::Tensor C, rows;
+  {
+    pybind11::gil_scoped_release unlocked;
+    C = at::empty(shape, A->options().requires_grad(false).memory_format(c10::nullopt));
+    // (a copy where the leading dimensions do not fold into one)
+    if (!A->is_contiguous() || k == 0) rows = A->reshape({-1, k});
   }
+  if (rows.defined()) A = &rows;
   const at::Tensor* const t[kMulTensors] = {A, B, &C, s, workspace};
   if (!check_mul(t)) return nullptr;
   if (!enqueue_mul(*A, *B, C, *s, *workspace, A->numel() / k, n, k, h)) return nullptr;
@@ -168,6 +172,7 @@ PyObject* py_dense(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
   at::Tensor C;
   if (args[2] == Py_None) {
+    pybind11::gil_scoped_release unlocked;
     C = at::empty({m, n}, A.options().requires_grad(false));
   } else {
     const at::Tensor* c = tensor(args[2], "C");

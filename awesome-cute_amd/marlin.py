@@ -141,14 +141,23 @@ _block_gather = torch.from_numpy((64 * _k_in_block + _n_in_block).reshape(-1).as
 # kernels read them; the tensor operations beside them serve every other device,
 # type and layout, and give the same bits.
 
+def _looked_on():
+    """Whether something wants to see the tensor operations themselves: a compiler, a tracer, a
+    dispatch mode, a function transform (vmap, grad, jvp) or forward-mode differentiation."""
+    return (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() != 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _on_gpu(*tensors):
-    """Whether the kernels may take these tensors: plain, on one GPU, 16-byte aligned, and no
-    compiler or autograd looking on."""
+    """Whether the kernels may take these tensors: plain, on one GPU, 16-byte aligned, without
+    gradients, and nothing looking on."""
     dev = tensors[0].device
-    return (dev.type == "cuda" and not torch.compiler.is_compiling()
+    return (dev.type == "cuda" and not _looked_on()
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
             and all(t.device == dev and type(t) in (torch.Tensor, nn.Parameter)
-                    and t.data_ptr() % 16 == 0 for t in tensors))
+                    and not t.is_neg() and t.data_ptr() % 16 == 0 for t in tensors))
 
 
 def _convert_check(rc):
@@ -240,8 +249,11 @@ class Layer(nn.Module):
         if not torch.compiler.is_compiling():
             # (the buffers by name: as attributes each costs a Python call)
             held = self._buffers
-            return _torch_binding.linear(A, held['B'], held['s'], held['workspace'],
-                                         self.cute_version)
+            try:
+                B, s, workspace = held['B'], held['s'], held['workspace']
+            except KeyError:  # made a parameter, or computed by a parametrisation
+                B, s, workspace = self.B, self.s, self.workspace
+            return _torch_binding.linear(A, B, s, workspace, self.cute_version)
         C = torch.empty(A.shape[:-1] + (self.s.shape[1],), dtype=A.dtype, device=A.device)
         mul(A.reshape((-1, A.shape[-1])), self.B, C.view((-1, C.shape[-1])), self.s,
             self.workspace, cute_version=self.cute_version)
@@ -255,15 +267,23 @@ class Layer(nn.Module):
         s = scales.t()                 # (groups, n)
         w = linear.weight.data.t()     # (k, n)
         groupwise = self.groupsize != self.k
-        if (s.dtype == torch.half and s.shape == self.s.shape and w.shape == (self.k, self.n)
+        B, packed = self.B, self.s
+        if (s.dtype == packed.dtype == torch.half and B.dtype == torch.int32
+                and s.shape == packed.shape == (self.k // self.groupsize, self.n)
+                and B.shape == (self.k // 16, 2 * self.n) and w.shape == (self.k, self.n)
                 and (w.is_contiguous() or w.t().is_contiguous())
-                and self.B.is_contiguous() and self.s.is_contiguous()
-                and _on_gpu(w, self.B, self.s) and s.device == w.device and not s.requires_grad):
+                and B.is_contiguous() and packed.is_contiguous()
+                and _on_gpu(w, B, packed) and s.device == w.device
+                and type(s) in (torch.Tensor, nn.Parameter) and not s.requires_grad
+                and not s.is_neg()):
             dev = w.get_device()
             _convert_check(_lib.marlin_amd_pack(
                 w.data_ptr(), self.k, self.n, self.groupsize if groupwise else -1,
-                not w.is_contiguous(), s.data_ptr(), s.stride(0), s.stride(1), self.B.data_ptr(),
-                self.s.data_ptr(), dev, _raw_stream(dev)))
+                not w.is_contiguous(), s.data_ptr(), s.stride(0), s.stride(1), B.data_ptr(),
+                packed.data_ptr(), dev, _raw_stream(dev)))
+            # written in place, as an assignment to them would be
+            torch.autograd.graph.increment_version(
+                [t for t in (B, packed) if not t.is_inference()])
             return
         s_full = s.repeat_interleave(self.groupsize, dim=0) if groupwise else s
         q = torch.clamp(torch.round(w / s_full).int() + 8, 0, 15)

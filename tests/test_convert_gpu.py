@@ -90,3 +90,39 @@ def test_packed_integers(env, k, n):
     assert torch.equal(marlin.pack_weights(q).cpu(), want)
     assert torch.equal(marlin.pack_weights(q.t().contiguous().t()).cpu(), want)  # other layouts and types
     assert torch.equal(marlin.pack_weights(q.to(torch.int64)).cpu(), want)
+
+
+def test_what_looks_on_sees_the_tensor_operations(env):
+    torch, marlin = env
+    import torch.autograd.forward_ad as forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    w = torch.randn((3, 256, 64), device="cuda:0").half()
+    want = [torch.stack(x) for x in zip(*(_quantise(torch, x, 128) for x in w))]
+    for got, expected in zip(torch.vmap(lambda x: marlin.quantize(x, 128))(w), want):
+        _same(torch, got, expected)
+    graph = make_fx(lambda x: marlin.quantize(x, 128))(w[0])  # traced on one weight, run on another
+    for got, expected in zip(graph(w[1]), want):
+        _same(torch, got, expected[1])
+    with forward_ad.dual_level():
+        fake, _, s = marlin.quantize(forward_ad.make_dual(w[0], torch.ones_like(w[0])), 128)
+        assert forward_ad.unpack_dual(fake).tangent is not None
+        assert forward_ad.unpack_dual(s).tangent is not None
+
+
+def test_layers_whose_buffers_were_changed(env):
+    torch, marlin = env
+    k, n = 256, 512
+    fake, _, s = marlin.quantize(torch.randn((k, n), device="cuda:0").half() * 0.02, 128)
+    linear = torch.nn.Linear(k, n, bias=False, device="cuda:0", dtype=torch.half)
+    linear.weight.data = fake.t()
+    layer = marlin.Layer(k, n, 128).to("cuda:0")
+    versions = layer.B._version, layer.s._version
+    layer.pack(linear, s.t())
+    assert layer.B._version > versions[0] and layer.s._version > versions[1]
+    wide = marlin.Layer(k, n, 128).to("cuda:0").float()  # scales held in 32 bits
+    wide.pack(linear, s.t())
+    assert torch.equal(wide.s, layer.s.float()) and torch.equal(wide.B, layer.B)
+    x = torch.randn((3, k), device="cuda:0").half()
+    y = layer(x)
+    layer.B = torch.nn.Parameter(layer.B, requires_grad=False)  # a parameter in the buffer's place
+    assert torch.equal(layer(x), y)
