@@ -12,8 +12,8 @@
 // to memory, takes a ticket, and the last arrival adds all slices in slice
 // order and writes C.
 //
-// Whole tiles, 256 x 256 or (too few of them for the compute units) 128 x 256:
-// dense_kernel.  A workgroup of four waves, one per SIMD, each with a 128 x 128
+// Whole tiles, 256 x 256 or (too few of them for the compute units) 128 x 256,
+// and 128 x 256 in two slices where k is deep: dense_kernel.  A workgroup of four waves, one per SIMD, each with a 128 x 128
 // fp32 accumulator (all 256 AGPRs): a wave per quarter of the tile, or two
 // waves per 128 columns, each taking every other k step, their sums added
 // through LDS at the end.  The main loop is one assembly statement per tile
@@ -75,6 +75,7 @@ struct DnShape {
   static constexpr int kPitch = 256 * 2 + 16;   // bytes per row of the fp16 tile in LDS
   static constexpr int kRingBytes = kRing * kSlab, kTileBytes = TM * kPitch;
   static constexpr int kLds = kRingBytes > kTileBytes ? kRingBytes : kTileBytes;
+  static constexpr int kPartBytes = TM * 256 * 4;
   static_assert(kWK == 1 || kLds >= 128 * 1024, "room for the sums that waves hand each other");
 };
 // 128 x 128 tiles (dense_small_kernel)
@@ -89,6 +90,7 @@ struct DnSmall {
 };
 constexpr int kDnMaxSlots = 256;  // slices in flight per launch
 constexpr int kDnMaxSlices = 4;
+constexpr int kDnPairK = 7168;    // depth from which 128 x 256 tiles in two slices beat 128 x 128 ones
 constexpr int kDnCounterStride = 16;  // ints: a tile's slices meet in a cache line of their own
 
 struct DenseArgs {
@@ -246,8 +248,11 @@ __device__ __forceinline__ h4 dense_round(f4 v) {
   return (h4){(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
 }
 
-template <int TM>
+// SLICED (128 rows): every tile is cut into p.ksplit slices of the k range,
+// which finish it together.
+template <int TM, bool SLICED>
 __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
+  static_assert(!SLICED || TM == 128, "");
   extern __shared__ __attribute__((aligned(16))) char smem[];  // DnShape<TM>::kLds
   using Shape = DnShape<TM>;
   constexpr int WK = Shape::kWK, NF = Shape::kNF, TA = Shape::kTA, TB = Shape::kTB;
@@ -261,15 +266,26 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
   const int wk = WK == 1 ? 0 : wave >> 1;  // which of the k steps
 
   // every XCD gets a contiguous run of tile numbers (a placement hint only)
-  const int tile = xcd_work_index((int)blockIdx.x, p.dp_tiles);
+  // (neighbouring tiles of one k range, so that they share rows of A and B)
+  const int work = xcd_work_index((int)blockIdx.x, SLICED ? p.dp_tiles * p.ksplit : p.dp_tiles);
+  const int ks = SLICED ? work / p.dp_tiles : 0;
+  const int tile = SLICED ? work - ks * p.dp_tiles : work;
   int tm, tn;
   dn_tile_coord(tile, p.tiles_m, p.tiles_n, &tm, &tn);
   const int m0 = tm * TM;
   const int n0 = tn * 256;
   const int rows = min(TM, p.M - m0);
 
-  i4 ra_words = dn_rsrc_words((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
-  i4 rb_words = dn_rsrc_words((const char*)p.B + (size_t)n0 * p.K * 2, 256u * (unsigned)p.K * 2u);
+  // this workgroup's slabs [first, last) of the K/64
+  const int slabs_all = p.K / kDnStageK;
+  const int first = SLICED ? (int)((unsigned)ks * (unsigned)slabs_all / (unsigned)p.ksplit) : 0;
+  const int last =
+      SLICED ? (int)((unsigned)(ks + 1) * (unsigned)slabs_all / (unsigned)p.ksplit) : slabs_all;
+  const int skip = first * (kDnStageK * 2);  // bytes of a row before them
+  i4 ra_words = dn_rsrc_words((const char*)p.A + (size_t)m0 * p.K * 2 + skip,
+                              (unsigned)rows * (unsigned)p.K * 2u - (unsigned)skip);
+  i4 rb_words = dn_rsrc_words((const char*)p.B + (size_t)n0 * p.K * 2 + skip,
+                              256u * (unsigned)p.K * 2u - (unsigned)skip);
 
   // wave w fetches the w-th quarter of the A rows and of the B rows of a slab,
   // eight rows per instruction: lane (r = lane/8, c = lane%8) lands at [r][c] and
@@ -285,7 +301,7 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
       src[t] = r * p.K * 2 + 16 * c;
     }
   }
-  const int slabs = p.K / kDnStageK;
+  const int slabs = last - first;
   int s_at = 0;  // byte offset of the next slab to request
 
   // LDS: where this wave's loads of slot 0 go, and where its operand reads of
@@ -348,8 +364,68 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
     else
       add_up(std::integral_constant<int, NF>{});
     __syncthreads();
-    dense_write_tile<TM, 256, kPitch, 256, NF, 8>(smem, out, C, p.N, rows,
-                                                  [&](int i, int o) { return fin[i][o]; });
+    if constexpr (!SLICED) {
+      dense_write_tile<TM, 256, kPitch, 256, NF, 8>(smem, out, C, p.N, rows,
+                                                    [&](int i, int o) { return fin[i][o]; });
+    } else {
+      // as in dense_small_kernel, with eight pieces of half the columns of a row
+      // block (operands 4 (e % 2) ... + 3 of block e / 2 of every wave)
+      __shared__ int s_shares;
+      const __amdgpu_buffer_rsrc_t rP = dn_rsrc(p.scratch, 0x7fffffffu);
+      int* const word = &p.locks[tile * kDnCounterStride];
+      const int at = wave * (NF * 8 * 1024) + lane * 16;
+      const auto part = [&](int k2) { return (tile * p.ksplit + k2) * Shape::kPartBytes; };
+      const auto write_out = [&](int which) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          if (!(which >> e & 1)) continue;
+#pragma unroll
+          for (int o = 4 * (e & 1); o < 4 * (e & 1) + 4; o++)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, fin[e >> 1][o]), rP,
+                                                   at + (8 * (e >> 1) + o) * 1024, part(ks), 16 /* sc1 */);
+        }
+        __builtin_amdgcn_s_waitcnt(dn_vmcnt(0));  // my stores have been acknowledged
+        __syncthreads();
+      };
+      const int my_share = finish_pieces(1 << ks, p.ksplit, 8);
+      write_out(0xff & ~my_share);
+      if (tid == 0) s_shares = finish_arrive(word, p.ksplit, ks, p.finish_polls);
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(s_shares) == 0) {
+        write_out(my_share);
+        if (tid == 0) s_shares = finish_abandon(word, p.ksplit, ks);
+        __syncthreads();
+      }
+      const int pieces = __builtin_amdgcn_readfirstlane(finish_pieces(s_shares, p.ksplit, 8));
+      // two slices: the other one's sums of half my pieces requested at once
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        f4 v[4][4];
+#pragma unroll
+        for (int e = 4 * h; e < 4 * h + 4; e++) {
+          if (!(pieces >> e & 1)) continue;
+#pragma unroll
+          for (int o = 0; o < 4; o++)
+            v[e & 3][o] = __builtin_bit_cast(
+                f4, __builtin_amdgcn_raw_buffer_load_b128(
+                        rP, at + (8 * (e >> 1) + 4 * (e & 1) + o) * 1024, part(1 - ks), 16 /* sc1 */));
+        }
+#pragma unroll
+        for (int e = 4 * h; e < 4 * h + 4; e++) {
+          if (!(pieces >> e & 1)) continue;
+#pragma unroll
+          for (int o = 0; o < 4; o++)  // (a sum of two does not depend on their order)
+            *(h4*)(out + 16 * (e >> 1) * kPitch + 32 * (4 * (e & 1) + o)) =
+                dense_round(fin[e >> 1][4 * (e & 1) + o] + v[e & 3][o]);
+        }
+      }
+      __syncthreads();
+      // (row 64 (m / 64) + 16 i + ..., operand c % 8 of its wave)
+      dense_store_tile<TM, 256, kPitch, 256>(smem, C, p.N, rows, [&](int m, int c) {
+        return pieces >> (2 * ((m >> 4) & 3) + ((c >> 2) & 1)) & 1;
+      });
+      if (tid == 0) finish_leave(word, p.ksplit);
+    }
   }
 }
 
@@ -736,10 +812,13 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
       }
       cus = d.cus;
       if (!d.configured) {
-        e = hipFuncSetAttribute((const void*)dense_kernel<256>,
+        e = hipFuncSetAttribute((const void*)dense_kernel<256, false>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, DnShape<256>::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_kernel<128>,
+          e = hipFuncSetAttribute((const void*)dense_kernel<128, false>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnShape<128>::kLds);
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute((const void*)dense_kernel<128, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, DnShape<128>::kLds);
         if (e == hipSuccess)
           e = hipFuncSetAttribute((const void*)dense_small_kernel<false>,
@@ -774,6 +853,22 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
         !scratch_acquire(dev, stream, (size_t)cut_tiles * slices * DnSmall::kPartBytes, &view,
                          g_dn_error, sizeof(g_dn_error)))
       break;
+    // Problems of 128 x 128 tiles for more than half of the compute units, one
+    // workgroup each, wait for operands: a tile of 128 x 256 brings half as many
+    // rows of A per column, so in two slices along k the same workgroups take
+    // in three quarters of the bytes and run dense_kernel's loop.  The slices'
+    // meeting costs some 10 us, which a deep k earns back.  Twenty in a row, 128 x
+    // 128 against pairs: 777 x 4352 at k = 4096 35.3 and 35.9 us, 6144 50.9 and
+    // 47.3, 10240 79.9 and 71.1; 513 x 3584 28.6 and 30.0, 41.4 and 41.3, 65.9 and
+    // 62.2; 2048 x 2048 32.9 and 35.4, 48.1 and 47.5, 79.2 and 72.5.  Under
+    // capture, and where scratch cannot be had, the tiles are computed whole: such
+    // a graph names no scratch, and may be replayed on any stream beside others.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool pairs = small && pl.sk_tiles == 0 && 2 * pl.dp_tiles > cus && k >= kDnPairK &&
+                       hipStreamIsCapturing(stream, &capture) == hipSuccess &&
+                       capture == hipStreamCaptureStatusNone &&
+                       scratch_acquire(dev, stream, (size_t)pl.dp_tiles * DnShape<128>::kPartBytes, &view,
+                                       g_dn_error, sizeof(g_dn_error));
     (void)hipGetLastError();  // an earlier call's error is not this launch's
     DenseArgs a;
     a.A = A;
@@ -793,16 +888,21 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     a.scratch = view.partials;
     a.finish_polls = t_finish_polls < 0 ? kFinishPolls : t_finish_polls;
     constexpr int lds_small = DnSmall::kLds, lds_half = DnShape<128>::kLds, lds_large = DnShape<256>::kLds;
-    if (cut_tiles > 0)
+    if (pairs) {
+      a.tiles_n = n / kDnTile;
+      a.dp_tiles = pl.dp_tiles / 2;
+      a.ksplit = 2;
+      hipLaunchKernelGGL((dense_kernel<128, true>), dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
+    } else if (cut_tiles > 0)
       hipLaunchKernelGGL(dense_small_kernel<true>, dim3((small ? pl.dp_tiles : 0) + cut_tiles * slices),
                          dim3(512), lds_small, stream, a);
     else if (small)
       hipLaunchKernelGGL(dense_small_kernel<false>, dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
     if (!small && pl.dp_tiles > 0) {
       if (pl.tile_rows == 128)
-        hipLaunchKernelGGL(dense_kernel<128>, dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
+        hipLaunchKernelGGL((dense_kernel<128, false>), dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
       else
-        hipLaunchKernelGGL(dense_kernel<256>, dim3(pl.dp_tiles), dim3(256), lds_large, stream, a);
+        hipLaunchKernelGGL((dense_kernel<256, false>), dim3(pl.dp_tiles), dim3(256), lds_large, stream, a);
     }
     e = hipGetLastError();
     if (e != hipSuccess) {

@@ -26,9 +26,9 @@ extern "C" {
  * fp32 accumulation.  m is arbitrary; n % 256 == 0 and k % 64 == 0.
  * Partial sums of the stream-K tiles live in the library-owned buffer of this
  * (device, stream) that marlin_gemm uses too (include/marlin_amd.h): sized by
- * the launch (64 KiB per slice of a 128 x 128 tile), grown on demand, none for
- * launches without slices.  Calls on one stream may follow each other
- * freely, calls that overlap must use different streams; a call that would have
+ * the launch (64 KiB per slice of a 128 x 128 tile, 128 KiB of a 128 x 256
+ * one), grown on demand, none for launches without slices.  Calls on one stream
+ * may follow each other freely, calls that overlap must use different streams; a call that would have
  * to allocate under graph capture returns STREAMK_ERR_RUNTIME. */
 int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, int dev,
                     void* hip_stream);
@@ -42,7 +42,9 @@ int streamk_amd_check(int m, int n, int k);
  * tiles (the last ones in tile order), k slices per stream-K tile, (tile, slice)
  * pairs (workgroups, except that the stream-K tiles of 256 x 256 are computed as
  * four 128 x 128 quarters each, in as many slices as leave none without a
- * compute unit), rows of a tile (256, or 128 when 256 x 256 tiles would occupy at most half
+ * compute unit, and from k = 7168, outside a capture, two neighbouring whole
+ * 128 x 128 tiles as two slices of a 128 x 256 one), rows of a tile (256, or 128
+ * when 256 x 256 tiles would occupy at most half
  * of the compute units), columns of a tile (256, or 128 when 128 x 256 tiles
  * would occupy at most half of them too) */
 int streamk_amd_plan(int m, int n, int k, int cus, int* out);

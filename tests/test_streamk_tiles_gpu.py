@@ -54,6 +54,8 @@ def test_stages(env, m, n, stages, tile):
     (4000, 4352, 832, (256, 256)),    # 16 tiles, 64 quarters, up to three slices
     (129, 256, 512, (128, 128)), (300, 1280, 768, (128, 128)), (128, 512, 1216, (128, 128)),
     (5000, 512, 576, (128, 128)),     # whole tiles only
+    (777, 4352, 7232, (128, 128)),    # 119 tiles of 128 x 256 in two slices of unequal length, 9 rows in the last
+    (2048, 2048, 7168, (128, 128)), (129, 16384, 7232, (128, 128)),
 ])
 def test_slices(env, m, n, k, tile, polls):
     torch, streamk = env
@@ -63,3 +65,25 @@ def test_slices(env, m, n, k, tile, polls):
             _check(env, m, n, k, 1, tile)
     finally:
         streamk.force_finish_polls(-1)
+
+
+def test_deep_tiles_under_capture(env):
+    """Sizes that run in slices outside a capture are captured on a stream without scratch."""
+    torch, streamk = env
+    m, n, k = 777, 4352, 7168
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(5)
+    A, B = (torch.randint(-1, 2, (r, k), device="cuda:0", generator=gen).half() for r in (m, n))
+    C = streamk.gemm(A, B)
+    want = A.float() @ B.float().t()
+    assert torch.equal(C.float(), want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        streamk.gemm(A, B, C)
+    for _ in range(3):
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C.float(), want)
+        assert torch.equal(streamk.gemm(A, B).float(), want)
