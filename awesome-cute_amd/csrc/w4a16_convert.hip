@@ -337,6 +337,10 @@ constexpr int kMaxGridY = 65535;
 
 bool aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
+bool apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  return (uintptr_t)a + a_bytes <= (uintptr_t)b || (uintptr_t)b + b_bytes <= (uintptr_t)a;
+}
+
 }  // namespace
 
 }  // namespace w4a16
@@ -379,7 +383,15 @@ int marlin_amd_pack(const void* w, int k, int n, int groupsize, int by_column, c
                     void* stream) {
   const int gs = groupsize == -1 ? k : groupsize;
   if (k <= 0 || n <= 0 || gs <= 0 || n % 64 != 0 || k % 64 != 0 || gs % 64 != 0 || k % gs != 0 ||
-      k / 16 > kMaxGridY || !aligned(w) || !aligned(B))
+      k / 16 > kMaxGridY || !aligned(w) || !aligned(B) || s_group < 0 || s_col < 0)
+    return MARLIN_ERR_PROB_SHAPE;
+  // every workgroup reads scales while others write packed ones
+  const int groups = k / gs;
+  const size_t w_bytes = (size_t)k * n * 2, b_bytes = (size_t)k * n / 2, p_bytes = (size_t)groups * n * 2;
+  const size_t s_bytes = (size_t)((groups - 1) * s_group + (n - 1) * s_col + 1) * 2;
+  if (!apart(B, b_bytes, w, w_bytes) || !apart(B, b_bytes, scales, s_bytes) ||
+      !apart(B, b_bytes, s_packed, p_bytes) || !apart(s_packed, p_bytes, w, w_bytes) ||
+      !apart(s_packed, p_bytes, scales, s_bytes))
     return MARLIN_ERR_PROB_SHAPE;
   OnDevice on(dev);
   if (on.e != hipSuccess) return on.done();

@@ -160,6 +160,18 @@ def _on_gpu(*tensors):
                     and not t.is_neg() and t.data_ptr() % 16 == 0 for t in tensors))
 
 
+def _apart(written, *read):
+    """Whether no tensor of `read` has bytes between the first and the last of the contiguous
+    tensor `written`: a kernel would read what it is overwriting, the tensor operations read
+    everything first."""
+    lo, hi = written.data_ptr(), written.data_ptr() + written.numel() * written.element_size()
+    for t in read:
+        last = sum((size - 1) * stride for size, stride in zip(t.shape, t.stride()))
+        if t.data_ptr() < hi and t.data_ptr() + (last + 1) * t.element_size() > lo:
+            return False
+    return True
+
+
 def _convert_check(rc):
     if rc != 0:
         raise RuntimeError(f"weight conversion failed with code {rc}: "
@@ -275,7 +287,8 @@ class Layer(nn.Module):
                 and B.is_contiguous() and packed.is_contiguous()
                 and _on_gpu(w, B, packed) and s.device == w.device
                 and type(s) in (torch.Tensor, nn.Parameter) and not s.requires_grad
-                and not s.is_neg()):
+                and not s.is_neg()
+                and _apart(B, w, s, packed) and _apart(packed, w, s)):
             dev = w.get_device()
             _convert_check(_lib.marlin_amd_pack(
                 w.data_ptr(), self.k, self.n, self.groupsize if groupwise else -1,

@@ -33,8 +33,8 @@ int marlin_amd_quantize(const void *w, int k, int n, int groupsize, int by_colum
  * Fake-quantised weights and their scales to packed words and packed scales:
  * q = clamp(round(fp16(w / s)) + 8, 0, 15).  w as above, n a multiple of 64, k
  * of 64; scale of group g and column c at scales[g * s_group + c * s_col];
- * groupsize -1 or a multiple of 64.  B: (k/16, 2n) int32; s_packed: (groups,
- * n) fp16.
+ * groupsize -1 or a multiple of 64, no stride negative.  B: (k/16, 2n) int32;
+ * s_packed: (groups, n) fp16; neither may overlap the other, w or scales.
  */
 int marlin_amd_pack(const void *w, int k, int n, int groupsize, int by_column, const void *scales,
                     long long s_group, long long s_col, void *B, void *s_packed, int dev,

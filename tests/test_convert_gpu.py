@@ -126,3 +126,30 @@ def test_layers_whose_buffers_were_changed(env):
     y = layer(x)
     layer.B = torch.nn.Parameter(layer.B, requires_grad=False)  # a parameter in the buffer's place
     assert torch.equal(layer(x), y)
+
+
+@pytest.mark.parametrize("by_column", [False, True])
+@pytest.mark.parametrize("gs", [128, -1])
+def test_pack_reads_everything_before_it_writes(env, gs, by_column):
+    """Scales in the layer's own buffer, and a weight whose memory the packed words go to."""
+    torch, marlin = env
+    k, n = 512, 768
+    w = torch.randn((k, n), device="cuda:0").half() * 0.02
+    fake, _, s = marlin.quantize(w, gs)
+
+    def linear():
+        lin = torch.nn.Linear(k, n, bias=False, device="cuda:0", dtype=torch.half)
+        lin.weight.data = fake.t().contiguous() if by_column else fake.clone().t()
+        return lin
+
+    want = marlin.Layer(k, n, gs).to("cuda:0")
+    want.pack(linear(), s.t())
+    layer = marlin.Layer(k, n, gs).to("cuda:0")
+    layer.s.copy_(s)
+    layer.pack(linear(), layer.s.t())
+    assert torch.equal(layer.B, want.B) and torch.equal(layer.s, want.s)
+    layer, lin = marlin.Layer(k, n, gs).to("cuda:0"), linear()
+    memory = lin.weight.data if by_column else lin.weight.data.t()
+    layer.B = memory.view(torch.int32).view(-1)[:layer.B.numel()].view(layer.B.shape)
+    layer.pack(lin, s.t())
+    assert torch.equal(layer.B, want.B) and torch.equal(layer.s, want.s)

@@ -1,0 +1,25 @@
+"""CPU tests of the weight conversion's host side: what the C entries refuse before
+anything is launched.  No GPU work."""
+import os
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "awesome-cute_amd"))
+
+PROB_SHAPE = 1
+
+
+@pytest.mark.parametrize("B,s_packed,scales", [
+    (1 << 30, 1 << 29, 1 << 29),             # scales packed onto themselves
+    (1 << 30, 1 << 29, (1 << 29) + 2046),    # the last byte of the packed ones
+    (1 << 30, (1 << 20) + 1024, 1 << 29),    # inside the weight
+    ((1 << 20) + 1024, 1 << 29, 1 << 28),
+    (1 << 29, (1 << 29) + 1024, 1 << 28),    # the two outputs
+    (1 << 30, 1 << 29, (1 << 30) - 2046),    # scales that run into the words
+])
+def test_pack_refuses_operands_that_overlap(B, s_packed, scales):
+    import marlin
+    k, n, gs = 256, 512, 128
+    assert marlin._lib.marlin_amd_pack(1 << 20, k, n, gs, 0, scales, n, 1, B, s_packed, 0, None) == PROB_SHAPE
