@@ -333,7 +333,11 @@ struct OnDevice {
   }
 };
 
-constexpr int kMaxGridY = 65535;
+// a launch has at most 65535 rows of workgroups and 2^32 - 1 threads in a row
+bool grid_holds(long long x, int threads, long long y) {
+  return x * threads <= 0xffffffffLL && y <= 65535;
+}
+long long pieces_of(long long a, int b) { return (a + b - 1) / b; }
 
 bool aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -353,26 +357,29 @@ int marlin_amd_quantize(const void* w, int k, int n, int groupsize, int by_colum
                         void* q, void* s, int dev, void* stream) {
   const int gs = groupsize == -1 ? k : groupsize;
   if (k <= 0 || n <= 0 || gs <= 0 || k % gs != 0 || (by_column ? gs : n) % 4 != 0 ||
-      k / gs > kMaxGridY || !aligned(w) || !aligned(fake) || !aligned(q) || !aligned(s))
+      !aligned(w) || !aligned(fake) || !aligned(q) || !aligned(s))
     return MARLIN_ERR_PROB_SHAPE;
-  if (by_column && (k % 4 != 0 || (long long)n * (k / gs) > 0x7fffffffLL)) return MARLIN_ERR_PROB_SHAPE;
+  const long long teams = (long long)n * (k / gs);
+  const bool small = gs <= 128;
+  if (by_column ? !grid_holds(small ? pieces_of(teams, 8) : teams, kPThreads, 1)
+                : !grid_holds(pieces_of(n, small ? 256 : 64), kQThreads, k / gs))
+    return MARLIN_ERR_PROB_SHAPE;
   OnDevice on(dev);
   if (on.e != hipSuccess) return on.done();
   const half_t* in = (const half_t*)w;
   const hipStream_t st = (hipStream_t)stream;
   if (by_column) {
-    const long long teams = (long long)n * (k / gs);
-    if (gs <= 128)
-      hipLaunchKernelGGL(quantise_columns<32>, dim3((unsigned)((teams + 7) / 8)), dim3(kPThreads), 0,
+    if (small)
+      hipLaunchKernelGGL(quantise_columns<32>, dim3((unsigned)pieces_of(teams, 8)), dim3(kPThreads), 0,
                          st, in, n, k, gs, (half_t*)fake, (int*)q, (half_t*)s);
     else
       hipLaunchKernelGGL(quantise_columns<kPThreads>, dim3((unsigned)teams), dim3(kPThreads), 0, st,
                          in, n, k, gs, (half_t*)fake, (int*)q, (half_t*)s);
-  } else if (gs <= 128) {
-    hipLaunchKernelGGL(quantise_rows<64>, dim3(ceil_div(n, 256), k / gs), dim3(kQThreads), 0, st, in,
+  } else if (small) {
+    hipLaunchKernelGGL(quantise_rows<64>, dim3((unsigned)pieces_of(n, 256), k / gs), dim3(kQThreads), 0, st, in,
                        n, gs, (half_t*)fake, (int*)q, (half_t*)s);
   } else {
-    hipLaunchKernelGGL(quantise_rows<16>, dim3(ceil_div(n, 64), k / gs), dim3(kQThreads), 0, st, in, n,
+    hipLaunchKernelGGL(quantise_rows<16>, dim3((unsigned)pieces_of(n, 64), k / gs), dim3(kQThreads), 0, st, in, n,
                        gs, (half_t*)fake, (int*)q, (half_t*)s);
   }
   return on.done();
@@ -383,7 +390,9 @@ int marlin_amd_pack(const void* w, int k, int n, int groupsize, int by_column, c
                     void* stream) {
   const int gs = groupsize == -1 ? k : groupsize;
   if (k <= 0 || n <= 0 || gs <= 0 || n % 64 != 0 || k % 64 != 0 || gs % 64 != 0 || k % gs != 0 ||
-      k / 16 > kMaxGridY || !aligned(w) || !aligned(B) || s_group < 0 || s_col < 0)
+      !aligned(w) || !aligned(B) || s_group < 0 || s_col < 0 ||
+      (by_column ? !grid_holds(n / 64, kPThreads, pieces_of(k, 256))
+                 : !grid_holds(pieces_of(n, 2 * kPThreads), kPThreads, k / 16)))
     return MARLIN_ERR_PROB_SHAPE;
   // every workgroup reads scales while others write packed ones
   const int groups = k / gs;
@@ -398,21 +407,22 @@ int marlin_amd_pack(const void* w, int k, int n, int groupsize, int by_column, c
   const PackArgs p = {w, (const half_t*)scales, s_group, s_col, (int*)B, (half_t*)s_packed,
                       k, n, gs, groupsize != -1};
   if (by_column)
-    hipLaunchKernelGGL(pack_columns, dim3(n / 64, ceil_div(k, 256)), dim3(kPThreads), 0,
+    hipLaunchKernelGGL(pack_columns, dim3(n / 64, (unsigned)pieces_of(k, 256)), dim3(kPThreads), 0,
                        (hipStream_t)stream, p);
   else
-    hipLaunchKernelGGL(pack_rows<false>, dim3(ceil_div(n, 2 * kPThreads), k / 16), dim3(kPThreads), 0,
+    hipLaunchKernelGGL(pack_rows<false>, dim3((unsigned)pieces_of(n, 2 * kPThreads), k / 16), dim3(kPThreads), 0,
                        (hipStream_t)stream, p);
   return on.done();
 }
 
 int marlin_amd_pack_words(const void* q, int k, int n, void* B, int dev, void* stream) {
-  if (k <= 0 || n <= 0 || n % 64 != 0 || k % 16 != 0 || k / 16 > kMaxGridY || !aligned(q) || !aligned(B))
+  if (k <= 0 || n <= 0 || n % 64 != 0 || k % 16 != 0 || !aligned(q) || !aligned(B) ||
+      !grid_holds(pieces_of(n, 2 * kPThreads), kPThreads, k / 16))
     return MARLIN_ERR_PROB_SHAPE;
   OnDevice on(dev);
   if (on.e != hipSuccess) return on.done();
   const PackArgs p = {q, nullptr, 0, 0, (int*)B, nullptr, k, n, k, false};
-  hipLaunchKernelGGL(pack_rows<true>, dim3(ceil_div(n, 2 * kPThreads), k / 16), dim3(kPThreads), 0,
+  hipLaunchKernelGGL(pack_rows<true>, dim3((unsigned)pieces_of(n, 2 * kPThreads), k / 16), dim3(kPThreads), 0,
                      (hipStream_t)stream, p);
   return on.done();
 }

@@ -172,10 +172,12 @@ def _apart(written, *read):
     return True
 
 
-def _convert_check(rc):
-    if rc != 0:
+def _converted(rc):
+    """Whether a conversion kernel was launched; False where its grid cannot hold the problem."""
+    if rc not in (0, 1):
         raise RuntimeError(f"weight conversion failed with code {rc}: "
                            f"{_lib.marlin_amd_convert_last_error().decode()}")
+    return rc == 0
 
 
 def pack_weights(q):
@@ -186,9 +188,9 @@ def pack_weights(q):
     if q.dtype == torch.int32 and q.numel() and q.is_contiguous() and _on_gpu(q):
         B = torch.empty((k // 16, 2 * n), dtype=torch.int32, device=q.device)
         dev = q.get_device()
-        _convert_check(_lib.marlin_amd_pack_words(q.data_ptr(), k, n, B.data_ptr(), dev,
-                                                  _raw_stream(dev)))
-        return B
+        if _converted(_lib.marlin_amd_pack_words(q.data_ptr(), k, n, B.data_ptr(), dev,
+                                                 _raw_stream(dev))):
+            return B
     blocks = q.reshape(k // 16, 16, n // 64, 64).permute(0, 2, 1, 3).reshape(k // 16, n // 64, 1024)
     nib = blocks[:, :, _block_gather.to(q.device)].reshape(k // 16, n // 64, 128, 8).to(torch.int64)
     shifts = torch.arange(0, 32, 4, device=q.device, dtype=torch.int64)
@@ -213,18 +215,17 @@ def quantize(w, groupsize=-1):
     fake-quantised weight (k, n), q (k, n) int32 and s (groups, n)."""
     k, n = w.shape
     gs = k if groupsize == -1 else groupsize
-    if (w.dtype == torch.half and w.numel() and gs > 0 and k % gs == 0 and k // gs <= 65535
-            and _on_gpu(w)):
+    if w.dtype == torch.half and w.numel() and gs > 0 and k % gs == 0 and _on_gpu(w):
         by_column = not w.is_contiguous()
         if (w.t().is_contiguous() and gs % 4 == 0) if by_column else n % 4 == 0:
             fake = torch.empty_like(w, memory_format=torch.preserve_format, requires_grad=False)
             q = torch.empty_like(fake, dtype=torch.int32)
             s = torch.empty((k // gs, n), dtype=torch.half, device=w.device)
             dev = w.get_device()
-            _convert_check(_lib.marlin_amd_quantize(w.data_ptr(), k, n, gs, by_column,
-                                                    fake.data_ptr(), q.data_ptr(), s.data_ptr(),
-                                                    dev, _raw_stream(dev)))
-            return fake, q, s
+            if _converted(_lib.marlin_amd_quantize(w.data_ptr(), k, n, gs, by_column,
+                                                   fake.data_ptr(), q.data_ptr(), s.data_ptr(),
+                                                   dev, _raw_stream(dev))):
+                return fake, q, s
     wg = w.reshape(k // gs, gs, n)
     s = wg.abs().amax(dim=1, keepdim=True)
     s = s * (2 / 15)
@@ -290,14 +291,14 @@ class Layer(nn.Module):
                 and not s.is_neg()
                 and _apart(B, w, s, packed) and _apart(packed, w, s)):
             dev = w.get_device()
-            _convert_check(_lib.marlin_amd_pack(
-                w.data_ptr(), self.k, self.n, self.groupsize if groupwise else -1,
-                not w.is_contiguous(), s.data_ptr(), s.stride(0), s.stride(1), B.data_ptr(),
-                packed.data_ptr(), dev, _raw_stream(dev)))
-            # written in place, as an assignment to them would be
-            torch.autograd.graph.increment_version(
-                [t for t in (B, packed) if not t.is_inference()])
-            return
+            if _converted(_lib.marlin_amd_pack(
+                    w.data_ptr(), self.k, self.n, self.groupsize if groupwise else -1,
+                    not w.is_contiguous(), s.data_ptr(), s.stride(0), s.stride(1), B.data_ptr(),
+                    packed.data_ptr(), dev, _raw_stream(dev))):
+                # written in place, as an assignment to them would be
+                torch.autograd.graph.increment_version(
+                    [t for t in (B, packed) if not t.is_inference()])
+                return
         s_full = s.repeat_interleave(self.groupsize, dim=0) if groupwise else s
         q = torch.clamp(torch.round(w / s_full).int() + 8, 0, 15)
         self.B[:, :] = pack_weights(q).to(self.B.device)

@@ -7,7 +7,8 @@
  *
  * All pointers are device pointers, fp16 weights and scales, 16-byte aligned.
  * Calls are asynchronous on `stream` and need no workspace.  Returns one of
- * marlin_gemm's codes.
+ * marlin_gemm's codes; MARLIN_ERR_PROB_SHAPE also for a problem that no grid
+ * holds (some hundred million groups, a million rows).
  */
 #ifndef MARLIN_AMD_CONVERT_H
 #define MARLIN_AMD_CONVERT_H

@@ -153,3 +153,29 @@ def test_pack_reads_everything_before_it_writes(env, gs, by_column):
     layer.B = memory.view(torch.int32).view(-1)[:layer.B.numel()].view(layer.B.shape)
     layer.pack(lin, s.t())
     assert torch.equal(layer.B, want.B) and torch.equal(layer.s, want.s)
+
+
+def test_more_than_a_grid_holds(env):
+    """Sizes beyond the kernels' grids take the tensor operations: the same as in parts."""
+    torch, marlin = env
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(2)
+    k, n = 16 * 65536, 64
+    q = torch.randint(0, 16, (k, n), dtype=torch.int32, device="cuda:0", generator=gen)
+    assert torch.equal(marlin.pack_weights(q),
+                       torch.cat([marlin.pack_weights(half) for half in q.split(k // 2)]))
+    k, n = 128 * 8192, 256
+    w = torch.randint(-8, 8, (k, n), device="cuda:0", generator=gen).half()
+    s = torch.ones((k // 128, n), device="cuda:0").half()
+    linear = torch.nn.Linear(k, n, bias=False, device="meta", dtype=torch.half)
+    linear.weight = torch.nn.Parameter(w.t())
+    layer = marlin.Layer(k, n, 128).to("cuda:0")
+    layer.pack(linear, s.t())
+    assert torch.equal(layer.B, torch.cat([marlin.pack_weights((half + 8).int()) for half in w.split(k // 2)]))
+    del q, w, linear, layer
+    wide = torch.randn((65536, 8192), dtype=torch.half, device="cuda:0", generator=gen)  # columns
+    got = marlin.quantize(wide.t(), 4)
+    for part, rows in zip(got, (8192, 8192, 2048)):
+        assert part.shape == (rows, 65536)
+    half = marlin.quantize(wide[:32768].t(), 4)
+    assert all(torch.equal(a[:, :32768], b) for a, b in zip(got, half))

@@ -23,3 +23,16 @@ def test_pack_refuses_operands_that_overlap(B, s_packed, scales):
     import marlin
     k, n, gs = 256, 512, 128
     assert marlin._lib.marlin_amd_pack(1 << 20, k, n, gs, 0, scales, n, 1, B, s_packed, 0, None) == PROB_SHAPE
+
+
+def test_problems_no_grid_holds_are_refused():
+    """... with the code that sends the Python calls to the tensor operations."""
+    import marlin
+    lib, P = marlin._lib, 1 << 20
+    deep = 16 * 65536  # a row of workgroups per 16 rows: one too many
+    assert lib.marlin_amd_pack_words(P, deep, 64, 1 << 40, 0, None) == PROB_SHAPE
+    assert lib.marlin_amd_pack(P, deep, 64, 128, 0, 1 << 50, 64, 1, 1 << 40, 1 << 52, 0, None) == PROB_SHAPE
+    assert lib.marlin_amd_quantize(P, 4 * 65536, 64, 4, 0, P, P, P, 0, None) == PROB_SHAPE
+    # 32 threads, or 256, per group of a column: 2^32 threads
+    assert lib.marlin_amd_quantize(P, 8192, 65536, 4, 1, P, P, P, 0, None) == PROB_SHAPE
+    assert lib.marlin_amd_quantize(P, 132 * 256, 65536, 132, 1, P, P, P, 0, None) == PROB_SHAPE
