@@ -289,6 +289,9 @@ class Layer(nn.Module):
                 and _on_gpu(w, B, packed) and s.device == w.device
                 and type(s) in (torch.Tensor, nn.Parameter) and not s.requires_grad
                 and not s.is_neg()
+                # (writes to inference tensors elsewhere are refused by the assignments below)
+                and (torch.is_inference_mode_enabled()
+                     or not (B.is_inference() or packed.is_inference()))
                 and _apart(B, w, s, packed) and _apart(packed, w, s)):
             dev = w.get_device()
             if _converted(_lib.marlin_amd_pack(

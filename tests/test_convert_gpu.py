@@ -179,3 +179,22 @@ def test_more_than_a_grid_holds(env):
         assert part.shape == (rows, 65536)
     half = marlin.quantize(wide[:32768].t(), 4)
     assert all(torch.equal(a[:, :32768], b) for a, b in zip(got, half))
+
+
+def test_layers_made_in_inference_mode(env):
+    """Packing writes to the buffers: refused outside inference mode as any write to them is."""
+    torch, marlin = env
+    k, n = 128, 256
+    fake, _, s = marlin.quantize(torch.randn((k, n), device="cuda:0").half(), 128)
+    linear = torch.nn.Linear(k, n, bias=False, device="cuda:0", dtype=torch.half)
+    linear.weight.data = fake.t()
+    with torch.inference_mode():
+        layer = marlin.Layer(k, n, 128).to("cuda:0")
+        layer.pack(linear, s.t())
+        before = layer.B.clone()
+    with pytest.raises(RuntimeError, match="[Ii]nference"):
+        layer.pack(linear, s.t())
+    other = marlin.Layer(k, n, 128).to("cuda:0")
+    with torch.inference_mode():
+        other.pack(linear, s.t())
+    assert torch.equal(other.B, before)
