@@ -432,8 +432,13 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
 // CUT: some tiles are cut into slices, or are quarters of the plan's.  (One
 // kernel for both took whole tiles 0.25 us longer, 8.5 -> 8.75 us at 2048 x 2048
 // x 512.)
-template <bool CUT>
+// PAIRED (whole tiles): the sums in the order that dense_kernel adds them up in
+// two slices, the even and the odd k steps of either half of the k range by
+// themselves, so that a problem which runs in such slices where there is scratch
+// for them has the same bits where there is none.
+template <bool CUT, bool PAIRED>
 __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
+  static_assert(!CUT || !PAIRED, "");
   extern __shared__ __attribute__((aligned(16))) char smem[];  // DnSmall::kLds
   using Sh = DnSmall;
   __shared__ int s_shares;
@@ -509,10 +514,17 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   };
 
   f4 acc[4][2];
+  f4 odd[PAIRED ? 4 : 1][2];  // of the odd k steps
+  auto start = [&] {
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+    for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 2; j++) {
+        acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+        if constexpr (PAIRED) odd[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  start();
 
   i4 w[2][2];  // B operands of the two k steps of a stage
   i4 af[4];    // ring of A operands, three ahead of the MFMAs
@@ -587,27 +599,47 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
       }
       const h8 a = __builtin_bit_cast(h8, af[i]);
 #pragma unroll
-      for (int j = 0; j < 2; j++)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, w[h][j]), a,
-                                                           acc[i][j], 0, 0, 0);
+      for (int j = 0; j < 2; j++) {
+        f4& sum = PAIRED && h == 1 ? odd[PAIRED ? i : 0][j] : acc[i][j];
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, w[h][j]), a, sum, 0, 0, 0);
+      }
     }
   };
 
-  int slot = 0;  // ring slot of the stage being computed
-  for (int s = 0; s < stages; s++) {
-    const int slot_next = slot == Sh::kRing - 1 ? 0 : slot + 1;
-    const unsigned cur = slot * Sh::kSlab, nxt = slot_next * Sh::kSlab;
-    kstep(std::integral_constant<int, 0>{}, cur, nxt, s, slot);
-    kstep(std::integral_constant<int, 1>{}, cur, nxt, s, slot);
-    slot = slot_next;
+  int s = 0;     // the stage being computed
+  int slot = 0;  // its ring slot
+  auto run_to = [&](int stop) {
+    for (; s < stop; s++) {
+      const int slot_next = slot == Sh::kRing - 1 ? 0 : slot + 1;
+      const unsigned cur = slot * Sh::kSlab, nxt = slot_next * Sh::kSlab;
+      kstep(std::integral_constant<int, 0>{}, cur, nxt, s, slot);
+      kstep(std::integral_constant<int, 1>{}, cur, nxt, s, slot);
+      slot = slot_next;
+    }
+    // The last k step has requested the operands of the stage after it (which
+    // may not exist); they are still on their way into w and af.  Those registers
+    // stay taken until the reads have landed: the compiler, which believes they
+    // were written when the reads were issued and may see no further use, would
+    // otherwise hand them to the code below at once, and a late arrival would
+    // overwrite what that code keeps there.
+    drain_reads(w[0], w[1], af);
+  };
+  if constexpr (PAIRED) {
+    f4 first[4][2];
+    run_to(stages / 2);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) first[i][j] = acc[i][j] + odd[i][j];
+    start();
+    run_to(stages);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) acc[i][j] = first[i][j] + (acc[i][j] + odd[i][j]);
+  } else {
+    run_to(stages);
   }
-  // The last k step has requested the operands of a stage that does not
-  // exist; they are still on their way into w and af.  Those registers stay
-  // taken until the reads have landed: the compiler, which believes they were
-  // written when the reads were issued and sees no further use, would
-  // otherwise hand them to the code below at once, and a late arrival would
-  // overwrite what that code keeps there.
-  drain_reads(w[0], w[1], af);
   // Nothing of the ring may still be on its way when LDS is reused.
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
@@ -821,10 +853,13 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
           e = hipFuncSetAttribute((const void*)dense_kernel<128, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, DnShape<128>::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_small_kernel<false>,
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<false, false>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_small_kernel<true>,
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<true, false>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<false, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
         if (e != hipSuccess) {
           dn_set_error(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
@@ -861,11 +896,12 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     // 128 against pairs: 777 x 4352 at k = 4096 35.3 and 35.9 us, 6144 50.9 and
     // 47.3, 10240 79.9 and 71.1; 513 x 3584 28.6 and 30.0, 41.4 and 41.3, 65.9 and
     // 62.2; 2048 x 2048 32.9 and 35.4, 48.1 and 47.5, 79.2 and 72.5.  Under
-    // capture, and where scratch cannot be had, the tiles are computed whole: such
-    // a graph names no scratch, and may be replayed on any stream beside others.
+    // capture, and where scratch cannot be had, the tiles are computed whole, in
+    // the same order of sums and so to the same bits: such a graph names no
+    // scratch, and may be replayed on any stream beside others.
+    const bool paired = small && pl.sk_tiles == 0 && 2 * pl.dp_tiles > cus && k >= kDnPairK;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool pairs = small && pl.sk_tiles == 0 && 2 * pl.dp_tiles > cus && k >= kDnPairK &&
-                       hipStreamIsCapturing(stream, &capture) == hipSuccess &&
+    const bool pairs = paired && hipStreamIsCapturing(stream, &capture) == hipSuccess &&
                        capture == hipStreamCaptureStatusNone &&
                        scratch_acquire(dev, stream, (size_t)pl.dp_tiles * DnShape<128>::kPartBytes, &view,
                                        g_dn_error, sizeof(g_dn_error));
@@ -894,10 +930,12 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
       a.ksplit = 2;
       hipLaunchKernelGGL((dense_kernel<128, true>), dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
     } else if (cut_tiles > 0)
-      hipLaunchKernelGGL(dense_small_kernel<true>, dim3((small ? pl.dp_tiles : 0) + cut_tiles * slices),
+      hipLaunchKernelGGL((dense_small_kernel<true, false>), dim3((small ? pl.dp_tiles : 0) + cut_tiles * slices),
                          dim3(512), lds_small, stream, a);
+    else if (paired)
+      hipLaunchKernelGGL((dense_small_kernel<false, true>), dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
     else if (small)
-      hipLaunchKernelGGL(dense_small_kernel<false>, dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
+      hipLaunchKernelGGL((dense_small_kernel<false, false>), dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
     if (!small && pl.dp_tiles > 0) {
       if (pl.tile_rows == 128)
         hipLaunchKernelGGL((dense_kernel<128, false>), dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);

@@ -28,8 +28,10 @@ extern "C" {
  * (device, stream) that marlin_gemm uses too (include/marlin_amd.h): sized by
  * the launch (64 KiB per slice of a 128 x 128 tile, 128 KiB of a 128 x 256
  * one), grown on demand, none for launches without slices.  Calls on one stream
- * may follow each other freely, calls that overlap must use different streams; a call that would have
- * to allocate under graph capture returns STREAMK_ERR_RUNTIME. */
+ * may follow each other freely, calls that overlap must use different streams; a
+ * call that would have to allocate under graph capture returns
+ * STREAMK_ERR_RUNTIME.  What the launch is (slices or whole tiles, see below)
+ * may depend on the capture and on the scratch, the bits of C do not. */
 int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, int dev,
                     void* hip_stream);
 

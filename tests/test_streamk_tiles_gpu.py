@@ -87,3 +87,24 @@ def test_deep_tiles_under_capture(env):
         torch.cuda.synchronize()
         assert torch.equal(C.float(), want)
         assert torch.equal(streamk.gemm(A, B).float(), want)
+
+
+@pytest.mark.parametrize("m,n,k", [(777, 4352, 7232), (2048, 2048, 7168), (129, 16384, 7232), (1000, 4096, 10304)])
+def test_deep_tiles_have_the_same_bits_under_capture(env, m, n, k):
+    """In two slices outside a capture and whole within one: the sums are added up in the same order."""
+    torch, streamk = env
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(k)
+    A, B = (torch.randn((r, k), device="cuda:0", generator=gen).half() for r in (m, n))
+    want = streamk.gemm(A, B)
+    C = torch.zeros_like(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        streamk.gemm(A, B, C)
+    for _ in range(3):
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
+        assert torch.equal(streamk.gemm(A, B), want)
