@@ -772,7 +772,7 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
   if (cus > 0 && configure_device(dev)) {
     PlanCtx cx = {cus, use_static ? kStaticPartialBytes : kPoolPartialLimit, t_force};
     cx.counters = max_par > 16 ? 16 : max_par;  // the counters of a tile sit that many ints apart
-    const Plan pl = make_plan(m, n, k, sms, cx);
+    Plan pl = make_plan(m, n, k, sms, cx);
     ScratchView view = {nullptr, nullptr};
     bool ok = true;
     if (use_static) {
@@ -793,6 +793,18 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
     } else if (pl.partial_bytes > 0) {
       ok = scratch_acquire(dev, stream, pl.partial_bytes, &view, g_last_error,
                            sizeof(g_last_error));
+      if (!ok && pl.kernel == 2) {
+        // slices of prefill tiles are there for speed alone: where their scratch
+        // cannot be had (a stream under capture, a full pool) the problem is
+        // computed without any
+        cx.partial_limit = 0;
+        pl = make_plan(m, n, k, sms, cx);
+        if (pl.partial_bytes > 0) {
+          cx.force.kernel = 2;
+          pl = make_plan(m, n, k, sms, cx);
+        }
+        ok = pl.partial_bytes == 0;
+      }
     }
     if (ok)
       rc = enqueue(pl, view, A, B, C, s, m, n, k, workspace, groupsize, max_par, stream);

@@ -95,3 +95,45 @@ def test_dequantised_weights_bit_exact(env, rows, groupsize):
         marlin.force_kernel(0)
         marlin.force_tile_rows(0)
         marlin.force_k_slices(0)
+
+
+@pytest.mark.parametrize("m,n,k", [(690, 4608, 4096), (140, 11008, 4864), (542, 1280, 1280), (529, 768, 4992),
+                                   (56, 18432, 1280)])
+def test_slices_captured_without_scratch(env, m, n, k):
+    """Problems that run in slices are captured on a stream that has no scratch, without any:
+    nothing is allocated, and the replays are right whatever runs in between.  On a stream
+    that has scratch the graph repeats the bits of the eager call."""
+    torch, marlin = env
+    dev = torch.device("cuda:0")
+    assert marlin.plan(m, n, k, 128)[1]["k_slices"] > 1
+    A, _, _, B, sp = O.make_problem(m, n, k, 128, seed=m)
+    dA, dB, ds = (torch.from_numpy(x).to(dev) for x in (A, B, sp))
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int, device=dev)
+    eager = torch.empty((m, n), dtype=torch.half, device=dev)
+    marlin.mul(dA, dB, eager, ds, ws)
+    torch.cuda.synchronize()
+    rows = np.unique(np.linspace(0, m - 1, 24).astype(int))
+    want = O.gemm(A[rows], B, sp, n, 128)
+    marlin.release()  # (a new stream may have the handle of one that had scratch)
+    cold, warm = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(warm):
+        marlin.mul(dA, dB, eager, ds, ws)
+    torch.cuda.synchronize()
+    held = marlin.scratch_bytes()
+    for side in (cold, warm):
+        C = torch.zeros_like(eager)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            marlin.mul(dA, dB, C, ds, ws)
+        assert marlin.scratch_bytes() == held
+        for _ in range(3):
+            C.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert side is cold or torch.equal(C, eager)
+            r = O.compare(C[rows].cpu().numpy(), want)
+            assert r.max_abs_err <= 1e-2 * r.max_abs_ref and r.rel_mean_abs_err <= 1e-3
+            marlin.mul(dA[:17], dB, torch.empty((17, n), dtype=torch.half, device=dev), ds, ws)
+        held = marlin.scratch_bytes()
+        del graph
