@@ -141,13 +141,34 @@ _block_gather = torch.from_numpy((64 * _k_in_block + _n_in_block).reshape(-1).as
 # kernels read them; the tensor operations beside them serve every other device,
 # type and layout, and give the same bits.
 
+def _stacks():
+    """What torch keeps of those that look on; torch has no public names for them."""
+    from torch.overrides import _get_current_function_mode_stack as function_modes
+    from torch.utils._device import DeviceContext
+    return (torch._C._get_tracing_state, torch._C._len_torch_dispatch_stack,
+            torch._C._functorch.peek_interpreter_stack, torch.autograd.forward_ad,
+            torch._C._len_torch_function_stack, function_modes, DeviceContext)
+
+
+try:
+    (_tracing_state, _dispatch_modes, _function_transforms, _forward_ad, _count_function_modes,
+     _function_modes, _DeviceContext) = _stacks()
+    _forward_ad._current_level
+    _can_tell = True
+except (AttributeError, ImportError):  # another torch: the tensor operations are right for everyone
+    _can_tell = False
+
+
 def _looked_on():
     """Whether something wants to see the tensor operations themselves: a compiler, a tracer, a
-    dispatch mode, a function transform (vmap, grad, jvp) or forward-mode differentiation."""
-    return (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-            or torch._C._len_torch_dispatch_stack() != 0
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0)
+    dispatch or function mode (one that only says where new tensors go does not), a function
+    transform (vmap, grad, jvp) or forward-mode differentiation."""
+    if not _can_tell or torch.compiler.is_compiling():
+        return True
+    return (_tracing_state() is not None or _dispatch_modes() != 0
+            or _function_transforms() is not None or _forward_ad._current_level >= 0
+            or (_count_function_modes() != 0
+                and any(type(mode) is not _DeviceContext for mode in _function_modes())))
 
 
 def _on_gpu(*tensors):

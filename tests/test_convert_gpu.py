@@ -198,3 +198,26 @@ def test_layers_made_in_inference_mode(env):
     with torch.inference_mode():
         other.pack(linear, s.t())
     assert torch.equal(other.B, before)
+
+
+def test_function_modes_see_the_tensor_operations(env):
+    torch, marlin = env
+    from torch.overrides import TorchFunctionMode
+    seen = []
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    w = torch.randn((256, 128), device="cuda:0").half()
+    want = marlin.quantize(w, 128)
+    with Mode():
+        got = marlin.quantize(w, 128)
+    assert "round" in seen and "clamp" in seen
+    for g, x in zip(got, want):
+        _same(torch, g, x)
+    seen.clear()
+    with torch.device("cuda:0"):  # says where new tensors go, no more
+        for g, x in zip(marlin.quantize(w, 128), want):
+            _same(torch, g, x)

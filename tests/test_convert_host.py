@@ -36,3 +36,29 @@ def test_problems_no_grid_holds_are_refused():
     # 32 threads, or 256, per group of a column: 2^32 threads
     assert lib.marlin_amd_quantize(P, 8192, 65536, 4, 1, P, P, P, 0, None) == PROB_SHAPE
     assert lib.marlin_amd_quantize(P, 132 * 256, 65536, 132, 1, P, P, P, 0, None) == PROB_SHAPE
+
+
+def test_what_counts_as_looking_on():
+    """Function modes see the tensor operations; a default device does not ask to."""
+    import torch
+    import marlin
+    from torch.overrides import TorchFunctionMode
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert marlin._can_tell and not marlin._looked_on()
+    with torch.device("cpu"):
+        assert not marlin._looked_on()
+        with Mode():
+            assert marlin._looked_on()
+    with Mode():
+        assert marlin._looked_on()
+    assert not marlin._looked_on()
+
+
+def test_without_torchs_own_names_the_tensor_operations_run(monkeypatch):
+    import marlin
+    monkeypatch.setattr(marlin, "_can_tell", False)
+    assert marlin._looked_on()
