@@ -100,13 +100,12 @@ struct DenseArgs {
   int M, N, K;
   int tiles_m, tiles_n;
   int dp_tiles;  // tiles computed by one workgroup each
-  // dense_small_kernel: tiles (the last ones in tile order) cut into ksplit
-  // slices; with quarters, the plan's tiles are 256 x 256 and those after
-  // dp_tiles are computed as four tiles each
+  // dense_small_kernel, in a launch of its own: the tiles after the first
+  // dp_tiles, in ksplit slices each; with quarters, the plan's tiles are 256 x
+  // 256 and computed as four tiles each
   int sk_tiles;
   int ksplit;
   int quarters;
-  int slices_only;   // the launch has no whole tiles
   int* locks;        // one zeroed counter per cut tile, kDnCounterStride ints apart, zero again afterwards
   float* scratch;    // kPartBytes per slice
   int finish_polls;  // looks at a tile's other slices before leaving them a share
@@ -429,7 +428,7 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
   }
 }
 
-// CUT: some tiles are cut into slices, or are quarters of the plan's.  (One
+// CUT: the tiles are cut into slices, or are quarters of the plan's.  (One
 // kernel for both took whole tiles 0.25 us longer, 8.5 -> 8.75 us at 2048 x 2048
 // x 512.)
 // PAIRED (whole tiles): the sums in the order that dense_kernel adds them up in
@@ -450,23 +449,15 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   const int wm = wave >> 2;  // 64-row half of the tile
   const int wn = wave & 3;   // 32-column quarter
 
-  // Stream-K slices come first in the grid, so that they run beside the first
-  // wave of whole tiles; slices of the same k range and neighbouring tiles are
-  // neighbours in the grid.  Every XCD gets a contiguous run of slices and of
-  // tile numbers (a placement hint only).
+  // Every XCD gets a contiguous run of slices or of tile numbers (a placement
+  // hint only); slices of the same k range and neighbouring tiles are neighbours.
   int tile, ks = 0, ksplit = 1, cut = 0;
   if constexpr (CUT) {
-    const int sk_blocks = p.sk_tiles * p.ksplit;
-    int work = (int)blockIdx.x;
-    if (p.slices_only) work = xcd_work_index(work, sk_blocks);
-    if (work < sk_blocks) {
-      ks = work / p.sk_tiles;
-      cut = work - ks * p.sk_tiles;
-      tile = p.dp_tiles + (p.quarters ? cut >> 2 : cut);
-      ksplit = p.ksplit;
-    } else {
-      tile = xcd_work_index(work - sk_blocks, p.dp_tiles);
-    }
+    const int work = xcd_work_index((int)blockIdx.x, p.sk_tiles * p.ksplit);
+    ks = work / p.sk_tiles;
+    cut = work - ks * p.sk_tiles;
+    tile = p.dp_tiles + (p.quarters ? cut >> 2 : cut);
+    ksplit = p.ksplit;
   } else {
     tile = xcd_work_index((int)blockIdx.x, p.dp_tiles);
   }
@@ -875,7 +866,7 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     // for a quarter of a tile's time, their quarters 256 (4096 x 4352 x 4096
     // 142 us with one launch for both, 125 with two; 6230 x 3072 x 1280 67 and 52).
     const bool small = pl.tile_cols == 128;
-    const bool quarters = !small && pl.sk_tiles > 0;
+    const bool quarters = pl.tile_rows == kDnTile && pl.sk_tiles > 0;
     const int cut_tiles = quarters ? 4 * pl.sk_tiles : pl.sk_tiles;
     int slices = pl.ksplit;
     if (quarters) {
@@ -919,7 +910,6 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     a.sk_tiles = cut_tiles;
     a.ksplit = slices;
     a.quarters = quarters ? 1 : 0;
-    a.slices_only = quarters || pl.dp_tiles == 0 ? 1 : 0;
     a.locks = view.counters;
     a.scratch = view.partials;
     a.finish_polls = t_finish_polls < 0 ? kFinishPolls : t_finish_polls;
@@ -930,7 +920,7 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
       a.ksplit = 2;
       hipLaunchKernelGGL((dense_kernel<128, true>), dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
     } else if (cut_tiles > 0)
-      hipLaunchKernelGGL((dense_small_kernel<true, false>), dim3((small ? pl.dp_tiles : 0) + cut_tiles * slices),
+      hipLaunchKernelGGL((dense_small_kernel<true, false>), dim3(cut_tiles * slices),
                          dim3(512), lds_small, stream, a);
     else if (paired)
       hipLaunchKernelGGL((dense_small_kernel<false, true>), dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
