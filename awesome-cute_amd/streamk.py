@@ -13,6 +13,8 @@ _lib.streamk_amd_plan.restype = _I
 _lib.streamk_amd_plan.argtypes = [_I, _I, _I, _I, _P]
 _lib.streamk_amd_tile_coord.restype = None
 _lib.streamk_amd_tile_coord.argtypes = [_I, _I, _I, _P]
+_lib.streamk_amd_slice_coord.restype = None
+_lib.streamk_amd_slice_coord.argtypes = [_I, _I, _I, _P]
 _lib.streamk_amd_force_finish_polls.restype = None
 _lib.streamk_amd_force_finish_polls.argtypes = [_I]
 _lib.streamk_amd_last_error.restype = ctypes.c_char_p
@@ -35,6 +37,13 @@ def tile_coord(tile, tiles_m, tiles_n):
     """(row tile, column tile) of a tile number."""
     out = (ctypes.c_int * 2)()
     _lib.streamk_amd_tile_coord(tile, tiles_m, tiles_n, out)
+    return out[0], out[1]
+
+
+def slice_coord(block, tiles, slices):
+    """(tile, slice) of a workgroup of a launch of slices."""
+    out = (ctypes.c_int * 2)()
+    _lib.streamk_amd_slice_coord(block, tiles, slices, out)
     return out[0], out[1]
 
 

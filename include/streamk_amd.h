@@ -55,6 +55,10 @@ int streamk_amd_plan(int m, int n, int k, int cus, int* out);
  * tiles_m * tiles_n); for tests of the numbering */
 void streamk_amd_tile_coord(int tile, int tiles_m, int tiles_n, int* out);
 
+/* (tile, slice) that workgroup `block` of a launch of tiles * slices workgroups
+ * computes; for tests of the order */
+void streamk_amd_slice_coord(int block, int tiles, int slices, int* out);
+
 /* how often a workgroup looks whether the other slices of its tile have arrived
  * before it leaves them its share of the sums, for the calling thread: -1 = the
  * default, 0 = at once; for tests (results do not depend on it) */

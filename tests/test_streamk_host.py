@@ -112,6 +112,18 @@ def test_tile_numbering_is_a_bijection_in_panels(streamk, tm, tn):
     assert {r for r, _ in first} == set(range(tm))
 
 
+@pytest.mark.parametrize("tiles,slices", [(1, 2), (108, 2), (64, 4), (85, 3), (63, 4), (128, 2), (7, 3)])
+def test_slices_of_a_tile_meet_in_one_xcd(streamk, tiles, slices):
+    """Workgroups are dealt to the 8 XCDs round-robin: the slices of a tile go to one of them,
+    but for the tiles that one run ends in and the next begins with."""
+    at = {streamk.slice_coord(b, tiles, slices): b % 8 for b in range(tiles * slices)}
+    assert set(at) == {(t, s) for t in range(tiles) for s in range(slices)}
+    apart = sum(len({at[t, s] for s in range(slices)}) > 1 for t in range(tiles))
+    assert apart <= min(tiles, 7)
+    if tiles % 8 == 0:
+        assert apart == 0
+
+
 def test_dense_oracle_against_numpy():
     """f16_gemm_tn_ref is pinned by an independent routine: exact equality with numpy's
     float64 product where every sum is exactly representable (small integers), and
