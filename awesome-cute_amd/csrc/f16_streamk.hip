@@ -8,21 +8,24 @@
 // partial wave are cut along k into slices, one workgroup per slice, and the
 // slices of a tile meet through fp32 partial sums in memory and a counter.
 // Unlike the reference's turnstile (gemm_streamk.h:562-590: every block waits
-// for the one before it) nobody waits: a slice writes its partial tile through
-// to memory, takes a ticket, and the last arrival adds all slices in slice
-// order and writes C.
+// for the one before it) nobody waits for a turn: a slice writes what others
+// will add up through to memory and arrives, and the slices of a tile finish it
+// together, each a share of it, or leave their share to the last arrival when
+// the others do not come within a bounded wait (finish_arrive).
 //
-// Whole tiles, 256 x 256 or (too few of them for the compute units) 128 x 256,
-// and 128 x 256 in two slices where k is deep: dense_kernel.  A workgroup of four waves, one per SIMD, each with a 128 x 128
-// fp32 accumulator (all 256 AGPRs): a wave per quarter of the tile, or two
-// waves per 128 columns, each taking every other k step, their sums added
-// through LDS at the end.  The main loop is one assembly statement per tile
-// shape, written by gen_dense.py, which documents the schedule and the
-// registers; the build runs it.
+// dense_kernel: whole tiles, 256 x 256 or (too few of them for the compute
+// units) 128 x 256, unless k is shallow, and 128 x 256 in two slices where k is
+// deep.  A workgroup of four waves, one per SIMD, each with a 128 x 128 fp32
+// accumulator (all 256 AGPRs): a wave per quarter of the tile, or two waves per
+// 128 columns, each taking every other k step, their sums added through LDS at
+// the end.  The main loop is one assembly statement per tile shape, written by
+// gen_dense.py, which documents the schedule and the registers; the build runs it.
 //
-// 128 x 128 tiles, whole or slices: dense_small_kernel.  Eight waves of 64 x 32,
-// two per SIMD.  It computes the problems with few tiles, and the stream-K tiles
-// of the others, every 256 x 256 tile of the partial wave as four of its own.
+// dense_small_kernel: eight waves, two per SIMD, of half the tile's rows and a
+// quarter of its columns each.  128 x 128 tiles, whole or in slices: the problems
+// with few tiles, and the stream-K tiles of the others, every 256 x 256 tile of
+// the partial wave as four of its own.  And the large whole tiles over a shallow
+// k, where its shorter start and end count for more than dense_kernel's loop.
 //
 // In both, B is the first MFMA operand and A the second, so
 // v_mfma_f32_16x16x32_f16 yields D[n][m]; lane l = 16kg + nu of an operand holds
@@ -78,19 +81,27 @@ struct DnShape {
   static constexpr int kPartBytes = TM * 256 * 4;
   static_assert(kWK == 1 || kLds >= 128 * 1024, "room for the sums that waves hand each other");
 };
-// 128 x 128 tiles (dense_small_kernel)
+// Tiles of dense_small_kernel: 128 x 128, 128 x 256 or 256 x 256
+template <int TM, int TN>
 struct DnSmall {
-  static constexpr int kSlabA = 128 * 128;
-  static constexpr int kSlab = 2 * kSlabA;
-  static constexpr int kRing = 4;
-  static constexpr int kLoads = 4;              // per wave and slab
-  static constexpr int kPitch = 128 * 2 + 16;
-  static constexpr int kLds = kRing * kSlab;
-  static constexpr int kPartBytes = 128 * 128 * 4;
+  static constexpr int kRB = TM / 32;           // row blocks of 16 of a wave
+  static constexpr int kNJ = TN / 64;           // operands of 16 columns of a wave
+  static constexpr int kSlabA = TM * 128;
+  static constexpr int kSlab = kSlabA + TN * 128;
+  // A stage of a small tile is shorter than a load's way from L2 (0.4 us of MFMAs
+  // for 128 x 128), so its slabs are requested further ahead.
+  static constexpr int kRing = TN == 128 ? 4 : TM == 128 ? 3 : 2;
+  static constexpr int kTA = TM / 64;           // load instructions per wave and slab
+  static constexpr int kLoads = kTA + kNJ;
+  static constexpr int kPitch = TN * 2 + 16;
+  static constexpr int kRingBytes = kRing * kSlab, kTileBytes = TM * kPitch;
+  static constexpr int kLds = kRingBytes > kTileBytes ? kRingBytes : kTileBytes;
+  static constexpr int kPartBytes = TM * TN * 4;
 };
 constexpr int kDnMaxSlots = 256;  // slices in flight per launch
 constexpr int kDnMaxSlices = 4;
 constexpr int kDnPairK = 7168;    // depth from which 128 x 256 tiles in two slices beat 128 x 128 ones
+constexpr int kDnRunsK = 6144;    // depth from which 128 x 256 tiles are not dealt out in runs, see there
 constexpr int kDnCounterStride = 16;  // ints: a tile's slices meet in a cache line of their own
 
 struct DenseArgs {
@@ -197,6 +208,13 @@ __device__ __forceinline__ void drain_reads(i4 (&a)[2], i4 (&b)[2], i4 (&f)[4]) 
                  "+v"(f[3]));
 #endif
 }
+__device__ __forceinline__ void drain_reads(i4 (&a)[4], i4 (&b)[4], i4 (&f)[4]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]),
+                 "+v"(b[3]), "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]));
+#endif
+}
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding)
 constexpr int dn_vm_lgkm0(int n) { return (n & 15) | (7 << 4) | (0 << 8) | ((n >> 4) << 14); }
 // s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
@@ -279,7 +297,13 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
 
   // every XCD gets a contiguous run of tile numbers (a placement hint only)
   // (neighbouring tiles of one k range, so that they share rows of A and B)
-  const int work = xcd_work_index((int)blockIdx.x, SLICED ? p.dp_tiles * p.ksplit : p.dp_tiles);
+  // ... except 128 x 256 tiles over a deep k that the XCDs cannot share evenly: a
+  // run of 16 or 17 tiles that begins anywhere in a row of a panel reads up to
+  // eight tiles' rows of B, every eighth tile one or two (1306 x 3072 x 7232 90.2
+  // us, so 79.2; 1152 x 4352 x 8192 106.7 and 102.9; at k = 5376 58.4 and 59.1)
+  const bool runs = SLICED || TM == 256 || (p.dp_tiles & 7) == 0 || p.K < kDnRunsK;
+  const int work = runs ? xcd_work_index((int)blockIdx.x, SLICED ? p.dp_tiles * p.ksplit : p.dp_tiles)
+                        : (int)blockIdx.x;
   const int ks = SLICED ? work / p.dp_tiles : 0;
   const int tile = SLICED ? work - ks * p.dp_tiles : work;
   int tm, tn;
@@ -448,19 +472,20 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
 // two slices, the even and the odd k steps of either half of the k range by
 // themselves, so that a problem which runs in such slices where there is scratch
 // for them has the same bits where there is none.
-template <bool CUT, bool PAIRED>
+template <int TM, int TN, bool CUT, bool PAIRED>
 __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
-  static_assert(!CUT || !PAIRED, "");
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // DnSmall::kLds
-  using Sh = DnSmall;
+  static_assert(!(CUT && PAIRED) && (TM * TN == 128 * 128 || !(CUT || PAIRED)), "");
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // DnSmall<TM, TN>::kLds
+  using Sh = DnSmall<TM, TN>;
+  constexpr int RB = Sh::kRB, NJ = Sh::kNJ, TA = Sh::kTA;
   __shared__ int s_shares;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int kg = lane >> 4;
   const int nu = lane & 15;
-  const int wm = wave >> 2;  // 64-row half of the tile
-  const int wn = wave & 3;   // 32-column quarter
+  const int wm = wave >> 2;  // row half of the tile
+  const int wn = wave & 3;   // column quarter
 
   // Every XCD gets a contiguous run of slices or of tile numbers (a placement
   // hint only)
@@ -474,29 +499,31 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   }
   int tm, tn;
   dn_tile_coord(tile, p.tiles_m, p.tiles_n, &tm, &tn);
-  int m0 = 128 * tm, n0 = 128 * tn;
+  int m0 = TM * tm, n0 = TN * tn;
   if (CUT && p.quarters) {
     m0 = 256 * tm + 128 * ((cut >> 1) & 1);
     n0 = 256 * tn + 128 * (cut & 1);
   }
-  const int rows = min(128, p.M - m0);
+  const int rows = min(TM, p.M - m0);
   if (CUT && rows <= 0) return;  // a quarter below the last row, all its slices
 
   const __amdgpu_buffer_rsrc_t rA =
       dn_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
   const __amdgpu_buffer_rsrc_t rB =
-      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, 128u * (unsigned)p.K * 2u);
+      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)TN * (unsigned)p.K * 2u);
 
-  // wave w fetches rows 16 w ... of the A and of the B slab, as dense_kernel does
-  int a_src[2], b_src[2];
+  // wave w fetches the w-th eighth of the A rows and of the B rows of a slab, as
+  // dense_kernel does
+  int a_src[TA], b_src[NJ];
   {
     const int r8 = lane >> 3, c = (lane & 7) ^ r8;
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      const int r = 16 * wave + 8 * t + r8;
+    for (int t = 0; t < TA; t++) {
+      const int r = 8 * (TA * wave + t) + r8;
       a_src[t] = (r < rows ? r : rows - 1) * p.K * 2 + 16 * c;
-      b_src[t] = r * p.K * 2 + 16 * c;
     }
+#pragma unroll
+    for (int t = 0; t < NJ; t++) b_src[t] = (8 * (NJ * wave + t) + r8) * p.K * 2 + 16 * c;
   }
   // this workgroup's stages [st0, st1) of the K/64 stages
   const int stages_all = p.K / kDnStageK;
@@ -508,39 +535,44 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   auto issue_slab = [&](int s, int slot) {
     const int inv = s < stages ? 0 : kDnOob;  // a stage past the end fetches zeros
     const int at = (st0 + s) * (kDnStageK * 2);
-    char* base = smem + slot * Sh::kSlab + wave * 2048;
+    char* base = smem + slot * Sh::kSlab;
 #pragma unroll
-    for (int t = 0; t < 2; t++) dn_dma16(rA, base + t * 1024, a_src[t] | inv, at);
+    for (int t = 0; t < TA; t++) dn_dma16(rA, base + (TA * wave + t) * 1024, a_src[t] | inv, at);
 #pragma unroll
-    for (int t = 0; t < 2; t++) dn_dma16(rB, base + Sh::kSlabA + t * 1024, b_src[t] | inv, at);
+    for (int t = 0; t < NJ; t++)
+      dn_dma16(rB, base + Sh::kSlabA + (NJ * wave + t) * 1024, b_src[t] | inv, at);
   };
 
-  f4 acc[4][2];
-  f4 odd[PAIRED ? 4 : 1][2];  // of the odd k steps
+  f4 acc[RB][NJ];
+  f4 odd[PAIRED ? RB : 1][NJ];  // of the odd k steps
   auto start = [&] {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
         if constexpr (PAIRED) odd[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
       }
   };
   start();
 
-  i4 w[2][2];  // B operands of the two k steps of a stage
+  i4 w[2][NJ]; // B operands of the two k steps of a stage
   i4 af[4];    // ring of A operands, three ahead of the MFMAs
   // operand addresses in slab 0 for the two k steps
   unsigned a_rd[2], b_rd[2];
 #pragma unroll
   for (int h = 0; h < 2; h++) {
     const unsigned sw = 16 * ((4 * h + kg) ^ (nu & 7));
-    a_rd[h] = (unsigned)(size_t)smem + (64 * wm + nu) * 128 + sw;
-    b_rd[h] = (unsigned)(size_t)smem + Sh::kSlabA + (32 * wn + nu) * 128 + sw;
+    a_rd[h] = (unsigned)(size_t)smem + (16 * RB * wm + nu) * 128 + sw;
+    b_rd[h] = (unsigned)(size_t)smem + Sh::kSlabA + (16 * NJ * wn + nu) * 128 + sw;
   }
-  auto read_b = [&](unsigned at, i4 (&dst)[2]) {
+  auto read_b = [&](unsigned at, i4 (&dst)[NJ]) {
     dn_read16<0>(at, dst[0]);
     dn_read16<2048>(at, dst[1]);
+    if constexpr (NJ == 4) {
+      dn_read16<2 * 2048>(at, dst[2]);
+      dn_read16<3 * 2048>(at, dst[3]);
+    }
   };
 
   // prologue: every slot requested; slab 0 landed (loads complete in order); its
@@ -556,10 +588,11 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
 
   // One k step (H) of the stage in slab `cur`.  LDS reads in issue order, with
   // Ai the operand of row block i and primes the prefetches for the step after:
-  //   step 0:  | B(step 1) x 2  A3 | A0' | A1' | A2' |
-  //   step 1:  | A3 | barrier, B(next stage) x 2  A0' | A1' | A2' |
+  //   step 0:  | B(step 1) x NJ  A3 | A0' | A1' | A2' |
+  //   step 1:  | A3 | barrier, B(next stage) x NJ  A0' | A1' | A2' |
+  // (with eight row blocks A4 ... A7 follow A3 in the same way).
   // When row block i is used, the reads issued after Ai may still be pending:
-  // three A operands, plus the two B reads where those were issued in between
+  // three A operands, plus the NJ B reads where those were issued in between
   // (the three row blocks from the one that issues them).
   // The barrier of a stage sits where the first read from the next slab is
   // about to be issued: by then every wave has its own part of that slab (it
@@ -567,12 +600,12 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   // the current slab, which the request for the stage after next overwrites.
   auto kstep = [&](auto H, unsigned cur, unsigned nxt, int s, int slot) {
     constexpr int h = decltype(H)::value;
-    constexpr int ib = h;  // row block that issues the B reads
+    constexpr int ib = h ? RB - 3 : 0;  // row block that issues the B reads
     const unsigned ac = a_rd[h] + cur;                      // this step, this slab
     const unsigned an = h ? a_rd[0] + nxt : a_rd[1] + cur;  // the step after
     const unsigned bn = h ? b_rd[0] + nxt : b_rd[1] + cur;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < RB; i++) {
       if (i == ib) {
         if (h == 1) {
           // my loads of the next slab (the slabs after it may still be on
@@ -584,24 +617,32 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
         read_b(bn, w[h ^ 1]);
       }
       // operand of row block i + 3: of this step, or of the step after
+      auto read_a = [&](auto I) {
+        constexpr int x = decltype(I)::value;
+        dn_read16<(x < RB ? x : x - RB) * 2048>(x < RB ? ac : an, af[x & 3]);
+      };
       switch (i) {  // i is a constant after unrolling
-        case 0: dn_read16<3 * 2048>(ac, af[3]); break;
-        case 1: dn_read16<0>(an, af[0]); break;
-        case 2: dn_read16<2048>(an, af[1]); break;
-        case 3: dn_read16<2 * 2048>(an, af[2]); break;
+        case 0: read_a(std::integral_constant<int, 3>{}); break;
+        case 1: read_a(std::integral_constant<int, 4>{}); break;
+        case 2: read_a(std::integral_constant<int, 5>{}); break;
+        case 3: read_a(std::integral_constant<int, 6>{}); break;
+        case 4: read_a(std::integral_constant<int, 7>{}); break;
+        case 5: read_a(std::integral_constant<int, 8>{}); break;
+        case 6: read_a(std::integral_constant<int, 9>{}); break;
+        case 7: read_a(std::integral_constant<int, 10>{}); break;
       }
       if (i >= ib && i <= ib + 2)
-        dn_wait<5>(af[i]);
+        dn_wait<3 + NJ>(af[i & 3]);
       else
-        dn_wait<3>(af[i]);
+        dn_wait<3>(af[i & 3]);
       if (i == 0) {
         // the B operands of this step were requested before A0 was
 #pragma unroll
-        for (int j = 0; j < 2; j++) asm volatile("" : "+v"(w[h][j]));
+        for (int j = 0; j < NJ; j++) asm volatile("" : "+v"(w[h][j]));
       }
-      const h8 a = __builtin_bit_cast(h8, af[i]);
+      const h8 a = __builtin_bit_cast(h8, af[i & 3]);
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         f4& sum = PAIRED && h == 1 ? odd[PAIRED ? i : 0][j] : acc[i][j];
         sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, w[h][j]), a, sum, 0, 0, 0);
       }
@@ -627,18 +668,18 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
     drain_reads(w[0], w[1], af);
   };
   if constexpr (PAIRED) {
-    f4 first[4][2];
+    f4 first[RB][NJ];
     run_to(stages / 2);
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) first[i][j] = acc[i][j] + odd[i][j];
+      for (int j = 0; j < NJ; j++) first[i][j] = acc[i][j] + odd[i][j];
     start();
     run_to(stages);
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) acc[i][j] = first[i][j] + (acc[i][j] + odd[i][j]);
+      for (int j = 0; j < NJ; j++) acc[i][j] = first[i][j] + (acc[i][j] + odd[i][j]);
   } else {
     run_to(stages);
   }
@@ -647,11 +688,11 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   __syncthreads();
 
   // a lane holds, per (i, j), row 16i + nu and four consecutive columns
-  char* const out = smem + (64 * wm + nu) * Sh::kPitch + (32 * wn + 4 * (lane >> 4)) * 2;
+  char* const out = smem + (16 * RB * wm + nu) * Sh::kPitch + (16 * NJ * wn + 4 * (lane >> 4)) * 2;
   half_t* const C = (half_t*)p.C + (size_t)m0 * p.N + n0;
   if (!CUT || ksplit == 1) {
-    dense_write_tile<128, 128, Sh::kPitch, 512, 4, 2>(smem, out, C, p.N, rows,
-                                                      [&](int i, int j) { return acc[i][j]; });
+    dense_write_tile<TM, TN, Sh::kPitch, 512, RB, NJ>(smem, out, C, p.N, rows,
+                                                     [&](int i, int j) { return acc[i][j]; });
     return;
   }
 
@@ -753,8 +794,8 @@ struct DnPlan {
 
 // Whole waves of tiles go to one workgroup each; the tiles of the partial last
 // wave are cut into as many k slices as there are idle compute units per tile
-// (at most four: beyond that the partial-sum traffic of the one workgroup that
-// finishes a tile costs more than the slices save), each at least 256 deep.
+// (at most four, which is what dense_small_kernel has registers for where it adds
+// them up), each at least 256 deep.
 DnPlan dn_plan(int m, int n, int k, int cus) {
   DnPlan pl;
   // 256 x 256 tiles, unless they would occupy at most half of the compute
@@ -783,6 +824,26 @@ DnPlan dn_plan(int m, int n, int k, int cus) {
   pl.dp_tiles = tiles - pl.sk_tiles;
   pl.grid = pl.dp_tiles + pl.sk_tiles * s;
   return pl;
+}
+
+// Whether whole tiles of 256 columns go to dense_kernel's four waves, which read
+// less LDS per MFMA, or to dense_small_kernel's eight, which have half as many
+// sums each to clear, to add up (128 rows) and to write (1 to 2 us less per
+// launch) and request a slab at once.  Four waves save LDS time and power, so
+// they are ahead sooner when most of the compute units have a tile, and the
+// requests tell where deep operands come from memory and part of the compute
+// units have none.  Four and eight waves, us, operands from memory:
+//   256 x 256, 145 tiles (1076 x 7424)  k = 512 15.6 and 14.9, 1536 33.7 and 32.8, 2048 41.0 and 41.4,
+//                                       4096 78.1 and 81.3, 5376 120.6 and 114.4, 8192 174.7 and 162.0
+//              224 tiles (1900 x 7168)  2048 46.7 and 48.6, 5376 130.4 and 126.4, 8192 191.9 and 188.7
+//              256 tiles (4096 x 4096)  512 20.2 and 20.2, 1280 36.7 and 38.0, 8192 203.0 and 201.6 (and
+//                                       183.6 and 193.6 where they stay in the last-level cache)
+//   128 x 256, 132 tiles (1306 x 3072)  512 11.7 and 9.8, 2048 25.8 and 25.2, 3840 45.5 and 43.6, 4096 44.5 and 45.9
+//              256 tiles (1000 x 8192)  512 14.7 and 12.9, 2048 33.1 and 33.2, 3072 45.3 and 46.6
+bool dn_four_waves(int tile_rows, int tiles, int k, int cus) {
+  const bool most = 4 * tiles >= 3 * cus;
+  if (tile_rows != kDnTile) return k >= (most ? 3072 : 4096);
+  return k >= (most ? 768 : 2048) && (k < 5120 || tiles >= cus);
 }
 
 int dn_check(int m, int n, int k) {
@@ -855,14 +916,20 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
           e = hipFuncSetAttribute((const void*)dense_kernel<128, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, DnShape<128>::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_small_kernel<false, false>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<128, 128, false, false>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall<128, 128>::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_small_kernel<true, false>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<128, 128, true, false>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall<128, 128>::kLds);
         if (e == hipSuccess)
-          e = hipFuncSetAttribute((const void*)dense_small_kernel<false, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall::kLds);
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<128, 128, false, true>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall<128, 128>::kLds);
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<128, 256, false, false>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall<128, 256>::kLds);
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute((const void*)dense_small_kernel<256, 256, false, false>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall<256, 256>::kLds);
         if (e != hipSuccess) {
           dn_set_error(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
           break;
@@ -887,7 +954,7 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     // only slices exchange anything
     ScratchView view = {nullptr, nullptr};
     if (cut_tiles > 0 && slices > 1 &&
-        !scratch_acquire(dev, stream, (size_t)cut_tiles * slices * DnSmall::kPartBytes, &view,
+        !scratch_acquire(dev, stream, (size_t)cut_tiles * slices * DnSmall<128, 128>::kPartBytes, &view,
                          g_dn_error, sizeof(g_dn_error)))
       break;
     // Problems of 128 x 128 tiles for more than half of the compute units, one
@@ -924,24 +991,31 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     a.locks = view.counters;
     a.scratch = view.partials;
     a.finish_polls = t_finish_polls < 0 ? kFinishPolls : t_finish_polls;
-    constexpr int lds_small = DnSmall::kLds, lds_half = DnShape<128>::kLds, lds_large = DnShape<256>::kLds;
+    const auto launch = [&](auto kernel, int grid, int threads, int lds) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, a);
+    };
     if (pairs) {
       a.tiles_n = n / kDnTile;
       a.dp_tiles = pl.dp_tiles / 2;
       a.ksplit = 2;
-      hipLaunchKernelGGL((dense_kernel<128, true>), dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
-    } else if (cut_tiles > 0)
-      hipLaunchKernelGGL((dense_small_kernel<true, false>), dim3(cut_tiles * slices),
-                         dim3(512), lds_small, stream, a);
-    else if (paired)
-      hipLaunchKernelGGL((dense_small_kernel<false, true>), dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
-    else if (small)
-      hipLaunchKernelGGL((dense_small_kernel<false, false>), dim3(pl.dp_tiles), dim3(512), lds_small, stream, a);
+      launch(dense_kernel<128, true>, pl.dp_tiles, 256, DnShape<128>::kLds);
+    } else if (cut_tiles > 0) {
+      launch(dense_small_kernel<128, 128, true, false>, cut_tiles * slices, 512, DnSmall<128, 128>::kLds);
+    } else if (paired) {
+      launch(dense_small_kernel<128, 128, false, true>, pl.dp_tiles, 512, DnSmall<128, 128>::kLds);
+    } else if (small) {
+      launch(dense_small_kernel<128, 128, false, false>, pl.dp_tiles, 512, DnSmall<128, 128>::kLds);
+    }
     if (!small && pl.dp_tiles > 0) {
-      if (pl.tile_rows == 128)
-        hipLaunchKernelGGL((dense_kernel<128, false>), dim3(pl.dp_tiles), dim3(256), lds_half, stream, a);
+      const bool half = pl.tile_rows == 128, four = dn_four_waves(pl.tile_rows, pl.dp_tiles, k, cus);
+      if (half && four)
+        launch(dense_kernel<128, false>, pl.dp_tiles, 256, DnShape<128>::kLds);
+      else if (half)
+        launch(dense_small_kernel<128, 256, false, false>, pl.dp_tiles, 512, DnSmall<128, 256>::kLds);
+      else if (four)
+        launch(dense_kernel<256, false>, pl.dp_tiles, 256, DnShape<256>::kLds);
       else
-        hipLaunchKernelGGL((dense_kernel<256, false>), dim3(pl.dp_tiles), dim3(256), lds_large, stream, a);
+        launch(dense_small_kernel<256, 256, false, false>, pl.dp_tiles, 512, DnSmall<256, 256>::kLds);
     }
     e = hipGetLastError();
     if (e != hipSuccess) {

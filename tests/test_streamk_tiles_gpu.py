@@ -47,6 +47,16 @@ def test_stages(env, m, n, stages, tile):
     _check(env, m, n, 64 * stages, 2, tile)
 
 
+# ... and over a deeper k, in the loops of four waves (all but the last)
+@pytest.mark.parametrize("stages", [0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("m,n,k,tile", [(1999, 8192, 768, (256, 256)), (1535, 6400, 2048, (256, 256)),
+                                        (1001, 8192, 3072, (128, 256)), (767, 5632, 4096, (128, 256)),
+                                        (1300, 3328, 6144, (128, 256)),  # 143 tiles, dealt out one by one
+                                        (1076, 7424, 5120, (256, 256))])
+def test_deep_stages(env, m, n, k, stages, tile):
+    _check(env, m, n, k + 64 * stages, 1, tile)
+
+
 @pytest.mark.parametrize("polls", [-1, 0, 1])  # 0 and 1: shares left to the last arrival
 @pytest.mark.parametrize("m,n,k,tile", [
     (2049, 8192, 1024, (256, 256)),   # 32 stream-K tiles in quarters, most of them with one row or none
