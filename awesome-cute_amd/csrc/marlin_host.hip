@@ -151,31 +151,48 @@ struct PlanCtx {
   int cus;
   size_t partial_limit;
   Force force;
+  bool grouped;       // scales per group of 128, or one per column
   int counters = 16;  // ints of the workspace per column tile: min(max_par, 16)
 };
 
 // Cost in us of the prefill kernels with `tiles` tiles of tile_rows rows cut
-// into s slices, linear in what they do and fitted to 2700 launches on MI355X
-// (M = 65 ... 2100 on eleven (N, K) from 1024 x 1024 to 28672 x 8192, every
-// tile height and slice count; 4 % rms for 64 rows, 5 % for the others): a
-// launch, a round of workgroups, a 64-deep stage of each k half of a workgroup
-// (dearer the fuller the chip: the board's power), and with slices their
-// meeting, dearer with their number and with the traffic of a full chip.  R is
-// the row blocks of a tile of the four-wave kernel.
-double prefill_cost_slices(int tiles, int tile_rows, int k, int cus, int s) {
+// into s slices, linear in what they do: a launch, a round of workgroups, a
+// 64-deep stage of each k half of a workgroup (dearer the fuller the chip: the
+// board's power), and with slices their meeting, dearer with their number and
+// with the traffic of a full chip.  R is the row blocks of a tile of the
+// four-wave kernel.  Fitted to launches on MI355X, by themselves with group scales
+// (2700, M = 65 ... 2100 on eleven (N, K) from 1024 x 1024 to 28672 x 8192, every
+// tile height and slice count; 4 % rms for 64 rows, 5 % for the others) and with
+// one scale per column (32000 over 1300 problems, M = 33 ... 8192; 5 and 6 %),
+// whose weights are unpacked without a scale to multiply: a stage of a 64-row
+// tile takes 0.83 of the time, one of a 128-row tile 0.92.  By the first fit for
+// both, one problem in thirty with a scale per column was given slices or rows that
+// took 5 to 20 % longer than others (M = 313, N = 4096, K = 9728: five slices of 112
+// rows 33.1 us, three of 64 29.2).
+double prefill_cost_slices(int tiles, int tile_rows, int k, const PlanCtx& cx, int s) {
   // more workgroups than CUs run in rounds, the last of which is faster the
   // emptier it is: half way between whole rounds and the plain ratio fits
-  const double ratio = (double)tiles * s / cus;
-  const double rounds = ratio <= 1.0 ? 1.0 : 0.5 * (ceil_div(tiles * s, cus) + ratio);
+  const double ratio = (double)tiles * s / cx.cus;
+  const int whole = ceil_div(tiles * s, cx.cus);
+  const double rounds = ratio <= 1.0 ? 1.0 : 0.5 * (whole + ratio);
   const double fill = ratio < 1.0 ? ratio : 1.0;
-  const double stages = rounds * ceil_div(ceil_div(ceil_div(k, 64), s), 2);
-  if (tile_rows == 64)
+  const int depth = ceil_div(ceil_div(ceil_div(k, 64), s), 2);
+  const double stages = rounds * depth;
+  const double R = tile_rows / 16.0;
+  if (cx.grouped && tile_rows == 64)
     return -2.24 + 7.07 * rounds + (0.753 + 0.256 * fill) * stages +
            (s > 1 ? 0.86 + 0.61 * s + 1.90 * fill * rounds : 0.0);
-  const double R = tile_rows / 16.0;
-  return 5.16 - 1.97 * R + (2.63 * R - 2.42) * rounds +
-         (0.519 + (0.0586 + 0.0419 * fill) * R) * stages +
-         (s > 1 ? 2.12 + 0.302 * s + 0.625 * fill * rounds * R : 0.0);
+  if (cx.grouped)
+    return 5.16 - 1.97 * R + (2.63 * R - 2.42) * rounds +
+           (0.519 + (0.0586 + 0.0419 * fill) * R) * stages +
+           (s > 1 ? 2.12 + 0.302 * s + 0.625 * fill * rounds * R : 0.0);
+  const double late = ratio <= 1.0 ? 0.0 : (double)whole * depth;
+  if (tile_rows == 64)
+    return 2.34 + 3.22 * rounds + (0.656 + 0.116 * fill) * stages + 0.121 * late +
+           (s > 1 ? 0.508 + 0.629 * s + 2.16 * fill * rounds : 0.0);
+  return 3.92 - 0.318 * R + (0.960 * R - 0.802) * rounds +
+         (0.314 + (0.0704 + 0.0289 * fill) * R) * stages + 0.173 * late +
+         (s > 1 ? 3.33 + 0.290 * s + 0.501 * fill * rounds * R : 0.0);
 }
 
 // Whether a tile height is cut into s slices at all.  With 64 rows no more than
@@ -202,10 +219,10 @@ int prefill_k_slices(int tiles, int tile_rows, int k, const PlanCtx& cx) {
   if (cx.force.k_slices > 0) return cx.force.k_slices < most ? cx.force.k_slices : most;
   if (most > cx.cus / tiles) most = cx.cus / tiles;
   int best = 1;
-  double best_cost = prefill_cost_slices(tiles, tile_rows, k, cx.cus, 1);
+  double best_cost = prefill_cost_slices(tiles, tile_rows, k, cx, 1);
   for (int s = 2; s <= most; s++) {
     if (!slices_share(tile_rows, s)) continue;
-    const double c = prefill_cost_slices(tiles, tile_rows, k, cx.cus, s);
+    const double c = prefill_cost_slices(tiles, tile_rows, k, cx, s);
     if (c < best_cost) {
       best = s;
       best_cost = c;
@@ -216,7 +233,7 @@ int prefill_k_slices(int tiles, int tile_rows, int k, const PlanCtx& cx) {
 
 double prefill_cost_rows(int m, int n, int k, const PlanCtx& cx, int tile_rows) {
   const int tiles = ceil_div(m, tile_rows) * (n / 256);
-  return prefill_cost_slices(tiles, tile_rows, k, cx.cus,
+  return prefill_cost_slices(tiles, tile_rows, k, cx,
                              prefill_k_slices(tiles, tile_rows, k, cx));
 }
 
@@ -225,14 +242,18 @@ double prefill_cost_rows(int m, int n, int k, const PlanCtx& cx, int tile_rows) 
 // counts that 64-row tiles would pad -- M = 150, N = 12288, K = 4096: 31.6 us
 // with 64 rows, 31.7 with 128, 26.0 with 80; M = 300, N = K = 8192 59.1, 51.2
 // and 45.4; M = 203, N = 5120, K = 13568 46.8, 42.6 and 40.1 with 112; M = 300,
-// N = 28672, K = 8192 189, 172 and 142 -- and others are left to those two.
+// N = 28672, K = 8192 189, 172 and 142 -- and have to be ahead by 2 %, about what
+// the fit is worth.  Over 1660 problems that leaves 12 (14 with one scale per
+// column) that take 2 to 11 % longer than with 64 or 128 rows, 17 (54) without it
+// and with one fit for both; all together take 0.96 of the time.  (Where M is a
+// multiple of 64 they are not tried.)
 int prefill_tile_rows(int m, int n, int k, const PlanCtx& cx) {
   if (cx.force.tile_rows != 0) return cx.force.tile_rows;
   if (m <= 64) return 64;
   int best = 64;
   double best_cost = prefill_cost_rows(m, n, k, cx, 64);
   for (int rows = m % 64 == 0 ? 128 : 80; rows <= 128; rows += 16) {
-    const double c = prefill_cost_rows(m, n, k, cx, rows);
+    const double c = prefill_cost_rows(m, n, k, cx, rows) * (rows == 128 ? 1.0 : 1.02);
     if (c < best_cost) {
       best = rows;
       best_cost = c;
@@ -416,7 +437,11 @@ bool prefer_prefill(int m, int n, int k, const PlanCtx& cx) {
   // 1.1 at K = 8192, 1.5 at 11008), which the two fits, 15 % apart there in
   // opposite directions, do not resolve
   if (m <= kStreamMaxRows && n < 16384 && k < 8192) return false;
-  return prefill_cost(m, n, k, cx) <= stream_cost_as_planned(m, n, k, cx);
+  // (the streaming kernel's fit is that of group scales; one scale per column
+  // takes 0.96 of the time, and the fit is 5 % high where this is decided: M = 107,
+  // N = 8192, K = 4096 15.5 us streaming, 16.5 in four slices of 64 rows, by the fits
+  // 17.0 and 16.4)
+  return prefill_cost(m, n, k, cx) <= stream_cost_as_planned(m, n, k, cx) * (cx.grouped ? 1.0 : 0.9);
 }
 
 // Fitted time (us) of the column-strip kernel with `cs` strips per workgroup.
@@ -770,7 +795,7 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
   const int cus = device_cus(dev);
   rc = MARLIN_ERR_RUNTIME;
   if (cus > 0 && configure_device(dev)) {
-    PlanCtx cx = {cus, use_static ? kStaticPartialBytes : kPoolPartialLimit, t_force};
+    PlanCtx cx = {cus, use_static ? kStaticPartialBytes : kPoolPartialLimit, t_force, groupsize != -1};
     cx.counters = max_par > 16 ? 16 : max_par;  // the counters of a tile sit that many ints apart
     Plan pl = make_plan(m, n, k, sms, cx);
     ScratchView view = {nullptr, nullptr};
@@ -890,7 +915,7 @@ int marlin_amd_plan(int prob_m, int prob_n, int prob_k, int groupsize, int threa
   for (int i = 0; i < 13; i++) out[i] = 0;
   int rc = check_shape(prob_m, prob_n, prob_k, groupsize, thread_k, thread_n);
   if (rc != MARLIN_OK || prob_m == 0 || prob_n == 0 || prob_k == 0) return rc;
-  const PlanCtx cx = {cus, kPoolPartialLimit, t_force};
+  const PlanCtx cx = {cus, kPoolPartialLimit, t_force, groupsize != -1};
   Plan pl = make_plan(prob_m, prob_n, prob_k, sms, cx);
   out[0] = pl.kernel;
   out[1] = pl.grid;
@@ -913,7 +938,7 @@ int marlin_amd_plan_costs(int prob_m, int prob_n, int prob_k, int groupsize, int
   int thread_k = -1, thread_n = -1;
   int rc = check_shape(prob_m, prob_n, prob_k, groupsize, thread_k, thread_n);
   if (rc != MARLIN_OK || prob_m == 0 || prob_n == 0 || prob_k == 0) return rc;
-  const PlanCtx cx = {cus, kPoolPartialLimit, t_force};
+  const PlanCtx cx = {cus, kPoolPartialLimit, t_force, groupsize != -1};
   out[0] = stream_cost_as_planned(prob_m, prob_n, prob_k, cx);
   if (prob_n % 256 == 0) out[1] = prefill_cost(prob_m, prob_n, prob_k, cx);
   if (prob_m <= kStripMaxRows) {

@@ -210,6 +210,16 @@ def test_default_stream_plans_stay_inside_tiles(marlin, m, n, k):
                 assert (owner[t] == b).all()
 
 
+@pytest.mark.parametrize("m,n,k,groupsize,kernel,slices,rows", [
+    # one scale per column: cheaper to unpack, so fewer slices of lower tiles, and more streaming
+    (313, 4096, 9728, -1, 2, 3, 64), (106, 10240, 8064, -1, 2, 3, 64), (107, 8192, 4096, -1, 1, 1, 0),
+    (300, 8192, 8192, 128, 2, 2, 80),
+])
+def test_prefill_choice(marlin, m, n, k, groupsize, kernel, slices, rows):
+    rc, p = marlin.plan(m, n, k, groupsize)
+    assert rc == 0 and (p["kernel"], p["k_slices"], p["tile_rows"]) == (kernel, slices, rows), p
+
+
 def test_kernel_choice_by_cost(marlin):
     """Up to 16 rows over a few MiB of weights, and more rows (in parts of 16,
     a workgroup each) while the parts fill the compute units at most twice, go

@@ -97,8 +97,8 @@ def test_dequantised_weights_bit_exact(env, rows, groupsize):
         marlin.force_k_slices(0)
 
 
-@pytest.mark.parametrize("m,n,k", [(690, 4608, 4096), (140, 11008, 4864), (542, 1280, 1280), (529, 768, 4992),
-                                   (56, 18432, 1280)])
+@pytest.mark.parametrize("m,n,k", [(690, 4608, 4096), (140, 11008, 4864), (565, 1792, 2816), (529, 768, 4992),
+                                   (236, 3072, 4352)])
 def test_slices_captured_without_scratch(env, m, n, k):
     """Problems that run in slices are captured on a stream that has no scratch, without any:
     nothing is allocated, and the replays are right whatever runs in between.  On a stream
