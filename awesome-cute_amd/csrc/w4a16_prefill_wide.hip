@@ -114,13 +114,18 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   char* smem = smem_all + kh * Shape::kRingBytes;
 
   // Same numbering of the work as the other prefill kernel: every XCD
-  // (workgroup id mod 8) gets a contiguous run of tile numbers (whole tiles only
-  // if they share evenly), tiles are numbered in panels of 8 column tiles with the
-  // row tile next, and the k slices of a tile are consecutive work indices: they
-  // meet behind one L2.  (With slices dealt out one by one where their number is
-  // no multiple of 8, over M = 33 ... 8192, K < 6144: 1.09 times the time.)
+  // (workgroup id mod 8) gets a contiguous run of tile numbers, tiles are
+  // numbered in panels of 8 column tiles with the row tile next, and the k slices
+  // of a tile are consecutive work indices: they meet behind one L2.  (With slices
+  // dealt out one by one where their number is no multiple of 8, over M = 33 ...
+  // 8192, K < 6144: 1.09 times the time.)  Whole tiles of eight columns or more
+  // get runs only if their number is a multiple of 8 (else no difference on
+  // average, up to 6 % either way); of fewer, always, so that the columns of a row
+  // tile read A from one L2 (N = 256 ... 1792, M = 600 ... 8192: 1.02 times the time
+  // without, 1.05 with more tiles than compute units).
   const int total = tiles_m * tiles_n * ksplit;
-  const int work = SLICED || (total & 7) == 0 ? xcd_work_index((int)blockIdx.x, total) : (int)blockIdx.x;
+  const bool runs = SLICED || (total & 7) == 0 || tiles_n < 8;
+  const int work = runs ? xcd_work_index((int)blockIdx.x, total) : (int)blockIdx.x;
   const int tile = SLICED ? work / ksplit : work;
   const int ks = SLICED ? work - tile * ksplit : 0;
   int tm, tn;
