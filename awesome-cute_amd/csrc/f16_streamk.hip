@@ -846,6 +846,55 @@ bool dn_four_waves(int tile_rows, int tiles, int k, int cus) {
   return k >= (most ? 768 : 2048) && (k < 5120 || tiles >= cus);
 }
 
+// Whether 128 x 128 tiles are computed two by two, as slices of 128 x 256 ones.
+// Problems of 128 x 128 tiles for more than half of the compute units, one
+// workgroup each, wait for operands: a tile of 128 x 256 brings half as many rows
+// of A per column, so in two slices along k the same workgroups take in three
+// quarters of the bytes and run dense_kernel's loop.  The slices' meeting costs
+// some 10 us, which a deep k earns back: 128 x 128 against pairs, 777 x 4352 at k =
+// 4096 35.3 and 35.9 us, 6144 50.9 and 47.3, 10240 79.9 and 71.1; 513 x 3584 28.6
+// and 30.0, 41.4 and 41.3, 65.9 and 62.2; 2048 x 2048 32.9 and 35.4, 48.1 and 47.5,
+// 79.2 and 72.5.  At 6144 they are level but for the first, so the line lies above.
+// Under capture, and where scratch cannot be had, the tiles are computed whole, in
+// the same order of sums and so to the same bits: such a graph names no scratch,
+// and may be replayed on any stream beside others.
+bool dn_paired(const DnPlan& pl, int k, int cus) {
+  return pl.tile_cols == 128 && pl.sk_tiles == 0 && 2 * pl.dp_tiles > cus && k >= kDnPairK;
+}
+
+// One launch: `tiles` tiles of rows x cols in `slices` slices each, a workgroup
+// of 64 * waves threads per slice
+struct DnLaunch {
+  int rows, cols, waves, tiles, slices;
+};
+// The launches of a plan; `scratch`: whether pairs have room for their sums
+int dn_launches(const DnPlan& pl, int k, int cus, bool scratch, DnLaunch out[2]) {
+  int count = 0;
+  if (pl.tile_cols == 128) {
+    if (pl.sk_tiles > 0)  // (at most one wave of tiles: all of them)
+      out[count++] = {128, 128, 8, pl.sk_tiles, pl.ksplit};
+    else if (scratch && dn_paired(pl, k, cus))
+      out[count++] = {128, 256, 4, pl.dp_tiles / 2, 2};
+    else
+      out[count++] = {128, 128, 8, pl.dp_tiles, 1};
+    return count;
+  }
+  // The stream-K tiles of large tiles (256 x 256: 128 x 256 ones are less than one
+  // wave, and more than half of one) are computed as 128 x 128 quarters in a
+  // launch of their own, in slices while that leaves compute units idle: 16
+  // tiles of 256 x 256 in four slices are 64 workgroups, a quarter of the chip
+  // for a quarter of a tile's time, their quarters 256 (4096 x 4352 x 4096
+  // 142 us with one launch for both, 125 with two; 6230 x 3072 x 1280 67 and 52).
+  if (pl.sk_tiles > 0) {
+    int slices = cus / (4 * pl.sk_tiles);
+    if (slices > pl.ksplit) slices = pl.ksplit;
+    out[count++] = {128, 128, 8, 4 * pl.sk_tiles, slices < 1 ? 1 : slices};
+  }
+  if (pl.dp_tiles > 0)
+    out[count++] = {pl.tile_rows, 256, dn_four_waves(pl.tile_rows, pl.dp_tiles, k, cus) ? 4 : 8, pl.dp_tiles, 1};
+  return count;
+}
+
 int dn_check(int m, int n, int k) {
   if (m < 0 || n < 0 || k < 0) return STREAMK_ERR_SHAPE;
   if (n % kDnTile != 0 || k % kDnStageK != 0) return STREAMK_ERR_SHAPE;
@@ -938,42 +987,22 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
       }
     }
     const DnPlan pl = dn_plan(m, n, k, cus);
-    // The stream-K tiles of large tiles are computed as 128 x 128 quarters in a
-    // launch of their own, in slices while that leaves compute units idle: 16
-    // tiles of 256 x 256 in four slices are 64 workgroups, a quarter of the chip
-    // for a quarter of a tile's time, their quarters 256 (4096 x 4352 x 4096
-    // 142 us with one launch for both, 125 with two; 6230 x 3072 x 1280 67 and 52).
-    const bool small = pl.tile_cols == 128;
-    const bool quarters = pl.tile_rows == kDnTile && pl.sk_tiles > 0;
-    const int cut_tiles = quarters ? 4 * pl.sk_tiles : pl.sk_tiles;
-    int slices = pl.ksplit;
-    if (quarters) {
-      if (slices > cus / cut_tiles) slices = cus / cut_tiles;
-      if (slices < 1) slices = 1;
-    }
     // only slices exchange anything
+    DnLaunch launches[2];
+    int count = dn_launches(pl, k, cus, true, launches);
     ScratchView view = {nullptr, nullptr};
-    if (cut_tiles > 0 && slices > 1 &&
-        !scratch_acquire(dev, stream, (size_t)cut_tiles * slices * DnSmall<128, 128>::kPartBytes, &view,
-                         g_dn_error, sizeof(g_dn_error)))
-      break;
-    // Problems of 128 x 128 tiles for more than half of the compute units, one
-    // workgroup each, wait for operands: a tile of 128 x 256 brings half as many
-    // rows of A per column, so in two slices along k the same workgroups take
-    // in three quarters of the bytes and run dense_kernel's loop.  The slices'
-    // meeting costs some 10 us, which a deep k earns back.  Twenty in a row, 128 x
-    // 128 against pairs: 777 x 4352 at k = 4096 35.3 and 35.9 us, 6144 50.9 and
-    // 47.3, 10240 79.9 and 71.1; 513 x 3584 28.6 and 30.0, 41.4 and 41.3, 65.9 and
-    // 62.2; 2048 x 2048 32.9 and 35.4, 48.1 and 47.5, 79.2 and 72.5.  Under
-    // capture, and where scratch cannot be had, the tiles are computed whole, in
-    // the same order of sums and so to the same bits: such a graph names no
-    // scratch, and may be replayed on any stream beside others.
-    const bool paired = small && pl.sk_tiles == 0 && 2 * pl.dp_tiles > cus && k >= kDnPairK;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool pairs = paired && hipStreamIsCapturing(stream, &capture) == hipSuccess &&
-                       capture == hipStreamCaptureStatusNone &&
-                       scratch_acquire(dev, stream, (size_t)pl.dp_tiles * DnShape<128>::kPartBytes, &view,
-                                       g_dn_error, sizeof(g_dn_error));
+    const DnLaunch& first = launches[0];  // (whole tiles come last)
+    if (first.slices > 1) {
+      const bool paired = dn_paired(pl, k, cus);
+      const size_t bytes = (size_t)first.tiles * first.slices * first.rows * first.cols * 4;
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      const bool may = !paired || (hipStreamIsCapturing(stream, &capture) == hipSuccess &&
+                                   capture == hipStreamCaptureStatusNone);
+      if (!may || !scratch_acquire(dev, stream, bytes, &view, g_dn_error, sizeof(g_dn_error))) {
+        if (!paired) break;
+        count = dn_launches(pl, k, cus, false, launches);
+      }
+    }
     (void)hipGetLastError();  // an earlier call's error is not this launch's
     DenseArgs a;
     a.A = A;
@@ -984,38 +1013,41 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     a.K = k;
     a.tiles_m = pl.tiles_m;
     a.tiles_n = pl.tiles_n;
-    a.dp_tiles = pl.dp_tiles;
-    a.sk_tiles = cut_tiles;
-    a.ksplit = slices;
-    a.quarters = quarters ? 1 : 0;
     a.locks = view.counters;
     a.scratch = view.partials;
     a.finish_polls = t_finish_polls < 0 ? kFinishPolls : t_finish_polls;
-    const auto launch = [&](auto kernel, int grid, int threads, int lds) {
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, a);
-    };
-    if (pairs) {
-      a.tiles_n = n / kDnTile;
-      a.dp_tiles = pl.dp_tiles / 2;
-      a.ksplit = 2;
-      launch(dense_kernel<128, true>, pl.dp_tiles, 256, DnShape<128>::kLds);
-    } else if (cut_tiles > 0) {
-      launch(dense_small_kernel<128, 128, true, false>, cut_tiles * slices, 512, DnSmall<128, 128>::kLds);
-    } else if (paired) {
-      launch(dense_small_kernel<128, 128, false, true>, pl.dp_tiles, 512, DnSmall<128, 128>::kLds);
-    } else if (small) {
-      launch(dense_small_kernel<128, 128, false, false>, pl.dp_tiles, 512, DnSmall<128, 128>::kLds);
-    }
-    if (!small && pl.dp_tiles > 0) {
-      const bool half = pl.tile_rows == 128, four = dn_four_waves(pl.tile_rows, pl.dp_tiles, k, cus);
-      if (half && four)
-        launch(dense_kernel<128, false>, pl.dp_tiles, 256, DnShape<128>::kLds);
-      else if (half)
-        launch(dense_small_kernel<128, 256, false, false>, pl.dp_tiles, 512, DnSmall<128, 256>::kLds);
-      else if (four)
-        launch(dense_kernel<256, false>, pl.dp_tiles, 256, DnShape<256>::kLds);
-      else
-        launch(dense_small_kernel<256, 256, false, false>, pl.dp_tiles, 512, DnSmall<256, 256>::kLds);
+    for (int i = 0; i < count; i++) {
+      const DnLaunch& l = launches[i];
+      const bool pairs = l.cols > pl.tile_cols;
+      if (pairs) a.tiles_n = n / l.cols;
+      // (tiles in slices, and quarters, are the ones after the whole tiles)
+      const bool cut = l.slices > 1 || l.rows < pl.tile_rows;
+      a.dp_tiles = pairs ? l.tiles : pl.dp_tiles;
+      a.sk_tiles = cut ? l.tiles : 0;
+      a.ksplit = l.slices;
+      a.quarters = l.rows < pl.tile_rows ? 1 : 0;
+      const auto launch = [&](auto kernel, int lds) {
+        hipLaunchKernelGGL(kernel, dim3(l.tiles * l.slices), dim3(64 * l.waves), lds, stream, a);
+      };
+      if (l.waves == 4) {
+        if (pairs)
+          launch(dense_kernel<128, true>, DnShape<128>::kLds);
+        else if (l.rows == 128)
+          launch(dense_kernel<128, false>, DnShape<128>::kLds);
+        else
+          launch(dense_kernel<256, false>, DnShape<256>::kLds);
+      } else if (l.cols == 128) {
+        if (cut)
+          launch(dense_small_kernel<128, 128, true, false>, DnSmall<128, 128>::kLds);
+        else if (dn_paired(pl, k, cus))
+          launch(dense_small_kernel<128, 128, false, true>, DnSmall<128, 128>::kLds);
+        else
+          launch(dense_small_kernel<128, 128, false, false>, DnSmall<128, 128>::kLds);
+      } else if (l.rows == 128) {
+        launch(dense_small_kernel<128, 256, false, false>, DnSmall<128, 256>::kLds);
+      } else {
+        launch(dense_small_kernel<256, 256, false, false>, DnSmall<256, 256>::kLds);
+      }
     }
     e = hipGetLastError();
     if (e != hipSuccess) {
@@ -1043,6 +1075,18 @@ int streamk_amd_plan(int m, int n, int k, int cus, int* out) {
   out[6] = pl.tile_rows;
   out[7] = pl.tile_cols;
   return STREAMK_OK;
+}
+
+int streamk_amd_launches(int m, int n, int k, int cus, int scratch, int* out) {
+  if (dn_check(m, n, k) != STREAMK_OK || m == 0 || n == 0 || k == 0) return 0;
+  DnLaunch launches[2];
+  const int count = dn_launches(dn_plan(m, n, k, cus), k, cus, scratch != 0, launches);
+  for (int i = 0; i < count; i++) {
+    const DnLaunch& l = launches[i];
+    const int fields[5] = {l.rows, l.cols, l.waves, l.tiles, l.slices};
+    for (int j = 0; j < 5; j++) out[5 * i + j] = fields[j];
+  }
+  return count;
 }
 
 void streamk_amd_tile_coord(int tile, int tiles_m, int tiles_n, int* out) {

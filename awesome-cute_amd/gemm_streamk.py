@@ -44,10 +44,15 @@ def run(m, n, k, repeat=200, warmup=5, seed=0, dev="cuda:0", log=print):
     A = (torch.rand((m, k), device=dev, generator=gen) * 4 - 2).half()
     B = (torch.rand((n, k), device=dev, generator=gen) * 4 - 2).half()
     C = torch.empty((m, n), dtype=torch.half, device=dev)
-    _, plan = streamk.plan(m, n, k, torch.cuda.get_device_properties(dev).multi_processor_count)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    _, plan = streamk.plan(m, n, k, cus)
+    launches = streamk.launches(m, n, k, cus, scratch=False)  # (timed from a graph)
     log(f"fp16 gemm m:{m} n:{n} k:{k}")
     log(f"output tiles: {plan['dp_tiles'] + plan['sk_tiles']}, dp tiles: {plan['dp_tiles']}, "
-        f"sk tiles: {plan['sk_tiles']} x {plan['k_slices']} slices, workgroups: {plan['grid']}")
+        f"sk tiles: {plan['sk_tiles']}")
+    for one in launches:
+        log(f"launch: {one['tiles']} tiles of {one['rows']} x {one['cols']} x {one['slices']} slices, "
+            f"{one['waves']} waves each")
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
         for _ in range(max(warmup, 1)):  # the first call on a stream allocates the scratch

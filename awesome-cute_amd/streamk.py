@@ -11,6 +11,8 @@ _lib.streamk_amd_check.restype = _I
 _lib.streamk_amd_check.argtypes = [_I, _I, _I]
 _lib.streamk_amd_plan.restype = _I
 _lib.streamk_amd_plan.argtypes = [_I, _I, _I, _I, _P]
+_lib.streamk_amd_launches.restype = _I
+_lib.streamk_amd_launches.argtypes = [_I, _I, _I, _I, _I, _P]
 _lib.streamk_amd_tile_coord.restype = None
 _lib.streamk_amd_tile_coord.argtypes = [_I, _I, _I, _P]
 _lib.streamk_amd_slice_coord.restype = None
@@ -31,6 +33,14 @@ def plan(m, n, k, cus=256):
     rc = _lib.streamk_amd_plan(m, n, k, cus, out)
     keys = ("tiles_m", "tiles_n", "dp_tiles", "sk_tiles", "k_slices", "grid", "tile_rows", "tile_cols")
     return rc, dict(zip(keys, out))
+
+
+def launches(m, n, k, cus=256, scratch=True):
+    """The launches that compute the tiles; `scratch`: whether there is room for partial sums."""
+    out = (ctypes.c_int * 10)()
+    count = _lib.streamk_amd_launches(m, n, k, cus, int(scratch), out)
+    keys = ("rows", "cols", "waves", "tiles", "slices")
+    return [dict(zip(keys, out[5 * i:5 * i + 5])) for i in range(count)]
 
 
 def tile_coord(tile, tiles_m, tiles_n):

@@ -42,14 +42,21 @@ int streamk_amd_check(int m, int n, int k);
  * SK_DP_Block_Wrapper, dp_sk_block.h:31-80): out[0..7] = tiles along m, tiles
  * along n (tiles numbered in panels of 8 column tiles), data-parallel tiles, stream-K
  * tiles (the last ones in tile order), k slices per stream-K tile, (tile, slice)
- * pairs (workgroups, except that the stream-K tiles of 256 x 256 are computed as
- * four 128 x 128 quarters each, in as many slices as leave none without a
- * compute unit, and from k = 7168, outside a capture, two neighbouring whole
- * 128 x 128 tiles as two slices of a 128 x 256 one), rows of a tile (256, or 128
- * when 256 x 256 tiles would occupy at most half
- * of the compute units), columns of a tile (256, or 128 when 128 x 256 tiles
- * would occupy at most half of them too) */
+ * pairs, rows of a tile (256, or 128 when 256 x 256 tiles would occupy at most
+ * half of the compute units), columns of a tile (256, or 128 when 128 x 256 tiles
+ * would occupy at most half of them too).  streamk_amd_launches says how the
+ * tiles are computed. */
 int streamk_amd_plan(int m, int n, int k, int cus, int* out);
+
+/* the launches that compute these tiles, at most two, five numbers each: rows and
+ * columns of a workgroup's tile, waves of a workgroup, tiles, slices of the k
+ * range per tile (a workgroup per tile and slice).  The stream-K tiles of 256 x 256
+ * are computed as four 128 x 128 quarters each, in as many slices as leave none
+ * without a compute unit; and from k = 7168, with scratch != 0, two neighbouring
+ * whole 128 x 128 tiles as two slices of a 128 x 256 one (a call under capture,
+ * or whose scratch cannot be had, goes without).  Returns their number; 0 for
+ * sizes that are refused or empty. */
+int streamk_amd_launches(int m, int n, int k, int cus, int scratch, int* out);
 
 /* out[0], out[1] = row and column tile of tile number `tile` (0 <= tile <
  * tiles_m * tiles_n); for tests of the numbering */

@@ -112,6 +112,39 @@ def test_tile_numbering_is_a_bijection_in_panels(streamk, tm, tn):
     assert {r for r, _ in first} == set(range(tm))
 
 
+def test_launches_cover_the_plan(streamk):
+    """Every tile of the plan is in a launch, whole, in quarters or two to a pair, and no launch of
+    slices has more workgroups than compute units."""
+    rng = np.random.default_rng(3)
+    seen = set()
+    for _ in range(3000):
+        m, n = int(rng.integers(1, 9000)), 256 * int(rng.integers(1, 40))
+        k = 64 * int(rng.integers(1, 180))
+        for scratch in (True, False):
+            _, p = streamk.plan(m, n, k)
+            launches = streamk.launches(m, n, k, scratch=scratch)
+            assert 1 <= len(launches) <= 2
+            area = sum(l["rows"] * l["cols"] * l["tiles"] for l in launches)
+            assert area == p["tile_rows"] * p["tile_cols"] * p["tiles_m"] * p["tiles_n"]
+            for l in launches:
+                assert l["waves"] in (4, 8) and (l["rows"], l["cols"]) in {(128, 128), (128, 256), (256, 256)}
+                assert l["slices"] == 1 or l["tiles"] * l["slices"] <= 256
+                pair = (l["cols"] > p["tile_cols"])
+                assert not pair or (scratch and k >= 7168 and l["slices"] == 2)
+                seen.add((l["rows"], l["cols"], l["waves"], l["slices"]))
+    assert {(128, 128, 8, 1), (128, 128, 8, 4), (128, 256, 4, 2), (128, 256, 4, 1), (128, 256, 8, 1),
+            (256, 256, 4, 1), (256, 256, 8, 1)} <= seen
+    assert streamk.launches(16, 256, 0) == [] and streamk.launches(16, 128, 64) == []
+
+
+@pytest.mark.parametrize("m,n,k,waves", [
+    (931, 5120, 768, 8), (1306, 3072, 3840, 8), (1306, 3072, 4096, 4), (1000, 8192, 3072, 4),
+    (1076, 7424, 1536, 8), (1076, 7424, 4096, 4), (1076, 7424, 5376, 8), (4096, 4096, 512, 8),
+    (4096, 4096, 1024, 4), (4096, 4096, 8192, 4)])
+def test_waves_of_whole_tiles(streamk, m, n, k, waves):
+    assert streamk.launches(m, n, k)[-1]["waves"] == waves
+
+
 @pytest.mark.parametrize("tiles,slices", [(1, 2), (108, 2), (64, 4), (85, 3), (63, 4), (128, 2), (7, 3)])
 def test_slices_of_a_tile_meet_in_one_xcd(streamk, tiles, slices):
     """Workgroups are dealt to the 8 XCDs round-robin: the slices of a tile go to one of them,

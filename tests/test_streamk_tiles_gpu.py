@@ -44,6 +44,9 @@ def _check(env, m, n, k, top, tile):
 @pytest.mark.parametrize("m,n,tile", [(1281, 8192, (256, 256)), (1535, 6400, (256, 256)), (601, 8192, (128, 256)),
                                       (767, 5632, (128, 256)), (1, 256, (128, 128)), (300, 1024, (128, 128))])
 def test_stages(env, m, n, stages, tile):
+    assert env[1].launches(m, n, 64 * stages)[0] == {
+        "rows": tile[0], "cols": tile[1], "waves": 8, "slices": 1,
+        "tiles": -(-m // tile[0]) * (n // tile[1])}
     _check(env, m, n, 64 * stages, 2, tile)
 
 
@@ -54,6 +57,7 @@ def test_stages(env, m, n, stages, tile):
                                         (1300, 3328, 6144, (128, 256)),  # 143 tiles, dealt out one by one
                                         (1076, 7424, 5120, (256, 256))])
 def test_deep_stages(env, m, n, k, stages, tile):
+    assert env[1].launches(m, n, k + 64 * stages)[0]["waves"] == (8 if m == 1076 else 4)
     _check(env, m, n, k + 64 * stages, 1, tile)
 
 
@@ -68,13 +72,21 @@ def test_deep_stages(env, m, n, k, stages, tile):
     (2048, 2048, 7168, (128, 128)), (129, 16384, 7232, (128, 128)),
 ])
 def test_slices(env, m, n, k, tile, polls):
+    import marlin
     torch, streamk = env
+    first = streamk.launches(m, n, k)[0]
+    sliced = first["slices"] > 1
+    assert sliced == (m != 5000) and (first["rows"], first["cols"]) == ((128, 256) if k >= 7168 else (128, 128))
+    marlin.release()
     streamk.force_finish_polls(polls)
     try:
         for _ in range(2):
             _check(env, m, n, k, 1, tile)
     finally:
         streamk.force_finish_polls(-1)
+    # the slices' sums had their room: nothing ran in the place of the launch above
+    sums = first["tiles"] * first["slices"] * first["rows"] * first["cols"] * 4
+    assert (marlin.scratch_bytes()[0] >= sums) if sliced else marlin.scratch_bytes() == (0, 0)
 
 
 def test_deep_tiles_under_capture(env):
