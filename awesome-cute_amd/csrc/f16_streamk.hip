@@ -40,10 +40,11 @@
 // lane's bytes land, the swizzle is applied to the address the lane fetches.
 //
 // What bounds it: LDS and the way into it, then the board's power.  The large
-// tiles with eight waves of 128 x 64 (twelve operand reads per 32 MFMAs) kept LDS
-// as busy as the matrix pipe; 128 x 128 per wave reads 16 per 64: 4096^3 101 ->
-// 96 us, 8192 x 8192 x 2048 217 -> 208, 1152 x 4352 x 4096 (128-row tiles) 50.8 ->
-// 49.5; 8192^3, at the power limit, 1.39 PFLOP/s either way.  The small tiles
+// tiles with eight waves of 128 x 64 take twelve operand reads per 32 MFMAs, with
+// 128 x 128 per wave 16 per 64: 4096^3 101 -> 96 us, 8192 x 8192 x 2048 217 -> 208,
+// where the operands stay in the last-level cache (the matrix pipe is then busy 76 %
+// of the cycles and LDS reads 21 %); 8192^3, at the power limit, 1.39 PFLOP/s
+// either way.  The small tiles
 // wait for operands: a compute unit takes in a stage's 32 KiB at 90 to 120 GB/s
 // from L2, 57 where A and B come from memory.
 #include <hip/hip_runtime.h>

@@ -13,9 +13,10 @@ move and spill them, and the LDS reads have to be placed and waited for one by
 one.
 
 Why that shape: every operand read from LDS (one ds_read_b128) feeds eight
-MFMAs.  With eight waves of 128 x 64 the reads of a stage and the loads' writes
-took LDS as long as the MFMAs took the matrix pipe (2048 of 2048 cycles at 128
-bytes a cycle); here they take 1536, and 896 instead of 1152 with 128-row tiles.
+MFMAs, 16 reads per 64 MFMAs where eight waves of 128 x 64 take 24, and 16 instead
+of 32 with 128-row tiles (64 x 64 each).  Fewer reads leave the matrix pipe more of
+the power that bounds the loop: 4096^3 101 -> 96 us, the pipe busy 76 % of the
+cycles, LDS reads 21 %.
 
 A step is 64 MFMAs: row blocks i = 0 ... 7 of 16 rows, operands o = 0 ... 7 of
 16 columns.  Its A operands are read three row blocks ahead into a ring of four,

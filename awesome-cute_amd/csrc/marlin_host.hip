@@ -711,7 +711,7 @@ int enqueue(const Plan& pl, const ScratchView& view, const void* A, const void* 
     a.row_parts = 1;
     a.part_rows = 0;
     a.finish_polls = t_force.finish_polls < 0 ? kFinishPolls : t_force.finish_polls;
-    // 128-row tiles: four waves with 128 x 128 accumulators; 64-row tiles: eight
+    // tiles of 80 to 128 rows: four waves with accumulators of all rows x 128 columns; 64-row tiles: eight
     // waves with 64 x 64
     rc = pl.tile_rows > 64 ? launch_prefill_wide(a, groupsize != -1, pl.tile_rows, pl.ksplit, stream)
                            : launch_prefill(a, groupsize != -1, pl.ksplit, stream);

@@ -6,7 +6,7 @@
 // a layer, so a decoder's linear layers ran at the host's pace.  Here they take
 // 3.3 and 5.0 us (of which the output's allocation 1.2), the launch itself
 // about 2.5: one row through the sixteen layers of four blocks of a 7B model
-// 200 -> 121 us, which is the kernels' time.
+// 206 -> 122 us on one box, 189 -> 135 on another.
 //
 // Tensors are allocated and the library is entered with the interpreter lock
 // released, as torch's own calls and ctypes do: a launch may wait for room in

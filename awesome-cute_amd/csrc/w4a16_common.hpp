@@ -165,7 +165,8 @@ struct GemmArgs {
   void* C;          // (M, N) fp16 row-major
   const void* S;    // (K/128, N) or (1, N) fp16, Marlin-permuted
   int M, N, K;
-  int* locks;       // N/128 counters, lock_stride ints apart; zero on entry and on exit
+  int* locks;       // a counter per column tile (streaming) or tile cut into slices
+                    // (prefill), lock_stride ints apart; zero on entry and on exit
   int lock_stride;  // >= 1; spreads the counters over separate cache lines
   float* scratch;   // partial sums of shared tiles (null if no tile is shared)
   int gpb;          // granules per workgroup (streaming kernel; the most, when wpt > 0)
