@@ -51,12 +51,13 @@ extern "C" {
  * library-owned buffer per (device, stream), sized by the call's plan and
  * grown on demand (hipMalloc on the first call that needs more; 64 KiB of tile
  * counters + whole MiB of partial sums, 4 MiB for N = K = 4096 at one row).  Nothing
- * is allocated while `stream` is being captured into a graph.  A call that would
- * have to then runs without scratch if it has the rows for the prefill kernel:
- * its tiles are computed whole instead of in slices of the k range, which may
- * take longer and may round the last bit of an element the other way.  Other
- * calls return MARLIN_ERR_RUNTIME.  Run the call once on that stream before the
- * capture, or use marlin_gemm_static.
+ * is allocated while `stream` is being captured into a graph, and no more than
+ * 256 buffers per device.  A call that cannot have its scratch for that runs
+ * without if it has the rows for the prefill kernel: its tiles are computed whole
+ * instead of in slices of the k range, which may take longer and may round the
+ * last bit of an element the other way.  Other calls return
+ * MARLIN_ERR_RUNTIME.  Run the call once on that stream before the capture, or use
+ * marlin_gemm_static.
  */
 int marlin_gemm(const void *A, const void *B, void *C, const void *s, int prob_m, int prob_n,
                 int prob_k, void *workspace, int groupsize, int dev, void *stream, int thread_k,
