@@ -25,6 +25,7 @@ SOURCES = {
     "w4a16_prefill_wide.hip": [],
     "w4a16_convert.hip": [],
     "f16_streamk.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "f16_tiles.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

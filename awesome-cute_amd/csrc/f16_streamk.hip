@@ -23,7 +23,7 @@
 //
 // dense_small_kernel: eight waves, two per SIMD, of half the tile's rows and a
 // quarter of its columns each.  128 x 128 tiles, whole or in slices: the problems
-// with few tiles, and the stream-K tiles of the others, every 256 x 256 tile of
+// with few tiles (those with fewer still go to f16_tiles.hip), and the stream-K tiles of the others, every 256 x 256 tile of
 // the partial wave as four of its own.  And the large whole tiles over a shallow
 // k, where its shorter start and end count for more than dense_kernel's loop.
 //
@@ -54,6 +54,7 @@
 #include <type_traits>
 
 #include "../../include/streamk_amd.h"
+#include "f16_dense.hpp"
 #include "scratch_pool.hpp"
 #include "w4a16_common.hpp"
 
@@ -62,8 +63,6 @@ namespace w4a16 {
 namespace {
 
 constexpr int kDnTile = 256;     // rows and columns of the large tile of C
-constexpr int kDnStageK = 64;    // k depth of a stage (two MFMA k steps); k is a multiple
-constexpr int kDnOob = (int)0x80000000;
 
 // Tiles of dense_kernel, TM rows and 256 columns: 256 x 256 or 128 x 256
 template <int TM>
@@ -100,96 +99,14 @@ struct DnSmall {
   static constexpr int kPartBytes = TM * TN * 4;
 };
 constexpr int kDnMaxSlots = 256;  // slices in flight per launch
-constexpr int kDnMaxSlices = 4;
 constexpr int kDnPairK = 7168;    // depth from which 128 x 256 tiles in two slices beat 128 x 128 ones
 constexpr int kDnRunsK = 6144;    // depth from which 128 x 256 tiles are not dealt out in runs, see there
-constexpr int kDnCounterStride = 16;  // ints: a tile's slices meet in a cache line of their own
-
-struct DenseArgs {
-  const void* A;
-  const void* B;
-  void* C;
-  int M, N, K;
-  int tiles_m, tiles_n;
-  int dp_tiles;  // tiles computed by one workgroup each
-  // dense_small_kernel, in a launch of its own: the tiles after the first
-  // dp_tiles, in ksplit slices each; with quarters, the plan's tiles are 256 x
-  // 256 and computed as four tiles each
-  int sk_tiles;
-  int ksplit;
-  int quarters;
-  int* locks;        // one zeroed counter per cut tile, kDnCounterStride ints apart, zero again afterwards
-  float* scratch;    // kPartBytes per slice
-  int finish_polls;  // looks at a tile's other slices before leaving them a share
-};
-
-// Tiles are numbered panel by panel: a panel is kDnPanel column tiles wide
-// (the last one narrower), and inside a panel the column tile runs fastest, or
-// the row tile where there are fewer than kDnPanel of them.  A run of
-// consecutive tile numbers then covers a compact block of C, so the workgroups
-// that share an L2 read few distinct rows of A and B, and with few row tiles
-// every row of B comes from memory into one L2 only (777 x 4352 x 10240: 91.5 us,
-// with columns first 98.7).
-constexpr int kDnPanel = 8;
-__host__ __device__ __forceinline__ void dn_tile_coord(int t, int tiles_m, int tiles_n, int* tm,
-                                                       int* tn) {
-  const int per_panel = tiles_m * kDnPanel;
-  const int p = t / per_panel;
-  const int first = p * kDnPanel;
-  const int width = tiles_n - first < kDnPanel ? tiles_n - first : kDnPanel;
-  const int o = t - p * per_panel;
-  if (tiles_m < kDnPanel) {
-    *tn = first + o / tiles_m;
-    *tm = o - (*tn - first) * tiles_m;
-  } else {
-    *tm = o / width;
-    *tn = first + o - *tm * width;
-  }
-}
-
-// (tile, slice) of a workgroup of dense_small_kernel: the slices of a tile are
-// neighbours behind one L2, where they meet.  With the slices of one k range as
-// neighbours instead, rows of B were shared by more tiles, but the sums passed
-// between XCDs: 2226 x 768 x 1536 15.3 us, with this 12.9; 560 x 2560 x 2304 17.0
-// and 15.0; four slices, 488 x 2048 x 1152 15.6 and 11.2; 350 x 2048 x 4096 17.9 and
-// 15.0; quarters, 4096 x 4352 x 4096 118.0 and 118.2.
-__host__ __device__ __forceinline__ void dn_slice_coord(int block, int tiles, int slices, int* tile,
-                                                        int* slice) {
-  const int work = xcd_work_index(block, tiles * slices);
-  *tile = work / slices;
-  *slice = work - *tile * slices;
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t dn_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
 
 // the four words of a raw buffer resource: 48-bit base, stride 0, size in
 // bytes, data format flags
 __device__ __forceinline__ i4 dn_rsrc_words(const void* p, unsigned bytes) {
   const unsigned long long a = (unsigned long long)p;
   return (i4){(int)(unsigned)a, (int)(unsigned)((a >> 32) & 0xffffu), (int)bytes, 0x00020000};
-}
-
-// 16 bytes per lane from a buffer straight into LDS: lane l's bytes land at
-// dst + 16*l (dst is wave-uniform).  The instruction's immediate offset stays
-// zero: the hardware would add it to the LDS address as well.  (Device pass
-// only; the host pass just needs the kernel's launch stub.)
-__device__ __forceinline__ void dn_dma16(__amdgpu_buffer_rsrc_t rsrc, char* dst, int voffset,
-                                         int soffset) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, voffset, soffset, 0, 0);
-#endif
-}
-
-// LDS reads of a main loop, outside the compiler's dependence tracking (it
-// would wait for every load in flight before each of them)
-template <int OFF>
-__device__ __forceinline__ void dn_read16(unsigned at, i4& v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF) : "memory");
-#endif
 }
 
 // wait until at most PENDING later LDS reads are outstanding; `v` is the
@@ -218,8 +135,6 @@ __device__ __forceinline__ void drain_reads(i4 (&a)[4], i4 (&b)[4], i4 (&f)[4]) 
 }
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding)
 constexpr int dn_vm_lgkm0(int n) { return (n & 15) | (7 << 4) | (0 << 8) | ((n >> 4) << 14); }
-// s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
-constexpr int dn_vmcnt(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 
 }  // namespace
 
@@ -273,10 +188,6 @@ __device__ __forceinline__ void dense_write_tile(const char* smem, char* out, ha
       }
     }
   }
-}
-
-__device__ __forceinline__ h4 dense_round(f4 v) {
-  return (h4){(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
 }
 
 // SLICED (128 rows): every tile is cut into p.ksplit slices of the k range,
@@ -774,6 +685,7 @@ constexpr int kDnMaxDevices = 16;
 
 thread_local char g_dn_error[256] = "";
 thread_local int t_finish_polls = -1;  // streamk_amd_force_finish_polls
+thread_local DnTile t_tile = {0, 0, 0};  // streamk_amd_force_tile
 
 void dn_set_error(hipError_t e, const char* what) {
   snprintf(g_dn_error, sizeof(g_dn_error), "%s: %s", what, hipGetErrorString(e));
@@ -896,6 +808,25 @@ int dn_launches(const DnPlan& pl, int k, int cus, bool scratch, DnLaunch out[2])
   return count;
 }
 
+// The tiles of less than 128 x 128 that compute the problem in place of dn_launches
+// (rows = 0: none).  Only where those would be 128 x 128 tiles, at most one per
+// compute unit, and only in slices where those are in slices, and no more of them:
+// the room acquired for their sums then holds these as well, and what a stream must
+// have seen before it can be captured does not depend on a choice that is a matter
+// of speed.
+DnTile dn_small_tile(const DnPlan& pl, int m, int n, int k, int cus) {
+  const int most = pl.tile_cols == 128 && pl.sk_tiles > 0 ? pl.ksplit : 1;
+  if (t_tile.rows < 0) return {0, 0, 0};
+  if (t_tile.rows > 0) {
+    DnTile t = t_tile;
+    const int tiles = ceil_div(m, t.rows) * (n / t.cols);
+    if (t.slices > most || tiles > kMaxCounters / kDnCounterStride) t.slices = 1;
+    return t;
+  }
+  if (pl.tile_cols != 128 || dn_paired(pl, k, cus)) return {0, 0, 0};
+  return dn_tile(m, n, k, cus, most);
+}
+
 int dn_check(int m, int n, int k) {
   if (m < 0 || n < 0 || k < 0) return STREAMK_ERR_SHAPE;
   if (n % kDnTile != 0 || k % kDnStageK != 0) return STREAMK_ERR_SHAPE;
@@ -980,6 +911,7 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
         if (e == hipSuccess)
           e = hipFuncSetAttribute((const void*)dense_small_kernel<256, 256, false, false>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, DnSmall<256, 256>::kLds);
+        if (e == hipSuccess) e = configure_dense_tiles();
         if (e != hipSuccess) {
           dn_set_error(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
           break;
@@ -991,6 +923,7 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     // only slices exchange anything
     DnLaunch launches[2];
     int count = dn_launches(pl, k, cus, true, launches);
+    const DnTile small = dn_small_tile(pl, m, n, k, cus);
     ScratchView view = {nullptr, nullptr};
     const DnLaunch& first = launches[0];  // (whole tiles come last)
     if (first.slices > 1) {
@@ -1017,6 +950,10 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     a.locks = view.counters;
     a.scratch = view.partials;
     a.finish_polls = t_finish_polls < 0 ? kFinishPolls : t_finish_polls;
+    if (small.rows > 0) {
+      launch_dense_tiles(a, small, stream);
+      count = 0;  // in place of the plan's launches
+    }
     for (int i = 0; i < count; i++) {
       const DnLaunch& l = launches[i];
       const bool pairs = l.cols > pl.tile_cols;
@@ -1078,6 +1015,17 @@ int streamk_amd_plan(int m, int n, int k, int cus, int* out) {
   return STREAMK_OK;
 }
 
+int streamk_amd_tile(int m, int n, int k, int cus, int* out) {
+  out[0] = out[1] = out[2] = 0;
+  const int rc = dn_check(m, n, k);
+  if (rc != STREAMK_OK || m == 0 || n == 0 || k == 0) return rc;
+  const DnTile t = dn_small_tile(dn_plan(m, n, k, cus), m, n, k, cus);
+  out[0] = t.rows;
+  out[1] = t.cols;
+  out[2] = t.slices;
+  return STREAMK_OK;
+}
+
 int streamk_amd_launches(int m, int n, int k, int cus, int scratch, int* out) {
   if (dn_check(m, n, k) != STREAMK_OK || m == 0 || n == 0 || k == 0) return 0;
   DnLaunch launches[2];
@@ -1100,6 +1048,12 @@ void streamk_amd_slice_coord(int block, int tiles, int slices, int* out) {
 
 void streamk_amd_force_finish_polls(int polls) {
   t_finish_polls = polls < 0 || polls > kFinishPolls ? -1 : polls;
+}
+
+void streamk_amd_force_tile(int rows, int cols, int slices) {
+  const bool exists = dn_tile_exists(rows, cols);
+  t_tile = {rows < 0 ? -1 : exists ? rows : 0, exists ? cols : 0,
+            slices < 1 ? 1 : slices > kDnMaxSlices ? kDnMaxSlices : slices};
 }
 
 long long streamk_amd_release(int dev) { return (long long)scratch_release(dev); }

@@ -1,0 +1,382 @@
+// Dense fp16 GEMM on small tiles, 32 x 32 to 64 x 128: the problems that have too
+// few 128 x 128 tiles for the compute units.  Same operands, slabs and order of
+// MFMA operands as the kernels of f16_streamk.hip.
+//
+// What bounds such a problem is latency: the launch, the first loads, and per
+// stage a barrier and the trip of its operands from LDS, about 0.18 us whatever
+// the tile.  In slices of 128 x 128 tiles it also paid for the slices' meeting,
+// some 4 us of a launch of 9.  Small tiles fill the compute units without slices,
+// unless k is deep and C so small that even these leave most of the chip idle.
+// Measured, slices of 128 x 128 tiles against this kernel (us): 291 x 1280 x 896
+// 9.2 and 4.5, 1024^3 11.4 and 5.9, 777 x 2048 x 1024 11.1 and 7.9, 64 x 2048 x
+// 4096 13.8 and 8.6, 100 x 512 x 10240 22.7 and 9.3.
+//
+// A wave computes 16 or 32 rows x 16 or 32 columns.  Per 64-deep stage it reads
+// all operands of the next stage from LDS while the MFMAs of this one run, so a
+// slab is free again as soon as every wave has its operands, and one barrier per
+// stage does.  The ring holds as many slabs as leave room for a second workgroup
+// on the compute unit (64 x 128: one workgroup and six slabs, 48 KiB more in
+// flight: 777 x 2048 x 1024 7.9 us, with three slabs and room for a second one
+// 8.2).  Operands loaded straight from memory into registers, with the waves along
+// k and no barrier at all, took two to three times as long: sixteen rows of 64
+// bytes per load instruction.
+#include <hip/hip_runtime.h>
+
+#include "f16_dense.hpp"
+#include "scratch_pool.hpp"
+
+namespace w4a16 {
+
+namespace {
+
+// TM x TN tiles, WM x WN waves
+template <int TM, int TN, int WM, int WN, int RING>
+struct DnTiles {
+  static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
+  static constexpr int kRB = TM / 16 / WM, kNJ = TN / 16 / WN;  // operands of a wave per k step
+  static constexpr int kOps = 2 * (kRB + kNJ);                  // ... per stage
+  static constexpr int kSlabA = TM * 128, kSlab = kSlabA + TN * 128;
+  static constexpr int kTA = TM / 8 / kWaves, kTB = TN / 8 / kWaves;  // load instructions per wave and slab
+  static constexpr int kLoads = kTA + kTB;
+  static constexpr int kPitch = TN * 2 + 16;  // bytes per row of the fp16 tile in LDS
+  static constexpr int kRingBytes = RING * kSlab, kTileBytes = TM * kPitch;
+  static constexpr int kLds = kRingBytes > kTileBytes ? kRingBytes : kTileBytes;
+  static constexpr int kPartBytes = TM * TN * 4;
+  static_assert(kTA * 8 * kWaves == TM && kTB * 8 * kWaves == TN, "whole instructions");
+  static_assert(kRB >= 1 && kRB <= 2 && kNJ >= 1 && kNJ <= 2, "operands that the reads below name");
+};
+
+// wait for every LDS read in flight; the registers are named so that they count
+// as in use up to here
+template <int N>
+__device__ __forceinline__ void dn_landed(i4 (&v)[N]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(N == 4 || N == 6 || N == 8, "");
+  if constexpr (N == 4)
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+  else if constexpr (N == 6)
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
+  else
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]),
+                   "+v"(v[7]));
+#endif
+}
+
+}  // namespace
+
+// p.tiles_m x p.tiles_n tiles, all of them in p.ksplit slices (CUT) or whole
+template <int TM, int TN, int WM, int WN, int RING, bool CUT>
+__global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
+  using Sh = DnTiles<TM, TN, WM, WN, RING>;
+  constexpr int RB = Sh::kRB, NJ = Sh::kNJ, TA = Sh::kTA, TB = Sh::kTB;
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // Sh::kLds
+  __shared__ int s_shares;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int kg = lane >> 4;
+  const int nu = lane & 15;
+  const int wm = wave / WN;
+  const int wn = wave % WN;
+
+  int tile, ks = 0;
+  if constexpr (CUT)
+    dn_slice_coord((int)blockIdx.x, p.tiles_m * p.tiles_n, p.ksplit, &tile, &ks);
+  else
+    tile = xcd_work_index((int)blockIdx.x, p.tiles_m * p.tiles_n);
+  int tm, tn;
+  dn_tile_coord(tile, p.tiles_m, p.tiles_n, &tm, &tn);
+  const int m0 = TM * tm, n0 = TN * tn;
+  const int rows = min(TM, p.M - m0);
+  const __amdgpu_buffer_rsrc_t rA =
+      dn_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
+  const __amdgpu_buffer_rsrc_t rB =
+      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)TN * (unsigned)p.K * 2u);
+
+  // a wave fetches its share of the rows of A and of B, eight rows per
+  // instruction; rows past the end of A repeat the last one (never stored)
+  int a_src[TA], b_src[TB];
+  {
+    const int r8 = lane >> 3, c = (lane & 7) ^ r8;
+#pragma unroll
+    for (int t = 0; t < TA; t++) {
+      const int r = 8 * (TA * wave + t) + r8;
+      a_src[t] = (r < rows ? r : rows - 1) * p.K * 2 + 16 * c;
+    }
+#pragma unroll
+    for (int t = 0; t < TB; t++) b_src[t] = (8 * (TB * wave + t) + r8) * p.K * 2 + 16 * c;
+  }
+  // this workgroup's stages (at most 4 slices of at most 2^24 stages: 32 bits do)
+  const int all = p.K / kDnStageK;
+  const int st0 = CUT ? (int)((unsigned)ks * (unsigned)all / (unsigned)p.ksplit) : 0;
+  const int st1 = CUT ? (int)((unsigned)(ks + 1) * (unsigned)all / (unsigned)p.ksplit) : all;
+  const int stages = st1 - st0;
+
+  auto issue_slab = [&](int s, int slot) {
+    const int inv = s < stages ? 0 : kDnOob;  // a stage past the end fetches zeros
+    const int at = (st0 + s) * (kDnStageK * 2);
+    char* const base = smem + slot * Sh::kSlab;
+#pragma unroll
+    for (int t = 0; t < TA; t++) dn_dma16(rA, base + (TA * wave + t) * 1024, a_src[t] | inv, at);
+#pragma unroll
+    for (int t = 0; t < TB; t++)
+      dn_dma16(rB, base + Sh::kSlabA + (TB * wave + t) * 1024, b_src[t] | inv, at);
+  };
+
+  // operands of a stage, per k step B then A; where they sit in slab 0
+  unsigned a_rd[2], b_rd[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const unsigned sw = 16 * ((4 * h + kg) ^ (nu & 7));
+    a_rd[h] = (unsigned)(size_t)smem + (16 * RB * wm + nu) * 128 + sw;
+    b_rd[h] = (unsigned)(size_t)smem + Sh::kSlabA + (16 * NJ * wn + nu) * 128 + sw;
+  }
+  auto read = [&](i4 (&o)[Sh::kOps], unsigned slab) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      i4* const b = o + h * (RB + NJ);
+      dn_read16<0>(b_rd[h] + slab, b[0]);
+      if constexpr (NJ == 2) dn_read16<2048>(b_rd[h] + slab, b[1]);
+      dn_read16<0>(a_rd[h] + slab, b[NJ]);
+      if constexpr (RB == 2) dn_read16<2048>(a_rd[h] + slab, b[NJ + 1]);
+    }
+  };
+
+  f4 acc[RB][NJ];
+#pragma unroll
+  for (int i = 0; i < RB; i++)
+#pragma unroll
+    for (int j = 0; j < NJ; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](i4 (&o)[Sh::kOps]) {
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(h8, o[h * (RB + NJ) + j]),
+              __builtin_bit_cast(h8, o[h * (RB + NJ) + NJ + i]), acc[i][j], 0, 0, 0);
+  };
+
+  // Every slot requested; slab 0 landed (loads complete in order), its operands
+  // read.  The reads are written by hand (the compiler would wait for every load
+  // in flight before each of them); between the reads into a set of registers and
+  // the wait that names them stand the MFMAs of the other set and nothing else.
+  i4 even[Sh::kOps], odd[Sh::kOps];
+#pragma unroll
+  for (int r = 0; r < RING; r++) issue_slab(r, r);
+  __builtin_amdgcn_s_waitcnt(dn_vmcnt((RING - 1) * Sh::kLoads));
+  __builtin_amdgcn_s_barrier();
+  read(even, 0);
+  dn_landed(even);
+  int slot = 0;
+  // Stage s, its operands in `cur`: once my loads of the next slab have landed and
+  // everybody's have (the barrier, which every wave reaches with its operands of
+  // this slab in registers), read the next stage's operands, request the slab
+  // after the ring's last in this one's place, and multiply.
+  auto stage = [&](int s, i4 (&cur)[Sh::kOps], i4 (&next)[Sh::kOps]) {
+    __builtin_amdgcn_s_waitcnt(dn_vmcnt((RING - 2) * Sh::kLoads));
+    __builtin_amdgcn_s_barrier();
+    const int slot_next = slot == RING - 1 ? 0 : slot + 1;
+    __builtin_amdgcn_sched_barrier(0);
+    read(next, slot_next * Sh::kSlab);
+    issue_slab(s + RING, slot);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(cur);
+    __builtin_amdgcn_sched_barrier(0);
+    dn_landed(next);
+    slot = slot_next;
+  };
+  int s = 0;
+  for (; s + 1 < stages; s += 2) {
+    stage(s, even, odd);
+    stage(s + 1, odd, even);
+  }
+  if (s < stages) multiply(even);
+  // nothing of the ring may still be on its way when LDS is reused
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+
+  // a lane holds, per (i, j), row 16i + nu and four consecutive columns; the tile
+  // leaves through LDS as whole rows, the parts of the waves in `waves`
+  char* const out = smem + (16 * RB * wm + nu) * Sh::kPitch + (16 * NJ * wn + 4 * kg) * 2;
+  half_t* const C = (half_t*)p.C + (size_t)m0 * p.N + n0;
+  auto put = [&](int i, int j, f4 v) { *(h4*)(out + 16 * i * Sh::kPitch + 32 * j) = dense_round(v); };
+  auto store = [&](int waves) {
+    __syncthreads();
+    constexpr int PR = TN / 8;  // 16-byte pieces of a row
+#pragma unroll
+    for (int at0 = 0; at0 < TM * PR; at0 += Sh::kThreads) {
+      const int at = at0 + tid;
+      const int m = at / PR, c = at % PR;
+      if ((TM * PR % Sh::kThreads != 0 && at >= TM * PR) || m >= rows ||
+          !(waves >> (m / (16 * RB) * WN + c / (2 * NJ)) & 1))
+        continue;
+      // nobody reads C again in this launch
+      __builtin_nontemporal_store(*(const i4*)(smem + m * Sh::kPitch + c * 16),
+                                  (i4*)(C + (size_t)m * p.N + c * 8));
+    }
+  };
+  if constexpr (!CUT) {
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+      for (int j = 0; j < NJ; j++) put(i, j, acc[i][j]);
+    store(-1);
+  } else {
+    // slices: as in dense_small_kernel, the pieces of a tile being its waves' parts
+    const __amdgpu_buffer_rsrc_t rP = dn_rsrc(p.scratch, 0x7fffffffu);
+    int* const word = &p.locks[tile * kDnCounterStride];
+    const int at = wave * (RB * NJ * 1024) + lane * 16;
+    const auto part = [&](int k2) { return (tile * p.ksplit + k2) * Sh::kPartBytes; };
+    const auto write_out = [&](int waves) {
+      if (waves >> wave & 1) {
+#pragma unroll
+        for (int e = 0; e < RB * NJ; e++)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, acc[e / NJ][e % NJ]), rP,
+                                                 at + e * 1024, part(ks), 16 /* sc1 */);
+      }
+      __builtin_amdgcn_s_waitcnt(dn_vmcnt(0));  // my stores have been acknowledged
+      __syncthreads();
+    };
+    const int my_share = finish_pieces(1 << ks, p.ksplit, Sh::kWaves);
+    write_out(~my_share);
+    if (tid == 0) s_shares = finish_arrive(word, p.ksplit, ks, p.finish_polls);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_shares) == 0) {
+      write_out(my_share);
+      if (tid == 0) s_shares = finish_abandon(word, p.ksplit, ks);
+      __syncthreads();
+    }
+    const int waves = __builtin_amdgcn_readfirstlane(finish_pieces(s_shares, p.ksplit, Sh::kWaves));
+    if (waves >> wave & 1) {
+      f4 v[RB * NJ][kDnMaxSlices];  // all of it requested at once
+#pragma unroll
+      for (int e = 0; e < RB * NJ; e++)
+#pragma unroll
+        for (int x = 0; x < kDnMaxSlices; x++)
+          v[e][x] = x >= p.ksplit ? (f4){0.f, 0.f, 0.f, 0.f}
+                    : x == ks     ? acc[e / NJ][e % NJ]
+                                  : __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                               rP, at + e * 1024, part(x), 16 /* sc1 */));
+#pragma unroll
+      for (int e = 0; e < RB * NJ; e++) {
+        f4 sum = v[e][0];
+#pragma unroll
+        for (int x = 1; x < kDnMaxSlices; x++) sum += v[e][x];
+        put(e / NJ, e % NJ, sum);
+      }
+    }
+    store(waves);
+    if (tid == 0) finish_leave(word, p.ksplit);
+  }
+}
+
+namespace {
+
+// calls f(kernel, LDS bytes, threads) for the tile's kernel
+template <class F>
+void with_tile_kernel(int rows, int cols, bool cut, F f) {
+  const auto one = [&](auto shape, auto whole, auto sliced) {
+    using Sh = decltype(shape);
+    f(cut ? sliced : whole, Sh::kLds, Sh::kThreads);
+  };
+#define DN_TILE(TM, TN, WM, WN, RING)                                                       \
+  if (rows == TM && cols == TN)                                                             \
+  return one(DnTiles<TM, TN, WM, WN, RING>{}, dense_tile_kernel<TM, TN, WM, WN, RING, false>, \
+             dense_tile_kernel<TM, TN, WM, WN, RING, true>)
+  DN_TILE(32, 32, 2, 2, 8);
+  DN_TILE(32, 64, 2, 2, 6);
+  DN_TILE(64, 64, 2, 4, 4);
+  DN_TILE(64, 128, 2, 4, 6);
+#undef DN_TILE
+}
+
+}  // namespace
+
+bool dn_tile_exists(int rows, int cols) {
+  bool found = false;
+  with_tile_kernel(rows, cols, false, [&](auto, int, int) { found = true; });
+  return found;
+}
+
+hipError_t configure_dense_tiles() {
+  hipError_t e = hipSuccess;
+  for (const int rows : {32, 64})
+    for (const int cols : {32, 64, 128})
+      for (const bool cut : {false, true})
+        with_tile_kernel(rows, cols, cut, [&](auto kernel, int lds, int) {
+          if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        });
+  return e;
+}
+
+void launch_dense_tiles(DenseArgs a, const DnTile& t, hipStream_t stream) {
+  a.tiles_m = ceil_div(a.M, t.rows);
+  a.tiles_n = a.N / t.cols;
+  a.ksplit = t.slices;
+  with_tile_kernel(t.rows, t.cols, t.slices > 1, [&](auto kernel, int lds, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.tiles_n * t.slices), dim3(threads), lds, stream, a);
+  });
+}
+
+// Costs in us, fitted to launches of 260 problems (m = 1 ... 8192, n = 512 ...
+// 8192, k = 512 ... 10240, 128 x 128 tiles for at most one wave of compute units;
+// 5 to 7 % rms): a launch, its stages (dearer the fuller the chip), those of
+// workgroups beyond one per compute unit, the slices' meeting.
+static double dn_tile_cost(int rows, int cols, int tiles, int stages, int slices, int cus) {
+  struct Fit {
+    int rows, cols;
+    double launch, stage, fill, more, more_stage, meet, slice;
+  };
+  static const Fit fits[] = {{32, 32, 2.23, 0.084, 0.017, 0.89, 0.079, 2.24, 0.08},
+                             {32, 64, 2.38, 0.118, 0.031, 1.12, 0.124, 2.35, 0.30},
+                             {64, 64, 2.56, 0.159, 0.036, 0.98, 0.187, 2.14, 0.40},
+                             {64, 128, 3.14, 0.232, 0.074, 7.28, 0.287, 3.00, 0.46}};
+  for (const Fit& f : fits) {
+    if (f.rows != rows || f.cols != cols) continue;
+    const double r = (double)tiles * slices / cus;
+    // workgroups beyond one per compute unit: half way between the rounds they
+    // make and their share of one
+    const double more = r > 1.0 ? 0.5 * (ceil_div(tiles * slices, cus) + r) - 1.0 : 0.0;
+    const int st = ceil_div(stages, slices);
+    return f.launch + f.more * more + st * (f.stage + f.fill * (r < 1.0 ? r : 1.0) + f.more_stage * more) +
+           (slices > 1 ? f.meet + f.slice * slices : 0.0);
+  }
+  return 1e30;
+}
+
+// The cheapest small tile, if it is 3 % cheaper than 128 x 128 ones (costs fitted
+// to the same problems: 4.5 % rms in slices, 3 % whole).  In 2 or 4 slices (waves
+// share a tile unevenly with 3), at most one workgroup per compute unit.  Over the
+// 260 problems that is 1.466 times the speed of 128 x 128 tiles, the best choice
+// for each 1.480; none is slower than it was.
+DnTile dn_tile(int m, int n, int k, int cus, int max_slices) {
+  const int stages = k / kDnStageK;
+  const int large = ceil_div(m, 128) * (n / 128);
+  const double fill = (double)large * max_slices / cus;
+  const double large_cost =
+      max_slices > 1 ? 6.48 + 0.30 * max_slices + (double)stages / max_slices * (0.294 + 0.258 * fill)
+                     : 3.62 + stages * (0.259 + 0.252 * fill);
+  DnTile best = {0, 0, 0};
+  double best_cost = large_cost;
+  for (const DnTile& t : {DnTile{32, 32, 1}, DnTile{32, 64, 1}, DnTile{64, 64, 1}, DnTile{64, 128, 1}}) {
+    const int tiles = ceil_div(m, t.rows) * (n / t.cols);
+    if (tiles > 5 * cus) continue;  // (beyond what was fitted; never the best there)
+    for (int s = 1; s <= max_slices && s <= 4; s *= 2) {
+      if (s > 1 && (tiles * s > cus || tiles > kMaxCounters / kDnCounterStride)) break;
+      const double c = 1.03 * dn_tile_cost(t.rows, t.cols, tiles, stages, s, cus);
+      if (c < best_cost) {
+        best = {t.rows, t.cols, s};
+        best_cost = c;
+      }
+    }
+  }
+  return best;
+}
+
+}  // namespace w4a16

@@ -44,11 +44,22 @@ int streamk_amd_check(int m, int n, int k);
  * tiles (the last ones in tile order), k slices per stream-K tile, (tile, slice)
  * pairs, rows of a tile (256, or 128 when 256 x 256 tiles would occupy at most
  * half of the compute units), columns of a tile (256, or 128 when 128 x 256 tiles
- * would occupy at most half of them too).  streamk_amd_launches says how the
- * tiles are computed. */
+ * would occupy at most half of them too).  streamk_amd_launches and
+ * streamk_amd_tile say how the problem is computed. */
 int streamk_amd_plan(int m, int n, int k, int cus, int* out);
 
-/* the launches that compute these tiles, at most two, five numbers each: rows and
+/* out[0..2] = rows, columns and k slices of the tiles of less than 128 x 128 that
+ * compute the problem, in one launch of a workgroup per tile and slice, in place
+ * of streamk_amd_launches: 32 x 32, 32 x 64, 64 x 64 or 64 x 128, where that is
+ * cheaper; zeros where it is not.  Returns what streamk_amd_check does. */
+int streamk_amd_tile(int m, int n, int k, int cus, int* out);
+
+/* the tile for every problem of the calling thread, whatever its cost, in at most
+ * the plan's slices: rows = 0 back to the choice by cost, < 0 never a small tile;
+ * for tests and tools */
+void streamk_amd_force_tile(int rows, int cols, int slices);
+
+/* the launches that compute the plan's tiles, at most two, five numbers each: rows and
  * columns of a workgroup's tile, waves of a workgroup, tiles, slices of the k
  * range per tile (a workgroup per tile and slice).  The stream-K tiles of 256 x 256
  * are computed as four 128 x 128 quarters each, in as many slices as leave none
