@@ -63,8 +63,9 @@ __device__ __forceinline__ int quantised(half_t w, float s, float r) {
   q = __builtin_fmaf(e, r, q);
   if (__builtin_expect(!(__builtin_fabsf(e) < __builtin_inff()), 0)) q = x / s;
   const float h = (float)(half_t)q;
-  // a NaN becomes 0 and an infinity the largest integer, which wraps
-  const int i = (int)((unsigned)__float2int_rn(h) + 8u);
+  // a NaN becomes 0 and an infinity the largest integer, which wraps (said in so
+  // many words: of an integer sum the compiler keeps the clamp at 15)
+  const int i = h == __builtin_inff() ? -8 : __float2int_rn(h) + 8;
   return i < 0 ? 0 : i > 15 ? 15 : i;
 }
 

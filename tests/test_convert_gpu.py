@@ -80,6 +80,27 @@ def test_pack_is_the_tensor_sequence(env, k, n, gs, by_column):
         _same(torch, layer.s, marlin.pack_scales(s, groups > 1))
 
 
+@pytest.mark.parametrize("by_column", [False, True])
+def test_pack_takes_any_half(env, by_column):
+    """Every bit pattern as a weight, under scales of any bits: zeros, infinities, NaN, negative
+    and subnormal ones, quotients beyond a half and beyond an integer."""
+    torch, marlin = env
+    gen = torch.Generator(device="cuda:0")
+    k = n = 256
+    linear = torch.nn.Linear(k, n, bias=False, device="cuda:0", dtype=torch.half)
+    layer = marlin.Layer(k, n, 128).to("cuda:0")
+    for seed in range(8):
+        gen.manual_seed(seed)
+        w = torch.randperm(65536, device="cuda:0", generator=gen).to(torch.int16).view(torch.half).reshape(n, k)
+        s = torch.randint(-32768, 32768, (n, 2), device="cuda:0", generator=gen).to(torch.int16).view(torch.half)
+        s[:6, 0] = torch.tensor([0.0, -0.0, float("inf"), float("nan"), 2.0 ** -24, 65504.0])
+        s[6:n // 2] = torch.rand((n // 2 - 6, 2), device="cuda:0", generator=gen).half() * 0.02
+        linear.weight.data = w if by_column else w.t().contiguous().t()
+        layer.pack(linear, s)
+        q = torch.clamp(torch.round(w.t() / s.t().repeat_interleave(128, 0)).int() + 8, 0, 15)
+        assert torch.equal(layer.B.cpu(), marlin.pack_weights(q.cpu()))
+
+
 @pytest.mark.parametrize("k,n", [(16, 64), (48, 576), (256, 1088)])
 def test_packed_integers(env, k, n):
     torch, marlin = env
