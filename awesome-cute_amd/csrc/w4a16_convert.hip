@@ -7,8 +7,9 @@
 // passes over the weight, half of them over 64-bit integers (n = 11008, k =
 // 4096: 1712 us for the pair).  Here each is one pass: the quantiser reads a
 // weight once (twice where a group does not fit into registers) and writes its
-// 6 bytes, the packer reads it once and writes its half byte: 97 us for the
-// pair, 70 of it the quantiser.
+// 6 bytes, the packer reads it once and writes its half byte: 91 us for the
+// pair, 65 of it the quantiser, whose traffic alone (read, write, nothing computed)
+// takes 68.
 //
 // Every rounding is that of the tensor operations: fp16(w / s) is the rounded
 // fp32 quotient rounded once more, the integer is rounded half to even, and
@@ -67,6 +68,24 @@ __device__ __forceinline__ int quantised(half_t w, float s, float r) {
   // many words: of an integer sum the compiler keeps the clamp at 15)
   const int i = h == __builtin_inff() ? -8 : __float2int_rn(h) + 8;
   return i < 0 ? 0 : i > 15 ? 15 : i;
+}
+
+// quantised() of two halves with one scale, in bits 0-3 and 16-19.  Numbers are
+// clamped to -8 ... 7 as halves and rounded to whole ones by adding 1544: halves
+// from 1024 to 2048 are whole, sums are rounded half to even, and the low four bits
+// of 1544 + i are those of 8 + i.  Quotients that no half is near (a zero or infinite
+// operand, NaN, overflow) go through quantised().
+__device__ __forceinline__ int quantised_pair(half_t a, half_t b, float s, float r) {
+  const float x = (float)a, y = (float)b;
+  float p = x * r, q = y * r;
+  p = __builtin_fmaf(__builtin_fmaf(-p, s, x), r, p);
+  q = __builtin_fmaf(__builtin_fmaf(-q, s, y), r, q);
+  if (__builtin_expect(!(__builtin_fabsf(p) < 65520.f) || !(__builtin_fabsf(q) < 65520.f), 0))
+    return quantised(a, s, r) | (quantised(b, s, r) << 16);
+  const h2 top = {(half_t)7.f, (half_t)7.f}, bottom = {(half_t)-8.f, (half_t)-8.f};
+  const h2 whole = {(half_t)1544.f, (half_t)1544.f};
+  const h2 v = {(half_t)p, (half_t)q};
+  return as_int(__builtin_elementwise_max(__builtin_elementwise_min(v, top), bottom) + whole) & 0x000f000f;
 }
 
 template <int N>
@@ -227,18 +246,39 @@ struct PackArgs {
 // 16j + c and 16j + c + 8 (reference marlin.py:29-48): thread (t, 8 columns)
 // reads those four rows, has one half of eight words, and exchanges four
 // halves with the thread of the other eight columns.  Four t and sixteen
-// column threads in a wave: a row is read in runs of 256 bytes, and a store
-// instruction writes runs of 64.
+// column threads in a wave: a row is read in runs of 256 bytes.  A thread then
+// has four c of one j, and exchanges them with the threads of the other three j
+// for four j of one c, 16 bytes of B: 32 threads store 512 bytes in a row.
+// (Stored as words, every 16 bytes, and quantised one by one: n = 11008, k = 4096,
+// weights from memory, 31.2 us; so 23.4, 4.8 TB/s.)
 template <bool INTS>
 __global__ __launch_bounds__(kPThreads) void pack_rows(PackArgs p) {
   const int t = threadIdx.x & 3;
   const int c0 = ((int)blockIdx.x * (kPThreads / 4) + (int)(threadIdx.x >> 2)) * 8;
-  if (c0 >= p.n) return;  // (both threads of an exchange or neither: n is a multiple of 64)
+  if (c0 >= p.n) return;  // (all threads of an exchange or none: n is a multiple of 64)
   const int kt = blockIdx.y;
   int half[8];
-  Columns<8> col;
-  if (!INTS) {
+  if constexpr (INTS) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = 16 * kt + 2 * t + (r & 1) + 8 * (r >> 1);
+      const int shift = 16 * (r & 1) + 4 * (r >> 1);
+      const int* const q = (const int*)p.w + (size_t)row * p.n + c0;
+      int v[8];
+      *(i4*)v = *(const i4*)q;
+      *(i4*)(v + 4) = *(const i4*)(q + 4);
+#pragma unroll
+      for (int i = 0; i < 8; i++) half[i] = r == 0 ? v[i] : half[i] | (v[i] << shift);
+    }
+  } else {
+    h8 w[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = 16 * kt + 2 * t + (r & 1) + 8 * (r >> 1);
+      w[r] = *(const h8*)((const half_t*)p.w + (size_t)row * p.n + c0);
+    }
     const int g = 16 * kt / p.gs;
+    Columns<8> col;
     half_t sv[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -250,64 +290,84 @@ __global__ __launch_bounds__(kPThreads) void pack_rows(PackArgs p) {
 #pragma unroll
       for (int i = 0; i < 8; i++) out[scale_slot(c0 + i, p.grouped)] = sv[i];
     }
-  }
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int row = 16 * kt + 2 * t + (r & 1) + 8 * (r >> 1);
-    const int shift = 16 * (r & 1) + 4 * (r >> 1);
-    const size_t at = (size_t)row * p.n + c0;
-    int v[8];
-    if (INTS) {
-      *(i4*)v = *(const i4*)((const int*)p.w + at);
-      *(i4*)(v + 4) = *(const i4*)((const int*)p.w + at + 4);
-    } else {
-      const h8 w = *(const h8*)((const half_t*)p.w + at);
-#pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = quantised(w[i], col.s[i], col.r[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; i++) half[i] = r == 0 ? v[i] : half[i] | (v[i] << shift);
+    for (int i = 0; i < 8; i++)
+      half[i] = quantised_pair(w[0][i], w[1][i], col.s[i], col.r[i]) |
+                (quantised_pair(w[2][i], w[3][i], col.s[i], col.r[i]) << 4);
   }
   const int odd = (c0 >> 3) & 1;  // columns 8 ... 15 of their sixteen
-  int* B = p.B + (size_t)kt * 2 * p.n + (c0 >> 6) * 128 + ((c0 >> 4) & 3) + 4 * t;
+  const int j0 = (c0 >> 4) & 1, j1 = (c0 >> 5) & 1;
+  int word[4];  // c = i + 4 odd, my j
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int got = __shfl_xor(odd ? half[i] : half[i + 4], 4);
     // even: c = i with the partner's columns above; odd: c = i + 4
-    const int word = odd ? got | (half[i + 4] << 8) : half[i] | (got << 8);
-    B[16 * (i + 4 * odd)] = word;
+    word[i] = odd ? got | (half[i + 4] << 8) : half[i] | (got << 8);
   }
+  int pair[2][2];  // c = 2i + j0 + 4 odd; j = its second index + 2 j1
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int got = __shfl_xor(j0 ? word[2 * i] : word[2 * i + 1], 8);
+    pair[i][0] = j0 ? got : word[2 * i];
+    pair[i][1] = j0 ? word[2 * i + 1] : got;
+  }
+  i4 out;  // c = 2 j1 + j0 + 4 odd, all j
+#pragma unroll
+  for (int x = 0; x < 2; x++) {
+    const int got = __shfl_xor(j1 ? pair[0][x] : pair[1][x], 16);
+    out[x] = j1 ? got : pair[0][x];
+    out[2 + x] = j1 ? pair[1][x] : got;
+  }
+  *(i4*)(p.B + (size_t)kt * 2 * p.n + (c0 >> 6) * 128 + 16 * (2 * j1 + j0 + 4 * odd) + 4 * t) = out;
 }
 
-// Fake weights stored column by column, (n, k): a thread takes 64 k-values of
-// one column (a whole cache line), a wave a 64-column block, whose four rows of
-// B it writes completely.
+// Fake weights stored column by column, (n, k): a wave takes 64 k-values of a
+// 64-column block, eight lanes a column's 128 bytes at a time, and writes four
+// rows of B of it completely.  A thread then has eight k-values (low or high
+// ones of a row of B, by its lane's lowest bit) of columns 8 i + lane / 8, both
+// halves of sixteen columns, and exchanges with its neighbour: the even one takes
+// t = 0, 1, the odd one 2, 3, all j of them, 32 bytes in a row.  (With a column per
+// lane, whose load instructions touch 64 lines each, n = 11008, k = 4096 took 50
+// us, so 27.3.)
 __global__ __launch_bounds__(kPThreads) void pack_columns(PackArgs p) {
   const int lane = threadIdx.x & 63;
   const int blk = (int)blockIdx.x;
   const int k0 = ((int)blockIdx.y * (kPThreads / kWave) + (int)(threadIdx.x >> 6)) * 64;
   if (k0 >= p.k) return;
-  const int c = blk * 64 + lane;
+  const int c = blk * 64 + (lane >> 3), chunk = lane & 7, odd = lane & 1;
+  const h8* src = (const h8*)((const half_t*)p.w + (size_t)c * p.k + k0) + chunk;
+  h8 w[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) w[i] = src[(size_t)i * p.k];
   const int g = k0 / p.gs;
-  const half_t sv = p.scales[g * p.s_group + c * p.s_col];
-  const float s = (float)sv, rs = __builtin_amdgcn_rcpf(s);
-  if (k0 == g * p.gs) p.s_packed[(size_t)g * p.n + scale_slot(c, p.grouped)] = sv;
-  const h8* src = (const h8*)((const half_t*)p.w + (size_t)c * p.k + k0);
-  const int hi = (lane >> 3) & 1;
+  half_t sv[8];
 #pragma unroll
-  for (int kt = 0; kt < 4; kt++) {
-    const h8 a = src[2 * kt], b = src[2 * kt + 1];
-    int half[4];
+  for (int i = 0; i < 8; i++) sv[i] = p.scales[g * p.s_group + (c + 8 * i) * p.s_col];
+  if (chunk == 0 && k0 == g * p.gs) {
+    half_t* const out = p.s_packed + (size_t)g * p.n;
 #pragma unroll
-    for (int t = 0; t < 4; t++)
-      half[t] = quantised(a[2 * t], s, rs) | (quantised(a[2 * t + 1], s, rs) << 16) |
-                (quantised(b[2 * t], s, rs) << 4) | (quantised(b[2 * t + 1], s, rs) << 20);
-    int* B = p.B + (size_t)(k0 / 16 + kt) * 2 * p.n + blk * 128 + 16 * (lane & 7) + (lane >> 4);
+    for (int i = 0; i < 8; i++) out[scale_slot(c + 8 * i, p.grouped)] = sv[i];
+  }
+  int half[4][4];  // [t][j]: my four bits of both columns
 #pragma unroll
-    for (int i = 0; i < 2; i++) {  // columns c: words t = 0, 1; columns c + 8: t = 2, 3
-      const int got = __shfl_xor(hi ? half[i] : half[i + 2], 8);
-      B[4 * (i + 2 * hi)] = hi ? got | (half[i + 2] << 8) : half[i] | (got << 8);
+  for (int i = 0; i < 8; i++) {
+    const float s = (float)sv[i], rs = __builtin_amdgcn_rcpf(s);
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const int v = quantised_pair(w[i][2 * t], w[i][2 * t + 1], s, rs);
+      half[t][i >> 1] = (i & 1) == 0 ? v : half[t][i >> 1] | (v << 8);
     }
+  }
+  int* const B = p.B + (size_t)((k0 >> 4) + (chunk >> 1)) * 2 * p.n + blk * 128 + 16 * (lane >> 3) + 8 * odd;
+#pragma unroll
+  for (int x = 0; x < 2; x++) {
+    i4 out;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int got = __shfl_xor(odd ? half[x][j] : half[2 + x][j], 1);
+      out[j] = odd ? got | (half[2 + x][j] << 4) : half[x][j] | (got << 4);
+    }
+    *(i4*)(B + 4 * x) = out;
   }
 }
 
