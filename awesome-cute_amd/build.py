@@ -21,6 +21,7 @@ SOURCES = {
     "scratch_pool.hip": [],
     "w4a16_stream.hip": [],
     "w4a16_strip.hip": [],
+    "w4a16_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "w4a16_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "w4a16_prefill_wide.hip": [],
     "w4a16_convert.hip": [],

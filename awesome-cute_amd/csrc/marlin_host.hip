@@ -63,7 +63,8 @@ bool configure_device(int dev) {
   std::lock_guard<std::mutex> lk(g_mu);
   if (g_dev[dev].configured) return true;
   if (configure_stream_kernels() != 0 || configure_prefill_kernels() != 0 ||
-      configure_prefill_wide_kernels() != 0 || configure_strip_kernels() != 0) {
+      configure_prefill_wide_kernels() != 0 || configure_strip_kernels() != 0 ||
+      configure_rows_kernels() != 0) {
     set_error(hipGetLastError(), "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
     return false;
   }
@@ -141,7 +142,12 @@ struct Force {
   int kernel = 0, k_slices = 0, tile_rows = 0;
   int row_halves = 0;  // streaming kernel: 0 = by cost, 1 = never cut the rows, 2 = cut them where possible
   int strips = 0;      // column-strip kernel: 0 = by cost, or 1 to 4 strips per workgroup
+  int rows_strips = 0, rows_blocks = 0;  // rows of a strip set in one workgroup: 0 = by cost, strips -1 = never
   int finish_polls = -1;  // looks at the other slices of a tile before leaving; -1 = kFinishPolls
+  bool any() const {
+    return kernel != 0 || k_slices != 0 || tile_rows != 0 || row_halves != 0 || strips != 0 ||
+           rows_strips != 0 || finish_polls >= 0;
+  }
 };
 thread_local Force t_force;
 
@@ -663,6 +669,115 @@ Plan make_plan(int m, int n, int k, int sms, const PlanCtx& cx) {
   return pl;
 }
 
+// The strips and row blocks of 16 of a workgroup of w4a16_rows.hip where that
+// kernel computes the problem in place of the plan (strips 0: not).
+struct RowsPlan {
+  int strips, blocks;
+};
+
+// Fitted time (us) of that kernel: a launch, the meeting of the waves' sums, the
+// activations and weights a workgroup takes in and what it computes, dearer the
+// fuller the chip, the same again for workgroups beyond one per compute unit (half
+// way between the rounds they make and their share of one), and the weights'
+// way from memory.  2800 launches over 320 problems, M = 17 ... 1500, N = 512 ...
+// 28672, K = 512 ... 13824; 6 % rms.
+double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx) {
+  const int wgs = ceil_div(n / 16, strips) * ceil_div(m, 16 * blocks);
+  const double r = (double)wgs / cx.cus;
+  const double fill = r < 1.0 ? r : 1.0;
+  const double more = r > 1.0 ? 0.5 * (ceil_div(wgs, cx.cus) + r) - 1.0 : 0.0;
+  const double K = k / 1000.0, sums = strips * blocks;
+  const double memory = 0.5e-7 * n * k;
+  if (cx.grouped)
+    return 2.88 + 0.167 * sums +
+           K * (0.335 * blocks + 0.239 * strips + fill * (0.075 * blocks + 0.033 * strips) +
+                more * (0.297 * blocks + 0.202 * strips + 0.080 * sums)) +
+           0.240 * more * sums + 0.180 * memory;
+  return 2.71 + 0.174 * sums +
+         K * (0.363 * blocks + 0.186 * strips + fill * (0.086 * blocks + 0.032 * strips) +
+              more * (0.285 * blocks + 0.188 * strips + 0.039 * sums)) +
+         0.294 * more * sums + 0.149 * memory;
+}
+
+// For 17 rows and more, where it is 4 % cheaper than the plan -- by the plan's own
+// fits, which on these problems read 3 to 7 % low with group scales, 1 % high to 4 %
+// low without (the factors below).  Not over k ranges below 640, nor, with 16 rows
+// per workgroup, below 2048: a wave has a chunk or two there, which the column strips
+// take in at once (M = 51, N = 11520, K = 512 5.7 us streaming, 6.6 by the fit's
+// choice; M = 123, N = 512, K = 1536 4.1 and 5.0).  Over the 320 problems it is taken
+// for half, which makes all of them 1.074 times as fast, the best choice for each
+// 1.094, and three 2 to 4 % slower.  M = 46, N = 18432, K = 4480 29.2 -> 18.4 us, 45 x
+// 12288 x 4096 15.1 -> 12.9, 144 x 2048 x 1792 9.0 -> 6.6, 501 x 1024 x 2176 11.1 -> 8.5.
+RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& cx) {
+  if (cx.force.rows_strips > 0 && sms <= 0) return {cx.force.rows_strips, cx.force.rows_blocks};
+  if (sms > 0 || m <= 16 || k < 640 || cx.force.any()) return {0, 0};
+  double limit;
+  if (pl.kernel == 1)
+    limit = stream_cost_as_planned(m, n, k, cx) * (cx.grouped ? 1.03 : 0.99);
+  else if (pl.kernel == 2)
+    limit = prefill_cost(m, n, k, cx) * (cx.grouped ? 1.03 : 1.04);
+  else
+    limit = strip_cost(m, n, k, pl.strips, cx.cus) * (cx.grouped ? 1.07 : 1.0);
+  limit /= 1.04;
+  // the pairs, and how much longer than the fit each takes
+  static const struct {
+    int strips, blocks;
+    double by;
+  } pairs[] = {{1, 1, 1.06}, {2, 1, 0.97}, {3, 1, 1.03}, {2, 2, 0.96}, {3, 2, 1.08}, {4, 2, 1.00},
+               {6, 2, 0.97}, {2, 3, 0.99}, {3, 3, 1.03}, {4, 3, 0.97}, {5, 3, 0.98}, {6, 3, 0.98},
+               {4, 4, 0.98}, {5, 4, 1.00}, {6, 4, 0.98}, {7, 4, 1.02}};
+  RowsPlan best = {0, 0};
+  for (const auto& p : pairs) {
+    if (m <= 16 * (p.blocks - 1) || (p.blocks == 1 && k < 2048)) continue;  // (fewer blocks hold all rows)
+    // (beyond what was fitted, and never the best there)
+    if (ceil_div(n / 16, p.strips) * ceil_div(m, 16 * p.blocks) > 2.7 * cx.cus) continue;
+    const double c = rows_cost(m, n, k, p.strips, p.blocks, cx) * p.by;
+    if (c < limit) {
+      best = {p.strips, p.blocks};
+      limit = c;
+    }
+  }
+  return best;
+}
+
+// A thread's last plans, by everything that they are made from (no overrides among
+// it): planning takes the host up to a microsecond, a third of a launch, and a
+// decoder calls the same few sizes over and over.
+struct Planned {
+  int m = 0, n = 0, k = 0, sms = 0, cus = 0, counters = 0;
+  size_t partial_limit = 0;
+  bool grouped = false;
+  Plan plan;
+  RowsPlan rows;
+};
+constexpr int kPlansKept = 32;
+thread_local Planned t_plans[kPlansKept];
+
+Planned make_plans(int m, int n, int k, int sms, const PlanCtx& cx) {
+  Planned p;
+  p.m = m;
+  p.n = n;
+  p.k = k;
+  p.sms = sms;
+  p.cus = cx.cus;
+  p.counters = cx.counters;
+  p.partial_limit = cx.partial_limit;
+  p.grouped = cx.grouped;
+  p.plan = make_plan(m, n, k, sms, cx);
+  p.rows = rows_plan(m, n, k, sms, p.plan, cx);
+  return p;
+}
+
+Planned plans_for(int m, int n, int k, int sms, const PlanCtx& cx) {
+  if (cx.force.any()) return make_plans(m, n, k, sms, cx);
+  const unsigned mix = (unsigned)m * 0x9e3779b1u ^ (unsigned)n * 0x85ebca6bu ^ (unsigned)k * 0xc2b2ae35u;
+  Planned& kept = t_plans[(mix >> 16) % kPlansKept];
+  if (kept.m != m || kept.n != n || kept.k != k || kept.sms != sms || kept.cus != cx.cus ||
+      kept.counters != cx.counters || kept.partial_limit != cx.partial_limit || kept.grouped != cx.grouped)
+    kept = make_plans(m, n, k, sms, cx);
+  return kept;
+}
+
 // Enqueue the launches of plan pl with the scratch of `view` (null pointers
 // when the plan exchanges nothing through scratch).
 int enqueue(const Plan& pl, const ScratchView& view, const void* A, const void* B, void* C,
@@ -741,6 +856,22 @@ int enqueue(const Plan& pl, const ScratchView& view, const void* A, const void* 
   return rc;
 }
 
+int enqueue_rows(const RowsPlan& rows, const void* A, const void* B, void* C, const void* s, int m,
+                 int n, int k, int groupsize, hipStream_t stream) {
+  (void)hipGetLastError();  // an earlier call's error is not this launch's
+  GemmArgs a = {};
+  a.A = A;
+  a.B = B;
+  a.C = C;
+  a.S = s;
+  a.M = m;
+  a.N = n;
+  a.K = k;
+  const int rc = launch_rows(a, groupsize != -1, rows.strips, rows.blocks, stream);
+  if (rc == MARLIN_ERR_RUNTIME) set_error(w4a16::last_launch_error(), "kernel launch");
+  return rc;
+}
+
 // With `dev` current: this device's copy of the fixed scratch array.  Its
 // counters need no clearing: the array is zero when the module is loaded and
 // every launch hands its counters back zeroed.  (A clearing kernel on the first
@@ -797,7 +928,8 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
   if (cus > 0 && configure_device(dev)) {
     PlanCtx cx = {cus, use_static ? kStaticPartialBytes : kPoolPartialLimit, t_force, groupsize != -1};
     cx.counters = max_par > 16 ? 16 : max_par;  // the counters of a tile sit that many ints apart
-    Plan pl = make_plan(m, n, k, sms, cx);
+    const Planned planned = plans_for(m, n, k, sms, cx);
+    Plan pl = planned.plan;
     ScratchView view = {nullptr, nullptr};
     bool ok = true;
     if (use_static) {
@@ -831,7 +963,11 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
         ok = pl.partial_bytes == 0;
       }
     }
-    if (ok)
+    // (with the plan's scratch in hand: what a stream must have seen before it can be
+    // captured does not depend on a choice that is a matter of speed)
+    if (ok && planned.rows.strips > 0)
+      rc = enqueue_rows(planned.rows, A, B, C, s, m, n, k, groupsize, stream);
+    else if (ok)
       rc = enqueue(pl, view, A, B, C, s, m, n, k, workspace, groupsize, max_par, stream);
   }
   if (prev != dev) (void)hipSetDevice(prev);
@@ -933,6 +1069,19 @@ int marlin_amd_plan(int prob_m, int prob_n, int prob_k, int groupsize, int threa
   return rc;
 }
 
+int marlin_amd_rows_plan(int prob_m, int prob_n, int prob_k, int groupsize, int cus, int* out) {
+  out[0] = out[1] = 0;
+  int thread_k = -1, thread_n = -1;
+  int rc = check_shape(prob_m, prob_n, prob_k, groupsize, thread_k, thread_n);
+  if (rc != MARLIN_OK || prob_m == 0 || prob_n == 0 || prob_k == 0) return rc;
+  const PlanCtx cx = {cus, kPoolPartialLimit, t_force, groupsize != -1};
+  const RowsPlan rows =
+      rows_plan(prob_m, prob_n, prob_k, -1, make_plan(prob_m, prob_n, prob_k, -1, cx), cx);
+  out[0] = rows.strips;
+  out[1] = 16 * rows.blocks;
+  return rc;
+}
+
 int marlin_amd_plan_costs(int prob_m, int prob_n, int prob_k, int groupsize, int cus, double* out) {
   for (int i = 0; i < 4; i++) out[i] = -1.0;
   int thread_k = -1, thread_n = -1;
@@ -960,6 +1109,12 @@ void marlin_amd_force_row_halves(int mode) { t_force.row_halves = mode == 1 || m
 
 void marlin_amd_force_tile_rows(int rows) {
   t_force.tile_rows = rows >= 64 && rows <= 128 && rows % 16 == 0 ? rows : 0;
+}
+
+void marlin_amd_force_rows(int strips, int blocks) {
+  const bool exists = rows_exist(strips, blocks);
+  t_force.rows_strips = strips < 0 ? -1 : exists ? strips : 0;
+  t_force.rows_blocks = exists ? blocks : 0;
 }
 
 void marlin_amd_force_finish_polls(int polls) {

@@ -258,6 +258,12 @@ int launch_stream(const GemmArgs& a, bool group, int grid, hipStream_t stream);
 constexpr int kStripMaxRows = 1024;
 int configure_strip_kernels();
 int launch_strip(const GemmArgs& a, bool group, int strips, hipStream_t stream);
+// any rows in parts of 16 `blocks`, `strips` 16-column strips per workgroup, over
+// the whole k range (w4a16_rows.hip); not every pair exists
+constexpr int kRowsMaxStrips = 7, kRowsMaxBlocks = 4;
+bool rows_exist(int strips, int blocks);
+int configure_rows_kernels();
+int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream_t stream);
 // ksplit >= 1 slices of the k range per tile; above 1 the launch needs
 // a.scratch (ksplit * tiles * tile bytes of fp32) and a.locks (one zeroed
 // counter per tile, zero again afterwards)

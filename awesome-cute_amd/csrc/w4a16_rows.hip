@@ -1,0 +1,358 @@
+// Column strips with up to 64 rows per workgroup: a workgroup owns CS 16-column
+// strips (w4a16_strip.hip says what a strip is) and 16 MB rows over the whole k
+// range.  For 17 rows and more, where a workgroup per 16 rows unpacks every weight
+// several times, and a column tile that shares its k range among workgroups pays
+// for their meeting (2 to 4 us of a launch of 10 to 15).
+//
+// What bounds it: what a compute unit takes in, 55 to 60 GB/s with all of them at
+// work -- 32 MB k bytes of activations from the L2s beside 8 CS k bytes of weights
+// -- and what its LDS takes in, 64 bytes per clock whatever the width of the stores
+// (reads come at 230).  So the activations go straight to LDS (buffer_load ... lds)
+// and are read once, as whole operands: sets of strips and rows are chosen to keep
+// both streams short (rows_plan in marlin_host.hip).  M = 45, N = 12288, K = 4096:
+// 15.1 us streaming, 12.7 so; M = 46, N = 18432, K = 4480 29.2 and 18.4.
+//
+// Eight waves split the k range into contiguous runs of chunks of 64 k-values and
+// meet once, at the end: no barrier in the loop, no scratch, no counters.  The
+// weights of a chunk are fetched 16 bytes per lane, four rows of B, and pass
+// through LDS into operand order.  MFMA lane (kg, nu) takes the sixteen k-values of
+// row kg of the four for column slot nu -- word j = (nu/2)%4 of the Marlin lanes
+// (t, c = 2s + e), t = 0 ... 3, e = nu/8 -- so that an activation operand is eight
+// neighbouring k-values of a row, 16 bytes.
+//
+// The more chunks a wave has in flight the longer each takes to come: two where
+// strips and rows are few (a launch then waits for its first ones), else one, whose
+// successor is requested before its arithmetic (M = 45, N = 12288, K = 4096: one
+// 12.9 us, two 13.6; M = 111, N = 512, K = 4992, one strip and 16
+// rows: two 6.6 us).
+#include <type_traits>
+
+#include "w4a16_common.hpp"
+
+namespace w4a16 {
+
+namespace {
+
+constexpr int kRowsOob = (int)0x80000000;  // offset past any buffer (sizes are < 2 GiB)
+constexpr int kRowsWaves = 8;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+
+// 16 bytes per lane from a buffer straight into LDS, lane l's at dst + 16*l
+__device__ __forceinline__ void rows_dma16(__amdgpu_buffer_rsrc_t rsrc, char* dst, int voffset,
+                                           int soffset) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, voffset, soffset, 0, 0);
+#endif
+}
+
+// LDS accesses of the loop, outside the compiler's dependence tracking (it would
+// wait for every load in flight before each of them)
+template <int OFF>
+__device__ __forceinline__ void rows_read16(unsigned at, i4& v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF) : "memory");
+#endif
+}
+template <int DW0, int DW1>  // offsets in dwords
+__device__ __forceinline__ void rows_read2(unsigned at, i2& v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("ds_read2_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(at), "n"(DW0), "n"(DW1) : "memory");
+#endif
+}
+__device__ __forceinline__ void rows_write16(unsigned at, i4 v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("ds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory");
+#endif
+}
+// s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
+constexpr int rows_vmcnt(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
+
+template <int N, class F>
+__device__ __forceinline__ void rows_each(F f) {
+  if constexpr (N > 0) {
+    rows_each<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+}  // namespace
+
+template <int CS, int MB, int DEPTH>
+struct RowsShape {
+  static constexpr int kBLoads = (CS + 1) / 2;  // of 1 KiB per wave and chunk, eight lines of 128 bytes
+  static constexpr int kALoads = 2 * MB;        // ... eight rows
+  static constexpr int kSlot = 2048 * MB;       // activations of a chunk
+  static constexpr int kBRow = CS * 128 + 16;   // a row of B in LDS
+  static constexpr int kStagePerWave = DEPTH * kSlot + 4 * kBRow;
+  // the waves' sums meet through LDS in passes of at most 16 blocks of 16 x 16
+  static constexpr int kBlocks = CS * MB;
+  static constexpr int kPasses = (kBlocks + 15) / 16;
+  static constexpr int kPass = (kBlocks + kPasses - 1) / kPasses;
+  static constexpr int kReduce = kRowsWaves * kPass * 1024;
+  static constexpr int kLds =
+      kRowsWaves * kStagePerWave > kReduce ? kRowsWaves * kStagePerWave : kReduce;
+  static_assert(kLds <= 160 * 1024, "LDS of a compute unit");
+};
+
+template <int CS, int MB, bool GROUP, int DEPTH>
+__global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
+  using Sh = RowsShape<CS, MB, DEPTH>;
+  constexpr int NA = Sh::kALoads, NB = Sh::kBLoads;
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // Sh::kLds
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int kg = lane >> 4;
+  const int nu = lane & 15;
+  // the parts of a strip set are neighbours behind one L2 (p.gpb carries the grid)
+  const int wid = xcd_work_index((int)blockIdx.x, p.gpb);
+  const int set = wid / p.row_parts;
+  const int row0 = 16 * MB * (wid - set * p.row_parts);
+  const int strip0 = set * CS;
+  const int n_strips = p.N >> 4;  // (the last set may have fewer strips than CS)
+
+  // my chunks [c0, c1): whole groups where there are groups
+  const int chunks = p.K / 64;
+  const int c0 = GROUP ? 2 * (wave * (chunks / 2) / kRowsWaves) : wave * chunks / kRowsWaves;
+  const int c1 = GROUP ? 2 * ((wave + 1) * (chunks / 2) / kRowsWaves) : (wave + 1) * chunks / kRowsWaves;
+
+  const __amdgpu_buffer_rsrc_t rB = rows_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
+  const __amdgpu_buffer_rsrc_t rA = rows_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
+  const __amdgpu_buffer_rsrc_t rS =
+      rows_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
+  const int b_row = p.N * 8;  // bytes per row of B
+
+  char* const stage = smem + wave * Sh::kStagePerWave;
+  const unsigned lds_a = (unsigned)(size_t)stage, lds_b = lds_a + DEPTH * Sh::kSlot;
+  // weights: lines in the order [row][strip]; lanes past the last line fetch
+  // nothing and write to the padding
+  int b_src[NB];
+  unsigned b_wr[NB];
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    const int line = 8 * i + lane / 8, row = line / CS, strip = strip0 + line % CS;
+    const bool on = line < 4 * CS;
+    b_src[i] = on && strip < n_strips ? row * b_row + 128 * strip + 16 * (lane % 8) : kRowsOob;
+    b_wr[i] = lds_b + (on ? row * Sh::kBRow + 128 * (line % CS) + 16 * (lane % 8) : 3 * Sh::kBRow + CS * 128);
+  }
+  const unsigned b_rd = lds_b + kg * Sh::kBRow + 64 * (nu >> 3) + 4 * ((nu >> 1) & 3);
+  const int shift = 8 * (nu & 1);  // h = nu%2 picks the low or the high byte pairs
+  // activations: 128 bytes of eight rows per load; piece p of row r sits at position
+  // p ^ (r % 8), so that the operand reads (piece 2 kg + q of row nu) meet no bank
+  // twice.  Rows past M are zeros.
+  int a_src[NA];
+#pragma unroll
+  for (int i = 0; i < NA; i++) {
+    const int r = row0 + 8 * i + lane / 8;
+    a_src[i] = r < p.M ? r * p.K * 2 + 16 * ((lane % 8) ^ (lane / 8)) : kRowsOob;
+  }
+  unsigned a_rd[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) a_rd[q] = lds_a + nu * 128 + 16 * ((2 * kg + q) ^ (nu & 7));
+  const int s_src = 2 * (16 * strip0 + nu);  // a group's scale of slot nu, 32 bytes per strip
+
+  const DequantConsts dc;
+  i4 bq[DEPTH][NB];
+  unsigned short sq[CS], sc[CS];
+
+  // Request chunk c into slot d, and with an even one the scales of its group; a
+  // chunk that is not mine is requested at an offset past everything.
+  auto issue = [&](int d, int c, bool even) {
+    __builtin_amdgcn_sched_barrier(0);
+    const int inv = c < c1 ? 0 : kRowsOob;
+    if (GROUP && even) {
+#pragma unroll
+      for (int s = 0; s < CS; s++)
+        sq[s] = __builtin_amdgcn_raw_buffer_load_b16(rS, (s_src + 32 * s) | inv, (c >> 1) * p.N * 2, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+      bq[d][i] = __builtin_amdgcn_raw_buffer_load_b128(rB, b_src[i] | inv, 4 * c * b_row, 2);
+#pragma unroll
+    for (int i = 0; i < NA; i++) rows_dma16(rA, stage + d * Sh::kSlot + 1024 * i, a_src[i] | inv, 128 * c);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  f4 acc[CS][MB];
+#pragma unroll
+  for (int s = 0; s < CS; s++)
+#pragma unroll
+    for (int m = 0; m < MB; m++) acc[s][m] = (f4){0.f, 0.f, 0.f, 0.f};
+
+  const h2 sub = {(half_t)1032.f, (half_t)1032.f};
+  const h2 mul = {(half_t)0.0625f, (half_t)0.0625f};
+  const h2 add = {(half_t)-72.f, (half_t)-72.f};
+  auto step = [&](int d, int c, auto EVEN) {
+    constexpr bool even = decltype(EVEN)::value;
+    // chunk c has landed; the one after it may still be on its way
+    constexpr int later = DEPTH == 1 ? 0 : NA + NB + (GROUP && !even ? CS : 0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(rows_vmcnt(later));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NB; i++) rows_write16(b_wr[i], bq[d][i]);
+    i4 av[MB][2];
+    i2 wv[CS][2];
+    const unsigned slot = d * Sh::kSlot;
+    rows_each<MB>([&](auto I) {
+      rows_read16<2048 * I.value>(a_rd[0] + slot, av[I.value][0]);
+      rows_read16<2048 * I.value>(a_rd[1] + slot, av[I.value][1]);
+    });
+    rows_each<CS>([&](auto I) {
+      rows_read2<32 * I.value, 32 * I.value + 4>(b_rd, wv[I.value][0]);
+      rows_read2<32 * I.value + 8, 32 * I.value + 12>(b_rd, wv[I.value][1]);
+    });
+    // every operand has come back: nothing stands between the reads and this, and
+    // the registers are named so that they count as in use up to here
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(av[0][0]), "+v"(av[0][1]), "+v"(wv[0][0]), "+v"(wv[0][1]));
+#pragma unroll
+    for (int m = 1; m < MB; m++) asm volatile("" : "+v"(av[m][0]), "+v"(av[m][1]));
+#pragma unroll
+    for (int s = 1; s < CS; s++) asm volatile("" : "+v"(wv[s][0]), "+v"(wv[s][1]));
+#endif
+    if (GROUP && even) {
+#pragma unroll
+      for (int s = 0; s < CS; s++) sc[s] = sq[s];
+    }
+    issue(d, c + DEPTH, DEPTH == 1 ? !even : even);
+#pragma unroll
+    for (int s = 0; s < CS; s++) {
+      h2 lo[4], hi[4];  // k-values 2t, 2t + 1 and 2t + 8, 2t + 9 of the lane's sixteen
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const int w = (int)((unsigned)wv[s][t >> 1][t & 1] >> shift);
+        lo[t] = as_h2((w & dc.lo_mask) | dc.ex) - sub;
+        hi[t] = __builtin_elementwise_fma(as_h2((w & dc.hi_mask) | dc.ex), mul, add);
+        if constexpr (GROUP) {
+          const half_t x = __builtin_bit_cast(half_t, sc[s]);
+          const h2 s2 = {x, x};
+          lo[t] *= s2;
+          hi[t] *= s2;
+        }
+      }
+      const h8 w0 = make_h8(lo[0], lo[1], lo[2], lo[3]), w1 = make_h8(hi[0], hi[1], hi[2], hi[3]);
+#pragma unroll
+      for (int m = 0; m < MB; m++)
+        acc[s][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, __builtin_bit_cast(h8, av[m][0]), acc[s][m], 0, 0, 0);
+#pragma unroll
+      for (int m = 0; m < MB; m++)
+        acc[s][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, __builtin_bit_cast(h8, av[m][1]), acc[s][m], 0, 0, 0);
+    }
+  };
+
+#pragma unroll
+  for (int d = 0; d < DEPTH; d++) issue(d, c0 + d, d == 0);
+  for (int c = c0; c < c1; c += 2) {
+    step(0, c, std::true_type{});
+    if (c + 1 < c1) step(DEPTH - 1, c + 1, std::false_type{});
+  }
+  // nothing may still be on its way into LDS when it is reused
+  __builtin_amdgcn_s_waitcnt(0);
+
+  // ---- sum the eight waves, a block of 16 slots x 16 rows to a wave
+  f4* const red = (f4*)smem;
+#pragma unroll
+  for (int b0 = 0; b0 < Sh::kBlocks; b0 += Sh::kPass) {
+    __syncthreads();
+#pragma unroll
+    for (int b = b0; b < b0 + Sh::kPass && b < Sh::kBlocks; b++)
+      red[(wave * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (Sh::kPass + kRowsWaves - 1) / kRowsWaves; i++) {
+      const int b = b0 + i * kRowsWaves + wave;
+      if (b >= b0 + Sh::kPass || b >= Sh::kBlocks) continue;
+      f4 v = red[(b - b0) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < kRowsWaves; w++) v += red[(w * Sh::kPass + b - b0) * 64 + lane];
+      const int strip = strip0 + b / MB, row = row0 + 16 * (b % MB) + nu;
+      if (strip >= n_strips) continue;
+      // Register r of lane (row, kg) holds slot 4 kg + r, column 16j + 8h + 2s + e
+      // of the strip's block, e = kg / 2, j = 2 (kg % 2) + r / 2, h = r % 2.  The
+      // lanes of both e, 32 apart, exchange halves and store two columns at a time.
+      const int col = 64 * (strip >> 2) + 2 * (strip & 3) + 32 * (kg & 1);
+      const int e = kg >> 1;
+      unsigned o[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        half_t x = (half_t)v[r];
+        if constexpr (!GROUP) x *= ((const half_t*)p.S)[scale_index_single(col + e + 16 * (r >> 1) + 8 * (r & 1))];
+        o[r] = __builtin_bit_cast(unsigned short, x);
+      }
+      const unsigned got = __shfl_xor((int)(e ? o[0] | (o[1] << 16) : o[2] | (o[3] << 16)), 32);
+      if (row < p.M) {
+        unsigned* const out = (unsigned*)((half_t*)p.C + (size_t)row * p.N + col + 16 * e);
+        out[0] = e ? (got & 0xffffu) | (o[2] << 16) : o[0] | (got << 16);
+        out[4] = e ? (got >> 16) | (o[3] << 16) : o[1] | (got & 0xffff0000u);
+      }
+    }
+  }
+}
+
+namespace {
+
+// calls f(kernel, LDS bytes) for a set of strips and rows that exists
+template <class F>
+bool with_rows_kernel(int strips, int blocks, bool group, F f) {
+  const auto one = [&](auto shape, auto grouped, auto single) {
+    f(group ? grouped : single, decltype(shape)::kLds);
+    return true;
+  };
+#define ROWS(CS, MB, DEPTH)                                                                   \
+  if (strips == CS && blocks == MB)                                                           \
+  return one(RowsShape<CS, MB, DEPTH>{}, rows_kernel<CS, MB, true, DEPTH>, rows_kernel<CS, MB, false, DEPTH>)
+  ROWS(1, 1, 2);
+  ROWS(2, 1, 2);
+  ROWS(3, 1, 2);
+  ROWS(2, 2, 2);
+  ROWS(3, 2, 1);
+  ROWS(4, 2, 1);
+  ROWS(6, 2, 1);
+  ROWS(2, 3, 1);
+  ROWS(3, 3, 1);
+  ROWS(4, 3, 1);
+  ROWS(5, 3, 1);
+  ROWS(6, 3, 1);
+  ROWS(4, 4, 1);
+  ROWS(5, 4, 1);
+  ROWS(6, 4, 1);
+  ROWS(7, 4, 1);
+#undef ROWS
+  return false;
+}
+
+}  // namespace
+
+bool rows_exist(int strips, int blocks) {
+  return with_rows_kernel(strips, blocks, false, [](auto, int) {});
+}
+
+int configure_rows_kernels() {
+  bool ok = true;
+  for (int strips = 1; strips <= kRowsMaxStrips; strips++)
+    for (int blocks = 1; blocks <= kRowsMaxBlocks; blocks++)
+      for (const bool group : {false, true})
+        with_rows_kernel(strips, blocks, group, [&](auto kernel, int lds) {
+          ok = ok && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         lds) == hipSuccess;
+        });
+  return ok ? 0 : 3;
+}
+
+int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream_t stream) {
+  GemmArgs b = a;
+  b.row_parts = ceil_div(a.M, 16 * blocks);
+  b.part_rows = 16 * blocks;
+  b.gpb = ceil_div(a.N / 16, strips) * b.row_parts;
+  const bool found = with_rows_kernel(strips, blocks, group, [&](auto kernel, int lds) {
+    hipLaunchKernelGGL(kernel, dim3(b.gpb), dim3(64 * kRowsWaves), lds, stream, b);
+  });
+  return found ? launch_status() : 2;
+}
+
+}  // namespace w4a16

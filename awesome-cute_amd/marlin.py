@@ -39,6 +39,10 @@ _lib.marlin_amd_force_tile_rows.restype = None
 _lib.marlin_amd_force_tile_rows.argtypes = [_I]
 _lib.marlin_amd_force_finish_polls.restype = None
 _lib.marlin_amd_force_finish_polls.argtypes = [_I]
+_lib.marlin_amd_force_rows.restype = None
+_lib.marlin_amd_force_rows.argtypes = [_I, _I]
+_lib.marlin_amd_rows_plan.restype = _I
+_lib.marlin_amd_rows_plan.argtypes = [_I, _I, _I, _I, _I, _P]
 _lib.marlin_amd_force_row_halves.restype = None
 _lib.marlin_amd_force_row_halves.argtypes = [_I]
 _lib.marlin_amd_force_kernel.restype = None
@@ -385,6 +389,21 @@ def force_row_halves(mode):
     _lib.marlin_amd_force_row_halves(int(mode))
 
 
+def force_rows(strips, blocks=1):
+    """`strips` 16-column strips and `blocks` blocks of 16 rows per workgroup of the kernel that
+    keeps up to 64 rows of a strip set together, for every problem, where the pair exists; 0 = by
+    cost, -1 = never (calling thread only)."""
+    _lib.marlin_amd_force_rows(int(strips), int(blocks))
+
+
+def rows_plan(m, n, k, groupsize=-1, cus=256):
+    """(strips, rows) of a workgroup of that kernel where it computes the problem in place of
+    plan(), or None."""
+    out = (ctypes.c_int * 2)()
+    _lib.marlin_amd_rows_plan(m, n, k, groupsize, cus, out)
+    return tuple(out) if out[0] > 0 else None
+
+
 def work_order(grid):
     """Work index of every workgroup of a streaming launch of `grid` workgroups."""
     out = (ctypes.c_int * grid)()
@@ -393,7 +412,7 @@ def work_order(grid):
 
 
 def plan(m, n, k, groupsize=-1, thread_k=-1, thread_n=-1, sms=-1, cus=256):
-    """Kernel, grid and stream-K partition marlin_gemm would use."""
+    """Kernel, grid and stream-K partition marlin_gemm would use, unless rows_plan() names another."""
     out = (ctypes.c_int * 13)()
     rc = _lib.marlin_amd_plan(m, n, k, groupsize, thread_k, thread_n, sms, cus, out)
     keys = ("kernel", "grid", "granules_per_wg", "col_tiles", "granules_per_tile", "launches",

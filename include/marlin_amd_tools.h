@@ -119,6 +119,23 @@ void marlin_amd_force_tile_rows(int rows);
 void marlin_amd_force_finish_polls(int polls);
 
 /*
+ * out[0], out[1] = 16-column strips and rows of a workgroup of the kernel that
+ * keeps up to 64 rows of a set of strips in one workgroup, where it computes the
+ * problem in place of marlin_amd_plan's choice (17 rows and more; zeros where it
+ * does not).  The plan's scratch is acquired either way.  Returns the marlin_gemm
+ * error code for the shape.  No reference counterpart.
+ */
+int marlin_amd_rows_plan(int prob_m, int prob_n, int prob_k, int groupsize, int cus, int *out);
+
+/*
+ * That kernel with these strips (1 to 7) and row blocks of 16 (1 to 4) per
+ * workgroup for every call of the calling thread without an `sms` hint, where the
+ * pair exists; strips = 0: by cost (default; never beside another override),
+ * < 0: never.  No reference counterpart; for tests and tools.
+ */
+void marlin_amd_force_rows(int strips, int blocks);
+
+/*
  * out[0..4] = compute units, shader clock (kHz), memory clock (kHz), memory
  * bus width (bits), L2 size (bytes) of device dev, as the HIP runtime reports
  * them.  Returns MARLIN_OK or MARLIN_ERR_RUNTIME.

@@ -1,0 +1,134 @@
+"""Column strips with up to 64 rows per workgroup: where they are chosen (CPU), and the
+kernel at the edges of its strip sets, row blocks and k range (GPU) -- the oracle at the
+tolerance of the other kernels (one fp16 rounding of weights and result, fp32 sums:
+max|C - C_ref| <= 1e-2 max|C_ref|, mean 1e-3, as in test_gemm_gpu.py) and, with one-hot
+rows, the dequantised weights bit for bit."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+import _oracle as O
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "awesome-cute_amd"))
+
+PAIRS = [(1, 1), (2, 1), (3, 1), (2, 2), (3, 2), (4, 2), (6, 2), (2, 3), (3, 3), (4, 3), (5, 3), (6, 3),
+         (4, 4), (5, 4), (6, 4), (7, 4)]
+
+
+@pytest.mark.parametrize("groupsize", [128, -1])
+def test_where_the_rows_stay_together(groupsize):
+    import marlin
+    rng = np.random.default_rng(1)
+    seen = set()
+    for _ in range(2000):
+        m, n, k = int(2 ** rng.uniform(0, 11)), 256 * int(2 ** rng.uniform(0, 6.8)), 128 * int(2 ** rng.uniform(0, 7))
+        t = marlin.rows_plan(m, n, k, groupsize)
+        if t is None:
+            continue
+        strips, rows = t
+        seen.add((strips, rows // 16))
+        assert m > 16 and k >= (640 if rows > 16 else 2048) and (strips, rows // 16) in PAIRS
+        assert rows == 16 or m > rows - 16
+        assert -(-(n // 16) // strips) * -(-m // rows) <= 2.7 * 256
+    assert len(seen) > 8
+    for m, n, k in [(16, 4096, 4096), (2048, 4096, 4096), (64, 4096, 512)]:
+        assert marlin.rows_plan(m, n, k, groupsize) is None
+    # an override of the plan is an override of this choice, too
+    assert marlin.rows_plan(46, 18432, 4480, groupsize) is not None
+    for force, off in [(marlin.force_kernel, 0), (marlin.force_strips, 0), (marlin.force_k_slices, 0),
+                       (marlin.force_tile_rows, 0), (marlin.force_row_halves, 0), (marlin.force_finish_polls, -1)]:
+        force(64 if force is marlin.force_tile_rows else 1)
+        try:
+            assert marlin.rows_plan(46, 18432, 4480, groupsize) is None
+        finally:
+            force(off)
+
+
+def _gemm(A, B, s, n):
+    import torch
+    import marlin
+    dev = torch.device("cuda:0")
+    m = A.shape[0]
+    C = torch.full((m + 1, n), 7.0, dtype=torch.half, device=dev)
+    ws = torch.zeros(max(n // 128, 1) * 16, dtype=torch.int, device=dev)
+    marlin.mul(torch.from_numpy(A).to(dev), torch.from_numpy(B).to(dev), C[:m], torch.from_numpy(s).to(dev), ws)
+    torch.cuda.synchronize()
+    assert (C[m] == 7.0).all() and not ws.any().item()  # nothing past the last row
+    return C[:m].cpu().numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("strips,blocks", PAIRS)
+@pytest.mark.parametrize("groupsize", [128, -1])
+def test_rows_against_the_oracle(strips, blocks, groupsize):
+    """Row counts around a workgroup's, strip sets that do and do not divide the columns, and k
+    ranges of one chunk per wave, fewer, and an uneven number."""
+    import marlin
+    marlin.force_rows(strips, blocks)
+    try:
+        for m in (17, 16 * blocks + 1, 32 * blocks, 70):
+            for n, k in ((256, 512), (768, 1152), (1024, 2688 if groupsize == 128 else 2624)):
+                A, q, s, B, sp = O.make_problem(m, n, k, groupsize, seed=m + n + k)
+                r = O.compare(_gemm(A, B, sp, n), O.gemm(A, B, sp, n, groupsize))
+                assert r.max_abs_err <= 1e-2 * r.max_abs_ref and r.cosine >= 0.9999, (m, n, k, r)
+    finally:
+        marlin.force_rows(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("strips,blocks", PAIRS)
+@pytest.mark.parametrize("groupsize", [128, -1])
+def test_rows_return_dequantised_weights(strips, blocks, groupsize):
+    import marlin
+    n, k, m = 512, 640, 64
+    _, q, s, B, sp = O.make_problem(1, n, k, groupsize, seed=strips + blocks)
+    W = O.dequant(B, sp, k, n, groupsize)
+    if groupsize == -1:
+        W = W * O.unpack_scales(sp, False)  # fp16(q-8) * s, one rounding
+    marlin.force_rows(strips, blocks)
+    try:
+        for base in range(0, k, m):
+            A = np.zeros((m, k), np.float16)
+            A[np.arange(m), base + np.arange(m)] = 1.0
+            assert np.array_equal(_gemm(A, B, sp, n).view(np.uint16), W[base:base + m].view(np.uint16)), base
+    finally:
+        marlin.force_rows(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,g", [(46, 18432, 4480, 128), (45, 12288, 4096, -1), (144, 2048, 1792, 128), (111, 512, 4992, 128)])
+def test_chosen_and_captured(m, n, k, g):
+    """By cost, against fp32 of the same weights; twice the same bits, in a replayed graph too."""
+    import torch
+    import marlin
+    assert marlin.rows_plan(m, n, k, g) is not None
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(m)
+    q = torch.randint(0, 16, (k, n), dtype=torch.int32, device=dev, generator=gen)
+    s = (torch.rand((1 if g == -1 else k // g, n), device=dev, generator=gen) * 0.019 + 0.001).half()
+    A = torch.randn((m, k), device=dev, generator=gen).half()
+    B, sp = marlin.pack_weights(q), marlin.pack_scales(s, g != -1)
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int, device=dev)
+    C = torch.zeros((m, n), dtype=torch.half, device=dev)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        marlin.mul(A, B, C, sp, ws)
+        side.synchronize()
+        want = C.clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            marlin.mul(A, B, C, sp, ws)
+    ref = A.float() @ ((q - 8).float() * s.float().repeat_interleave(k // s.shape[0], 0))
+    assert (want.float() - ref).norm() <= 1.2e-3 * ref.norm()
+    for _ in range(3):
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
+        marlin.mul(A, B, C, sp, ws)
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
