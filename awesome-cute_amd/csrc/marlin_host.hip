@@ -709,7 +709,8 @@ double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx)
 // 1.094, and three 2 to 4 % slower.  M = 46, N = 18432, K = 4480 29.2 -> 18.4 us, 45 x
 // 12288 x 4096 15.1 -> 12.9, 144 x 2048 x 1792 9.0 -> 6.6, 501 x 1024 x 2176 11.1 -> 8.5.
 RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& cx) {
-  if (cx.force.rows_strips > 0 && sms <= 0) return {cx.force.rows_strips, cx.force.rows_blocks};
+  if (cx.force.rows_strips > 0 && sms <= 0 && (cx.force.rows_strips < 8 || n % 128 == 0))
+    return {cx.force.rows_strips, cx.force.rows_blocks};
   if (sms > 0 || m <= 16 || k < 640 || cx.force.any()) return {0, 0};
   double limit;
   if (pl.kernel == 1)
@@ -725,7 +726,8 @@ RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& 
     double by;
   } pairs[] = {{1, 1, 1.06}, {2, 1, 0.97}, {3, 1, 1.03}, {2, 2, 0.96}, {3, 2, 1.08}, {4, 2, 1.00},
                {6, 2, 0.97}, {2, 3, 0.99}, {3, 3, 1.03}, {4, 3, 0.97}, {5, 3, 0.98}, {6, 3, 0.98},
-               {4, 4, 0.98}, {5, 4, 1.00}, {6, 4, 0.98}, {7, 4, 1.02}};
+               {4, 4, 0.98}, {5, 4, 1.00}, {6, 4, 0.98}, {7, 4, 1.02},
+               {8, 2, 0.92}, {8, 3, 0.93}, {8, 4, 0.94}};
   RowsPlan best = {0, 0};
   for (const auto& p : pairs) {
     if (m <= 16 * (p.blocks - 1) || (p.blocks == 1 && k < 2048)) continue;  // (fewer blocks hold all rows)

@@ -259,8 +259,9 @@ constexpr int kStripMaxRows = 1024;
 int configure_strip_kernels();
 int launch_strip(const GemmArgs& a, bool group, int strips, hipStream_t stream);
 // any rows in parts of 16 `blocks`, `strips` 16-column strips per workgroup, over
-// the whole k range (w4a16_rows.hip); not every pair exists
-constexpr int kRowsMaxStrips = 7, kRowsMaxBlocks = 4;
+// the whole k range (w4a16_rows.hip); not every pair exists, and eight strips need
+// a.N % 128 == 0
+constexpr int kRowsMaxStrips = 8, kRowsMaxBlocks = 4;
 bool rows_exist(int strips, int blocks);
 int configure_rows_kernels();
 int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream_t stream);

@@ -128,7 +128,7 @@ void marlin_amd_force_finish_polls(int polls);
 int marlin_amd_rows_plan(int prob_m, int prob_n, int prob_k, int groupsize, int cus, int *out);
 
 /*
- * That kernel with these strips (1 to 7) and row blocks of 16 (1 to 4) per
+ * That kernel with these strips (1 to 8) and row blocks of 16 (1 to 4) per
  * workgroup for every call of the calling thread without an `sms` hint, where the
  * pair exists; strips = 0: by cost (default; never beside another override),
  * < 0: never.  No reference counterpart; for tests and tools.

@@ -15,7 +15,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 sys.path.insert(0, os.path.join(ROOT, "awesome-cute_amd"))
 
 PAIRS = [(1, 1), (2, 1), (3, 1), (2, 2), (3, 2), (4, 2), (6, 2), (2, 3), (3, 3), (4, 3), (5, 3), (6, 3),
-         (4, 4), (5, 4), (6, 4), (7, 4)]
+         (4, 4), (5, 4), (6, 4), (7, 4), (8, 2), (8, 3), (8, 4)]
 
 
 @pytest.mark.parametrize("groupsize", [128, -1])
