@@ -70,18 +70,18 @@ __device__ __forceinline__ int quantised(half_t w, float s, float r) {
   return i < 0 ? 0 : i > 15 ? 15 : i;
 }
 
-// quantised() of two halves with one scale, in bits 0-3 and 16-19.  Numbers are
-// clamped to -8 ... 7 as halves and rounded to whole ones by adding 1544: halves
-// from 1024 to 2048 are whole, sums are rounded half to even, and the low four bits
-// of 1544 + i are those of 8 + i.  Quotients that no half is near (a zero or infinite
-// operand, NaN, overflow) go through quantised().
-__device__ __forceinline__ int quantised_pair(half_t a, half_t b, float s, float r) {
+// quantised() of two halves, in bits 0-3 and 16-19.  Numbers are clamped to -8 ...
+// 7 as halves and rounded to whole ones by adding 1544: halves from 1024 to 2048 are
+// whole, sums are rounded half to even, and the low four bits of 1544 + i are those
+// of 8 + i.  Quotients that no half is near (a zero or infinite operand, NaN,
+// overflow) go through quantised().
+__device__ __forceinline__ int quantised_pair(half_t a, half_t b, float sa, float ra, float sb, float rb) {
   const float x = (float)a, y = (float)b;
-  float p = x * r, q = y * r;
-  p = __builtin_fmaf(__builtin_fmaf(-p, s, x), r, p);
-  q = __builtin_fmaf(__builtin_fmaf(-q, s, y), r, q);
+  float p = x * ra, q = y * rb;
+  p = __builtin_fmaf(__builtin_fmaf(-p, sa, x), ra, p);
+  q = __builtin_fmaf(__builtin_fmaf(-q, sb, y), rb, q);
   if (__builtin_expect(!(__builtin_fabsf(p) < 65520.f) || !(__builtin_fabsf(q) < 65520.f), 0))
-    return quantised(a, s, r) | (quantised(b, s, r) << 16);
+    return quantised(a, sa, ra) | (quantised(b, sb, rb) << 16);
   const h2 top = {(half_t)7.f, (half_t)7.f}, bottom = {(half_t)-8.f, (half_t)-8.f};
   const h2 whole = {(half_t)1544.f, (half_t)1544.f};
   const h2 v = {(half_t)p, (half_t)q};
@@ -107,10 +107,15 @@ __device__ __forceinline__ void write4(i2 v, const S& c, half_t* fake, int* q) {
   h4 f;
   i4 o;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int x = quantised(w[i], c.s[i], c.r[i]);
-    f[i] = (half_t)(x - 8) * (half_t)c.s[i];
-    o[i] = x;
+  for (int i = 0; i < 4; i += 2) {
+    const int x = quantised_pair(w[i], w[i + 1], c.s[i], c.r[i], c.s[i + 1], c.r[i + 1]);
+    // (1024 + x - 1032 is exact, and the product rounded once)
+    const h2 whole = as_h2(x | 0x64006400) - (h2){(half_t)1032.f, (half_t)1032.f};
+    const h2 y = whole * (h2){(half_t)c.s[i], (half_t)c.s[i + 1]};
+    f[i] = y[0];
+    f[i + 1] = y[1];
+    o[i] = x & 0xffff;
+    o[i + 1] = x >> 16;
   }
   *(h4*)fake = f;
   // (nothing reads the integers soon; the packer reads the fake weights)
@@ -119,8 +124,8 @@ __device__ __forceinline__ void write4(i2 v, const S& c, half_t* fake, int* q) {
 
 // (k, n), columns contiguous.  A workgroup takes one group of 4 CL columns, a
 // thread four of them and every (512 / CL)-th row.  CL = 64 for groups of up
-// to 128 rows, which then stay in registers; CL = 16 for longer ones, so that
-// one group per column still gives n / 64 workgroups (n = 11008: 172).
+// to 128 rows, which then stay in registers; CL = 16 for longer ones that are not
+// quantised in chunks (in_chunks).
 template <int CL>
 __global__ __launch_bounds__(kQThreads) void quantise_rows(const half_t* w, int n, int gs,
                                                            half_t* fake, int* q, half_t* s) {
@@ -174,6 +179,85 @@ __global__ __launch_bounds__(kQThreads) void quantise_rows(const half_t* w, int 
       const size_t at = base + (size_t)row * n;
       write4(*(const i2*)(w + at), col, fake + at, q + at);
     }
+  }
+}
+
+// Long groups, (k, n) with columns contiguous, in three launches, so that chunks of
+// 128 rows are workgroups of their own: the largest magnitudes of every chunk, the
+// scales from them, and the chunks quantised.  The magnitudes lie at the head of q,
+// which the last launch overwrites.
+constexpr int kChunkRows = 128;
+
+__global__ __launch_bounds__(kQThreads) void chunk_maxima(const half_t* w, int n, int gs, int per_group,
+                                                          unsigned short* part) {
+  __shared__ us4 top_of[kQThreads / kWave][kWave];
+  const int cl = threadIdx.x % kWave, rl = threadIdx.x / kWave;
+  const int c0 = ((int)blockIdx.x * kWave + cl) * 4;
+  const int g = (int)blockIdx.y / per_group, r0 = ((int)blockIdx.y - g * per_group) * kChunkRows;
+  const int rows = gs - r0 < kChunkRows ? gs - r0 : kChunkRows;
+  us4 top = (us4)0;
+  if (c0 < n) {
+    const half_t* const at = w + ((size_t)g * gs + r0) * n + c0;
+    i2 v[kKeep];
+#pragma unroll
+    for (int i = 0; i < kKeep; i++) {
+      const int row = rl + i * (kQThreads / kWave);
+      v[i] = row < rows ? *(const i2*)(at + (size_t)row * n) : (i2)0;
+    }
+#pragma unroll
+    for (int i = 0; i < kKeep; i++) top = max_of(top, abs_bits(v[i]));
+  }
+  top_of[rl][cl] = top;
+  __syncthreads();
+  if (rl != 0 || c0 >= n) return;
+#pragma unroll
+  for (int i = 1; i < kQThreads / kWave; i++) top = max_of(top, top_of[i][cl]);
+  *(us4*)(part + (size_t)blockIdx.y * n + c0) = top;
+}
+
+__global__ __launch_bounds__(kQThreads) void chunk_scales(const unsigned short* part, int n, int per_group,
+                                                          half_t* s) {
+  __shared__ us4 top_of[kQThreads / 16][16];
+  const int cl = threadIdx.x % 16, rl = threadIdx.x / 16;
+  const int c0 = ((int)blockIdx.x * 16 + cl) * 4;
+  us4 top = (us4)0;
+  if (c0 < n)
+    for (int i = rl; i < per_group; i += kQThreads / 16)
+      top = max_of(top, *(const us4*)(part + ((size_t)blockIdx.y * per_group + i) * n + c0));
+  top_of[rl][cl] = top;
+  __syncthreads();
+  if (rl != 0 || c0 >= n) return;
+#pragma unroll 8
+  for (int i = 1; i < kQThreads / 16; i++) top = max_of(top, top_of[i][cl]);
+  h4 sv;
+#pragma unroll
+  for (int i = 0; i < 4; i++) sv[i] = scale_of(top[i]);
+  *(h4*)(s + (size_t)blockIdx.y * n + c0) = sv;
+}
+
+__global__ __launch_bounds__(kQThreads) void quantise_chunks(const half_t* w, int n, int gs, int per_group,
+                                                             half_t* fake, int* q, const half_t* s) {
+  const int c0 = ((int)blockIdx.x * kWave + (int)(threadIdx.x % kWave)) * 4;
+  if (c0 >= n) return;
+  const int g = (int)blockIdx.y / per_group, r0 = ((int)blockIdx.y - g * per_group) * kChunkRows;
+  const int rows = gs - r0 < kChunkRows ? gs - r0 : kChunkRows;
+  const size_t base = ((size_t)g * gs + r0) * n + c0;
+  const int rl = threadIdx.x / kWave;
+  i2 v[kKeep];
+#pragma unroll
+  for (int i = 0; i < kKeep; i++) {
+    const int row = rl + i * (kQThreads / kWave);
+    v[i] = row < rows ? *(const i2*)(w + base + (size_t)row * n) : (i2)0;
+  }
+  const h4 sv = *(const h4*)(s + (size_t)g * n + c0);
+  Columns<4> col;
+#pragma unroll
+  for (int i = 0; i < 4; i++) col.set(i, sv[i]);
+#pragma unroll
+  for (int i = 0; i < kKeep; i++) {
+    const int row = rl + i * (kQThreads / kWave);
+    const size_t at = base + (size_t)row * n;
+    if (row < rows) write4(v[i], col, fake + at, q + at);
   }
 }
 
@@ -292,8 +376,8 @@ __global__ __launch_bounds__(kPThreads) void pack_rows(PackArgs p) {
     }
 #pragma unroll
     for (int i = 0; i < 8; i++)
-      half[i] = quantised_pair(w[0][i], w[1][i], col.s[i], col.r[i]) |
-                (quantised_pair(w[2][i], w[3][i], col.s[i], col.r[i]) << 4);
+      half[i] = quantised_pair(w[0][i], w[1][i], col.s[i], col.r[i], col.s[i], col.r[i]) |
+                (quantised_pair(w[2][i], w[3][i], col.s[i], col.r[i], col.s[i], col.r[i]) << 4);
   }
   const int odd = (c0 >> 3) & 1;  // columns 8 ... 15 of their sixteen
   const int j0 = (c0 >> 4) & 1, j1 = (c0 >> 5) & 1;
@@ -354,7 +438,7 @@ __global__ __launch_bounds__(kPThreads) void pack_columns(PackArgs p) {
     const float s = (float)sv[i], rs = __builtin_amdgcn_rcpf(s);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-      const int v = quantised_pair(w[i][2 * t], w[i][2 * t + 1], s, rs);
+      const int v = quantised_pair(w[i][2 * t], w[i][2 * t + 1], s, rs, s, rs);
       half[t][i >> 1] = (i & 1) == 0 ? v : half[t][i >> 1] | (v << 8);
     }
   }
@@ -400,6 +484,23 @@ bool grid_holds(long long x, int threads, long long y) {
 }
 long long pieces_of(long long a, int b) { return (a + b - 1) / b; }
 
+// Whether long groups are quantised in chunks.  In one launch, a workgroup per group
+// of 64 columns, a row takes a round of workgroups 14 to 30 ns, however few they
+// are; in chunks the chip is full whatever n is, but w is read twice and there are
+// three launches.  One scale per column, us in one launch and in chunks: n = 1024, k =
+// 1024 15.6 and 15.6, 2048 28.7 and 16.2, 8192 113.7 and 22.5; n = 4096 1024 17.1 and
+// 17.6, 4096 74.9 and 31.4, 8192 156 and 58; n = 8192 2048 40.4 and 30.3; n = 11008
+// 1024 23.9 and 24.2, 4096 100.8 and 82.0; n = 16384 2048 52.0 and 64.9, 4096 120.8
+// and 127.3; n = 28672 1024 46.6 and 49.7, 8192 556 and 454.
+bool in_chunks(int n, int k, int gs) {
+  constexpr double kUnits = 256;  // compute units of the chip
+  const double wgs = (double)pieces_of(n, 64) * (k / gs);
+  const double rounds = wgs <= kUnits ? 1.0 : (double)pieces_of((long long)wgs, (int)kUnits);
+  const double whole = gs * rounds * (0.0139 + 6.1e-5 * (wgs < kUnits ? wgs : kUnits));
+  const double chunks = 16.0 + gs * wgs * 1.02e-4;
+  return chunks < whole && pieces_of(gs, kChunkRows) * (k / gs) <= 65535;
+}
+
 bool aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 bool apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
@@ -439,6 +540,14 @@ int marlin_amd_quantize(const void* w, int k, int n, int groupsize, int by_colum
   } else if (small) {
     hipLaunchKernelGGL(quantise_rows<64>, dim3((unsigned)pieces_of(n, 256), k / gs), dim3(kQThreads), 0, st, in,
                        n, gs, (half_t*)fake, (int*)q, (half_t*)s);
+  } else if (in_chunks(n, k, gs)) {
+    const int per_group = (int)pieces_of(gs, kChunkRows);
+    const dim3 chunks((unsigned)pieces_of(n, 256), (unsigned)(k / gs) * per_group);
+    hipLaunchKernelGGL(chunk_maxima, chunks, dim3(kQThreads), 0, st, in, n, gs, per_group, (unsigned short*)q);
+    hipLaunchKernelGGL(chunk_scales, dim3((unsigned)pieces_of(n, 64), k / gs), dim3(kQThreads), 0, st,
+                       (const unsigned short*)q, n, per_group, (half_t*)s);
+    hipLaunchKernelGGL(quantise_chunks, chunks, dim3(kQThreads), 0, st, in, n, gs, per_group, (half_t*)fake,
+                       (int*)q, (const half_t*)s);
   } else {
     hipLaunchKernelGGL(quantise_rows<16>, dim3((unsigned)pieces_of(n, 64), k / gs), dim3(kQThreads), 0, st, in, n,
                        gs, (half_t*)fake, (int*)q, (half_t*)s);

@@ -80,6 +80,16 @@ def test_pack_is_the_tensor_sequence(env, k, n, gs, by_column):
         _same(torch, layer.s, marlin.pack_scales(s, groups > 1))
 
 
+@pytest.mark.parametrize("k,n,gs", [(2048, 64, -1), (1920, 1028, -1), (4352, 260, 2176), (1921, 132, -1)])
+def test_long_groups_in_chunks(env, k, n, gs):
+    """Groups of many chunks of 128 rows, whole and ragged, one and two per column."""
+    torch, marlin = env
+    w = _weights(torch, k, n, False, seed=k + n)
+    w[k - 1, 5] = 3.0e4  # the largest of its group, in the last chunk
+    for g, want in zip(marlin.quantize(w, gs), _quantise(torch, w, k if gs == -1 else gs)):
+        _same(torch, g, want)
+
+
 @pytest.mark.parametrize("by_column", [False, True])
 def test_pack_takes_any_half(env, by_column):
     """Every bit pattern as a weight, under scales of any bits: zeros, infinities, NaN, negative
