@@ -99,16 +99,21 @@ __device__ __forceinline__ h4 dense_round(f4 v) {
   return (h4){(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
 }
 
-// Tiles of less than 128 x 128 (f16_tiles.hip): rows x cols, in `slices` slices of
-// the k range each; rows = 0 where the larger tiles are the better ones.
+// One launch of a plan: `tiles` tiles of rows x cols in `slices` slices each, a
+// workgroup of 64 * waves threads per slice
+struct DnLaunch {
+  int rows, cols, waves, tiles, slices;
+};
+
+// Tiles of f16_tiles.hip: rows x cols, in `slices` slices of the k range each; rows = 0
+// where the plan's are the better ones.
 struct DnTile {
   int rows, cols, slices;
 };
-// for a problem that 128 x 128 tiles cut into max_slices slices would compute (1:
-// whole) on a device of `cus` compute units; no more slices than those
-DnTile dn_tile(int m, int n, int k, int cus, int max_slices);
-// of the sizes that exist: 32 x 32, 32 x 64, 64 x 64, 64 x 128
-bool dn_tile_exists(int rows, int cols);
+// for a problem that `plan` alone would compute on a device of `cus` compute units; no
+// more slices than that has
+DnTile dn_tile(int m, int n, int k, int cus, const DnLaunch& plan);
+bool dn_tile_exists(int rows, int cols, bool cut);
 hipError_t configure_dense_tiles();
 void launch_dense_tiles(DenseArgs a, const DnTile& t, hipStream_t stream);
 

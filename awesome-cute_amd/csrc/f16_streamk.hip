@@ -775,11 +775,6 @@ bool dn_paired(const DnPlan& pl, int k, int cus) {
   return pl.tile_cols == 128 && pl.sk_tiles == 0 && 2 * pl.dp_tiles > cus && k >= kDnPairK;
 }
 
-// One launch: `tiles` tiles of rows x cols in `slices` slices each, a workgroup
-// of 64 * waves threads per slice
-struct DnLaunch {
-  int rows, cols, waves, tiles, slices;
-};
 // The launches of a plan; `scratch`: whether pairs have room for their sums
 int dn_launches(const DnPlan& pl, int k, int cus, bool scratch, DnLaunch out[2]) {
   int count = 0;
@@ -808,23 +803,24 @@ int dn_launches(const DnPlan& pl, int k, int cus, bool scratch, DnLaunch out[2])
   return count;
 }
 
-// The tiles of less than 128 x 128 that compute the problem in place of dn_launches
-// (rows = 0: none).  Only where those would be 128 x 128 tiles, at most one per
-// compute unit, and only in slices where those are in slices, and no more of them:
-// the room acquired for their sums then holds these as well, and what a stream must
-// have seen before it can be captured does not depend on a choice that is a matter
-// of speed.
-DnTile dn_small_tile(const DnPlan& pl, int m, int n, int k, int cus) {
-  const int most = pl.tile_cols == 128 && pl.sk_tiles > 0 ? pl.ksplit : 1;
+// The tiles of f16_tiles.hip that compute the problem in place of dn_launches (rows =
+// 0: none).  Only in place of one launch, not of pairs of slices, and only in slices
+// where that is in slices, and no more of them: the room acquired for their sums then
+// holds these as well, and what a stream must have seen before it can be captured
+// does not depend on a choice that is a matter of speed.
+DnTile dn_tile_for(const DnPlan& pl, int m, int n, int k, int cus) {
   if (t_tile.rows < 0) return {0, 0, 0};
   if (t_tile.rows > 0) {
     DnTile t = t_tile;
-    const int tiles = ceil_div(m, t.rows) * (n / t.cols);
-    if (t.slices > most || tiles > kMaxCounters / kDnCounterStride) t.slices = 1;
+    const int most = pl.tile_cols == 128 && pl.sk_tiles > 0 ? pl.ksplit : 1;
+    const int tiles = ceil_div(m, t.rows) * ceil_div(n, t.cols);
+    if (t.slices > most || tiles > kMaxCounters / kDnCounterStride || !dn_tile_exists(t.rows, t.cols, true))
+      t.slices = 1;
     return t;
   }
-  if (pl.tile_cols != 128 || dn_paired(pl, k, cus)) return {0, 0, 0};
-  return dn_tile(m, n, k, cus, most);
+  DnLaunch launches[2];
+  if (dn_paired(pl, k, cus) || dn_launches(pl, k, cus, true, launches) != 1) return {0, 0, 0};
+  return dn_tile(m, n, k, cus, launches[0]);
 }
 
 int dn_check(int m, int n, int k) {
@@ -923,7 +919,7 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     // only slices exchange anything
     DnLaunch launches[2];
     int count = dn_launches(pl, k, cus, true, launches);
-    const DnTile small = dn_small_tile(pl, m, n, k, cus);
+    const DnTile tile = dn_tile_for(pl, m, n, k, cus);
     ScratchView view = {nullptr, nullptr};
     const DnLaunch& first = launches[0];  // (whole tiles come last)
     if (first.slices > 1) {
@@ -950,8 +946,8 @@ int streamk_gemm_tn(const void* A, const void* B, void* C, int m, int n, int k, 
     a.locks = view.counters;
     a.scratch = view.partials;
     a.finish_polls = t_finish_polls < 0 ? kFinishPolls : t_finish_polls;
-    if (small.rows > 0) {
-      launch_dense_tiles(a, small, stream);
+    if (tile.rows > 0) {
+      launch_dense_tiles(a, tile, stream);
       count = 0;  // in place of the plan's launches
     }
     for (int i = 0; i < count; i++) {
@@ -1019,7 +1015,7 @@ int streamk_amd_tile(int m, int n, int k, int cus, int* out) {
   out[0] = out[1] = out[2] = 0;
   const int rc = dn_check(m, n, k);
   if (rc != STREAMK_OK || m == 0 || n == 0 || k == 0) return rc;
-  const DnTile t = dn_small_tile(dn_plan(m, n, k, cus), m, n, k, cus);
+  const DnTile t = dn_tile_for(dn_plan(m, n, k, cus), m, n, k, cus);
   out[0] = t.rows;
   out[1] = t.cols;
   out[2] = t.slices;
@@ -1051,7 +1047,7 @@ void streamk_amd_force_finish_polls(int polls) {
 }
 
 void streamk_amd_force_tile(int rows, int cols, int slices) {
-  const bool exists = dn_tile_exists(rows, cols);
+  const bool exists = dn_tile_exists(rows, cols, false);
   t_tile = {rows < 0 ? -1 : exists ? rows : 0, exists ? cols : 0,
             slices < 1 ? 1 : slices > kDnMaxSlices ? kDnMaxSlices : slices};
 }

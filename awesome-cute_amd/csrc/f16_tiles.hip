@@ -1,8 +1,14 @@
-// Dense fp16 GEMM on small tiles, 32 x 32 to 64 x 128: the problems that have too
-// few 128 x 128 tiles for the compute units.  Same operands, slabs and order of
-// MFMA operands as the kernels of f16_streamk.hip.
+// Dense fp16 GEMM on tiles of many sizes, 32 x 32 to 128 x 256, of which the one is
+// taken that fills the compute units best: the problems that are less than a wave
+// or two of the tiles of f16_streamk.hip.  Same operands, slabs and order of MFMA
+// operands as the kernels there.
 //
-// What bounds such a problem is latency: the launch, the first loads, and per
+// Sizes between 64 x 128 and 128 x 256 are there for problems whose 128 x 256 tiles
+// leave a quarter to a half of the chip idle: 1514 x 3072 x 8576, 144 of those 115.7
+// us, 256 of 96 x 192 89.6; 701 x 5632 x 832 132 of them 13.8, 231 of 128 x 192 10.9;
+// 885 x 6912 x 1600 189 of them 25.8, 252 of 128 x 192 21.5.
+//
+// What bounds a problem of few small tiles is latency: the launch, the first loads, and per
 // stage a barrier and the trip of its operands from LDS, about 0.18 us whatever
 // the tile.  In slices of 128 x 128 tiles it also paid for the slices' meeting,
 // some 4 us of a launch of 9.  Small tiles fill the compute units without slices,
@@ -11,7 +17,8 @@
 // 9.2 and 4.5, 1024^3 11.4 and 5.9, 777 x 2048 x 1024 11.1 and 7.9, 64 x 2048 x
 // 4096 13.8 and 8.6, 100 x 512 x 10240 22.7 and 9.3.
 //
-// A wave computes 16 or 32 rows x 16 or 32 columns.  Per 64-deep stage it reads
+// A wave computes half the rows x a quarter (32 x 64 and less: half) of the columns.
+// Per 64-deep stage it reads
 // all operands of the next stage from LDS while the MFMAs of this one run, so a
 // slab is free again as soon as every wave has its operands, and one barrier per
 // stage does.  The ring holds as many slabs as leave room for a second workgroup
@@ -35,15 +42,15 @@ struct DnTiles {
   static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
   static constexpr int kRB = TM / 16 / WM, kNJ = TN / 16 / WN;  // operands of a wave per k step
   static constexpr int kOps = 2 * (kRB + kNJ);                  // ... per stage
-  static constexpr int kSlabA = TM * 128, kSlab = kSlabA + TN * 128;
-  static constexpr int kTA = TM / 8 / kWaves, kTB = TN / 8 / kWaves;  // load instructions per wave and slab
+  static constexpr int kTA = (TM / 8 + kWaves - 1) / kWaves, kTB = TN / 8 / kWaves;  // load instructions per wave and slab
+  static constexpr int kSlabA = kTA * kWaves * 1024, kSlab = kSlabA + TN * 128;  // (A: rows past TM stay empty)
   static constexpr int kLoads = kTA + kTB;
   static constexpr int kPitch = TN * 2 + 16;  // bytes per row of the fp16 tile in LDS
   static constexpr int kRingBytes = RING * kSlab, kTileBytes = TM * kPitch;
   static constexpr int kLds = kRingBytes > kTileBytes ? kRingBytes : kTileBytes;
   static constexpr int kPartBytes = TM * TN * 4;
-  static_assert(kTA * 8 * kWaves == TM && kTB * 8 * kWaves == TN, "whole instructions");
-  static_assert(kRB >= 1 && kRB <= 2 && kNJ >= 1 && kNJ <= 2, "operands that the reads below name");
+  static_assert(kTB * 8 * kWaves == TN && TM % (16 * WM) == 0 && TN % (16 * WN) == 0, "whole blocks");
+  static_assert(kLds <= 160 * 1024 - 256, "LDS of a compute unit");
 };
 
 // wait for every LDS read in flight; the registers are named so that they count
@@ -51,17 +58,18 @@ struct DnTiles {
 template <int N>
 __device__ __forceinline__ void dn_landed(i4 (&v)[N]) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  static_assert(N == 4 || N == 6 || N == 8, "");
-  if constexpr (N == 4)
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
-  else if constexpr (N == 6)
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
-  else
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]),
-                   "+v"(v[7]));
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#pragma unroll
+  for (int i = 4; i < N; i++) asm volatile("" : "+v"(v[i]));
 #endif
+}
+// operands of COUNT neighbouring row blocks of 16
+template <int COUNT>
+__device__ __forceinline__ void dn_read_blocks(unsigned at, i4* v) {
+  if constexpr (COUNT > 0) {
+    dn_read_blocks<COUNT - 1>(at, v);
+    dn_read16<2048 * (COUNT - 1)>(at, v[COUNT - 1]);
+  }
 }
 
 }  // namespace
@@ -90,10 +98,11 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
   dn_tile_coord(tile, p.tiles_m, p.tiles_n, &tm, &tn);
   const int m0 = TM * tm, n0 = TN * tn;
   const int rows = min(TM, p.M - m0);
+  const int cols = min(TN, p.N - n0);  // (192 columns: the last tile may have fewer)
   const __amdgpu_buffer_rsrc_t rA =
       dn_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
   const __amdgpu_buffer_rsrc_t rB =
-      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)TN * (unsigned)p.K * 2u);
+      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)cols * (unsigned)p.K * 2u);
 
   // a wave fetches its share of the rows of A and of B, eight rows per
   // instruction; rows past the end of A repeat the last one (never stored)
@@ -103,7 +112,7 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
 #pragma unroll
     for (int t = 0; t < TA; t++) {
       const int r = 8 * (TA * wave + t) + r8;
-      a_src[t] = (r < rows ? r : rows - 1) * p.K * 2 + 16 * c;
+      a_src[t] = r >= TM ? kDnOob : (r < rows ? r : rows - 1) * p.K * 2 + 16 * c;
     }
 #pragma unroll
     for (int t = 0; t < TB; t++) b_src[t] = (8 * (TB * wave + t) + r8) * p.K * 2 + 16 * c;
@@ -136,11 +145,8 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
   auto read = [&](i4 (&o)[Sh::kOps], unsigned slab) {
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-      i4* const b = o + h * (RB + NJ);
-      dn_read16<0>(b_rd[h] + slab, b[0]);
-      if constexpr (NJ == 2) dn_read16<2048>(b_rd[h] + slab, b[1]);
-      dn_read16<0>(a_rd[h] + slab, b[NJ]);
-      if constexpr (RB == 2) dn_read16<2048>(a_rd[h] + slab, b[NJ + 1]);
+      dn_read_blocks<NJ>(b_rd[h] + slab, o + h * (RB + NJ));
+      dn_read_blocks<RB>(a_rd[h] + slab, o + h * (RB + NJ) + NJ);
     }
   };
 
@@ -212,7 +218,7 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
     for (int at0 = 0; at0 < TM * PR; at0 += Sh::kThreads) {
       const int at = at0 + tid;
       const int m = at / PR, c = at % PR;
-      if ((TM * PR % Sh::kThreads != 0 && at >= TM * PR) || m >= rows ||
+      if ((TM * PR % Sh::kThreads != 0 && at >= TM * PR) || m >= rows || (TN == 192 && 8 * c >= cols) ||
           !(waves >> (m / (16 * RB) * WN + c / (2 * NJ)) & 1))
         continue;
       // nobody reads C again in this launch
@@ -292,21 +298,28 @@ void with_tile_kernel(int rows, int cols, bool cut, F f) {
   DN_TILE(32, 64, 2, 2, 6);
   DN_TILE(64, 64, 2, 4, 4);
   DN_TILE(64, 128, 2, 4, 6);
+  if (cut) return;  // only tiles of at most 64 x 128 are cut
+  DN_TILE(96, 128, 2, 4, 4);
+  DN_TILE(64, 192, 2, 4, 4);
+  DN_TILE(96, 192, 2, 4, 3);
+  DN_TILE(128, 192, 2, 4, 3);
+  DN_TILE(96, 256, 2, 4, 3);
+  DN_TILE(128, 256, 2, 4, 3);
 #undef DN_TILE
 }
 
 }  // namespace
 
-bool dn_tile_exists(int rows, int cols) {
+bool dn_tile_exists(int rows, int cols, bool cut) {
   bool found = false;
-  with_tile_kernel(rows, cols, false, [&](auto, int, int) { found = true; });
+  with_tile_kernel(rows, cols, cut, [&](auto, int, int) { found = true; });
   return found;
 }
 
 hipError_t configure_dense_tiles() {
   hipError_t e = hipSuccess;
-  for (const int rows : {32, 64})
-    for (const int cols : {32, 64, 128})
+  for (const int rows : {32, 64, 96, 128})
+    for (const int cols : {32, 64, 128, 192, 256})
       for (const bool cut : {false, true})
         with_tile_kernel(rows, cols, cut, [&](auto kernel, int lds, int) {
           if (e == hipSuccess)
@@ -317,62 +330,84 @@ hipError_t configure_dense_tiles() {
 
 void launch_dense_tiles(DenseArgs a, const DnTile& t, hipStream_t stream) {
   a.tiles_m = ceil_div(a.M, t.rows);
-  a.tiles_n = a.N / t.cols;
+  a.tiles_n = ceil_div(a.N, t.cols);
   a.ksplit = t.slices;
   with_tile_kernel(t.rows, t.cols, t.slices > 1, [&](auto kernel, int lds, int threads) {
     hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.tiles_n * t.slices), dim3(threads), lds, stream, a);
   });
 }
 
-// Costs in us, fitted to launches of 260 problems (m = 1 ... 8192, n = 512 ...
-// 8192, k = 512 ... 10240, 128 x 128 tiles for at most one wave of compute units;
-// 5 to 7 % rms): a launch, its stages (dearer the fuller the chip), those of
-// workgroups beyond one per compute unit, the slices' meeting.
-static double dn_tile_cost(int rows, int cols, int tiles, int stages, int slices, int cus) {
-  struct Fit {
-    int rows, cols;
-    double launch, stage, fill, more, more_stage, meet, slice;
-  };
-  static const Fit fits[] = {{32, 32, 2.23, 0.084, 0.017, 0.89, 0.079, 2.24, 0.08},
-                             {32, 64, 2.38, 0.118, 0.031, 1.12, 0.124, 2.35, 0.30},
-                             {64, 64, 2.56, 0.159, 0.036, 0.98, 0.187, 2.14, 0.40},
-                             {64, 128, 3.14, 0.232, 0.074, 7.28, 0.287, 3.00, 0.46}};
-  for (const Fit& f : fits) {
-    if (f.rows != rows || f.cols != cols) continue;
-    const double r = (double)tiles * slices / cus;
-    // workgroups beyond one per compute unit: half way between the rounds they
-    // make and their share of one
-    const double more = r > 1.0 ? 0.5 * (ceil_div(tiles * slices, cus) + r) - 1.0 : 0.0;
-    const int st = ceil_div(stages, slices);
-    return f.launch + f.more * more + st * (f.stage + f.fill * (r < 1.0 ? r : 1.0) + f.more_stage * more) +
-           (slices > 1 ? f.meet + f.slice * slices : 0.0);
-  }
-  return 1e30;
+namespace {
+
+// Costs in us, fitted to launches over m = 1 ... 8192, n = 512 ... 8192, k = 512 ...
+// 10240 (260 problems that 128 x 128 tiles would cut into slices or nearly so, 560 with
+// more tiles; 5 to 10 % rms): a launch, its stages (dearer the fuller the chip), those
+// of workgroups beyond one per compute unit, the slices' meeting.
+constexpr struct DnFit {
+  int rows, cols;
+  double launch, stage, fill, more, more_stage, meet, slice;
+} kDnFits[] = {{32, 32, 2.23, 0.084, 0.017, 0.89, 0.079, 2.24, 0.08},
+               {32, 64, 2.38, 0.118, 0.031, 1.12, 0.124, 2.35, 0.30},
+               {64, 64, 2.56, 0.159, 0.036, 0.98, 0.187, 2.14, 0.40},
+               {64, 128, 2.54, 0.204, 0.194, 1.32, 0.378, 3.00, 0.46},
+               {96, 128, 2.39, 0.320, 0.171, 1.45, 0.481, 0, 0},
+               {64, 192, 2.00, 0.364, 0.163, 0.96, 0.531, 0, 0},
+               {96, 192, 2.39, 0.459, 0.184, 1.88, 0.646, 0, 0},
+               {128, 192, 3.00, 0.523, 0.192, 2.16, 0.774, 0, 0},
+               {96, 256, 2.52, 0.605, 0.204, 1.80, 0.837, 0, 0},
+               {128, 256, 3.07, 0.697, 0.237, 3.23, 1.005, 0, 0}};
+
+// workgroups beyond one per compute unit: half way between the rounds they make and
+// their share of one
+double dn_more(int wgs, int cus) {
+  const double r = (double)wgs / cus;
+  return r > 1.0 ? 0.5 * (ceil_div(wgs, cus) + r) - 1.0 : 0.0;
 }
 
-// The cheapest small tile, if it is 3 % cheaper than 128 x 128 ones (costs fitted
-// to the same problems: 4.5 % rms in slices, 3 % whole).  In 2 or 4 slices (waves
-// share a tile unevenly with 3), at most one workgroup per compute unit.  Over the
-// 260 problems that is 1.466 times the speed of 128 x 128 tiles, the best choice
-// for each 1.480; none is slower than it was.
-DnTile dn_tile(int m, int n, int k, int cus, int max_slices) {
+double dn_cost(const DnFit& f, int tiles, int stages, int slices, int cus) {
+  const double r = (double)tiles * slices / cus, more = dn_more(tiles * slices, cus);
+  const int st = ceil_div(stages, slices);
+  return f.launch + f.more * more + st * (f.stage + f.fill * (r < 1.0 ? r : 1.0) + f.more_stage * more) +
+         (slices > 1 ? f.meet + f.slice * slices : 0.0);
+}
+
+// ... and of the launch that would compute the problem otherwise (3 to 6 % rms)
+double dn_plan_cost(const DnLaunch& l, int stages, int cus) {
+  const double r = (double)l.tiles * l.slices / cus, fill = r < 1.0 ? r : 1.0;
+  const double more = dn_more(l.tiles, cus);
+  if (l.cols == 128)
+    return l.slices > 1
+               ? 6.48 + 0.30 * l.slices + (double)stages / l.slices * (0.294 + 0.258 * fill)
+               : 2.50 + stages * (0.325 + 0.271 * fill);
+  if (l.rows == 128)
+    return l.waves == 4 ? 5.95 * fill + stages * (0.719 + 0.176 * fill)
+                        : 3.60 + 0.34 * fill + stages * (0.503 + 0.452 * fill);
+  return l.waves == 4 ? 4.23 + 1.87 * more + stages * (1.037 + 0.563 * fill + 1.92 * more)
+                      : 1.39 + 6.66 * fill + stages * (0.954 + 0.514 * fill + 2.23 * more);
+}
+
+}  // namespace
+
+// The cheapest tile, if it is 3 % cheaper than the plan's launch, 7 % where that has
+// 256 x 256 tiles.  In 2 or 4 slices (waves share a tile unevenly with 3) no more than
+// the plan, at most one workgroup per compute unit.  570 problems of at most one wave
+// of 128 x 128 tiles run at 1.46 times the speed, with the best choice for each at
+// 1.475; 700 with more tiles at 1.110, the best choice 1.117, two of them 3 and five 4
+// to 5 % slower.  (Operands from memory: the line of 64 x 128 is theirs; out of the
+// last-level cache a stage takes three quarters of that.)
+DnTile dn_tile(int m, int n, int k, int cus, const DnLaunch& plan) {
   const int stages = k / kDnStageK;
-  const int large = ceil_div(m, 128) * (n / 128);
-  const double fill = (double)large * max_slices / cus;
-  const double large_cost =
-      max_slices > 1 ? 6.48 + 0.30 * max_slices + (double)stages / max_slices * (0.294 + 0.258 * fill)
-                     : 3.62 + stages * (0.259 + 0.252 * fill);
   DnTile best = {0, 0, 0};
-  double best_cost = large_cost;
-  for (const DnTile& t : {DnTile{32, 32, 1}, DnTile{32, 64, 1}, DnTile{64, 64, 1}, DnTile{64, 128, 1}}) {
-    const int tiles = ceil_div(m, t.rows) * (n / t.cols);
-    if (tiles > 5 * cus) continue;  // (beyond what was fitted; never the best there)
-    for (int s = 1; s <= max_slices && s <= 4; s *= 2) {
+  double limit = dn_plan_cost(plan, stages, cus) / (plan.rows == 256 ? 1.07 : 1.03);
+  for (const DnFit& f : kDnFits) {
+    const int tiles = ceil_div(m, f.rows) * ceil_div(n, f.cols);
+    if (tiles > 4 * cus) continue;  // (never the best there)
+    for (int s = 1; s <= (f.meet > 0 ? plan.slices : 1); s *= 2) {
       if (s > 1 && (tiles * s > cus || tiles > kMaxCounters / kDnCounterStride)) break;
-      const double c = 1.03 * dn_tile_cost(t.rows, t.cols, tiles, stages, s, cus);
-      if (c < best_cost) {
-        best = {t.rows, t.cols, s};
-        best_cost = c;
+      const double c = dn_cost(f, tiles, stages, s, cus);
+      if (c < limit) {
+        best = {f.rows, f.cols, s};
+        limit = c;
       }
     }
   }

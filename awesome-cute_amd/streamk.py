@@ -39,21 +39,22 @@ def plan(m, n, k, cus=256):
     return rc, dict(zip(keys, out))
 
 
-def small_tile(m, n, k, cus=256):
-    """(rows, cols, slices) of the tiles of less than 128 x 128 that compute the problem in one
-    launch, in place of the plan's, or None."""
+def tile(m, n, k, cus=256):
+    """(rows, cols, slices) of the tiles that compute the problem in one launch, in place of the
+    plan's, or None."""
     out = (ctypes.c_int * 3)()
     _lib.streamk_amd_tile(m, n, k, cus, out)
     return tuple(out) if out[0] > 0 else None
 
 
-def force_small_tile(rows, cols=0, slices=1):
-    """Which small tiles compute every problem (0 = by cost, -1 = none; calling thread only)."""
+def force_tile(rows, cols=0, slices=1):
+    """Tiles that compute every problem, in place of the plan's (0 = by cost, -1 = never; calling
+    thread only)."""
     _lib.streamk_amd_force_tile(int(rows), int(cols), int(slices))
 
 
 def launches(m, n, k, cus=256, scratch=True):
-    """The launches that compute the plan's tiles, unless small_tile() names smaller ones;
+    """The launches that compute the plan's tiles, unless tile() names others;
     `scratch`: whether there is room for partial sums."""
     out = (ctypes.c_int * 10)()
     count = _lib.streamk_amd_launches(m, n, k, cus, int(scratch), out)

@@ -48,15 +48,15 @@ int streamk_amd_check(int m, int n, int k);
  * streamk_amd_tile say how the problem is computed. */
 int streamk_amd_plan(int m, int n, int k, int cus, int* out);
 
-/* out[0..2] = rows, columns and k slices of the tiles of less than 128 x 128 that
- * compute the problem, in one launch of a workgroup per tile and slice, in place
- * of streamk_amd_launches: 32 x 32, 32 x 64, 64 x 64 or 64 x 128, where that is
- * cheaper; zeros where it is not.  Returns what streamk_amd_check does. */
+/* out[0..2] = rows, columns and k slices of the tiles, 32 x 32 to 128 x 256, that
+ * compute the problem in one launch of a workgroup per tile and slice, in place of
+ * streamk_amd_launches, where they fill the compute units better; zeros where they
+ * do not.  Returns what streamk_amd_check does. */
 int streamk_amd_tile(int m, int n, int k, int cus, int* out);
 
-/* the tile for every problem of the calling thread, whatever its cost, in at most
- * the plan's slices: rows = 0 back to the choice by cost, < 0 never a small tile;
- * for tests and tools */
+/* such tiles for every problem of the calling thread, whatever their cost, in at
+ * most the plan's slices: rows = 0 back to the choice by cost, < 0 never; for tests
+ * and tools */
 void streamk_amd_force_tile(int rows, int cols, int slices);
 
 /* the launches that compute the plan's tiles, at most two, five numbers each: rows and

@@ -1,4 +1,4 @@
-"""Dense GEMM on tiles of less than 128 x 128: where they are chosen (CPU), and the
+"""Dense GEMM on tiles of many sizes: where they are chosen (CPU), and the
 kernel at the edges of its tiles, stages and slices (GPU; whole numbers whose sums
 are exact in fp16 and in any order, so the result is torch's fp32 product, bit for
 bit)."""
@@ -10,31 +10,34 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 sys.path.insert(0, os.path.join(ROOT, "awesome-cute_amd"))
 
-TILES = [(32, 32), (32, 64), (64, 64), (64, 128)]
+CUT = [(32, 32), (32, 64), (64, 64), (64, 128)]  # whole or in slices
+TILES = CUT + [(96, 128), (64, 192), (96, 192), (128, 192), (96, 256), (128, 256)]
 
 
 @pytest.mark.parametrize("cus", [256, 304, 64])
-def test_small_tiles_stand_in_for_128_x_128_ones_only(cus):
+def test_tiles_stand_in_for_one_launch(cus):
     import numpy as np
     import streamk
     rng = np.random.default_rng(cus)
     seen = set()
-    for _ in range(4000):
+    for _ in range(6000):
         m, n = int(2 ** rng.uniform(0, 13)), 256 * int(2 ** rng.uniform(0, 5.3))
         k = 64 * int(2 ** rng.uniform(0, 7.5))
-        t, (_, p) = streamk.small_tile(m, n, k, cus), streamk.plan(m, n, k, cus)
+        t, (_, p) = streamk.tile(m, n, k, cus), streamk.plan(m, n, k, cus)
         if t is None:
             continue
         seen.add(t[:2])
         rows, cols, slices = t
-        tiles = -(-m // rows) * (n // cols)
-        assert (p["tile_rows"], p["tile_cols"]) == (128, 128) and (rows, cols) in TILES
+        tiles = -(-m // rows) * -(-n // cols)
+        assert (rows, cols) in TILES and tiles <= 4 * cus
+        assert len(streamk.launches(m, n, k, cus)) == 1 and streamk.launches(m, n, k, cus)[0]["slices"] == p["k_slices"]
         assert slices in (1, 2, 4) and slices <= p["k_slices"]
         if slices > 1:  # the plan's scratch holds their sums and counters
+            assert (rows, cols) in CUT and p["tile_cols"] == 128
             assert tiles * slices <= cus and tiles <= 1024
             assert tiles * rows * cols * slices <= p["sk_tiles"] * 128 * 128 * p["k_slices"]
-    assert seen == set(TILES)
-    assert streamk.small_tile(4096, 4352, 4096) is None and streamk.small_tile(777, 4352, 10240) is None
+    assert len(seen) >= 9
+    assert streamk.tile(4096, 4352, 4096) is None and streamk.tile(777, 4352, 10240) is None
 
 
 def _check(m, n, k, top):
@@ -56,38 +59,42 @@ def _check(m, n, k, top):
 @pytest.mark.parametrize("tile", TILES)
 @pytest.mark.parametrize("m", [1, 31, 65, 200])
 def test_stages(tile, m):
-    """One stage to past the end of the longest ring, even and odd."""
+    """One stage to past the end of the longest ring, even and odd, and columns that 192 does
+    not divide."""
     import streamk
-    streamk.force_small_tile(*tile)
+    streamk.force_tile(*tile)
     try:
         for stages in (1, 2, 3, 4, 5, 6, 7, 8, 9, 11):
             _check(m, 512, 64 * stages, 1)
+        _check(m, 256, 320, 1)
+        _check(m, 1536, 320, 1)
     finally:
-        streamk.force_small_tile(0)
+        streamk.force_tile(0)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("polls", [-1, 0, 1])  # 0 and 1: shares left to the last arrival
-@pytest.mark.parametrize("tile", TILES + [(-1, 0)])
+@pytest.mark.parametrize("tile", CUT + [(-1, 0)])
 @pytest.mark.parametrize("m,n,k,slices", [(33, 256, 1024, 4), (100, 512, 1344, 4), (129, 512, 832, 3), (300, 1280, 576, 2)])
 def test_slices(tile, m, n, k, slices, polls):
     """Slices of equal and unequal length; (-1, 0): the 128 x 128 tiles they stand in for."""
     import streamk
-    streamk.force_small_tile(*tile, slices)
+    streamk.force_tile(*tile, slices)
     streamk.force_finish_polls(polls)
     try:
         if tile[0] > 0:
-            assert streamk.small_tile(m, n, k) == tile + (slices,)
+            assert streamk.tile(m, n, k) == tile + (slices,)
         for _ in range(2):
             _check(m, n, k, 1)
     finally:
         streamk.force_finish_polls(-1)
-        streamk.force_small_tile(0)
+        streamk.force_tile(0)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(64, 512, 512), (291, 1280, 896), (100, 512, 10240), (777, 2048, 1024)])
+@pytest.mark.parametrize("m,n,k", [(64, 512, 512), (291, 1280, 896), (100, 512, 10240), (777, 2048, 1024), (1514, 3072, 1600),
+                                   (885, 6912, 704), (701, 5632, 832)])
 def test_chosen_tiles(m, n, k):
     import streamk
-    assert streamk.small_tile(m, n, k) is not None
+    assert streamk.tile(m, n, k) is not None
     _check(m, n, k, 1)
