@@ -16,10 +16,13 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
 
 #include "../../include/marlin_amd.h"
+#include "../../include/marlin_amd_convert.h"
 #include "../../include/streamk_amd.h"
 
 namespace {
@@ -208,9 +211,138 @@ PyObject* py_dense(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// What the conversion kernels may take: plain tensors on one GPU, 16-byte aligned,
+// without gradients.  (That nothing looks on is the caller's to know.)
+//
+// Bound: host time for layers up to about 3000 x 3000; the two kernels of a
+// 1024 x 1024 one take 12 us, the same checks in Python and two calls through
+// ctypes took 32 for quantising and packing, here 17 (4096 x 4096: 38.8 -> 33.3).
+const at::Tensor* plain(PyObject* o) {
+  return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr;
+}
+bool convertible(const at::Tensor& t, const at::Device& dev) {
+  return t.device() == dev && !t.is_neg() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0 &&
+         !(t.requires_grad() && c10::GradMode::is_enabled());
+}
+// 1 launched, 0 not a problem for the kernels, -1 with an exception set
+int converted(int rc) {
+  if (rc == MARLIN_OK) return 1;
+  if (rc == MARLIN_ERR_PROB_SHAPE) return 0;
+  PyErr_Format(PyExc_RuntimeError, "weight conversion failed with code %d: %s", rc,
+               marlin_amd_convert_last_error());
+  return -1;
+}
+
+// quantize(w, groupsize) -> (fake, q, s), or None where the tensor operations have to do it
+PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  int gs;
+  if (nargs != 2) {
+    PyErr_SetString(PyExc_TypeError, "quantize takes 2 arguments");
+    return nullptr;
+  }
+  const at::Tensor* const pw = plain(args[0]);
+  if (!to_int(args[1], &gs)) {  // what else a group size may be, the tensor operations say
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  if (!pw || pw->dim() != 2 || pw->scalar_type() != at::kHalf || !pw->is_cuda() || pw->numel() == 0)
+    Py_RETURN_NONE;
+  const at::Tensor& w = *pw;
+  const int64_t k = w.size(0), n = w.size(1);
+  if (gs == -1 && k == (int)k) gs = (int)k;
+  const bool by_column = !w.is_contiguous();
+  if (gs <= 0 || k % gs != 0 || k != (int)k || n != (int)n || !convertible(w, w.device()) ||
+      (by_column ? !(w.stride(0) == 1 && w.stride(1) == k && gs % 4 == 0) : n % 4 != 0))
+    Py_RETURN_NONE;
+  const int dev = w.get_device();
+  void* const st = current_stream(dev);
+  at::Tensor fake, q, s;
+  int rc;
+  {
+    pybind11::gil_scoped_release unlocked;
+    const auto plain_options = w.options().requires_grad(false);
+    fake = at::empty_like(w, plain_options, at::MemoryFormat::Preserve);
+    q = at::empty_like(fake, plain_options.dtype(at::kInt), at::MemoryFormat::Preserve);
+    s = at::empty({k / gs, n}, plain_options);
+    rc = marlin_amd_quantize(w.data_ptr(), (int)k, (int)n, gs, by_column, fake.data_ptr(), q.data_ptr(),
+                             s.data_ptr(), dev, st);
+  }
+  const int done = converted(rc);
+  if (done < 0) return nullptr;
+  if (done == 0) Py_RETURN_NONE;
+  PyObject* const out[3] = {THPVariable_Wrap(std::move(fake)), THPVariable_Wrap(std::move(q)),
+                            THPVariable_Wrap(std::move(s))};
+  PyObject* const tuple = PyTuple_New(3);
+  if (!tuple) return nullptr;
+  for (int i = 0; i < 3; i++) PyTuple_SET_ITEM(tuple, i, out[i]);
+  return tuple;
+  END_HANDLE_TH_ERRORS
+}
+
+// whether `read` has no bytes between the first and the last of the contiguous `written`: a
+// kernel would read what it is overwriting, the tensor operations read everything first
+bool apart(const at::Tensor& written, const at::Tensor& read) {
+  const char* const lo = (const char*)written.data_ptr();
+  const char* const hi = lo + written.numel() * written.element_size();
+  int64_t last = 0;
+  for (int64_t d = 0; d < read.dim(); d++) last += (read.size(d) - 1) * read.stride(d);
+  const char* const at = (const char*)read.data_ptr();
+  return at >= hi || at + (last + 1) * read.element_size() <= lo;
+}
+
+// pack(w (k, n), s (groups, n), B, packed, k, n, groupsize or -1) -> whether B and the packed
+// scales have been written; False where the tensor operations have to do it
+PyObject* py_pack(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  int k, n, gs;
+  if (nargs != 7) {
+    PyErr_SetString(PyExc_TypeError, "pack takes 7 arguments");
+    return nullptr;
+  }
+  const at::Tensor *pw = plain(args[0]), *ps = plain(args[1]), *pb = plain(args[2]), *pp = plain(args[3]);
+  if (!to_int(args[4], &k) || !to_int(args[5], &n) || !to_int(args[6], &gs)) {
+    PyErr_Clear();
+    Py_RETURN_FALSE;
+  }
+  if (!pw || !ps || !pb || !pp || !pw->is_cuda() || (gs <= 0 && gs != -1)) Py_RETURN_FALSE;
+  const at::Tensor &w = *pw, &s = *ps, &B = *pb, &packed = *pp;
+  const auto is = [](const at::Tensor& t, at::ScalarType type, int64_t rows, int64_t columns) {
+    return t.scalar_type() == type && t.dim() == 2 && t.size(0) == rows && t.size(1) == columns;
+  };
+  const int64_t groups = gs == -1 ? 1 : k / gs;
+  const bool by_column = !w.is_contiguous();
+  const at::Device on = w.device();
+  if (!is(w, at::kHalf, k, n) || !is(s, at::kHalf, groups, n) || !is(packed, at::kHalf, groups, n) ||
+      !is(B, at::kInt, k / 16, 2 * (int64_t)n) || (by_column && !(w.stride(0) == 1 && w.stride(1) == k)) ||
+      !B.is_contiguous() || !packed.is_contiguous() || !convertible(w, on) || !convertible(B, on) ||
+      !convertible(packed, on) || s.device() != on || s.requires_grad() || s.is_neg() ||
+      // (writes to inference tensors elsewhere are refused by the tensor operations)
+      (!c10::InferenceMode::is_enabled() && (B.is_inference() || packed.is_inference())) ||
+      !apart(B, w) || !apart(B, s) || !apart(B, packed) || !apart(packed, w) || !apart(packed, s))
+    Py_RETURN_FALSE;
+  const int dev = w.get_device();
+  void* const st = current_stream(dev);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = marlin_amd_pack(w.data_ptr(), k, n, gs, by_column, s.data_ptr(), s.stride(0), s.stride(1),
+                       B.data_ptr(), packed.data_ptr(), dev, st);
+  Py_END_ALLOW_THREADS
+  const int done = converted(rc);
+  if (done < 0) return nullptr;
+  if (done == 0) Py_RETURN_FALSE;
+  // written in place, as an assignment to them would be
+  for (const at::Tensor* t : {&B, &packed})
+    if (!t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
     {"mul", (PyCFunction)(void (*)(void))py_mul, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void (*)(void))py_linear, METH_FASTCALL, nullptr},
+    {"quantize", (PyCFunction)(void (*)(void))py_quantize, METH_FASTCALL, nullptr},
+    {"pack", (PyCFunction)(void (*)(void))py_pack, METH_FASTCALL, nullptr},
     {"dense", (PyCFunction)(void (*)(void))py_dense, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -185,18 +185,6 @@ def _on_gpu(*tensors):
                     and not t.is_neg() and t.data_ptr() % 16 == 0 for t in tensors))
 
 
-def _apart(written, *read):
-    """Whether no tensor of `read` has bytes between the first and the last of the contiguous
-    tensor `written`: a kernel would read what it is overwriting, the tensor operations read
-    everything first."""
-    lo, hi = written.data_ptr(), written.data_ptr() + written.numel() * written.element_size()
-    for t in read:
-        last = sum((size - 1) * stride for size, stride in zip(t.shape, t.stride()))
-        if t.data_ptr() < hi and t.data_ptr() + (last + 1) * t.element_size() > lo:
-            return False
-    return True
-
-
 def _converted(rc):
     """Whether a conversion kernel was launched; False where its grid cannot hold the problem."""
     if rc not in (0, 1):
@@ -240,17 +228,10 @@ def quantize(w, groupsize=-1):
     fake-quantised weight (k, n), q (k, n) int32 and s (groups, n)."""
     k, n = w.shape
     gs = k if groupsize == -1 else groupsize
-    if w.dtype == torch.half and w.numel() and gs > 0 and k % gs == 0 and _on_gpu(w):
-        by_column = not w.is_contiguous()
-        if (w.t().is_contiguous() and gs % 4 == 0) if by_column else n % 4 == 0:
-            fake = torch.empty_like(w, memory_format=torch.preserve_format, requires_grad=False)
-            q = torch.empty_like(fake, dtype=torch.int32)
-            s = torch.empty((k // gs, n), dtype=torch.half, device=w.device)
-            dev = w.get_device()
-            if _converted(_lib.marlin_amd_quantize(w.data_ptr(), k, n, gs, by_column,
-                                                   fake.data_ptr(), q.data_ptr(), s.data_ptr(),
-                                                   dev, _raw_stream(dev))):
-                return fake, q, s
+    if not _looked_on():
+        done = _torch_binding.quantize(w, groupsize)
+        if done is not None:
+            return done
     wg = w.reshape(k // gs, gs, n)
     s = wg.abs().amax(dim=1, keepdim=True)
     s = s * (2 / 15)
@@ -305,28 +286,9 @@ class Layer(nn.Module):
         s = scales.t()                 # (groups, n)
         w = linear.weight.data.t()     # (k, n)
         groupwise = self.groupsize != self.k
-        B, packed = self.B, self.s
-        if (s.dtype == packed.dtype == torch.half and B.dtype == torch.int32
-                and s.shape == packed.shape == (self.k // self.groupsize, self.n)
-                and B.shape == (self.k // 16, 2 * self.n) and w.shape == (self.k, self.n)
-                and (w.is_contiguous() or w.t().is_contiguous())
-                and B.is_contiguous() and packed.is_contiguous()
-                and _on_gpu(w, B, packed) and s.device == w.device
-                and type(s) in (torch.Tensor, nn.Parameter) and not s.requires_grad
-                and not s.is_neg()
-                # (writes to inference tensors elsewhere are refused by the assignments below)
-                and (torch.is_inference_mode_enabled()
-                     or not (B.is_inference() or packed.is_inference()))
-                and _apart(B, w, s, packed) and _apart(packed, w, s)):
-            dev = w.get_device()
-            if _converted(_lib.marlin_amd_pack(
-                    w.data_ptr(), self.k, self.n, self.groupsize if groupwise else -1,
-                    not w.is_contiguous(), s.data_ptr(), s.stride(0), s.stride(1), B.data_ptr(),
-                    packed.data_ptr(), dev, _raw_stream(dev))):
-                # written in place, as an assignment to them would be
-                torch.autograd.graph.increment_version(
-                    [t for t in (B, packed) if not t.is_inference()])
-                return
+        if not _looked_on() and _torch_binding.pack(w, s, self.B, self.s, self.k, self.n,
+                                                    self.groupsize if groupwise else -1):
+            return
         s_full = s.repeat_interleave(self.groupsize, dim=0) if groupwise else s
         q = torch.clamp(torch.round(w / s_full).int() + 8, 0, 15)
         self.B[:, :] = pack_weights(q).to(self.B.device)

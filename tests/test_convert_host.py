@@ -62,3 +62,23 @@ def test_without_torchs_own_names_the_tensor_operations_run(monkeypatch):
     import marlin
     monkeypatch.setattr(marlin, "_can_tell", False)
     assert marlin._looked_on()
+
+
+def test_what_the_kernels_do_not_take_is_left_to_the_tensor_operations():
+    """... with its own results and its own refusals, group sizes of every kind among them."""
+    import torch
+    import marlin
+    binding = marlin._torch_binding
+    w, B = torch.ones(256, 256).half(), torch.empty(16, 512, dtype=torch.int32)
+    for tensor in (w, w.t(), w.float(), w[0], [1.0], None):
+        for group in (-1, 128, 0, 2 ** 40, 128.0, None):
+            assert binding.quantize(tensor, group) is None
+            assert binding.pack(tensor, w, B, w, 256, 256, group) is False
+    _, q, s = marlin.quantize(w, 128)
+    assert q.shape == w.shape and s.shape == (2, 256)
+    with pytest.raises(ZeroDivisionError):
+        marlin.quantize(w, 0)
+    with pytest.raises(RuntimeError):
+        marlin.quantize(w, 2 ** 40)
+    with pytest.raises(TypeError):
+        marlin.quantize(w, 128.0)
