@@ -47,6 +47,11 @@ def run(m, n, k, repeat=200, warmup=5, seed=0, dev="cuda:0", log=print):
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     _, plan = streamk.plan(m, n, k, cus)
     launches = streamk.launches(m, n, k, cus, scratch=False)  # (timed from a graph)
+    tile = streamk.tile(m, n, k, cus)
+    if tile:  # one launch of these in their place
+        rows, cols, slices = tile
+        launches = [{"rows": rows, "cols": cols, "slices": slices, "tiles": -(-m // rows) * -(-n // cols),
+                     "waves": 4 if rows * cols < 4096 else 8}]
     log(f"fp16 gemm m:{m} n:{n} k:{k}")
     log(f"output tiles: {plan['dp_tiles'] + plan['sk_tiles']}, dp tiles: {plan['dp_tiles']}, "
         f"sk tiles: {plan['sk_tiles']}")

@@ -70,7 +70,7 @@ MEASURED_TRAFFIC_BYTES = {
     "prefill": (("prefill", 256), int((33941.5 * 2.0 + 16389.5) * 1024)),     # 86.3 MB, 2.04 x (A and B read by 16 tiles each)
     "mlp_up": (("strips", 230), int((11930.9 * 2.0 + 356.0) * 1024)),         # 24.8 MB, 1.04 x
     "mlp_down": (("stream", 256), int((13714.5 * 2.0 + 2185.0) * 1024)),      # 30.3 MB, 1.28 x
-    "large_g128": (("prefill", 224), int((66886.0 * 2.0 + 17930.5) * 1024)),  # 155.3 MB, 1.23 x
+    "large_g128": (("rows", 224), int((63314.0 * 2.0 + 3584.0) * 1024)),      # 133.3 MB, 1.06 x
     "large_chan": (("prefill", 224), int((65121.5 * 2.0 + 17930.5) * 1024)),  # 151.7 MB, 1.24 x
     "decode_large": (("stream", 224), int((59281.0 * 2.0 + 56.0) * 1024)),    # 121.5 MB, 1.00 x
 }
@@ -242,8 +242,13 @@ def time_shape(torch, marlin, O, name, steps, warmup, check=True, with_floor=Fal
     kernel = {1: "stream", 2: "prefill", 3: "strips"}.get(plan["kernel"])
     res["plan"] = {"kernel": kernel, "grid": plan["grid"], "k_slices": plan["k_slices"],
                    "tile_rows": plan["tile_rows"]}
+    rows = marlin.rows_plan(M, N, K, g, marlin.device_info(0)["compute_units"])
+    if rows:  # in place of that plan
+        kernel = "rows"
+        res["plan"] = {"kernel": kernel, "grid": -(-N // (16 * rows[0])) * -(-M // rows[1]), "k_slices": 1,
+                       "tile_rows": rows[1]}
     measured_on, traffic = MEASURED_TRAFFIC_BYTES.get(name, (None, None))
-    if measured_on != (kernel, plan["grid"]):
+    if measured_on != (kernel, res["plan"]["grid"]):
         traffic = None  # measured on another plan: stale
     if bound == "hbm":
         ach = res["weight_GBps"]

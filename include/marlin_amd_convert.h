@@ -26,6 +26,7 @@ extern "C" {
  * by_column = 0: w, fake (fp16) and q (int32) are (k, n) with the columns
  * contiguous, n a multiple of 4; by_column = 1: the same values stored column
  * by column, i.e. as (n, k), groupsize a multiple of 4.  s: (groups, n) fp16.
+ * (Where groups are long, q holds intermediate values before its own.)
  */
 int marlin_amd_quantize(const void *w, int k, int n, int groupsize, int by_column, void *fake,
                         void *q, void *s, int dev, void *stream);
