@@ -339,23 +339,34 @@ void launch_dense_tiles(DenseArgs a, const DnTile& t, hipStream_t stream) {
 
 namespace {
 
-// Costs in us, fitted to launches over m = 1 ... 8192, n = 512 ... 8192, k = 512 ...
-// 10240 (260 problems that 128 x 128 tiles would cut into slices or nearly so, 560 with
-// more tiles; 5 to 10 % rms): a launch, its stages (dearer the fuller the chip), those
-// of workgroups beyond one per compute unit, the slices' meeting.
+// Costs in us: a launch, a stage of the longest workgroup (dearer the fuller the chip)
+// and, whole, workgroups beyond one per compute unit and their stages; in slices the
+// launch holds their meeting.  Fitted to every tile on 2500 problems, m = 1 ... 8192, n =
+// 256 ... 16384, k = 64 ... 20480, 4 to 8 % rms where a tile is near the best.  Each
+// time is that with operands from memory, as a model's weights are, to 0.7 times that
+// with operands in the last-level cache to 0.3: the small tiles, which wait for
+// memory, take 1.2 to 1.5 times as long by the first as by the second, slices of 128 x
+// 128 1.1 times.  (Fitted to operands in the cache alone, 44 problems of 900 were given
+// tiles that took 2 to 19 % longer from memory than the plan's launch: 576 x 1536 x
+// 4544 23.0 us in 64 x 64, 19.4 in slices; 240 x 3328 x 4096 21.4 and 18.7.)
+struct DnLine {
+  double launch, stage, fill;
+};
 constexpr struct DnFit {
   int rows, cols;
-  double launch, stage, fill, more, more_stage, meet, slice;
-} kDnFits[] = {{32, 32, 2.23, 0.084, 0.017, 0.89, 0.079, 2.24, 0.08},
-               {32, 64, 2.38, 0.118, 0.031, 1.12, 0.124, 2.35, 0.30},
-               {64, 64, 2.56, 0.159, 0.036, 0.98, 0.187, 2.14, 0.40},
-               {64, 128, 2.54, 0.204, 0.194, 1.32, 0.378, 3.00, 0.46},
-               {96, 128, 2.39, 0.320, 0.171, 1.45, 0.481, 0, 0},
-               {64, 192, 2.00, 0.364, 0.163, 0.96, 0.531, 0, 0},
-               {96, 192, 2.39, 0.459, 0.184, 1.88, 0.646, 0, 0},
-               {128, 192, 3.00, 0.523, 0.192, 2.16, 0.774, 0, 0},
-               {96, 256, 2.52, 0.605, 0.204, 1.80, 0.837, 0, 0},
-               {128, 256, 3.07, 0.697, 0.237, 3.23, 1.005, 0, 0}};
+  DnLine whole;
+  double more, more_stage;
+  DnLine by2, by4;  // (64 x 128: 1.04 times the fit, whose misses are there)
+} kDnFits[] = {{32, 32, {2.20, 0.096, 0.039}, 0.81, 0.083, {4.46, 0.099, 0.049}, {4.52, 0.092, 0.071}},
+               {32, 64, {2.31, 0.142, 0.055}, 0.86, 0.132, {4.92, 0.174, 0.044}, {5.27, 0.151, 0.108}},
+               {64, 64, {2.33, 0.209, 0.059}, 0.85, 0.182, {5.46, 0.221, 0.061}, {5.69, 0.214, 0.114}},
+               {64, 128, {3.06, 0.297, 0.095}, 2.30, 0.328, {7.09, 0.321, 0.118}, {7.65, 0.309, 0.203}},
+               {96, 128, {3.27, 0.389, 0.088}, 2.16, 0.438, {}, {}},
+               {64, 192, {3.16, 0.404, 0.118}, 2.23, 0.465, {}, {}},
+               {96, 192, {3.64, 0.499, 0.103}, 2.57, 0.612, {}, {}},
+               {128, 192, {4.11, 0.511, 0.170}, 3.05, 0.758, {}, {}},
+               {96, 256, {4.10, 0.574, 0.188}, 3.21, 0.849, {}, {}},
+               {128, 256, {4.53, 0.641, 0.265}, 4.42, 1.039, {}, {}}};
 
 // workgroups beyond one per compute unit: half way between the rounds they make and
 // their share of one
@@ -365,44 +376,49 @@ double dn_more(int wgs, int cus) {
 }
 
 double dn_cost(const DnFit& f, int tiles, int stages, int slices, int cus) {
-  const double r = (double)tiles * slices / cus, more = dn_more(tiles * slices, cus);
-  const int st = ceil_div(stages, slices);
-  return f.launch + f.more * more + st * (f.stage + f.fill * (r < 1.0 ? r : 1.0) + f.more_stage * more) +
-         (slices > 1 ? f.meet + f.slice * slices : 0.0);
+  const double r = (double)tiles * slices / cus, fill = r < 1.0 ? r : 1.0;
+  const DnLine& l = slices == 1 ? f.whole : slices == 2 ? f.by2 : f.by4;
+  const double cost = l.launch + ceil_div(stages, slices) * (l.stage + l.fill * fill);
+  const double more = slices == 1 ? dn_more(tiles, cus) : 0.0;
+  return cost + more * (f.more + f.more_stage * stages);
 }
 
-// ... and of the launch that would compute the problem otherwise (3 to 6 % rms)
+// ... and of the launch that would compute the problem otherwise (3 to 4 % rms)
 double dn_plan_cost(const DnLaunch& l, int stages, int cus) {
   const double r = (double)l.tiles * l.slices / cus, fill = r < 1.0 ? r : 1.0;
   const double more = dn_more(l.tiles, cus);
-  if (l.cols == 128)
-    return l.slices > 1
-               ? 6.48 + 0.30 * l.slices + (double)stages / l.slices * (0.294 + 0.258 * fill)
-               : 2.50 + stages * (0.325 + 0.271 * fill);
+  if (l.cols == 128) {
+    const double each = (double)stages / l.slices;
+    return l.slices == 1   ? 3.12 + 0.58 * fill + stages * (0.464 + 0.075 * fill)
+           : l.slices == 2 ? 7.31 + each * (0.403 + 0.197 * fill)
+           : l.slices == 3 ? 8.05 + each * (0.288 + 0.347 * fill)
+                           : 7.90 + each * (0.404 + 0.251 * fill);
+  }
   if (l.rows == 128)
-    return l.waves == 4 ? 5.95 * fill + stages * (0.719 + 0.176 * fill)
-                        : 3.60 + 0.34 * fill + stages * (0.503 + 0.452 * fill);
-  return l.waves == 4 ? 4.23 + 1.87 * more + stages * (1.037 + 0.563 * fill + 1.92 * more)
-                      : 1.39 + 6.66 * fill + stages * (0.954 + 0.514 * fill + 2.23 * more);
+    return l.waves == 4 ? 5.73 + stages * (0.635 + 0.216 * fill)
+                        : 3.93 + 0.80 * fill + stages * (0.644 + 0.223 * fill);
+  return l.waves == 4 ? 8.43 * fill + 1.87 * more + stages * (1.263 + 0.198 * fill + 1.92 * more)
+                      : 2.81 + 4.63 * fill + 6.70 * more + stages * (1.147 + 0.341 * fill + 1.74 * more);
 }
 
 }  // namespace
 
-// The cheapest tile, if it is 3 % cheaper than the plan's launch, 7 % where that has
-// 256 x 256 tiles.  In 2 or 4 slices (waves share a tile unevenly with 3) no more than
-// the plan, at most one workgroup per compute unit.  570 problems of at most one wave
-// of 128 x 128 tiles run at 1.46 times the speed, with the best choice for each at
-// 1.475; 700 with more tiles at 1.110, the best choice 1.117, two of them 3 and five 4
-// to 5 % slower.  (Operands from memory: the line of 64 x 128 is theirs; out of the
-// last-level cache a stage takes three quarters of that.)
+// The cheapest tile, if it is 3 % cheaper than the plan's slices, 5 % than its whole
+// tiles and 7 % than those of 256 x 256.  In 2 or 4 slices (waves share a tile unevenly
+// with 3) no more than the plan, at most one workgroup per compute unit.  2500 other
+// problems for which this or the line before it (one fit to operands in the cache)
+// takes a tile: operands from memory 1.48 times the speed of the plan's launches, 17
+// problems 2 to 9 % slower, most of them 10 to 20 % faster with operands in the cache;
+// by the line before 1.46 times, 131 slower, the worst by 20 %.  In the cache 1.59 times
+// and two slower; before 1.58 and 51.
 DnTile dn_tile(int m, int n, int k, int cus, const DnLaunch& plan) {
   const int stages = k / kDnStageK;
   DnTile best = {0, 0, 0};
-  double limit = dn_plan_cost(plan, stages, cus) / (plan.rows == 256 ? 1.07 : 1.03);
+  double limit = dn_plan_cost(plan, stages, cus) / (plan.slices > 1 ? 1.03 : plan.rows == 256 ? 1.07 : 1.05);
   for (const DnFit& f : kDnFits) {
     const int tiles = ceil_div(m, f.rows) * ceil_div(n, f.cols);
     if (tiles > 4 * cus) continue;  // (never the best there)
-    for (int s = 1; s <= (f.meet > 0 ? plan.slices : 1); s *= 2) {
+    for (int s = 1; s <= (f.by2.launch > 0 ? plan.slices : 1); s *= 2) {
       if (s > 1 && (tiles * s > cus || tiles > kMaxCounters / kDnCounterStride)) break;
       const double c = dn_cost(f, tiles, stages, s, cus);
       if (c < limit) {

@@ -40,6 +40,14 @@ def test_tiles_stand_in_for_one_launch(cus):
     assert streamk.tile(4096, 4352, 4096) is None and streamk.tile(777, 4352, 10240) is None
 
 
+@pytest.mark.parametrize("m,n,k", [(576, 1536, 4544), (130, 7424, 3328), (240, 3328, 4096), (571, 1792, 5440), (265, 3840, 3072),
+                                   (172, 5376, 9920), (1486, 5376, 3008), (4798, 2048, 128)])
+def test_tiles_that_were_slower_are_not_taken(m, n, k):
+    """Sizes at which a tile took 1.05 to 1.19 times the plan's launch, operands from memory."""
+    import streamk
+    assert streamk.tile(m, n, k) is None
+
+
 def _check(m, n, k, top):
     import torch
     import streamk
