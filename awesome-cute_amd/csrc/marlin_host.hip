@@ -681,19 +681,28 @@ struct RowsPlan {
 // way between the rounds they make and their share of one), and the weights'
 // way from memory.  2800 launches over 320 problems, M = 17 ... 1500, N = 512 ...
 // 28672, K = 512 ... 13824; 6 % rms.
+// And where the rows that an XCD's workgroups read outgrow its L2 -- an eighth of the
+// strip sets each, with fewer than eight an eighth of (set, row part) pairs -- 0.24 us
+// per MB beyond 3.5: over n of 256 to 1024 with a thousand rows the kernel was taken
+// for faster where it took up to 1.46 times the plan's time (M = 1015, N = 256, K = 7296
+// 13.6 us in column strips, 19.9; M = 1531, N = 512, K = 8448 25.7 on prefill tiles,
+// 33.7).
 double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx) {
-  const int wgs = ceil_div(n / 16, strips) * ceil_div(m, 16 * blocks);
+  const int sets = ceil_div(n / 16, strips);
+  const int wgs = sets * ceil_div(m, 16 * blocks);
   const double r = (double)wgs / cx.cus;
   const double fill = r < 1.0 ? r : 1.0;
   const double more = r > 1.0 ? 0.5 * (ceil_div(wgs, cx.cus) + r) - 1.0 : 0.0;
   const double K = k / 1000.0, sums = strips * blocks;
   const double memory = 0.5e-7 * n * k;
+  const double beyond = 2e-6 * m * k * (sets < 8 ? sets / 8.0 : 1.0) - 3.5;
+  const double rows = beyond > 0.0 ? 0.24 * beyond : 0.0;
   if (cx.grouped)
-    return 2.88 + 0.167 * sums +
+    return rows + 2.88 + 0.167 * sums +
            K * (0.335 * blocks + 0.239 * strips + fill * (0.075 * blocks + 0.033 * strips) +
                 more * (0.297 * blocks + 0.202 * strips + 0.080 * sums)) +
            0.240 * more * sums + 0.180 * memory;
-  return 2.71 + 0.174 * sums +
+  return rows + 2.71 + 0.174 * sums +
          K * (0.363 * blocks + 0.186 * strips + fill * (0.086 * blocks + 0.032 * strips) +
               more * (0.285 * blocks + 0.188 * strips + 0.039 * sums)) +
          0.294 * more * sums + 0.149 * memory;
@@ -704,17 +713,24 @@ double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx)
 // low without (the factors below).  Not over k ranges below 640, nor, with 16 rows
 // per workgroup, below 2048: a wave has a chunk or two there, which the column strips
 // take in at once (M = 51, N = 11520, K = 512 5.7 us streaming, 6.6 by the fit's
-// choice; M = 123, N = 512, K = 1536 4.1 and 5.0).  Over the 320 problems it is taken
-// for half, which makes all of them 1.074 times as fast, the best choice for each
-// 1.094, and three 2 to 4 % slower.  M = 46, N = 18432, K = 4480 29.2 -> 18.4 us, 45 x
-// 12288 x 4096 15.1 -> 12.9, 144 x 2048 x 1792 9.0 -> 6.6, 501 x 1024 x 2176 11.1 -> 8.5.
+// choice; M = 123, N = 512, K = 1536 4.1 and 5.0).  Nine to twelve groups leave some
+// waves two of them and others one, which the fit does not hold: the line against a
+// streaming launch that shares no tile lies 5 % lower there (M = 123, N = 6912, K = 1280
+// 9.0 us streaming, 10.1; M = 64, N = 25600 13.5 and 14.7).  2500 other problems for
+// which this or the line before it (neither that, nor the activations beyond an L2) takes
+// the kernel: 1.136 times the speed of the plans' launches, 37 problems more than 2 %
+// slower and 15 more than 5 %; by the line before 1.130, 107 and 60.  M = 46, N = 18432,
+// K = 4480 29.2 -> 18.4 us, 45 x 12288 x 4096 15.1 -> 12.9, 144 x 2048 x 1792 9.0 -> 6.6,
+// 501 x 1024 x 2176 11.1 -> 8.5.
 RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& cx) {
   if (cx.force.rows_strips > 0 && sms <= 0 && (cx.force.rows_strips < 8 || n % 128 == 0))
     return {cx.force.rows_strips, cx.force.rows_blocks};
   if (sms > 0 || m <= 16 || k < 640 || cx.force.any()) return {0, 0};
   double limit;
   if (pl.kernel == 1)
-    limit = stream_cost_as_planned(m, n, k, cx) * (cx.grouped ? 1.03 : 0.99);
+    limit = stream_cost_as_planned(m, n, k, cx) * (!cx.grouped                             ? 0.99
+                                                   : pl.sp.wpt == 1 && k > 1024 && k <= 1536 ? 0.98
+                                                                                             : 1.03);
   else if (pl.kernel == 2)
     limit = prefill_cost(m, n, k, cx) * (cx.grouped ? 1.03 : 1.04);
   else

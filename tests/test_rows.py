@@ -47,6 +47,15 @@ def test_where_the_rows_stay_together(groupsize):
             force(off)
 
 
+@pytest.mark.parametrize("m,n,k,groupsize", [(1015, 256, 7296, -1), (1531, 512, 8448, 128), (2008, 512, 5888, 128), (1229, 256, 10496, 128),
+                                              (1316, 512, 5504, -1), (1654, 1024, 5504, 128), (123, 6912, 1280, 128),
+                                              (161, 5376, 1280, 128), (64, 25600, 1280, 128)])
+def test_not_where_it_was_slower(m, n, k, groupsize):
+    """Sizes at which the kernel took 1.09 to 1.47 times the plan's launch."""
+    import marlin
+    assert marlin.rows_plan(m, n, k, groupsize) is None
+
+
 def _gemm(A, B, s, n):
     import torch
     import marlin
