@@ -723,7 +723,8 @@ double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx)
 // K = 4480 29.2 -> 18.4 us, 45 x 12288 x 4096 15.1 -> 12.9, 144 x 2048 x 1792 9.0 -> 6.6,
 // 501 x 1024 x 2176 11.1 -> 8.5.
 RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& cx) {
-  if (cx.force.rows_strips > 0 && sms <= 0 && (cx.force.rows_strips < 8 || n % 128 == 0))
+  if (cx.force.rows_strips > 0 && sms <= 0 && (cx.force.rows_strips < 8 || n % 128 == 0) &&
+      rows_exist(cx.force.rows_strips, cx.force.rows_blocks, cx.grouped))
     return {cx.force.rows_strips, cx.force.rows_blocks};
   if (sms > 0 || m <= 16 || k < 640 || cx.force.any()) return {0, 0};
   double limit;
@@ -742,11 +743,12 @@ RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& 
     double by;
   } pairs[] = {{1, 1, 1.06}, {2, 1, 0.97}, {3, 1, 1.03}, {2, 2, 0.96}, {3, 2, 1.08}, {4, 2, 1.00},
                {6, 2, 0.97}, {2, 3, 0.99}, {3, 3, 1.03}, {4, 3, 0.97}, {5, 3, 0.98}, {6, 3, 0.98},
-               {4, 4, 0.98}, {5, 4, 1.00}, {6, 4, 0.98}, {7, 4, 1.02},
+               {4, 4, 0.98}, {5, 4, 1.00}, {6, 4, 0.98},
                {8, 2, 0.92}, {8, 3, 0.93}, {8, 4, 0.94}};
   RowsPlan best = {0, 0};
   for (const auto& p : pairs) {
     if (m <= 16 * (p.blocks - 1) || (p.blocks == 1 && k < 2048)) continue;  // (fewer blocks hold all rows)
+    if (p.strips == 4 && p.blocks == 4 && !cx.grouped) continue;            // (does not exist)
     // (beyond what was fitted, and never the best there)
     if (ceil_div(n / 16, p.strips) * ceil_div(m, 16 * p.blocks) > 2.7 * cx.cus) continue;
     const double c = rows_cost(m, n, k, p.strips, p.blocks, cx) * p.by;
@@ -1130,7 +1132,7 @@ void marlin_amd_force_tile_rows(int rows) {
 }
 
 void marlin_amd_force_rows(int strips, int blocks) {
-  const bool exists = rows_exist(strips, blocks);
+  const bool exists = rows_exist(strips, blocks, true);  // (a pair of one scale per column has one of groups)
   t_force.rows_strips = strips < 0 ? -1 : exists ? strips : 0;
   t_force.rows_blocks = exists ? blocks : 0;
 }

@@ -169,14 +169,17 @@ struct GemmArgs {
                     // (prefill), lock_stride ints apart; zero on entry and on exit
   int lock_stride;  // >= 1; spreads the counters over separate cache lines
   float* scratch;   // partial sums of shared tiles (null if no tile is shared)
-  int gpb;          // granules per workgroup (streaming kernel; the most, when wpt > 0)
+  int gpb;          // granules per workgroup (streaming kernel; the most, when wpt > 0);
+                    // rows kernel: workgroups of the launch (launch_rows sets it)
   int wpt;          // workgroups per column tile, or 0 (see StreamPlan)
   int row_parts;    // streaming kernel, wpt > 0: 1, or the number of parts the rows are cut
                     // into, `part_rows` each (the last one the rest), that separate
                     // workgroups compute: wpt workgroups per column tile and part; needs
                     // lock_stride >= row_parts.  Column-strip kernel: 1, or the number
-                    // of 16-row parts, a workgroup per strip set and part
-  int part_rows;    // rows of a part: 16 or 32
+                    // of 16-row parts, a workgroup per strip set and part.  Rows kernel:
+                    // parts of 16 row blocks, a workgroup per strip set and part
+                    // (launch_rows sets it)
+  int part_rows;    // rows of a part: 16 or 32 (streaming and column-strip kernels)
   int finish_polls; // prefill kernels: looks at a tile's other slices before leaving them a share
 };
 
@@ -262,7 +265,7 @@ int launch_strip(const GemmArgs& a, bool group, int strips, hipStream_t stream);
 // the whole k range (w4a16_rows.hip); not every pair exists, and eight strips need
 // a.N % 128 == 0
 constexpr int kRowsMaxStrips = 8, kRowsMaxBlocks = 4;
-bool rows_exist(int strips, int blocks);
+bool rows_exist(int strips, int blocks, bool group);
 int configure_rows_kernels();
 int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream_t stream);
 // ksplit >= 1 slices of the k range per tile; above 1 the launch needs

@@ -372,40 +372,39 @@ namespace {
 // calls f(kernel, LDS bytes) for a set of strips and rows that exists
 template <class F>
 bool with_rows_kernel(int strips, int blocks, bool group, F f) {
-  const auto one = [&](auto shape, auto grouped, auto single) {
-    f(group ? grouped : single, decltype(shape)::kLds);
-    return true;
-  };
-#define ROWS(CS, MB, DEPTH)                                                                   \
-  if (strips == CS && blocks == MB)                                                           \
-  return one(RowsShape<CS, MB, DEPTH>{}, rows_kernel<CS, MB, true, DEPTH>, rows_kernel<CS, MB, false, DEPTH>)
-  ROWS(1, 1, 2);
-  ROWS(2, 1, 2);
-  ROWS(3, 1, 2);
-  ROWS(2, 2, 2);
-  ROWS(3, 2, 1);
-  ROWS(4, 2, 1);
-  ROWS(6, 2, 1);
-  ROWS(2, 3, 1);
-  ROWS(3, 3, 1);
-  ROWS(4, 3, 1);
-  ROWS(5, 3, 1);
-  ROWS(6, 3, 1);
-  ROWS(4, 4, 1);
-  ROWS(5, 4, 1);
-  ROWS(6, 4, 1);
-  ROWS(7, 4, 1);
-  ROWS(8, 2, 1);
-  ROWS(8, 3, 1);
-  ROWS(8, 4, 1);
+#define ROWS(CS, MB, DEPTH, GROUP)                                               \
+  if (strips == CS && blocks == MB && group == GROUP) {                         \
+    f(rows_kernel<CS, MB, GROUP, DEPTH>, RowsShape<CS, MB, DEPTH>::kLds);       \
+    return true;                                                                \
+  }
+#define ROWS_OF_BOTH(CS, MB, DEPTH) ROWS(CS, MB, DEPTH, true) ROWS(CS, MB, DEPTH, false)
+  ROWS_OF_BOTH(1, 1, 2)
+  ROWS_OF_BOTH(2, 1, 2)
+  ROWS_OF_BOTH(3, 1, 2)
+  ROWS_OF_BOTH(2, 2, 2)
+  ROWS_OF_BOTH(3, 2, 1)
+  ROWS_OF_BOTH(4, 2, 1)
+  ROWS_OF_BOTH(6, 2, 1)
+  ROWS_OF_BOTH(2, 3, 1)
+  ROWS_OF_BOTH(3, 3, 1)
+  ROWS_OF_BOTH(4, 3, 1)
+  ROWS_OF_BOTH(5, 3, 1)
+  ROWS_OF_BOTH(6, 3, 1)
+  ROWS(4, 4, 1, true)  // (never the cheapest with one scale per column)
+  ROWS_OF_BOTH(5, 4, 1)
+  ROWS_OF_BOTH(6, 4, 1)
+  ROWS_OF_BOTH(8, 2, 1)
+  ROWS_OF_BOTH(8, 3, 1)
+  ROWS_OF_BOTH(8, 4, 1)
+#undef ROWS_OF_BOTH
 #undef ROWS
   return false;
 }
 
 }  // namespace
 
-bool rows_exist(int strips, int blocks) {
-  return with_rows_kernel(strips, blocks, false, [](auto, int) {});
+bool rows_exist(int strips, int blocks, bool group) {
+  return with_rows_kernel(strips, blocks, group, [](auto, int) {});
 }
 
 int configure_rows_kernels() {
@@ -423,7 +422,6 @@ int configure_rows_kernels() {
 int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream_t stream) {
   GemmArgs b = a;
   b.row_parts = ceil_div(a.M, 16 * blocks);
-  b.part_rows = 16 * blocks;
   b.gpb = ceil_div(a.N / 16, strips) * b.row_parts;
   if (strips == 8 && a.N % 128 != 0) return 2;  // (whole blocks of 64 columns only)
   const bool found = with_rows_kernel(strips, blocks, group, [&](auto kernel, int lds) {

@@ -15,7 +15,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 sys.path.insert(0, os.path.join(ROOT, "awesome-cute_amd"))
 
 PAIRS = [(1, 1), (2, 1), (3, 1), (2, 2), (3, 2), (4, 2), (6, 2), (2, 3), (3, 3), (4, 3), (5, 3), (6, 3),
-         (4, 4), (5, 4), (6, 4), (7, 4), (8, 2), (8, 3), (8, 4)]
+         (4, 4), (5, 4), (6, 4), (8, 2), (8, 3), (8, 4)]
+CASES = [(pair, g) for pair in PAIRS for g in (128, -1) if (pair, g) != ((4, 4), -1)]
 
 
 @pytest.mark.parametrize("groupsize", [128, -1])
@@ -23,17 +24,27 @@ def test_where_the_rows_stay_together(groupsize):
     import marlin
     rng = np.random.default_rng(1)
     seen = set()
-    for _ in range(2000):
+    for _ in range(60000):
         m, n, k = int(2 ** rng.uniform(0, 11)), 256 * int(2 ** rng.uniform(0, 6.8)), 128 * int(2 ** rng.uniform(0, 7))
         t = marlin.rows_plan(m, n, k, groupsize)
         if t is None:
             continue
         strips, rows = t
         seen.add((strips, rows // 16))
-        assert m > 16 and k >= (640 if rows > 16 else 2048) and (strips, rows // 16) in PAIRS
+        assert m > 16 and k >= (640 if rows > 16 else 2048) and ((strips, rows // 16), groupsize) in CASES
         assert rows == 16 or m > rows - 16
         assert -(-(n // 16) // strips) * -(-m // rows) <= 2.7 * 256
-    assert len(seen) > 8
+    if groupsize == 128:
+        assert marlin.rows_plan(491, 2048, 5760, 128) == (4, 64)  # (one problem in a thousand)
+        seen.add((4, 4))
+    assert sorted(seen) == sorted(pair for pair, g in CASES if g == groupsize)  # none that nothing reaches
+    for pair in ((7, 4), (4, 4)):  # what does not exist cannot be forced
+        marlin.force_rows(*pair)
+        try:
+            forced = marlin.rows_plan(64, 4096, 4096, groupsize) == (pair[0], 16 * pair[1])
+            assert forced == ((pair, groupsize) in CASES)
+        finally:
+            marlin.force_rows(0)
     for m, n, k in [(16, 4096, 4096), (2048, 4096, 4096), (64, 4096, 512)]:
         assert marlin.rows_plan(m, n, k, groupsize) is None
     # an override of the plan is an override of this choice, too
@@ -70,14 +81,15 @@ def _gemm(A, B, s, n):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("strips,blocks", PAIRS)
-@pytest.mark.parametrize("groupsize", [128, -1])
-def test_rows_against_the_oracle(strips, blocks, groupsize):
+@pytest.mark.parametrize("pair,groupsize", CASES)
+def test_rows_against_the_oracle(pair, groupsize):
     """Row counts around a workgroup's, strip sets that do and do not divide the columns, and k
     ranges of one chunk per wave, fewer, and an uneven number."""
     import marlin
+    strips, blocks = pair
     marlin.force_rows(strips, blocks)
     try:
+        assert marlin.rows_plan(17, 256, 512, groupsize) == (strips, 16 * blocks)
         for m in (17, 16 * blocks + 1, 32 * blocks, 70):
             for n, k in ((256, 512), (768, 1152), (1024, 2688 if groupsize == 128 else 2624)):
                 A, q, s, B, sp = O.make_problem(m, n, k, groupsize, seed=m + n + k)
@@ -88,10 +100,10 @@ def test_rows_against_the_oracle(strips, blocks, groupsize):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("strips,blocks", PAIRS)
-@pytest.mark.parametrize("groupsize", [128, -1])
-def test_rows_return_dequantised_weights(strips, blocks, groupsize):
+@pytest.mark.parametrize("pair,groupsize", CASES)
+def test_rows_return_dequantised_weights(pair, groupsize):
     import marlin
+    strips, blocks = pair
     n, k, m = 512, 640, 64
     _, q, s, B, sp = O.make_problem(1, n, k, groupsize, seed=strips + blocks)
     W = O.dequant(B, sp, k, n, groupsize)
