@@ -2,16 +2,17 @@
 // a launch and a plain read of the packed weights cost on this device, with no
 // arithmetic, and what the matrix pipes sustain by themselves, to judge the
 // GEMM kernels against.  A library of its own, beside libmarlin_amd.so, which
-// it asks for the plan of the shape (marlin_amd_plan): the product library
-// carries no measurement code.
+// it asks for the plan of the shape (marlin_amd_rows_plan, marlin_amd_plan): the
+// product library carries no measurement code.
 //
 // probe_read_kernel walks the packed weights exactly as the streaming kernel
 // does for the same plan -- same work split, same workgroup-to-XCD order, same
 // 128-bit streaming buffer loads of 1 KiB per wave instruction, four rows per
 // granule -- keeps up to kProbeDepth granules in flight per wave, and throws
 // the data away; probe_read_strips_kernel does the same for the column-strip
-// kernel's split (a workgroup of eight waves per 16, 32 or 64 columns over the
-// whole k range, eight rows of a strip per wave instruction).
+// kernel's split (a workgroup of eight waves per 16 to 64 columns over the
+// whole k range, eight rows of a strip per wave instruction) and the rows kernel's
+// (per 16 to 128 columns and row part, four rows of B at a time).
 // probe_empty_kernel does nothing at all.  probe_mfma_kernel is
 // a loop of nothing but v_mfma_f32_16x16x32_f16 on pseudo-random operands, two
 // waves per SIMD and 32 independent accumulators per wave: what the matrix
@@ -79,11 +80,12 @@ __global__ __launch_bounds__(256) void probe_read_kernel(GemmArgs p, int* sink) 
   if ((acc[0] & acc[1] & acc[2] & acc[3]) == 0x12345678 && sink) sink[0] = 1;
 }
 
-template <int CS>
+// ROWS: the rows kernel's chunks of four rows of B
+template <int CS, bool ROWS>
 __global__ __launch_bounds__(512) void probe_read_strips_kernel(GemmArgs p, int* sink) {
   // rows of B per chunk: two loads of 1 KiB per wave (three for three strips)
-  constexpr int NL = CS == 3 ? 3 : 2;
-  constexpr int kRows = 8 * NL / CS;
+  constexpr int NL = ROWS ? (CS + 1) / 2 : CS == 3 ? 3 : 2;
+  constexpr int kRows = ROWS ? 4 : 8 * NL / CS;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -100,8 +102,9 @@ __global__ __launch_bounds__(512) void probe_read_strips_kernel(GemmArgs p, int*
   for (int i = 0; i < NL; i++) {
     const int idx = 64 * i + lane;
     const int strip = strip0 + (idx / 8) % CS;
-    // (a strip past the last one, of a last workgroup of three, is not read)
-    b_lane[i] = strip < (p.N >> 4)
+    // (strips past the last one, of a last workgroup with fewer, and lanes past the
+    // chunk's lines read nothing)
+    b_lane[i] = strip < (p.N >> 4) && idx < 8 * CS * kRows
                     ? (idx / (8 * CS)) * b_row + 128 * strip + 16 * (idx % 8)
                     : kProbeOob;
   }
@@ -298,11 +301,44 @@ bool run_and_fetch(int n, float* host_out, F fn) {
 
 extern "C" {
 
+// The grid and the work split of a launch of this shape with prob_m rows; where
+// that is the prefill kernel's, of a launch with 16 rows.  out[0] = the kernel whose it
+// is (1 streaming, 3 column strips, 4 rows), out[1] = workgroups, out[2] = 16-column strips
+// per workgroup (0: streaming), out[3] = parts the rows are cut into, out[4], out[5] =
+// the streaming kernel's granules per workgroup and workgroups per column tile.  (No part
+// of the interface; exported for tests.)
+int w4a16_probe_split(int prob_m, int prob_n, int prob_k, int groupsize, int cus, int* out) {
+  for (int i = 0; i < 6; i++) out[i] = 0;
+  int rows[2], plan[13];
+  int rc = marlin_amd_rows_plan(prob_m, prob_n, prob_k, groupsize, cus, rows);
+  if (rc != MARLIN_OK) return rc;
+  if (rows[0] > 0) {
+    out[0] = 4;
+    out[2] = rows[0];
+    out[3] = w4a16::ceil_div(prob_m, rows[1]);
+    out[1] = w4a16::ceil_div(prob_n / 16, rows[0]) * out[3];
+    return rc;
+  }
+  rc = marlin_amd_plan(prob_m, prob_n, prob_k, groupsize, -1, -1, -1, cus, plan);
+  if (rc == MARLIN_OK && plan[0] == 2)
+    rc = marlin_amd_plan(16, prob_n, prob_k, groupsize, -1, -1, -1, cus, plan);
+  if (rc != MARLIN_OK) return rc;
+  out[0] = plan[0];
+  out[1] = plan[1];
+  out[2] = plan[12];
+  out[3] = plan[10];
+  out[4] = plan[2];
+  out[5] = plan[8];
+  return rc;
+}
+
 int marlin_amd_probe(int kind, const void* B, int prob_m, int prob_n, int prob_k, int dev,
                      void* stream_) {
   using namespace w4a16;
   hipStream_t stream = (hipStream_t)stream_;
   g_probe_error[0] = 0;
+  const int groupsize = kind == 4 || kind == 5 ? 128 : -1;
+  if (groupsize == 128) kind -= 4;
   if (prob_m <= 0 || prob_n <= 0 || prob_k <= 0 || dev < 0 || kind < 0 || kind > 2)
     return MARLIN_ERR_PROB_SHAPE;
   int info[5] = {0, 0, 0, 0, 0};
@@ -311,12 +347,8 @@ int marlin_amd_probe(int kind, const void* B, int prob_m, int prob_n, int prob_k
     return MARLIN_ERR_RUNTIME;
   }
   const int cus = info[0];
-  // the grid and the work split of a launch of this shape with prob_m rows; where
-  // that is the prefill kernel's, of a launch with 16 rows
-  int plan[13];
-  int rc = marlin_amd_plan(prob_m, prob_n, prob_k, -1, -1, -1, -1, cus, plan);
-  if (rc == MARLIN_OK && plan[0] == 2)
-    rc = marlin_amd_plan(16, prob_n, prob_k, -1, -1, -1, -1, cus, plan);
+  int split[6];
+  const int rc = w4a16_probe_split(prob_m, prob_n, prob_k, groupsize, cus, split);
   if (rc != MARLIN_OK) return rc;
   int prev = -1;
   hipError_t e = hipGetDevice(&prev);
@@ -326,8 +358,8 @@ int marlin_amd_probe(int kind, const void* B, int prob_m, int prob_n, int prob_k
     return MARLIN_ERR_RUNTIME;
   }
   (void)hipGetLastError();
-  const int grid = plan[1];
-  const int strips = plan[0] == 3 ? plan[12] : 0;
+  const int grid = split[1];
+  const int strips = split[2];
   if (kind == 0) {
     hipLaunchKernelGGL(probe_empty_kernel, dim3(grid), dim3(strips ? 512 : 256), 0, stream);
   } else if (kind == 1 && strips) {
@@ -336,23 +368,29 @@ int marlin_amd_probe(int kind, const void* B, int prob_m, int prob_n, int prob_k
     a.M = 1;
     a.N = prob_n;
     a.K = prob_k;
-    a.row_parts = plan[10];
-    if (strips == 1)
-      hipLaunchKernelGGL(probe_read_strips_kernel<1>, dim3(grid), dim3(512), 0, stream, a, (int*)nullptr);
-    else if (strips == 2)
-      hipLaunchKernelGGL(probe_read_strips_kernel<2>, dim3(grid), dim3(512), 0, stream, a, (int*)nullptr);
-    else if (strips == 3)
-      hipLaunchKernelGGL(probe_read_strips_kernel<3>, dim3(grid), dim3(512), 0, stream, a, (int*)nullptr);
-    else
-      hipLaunchKernelGGL(probe_read_strips_kernel<4>, dim3(grid), dim3(512), 0, stream, a, (int*)nullptr);
+    a.row_parts = split[3];
+    const auto read = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, stream, a, (int*)nullptr);
+    };
+    const bool rows = split[0] == 4;
+    switch (strips) {
+      case 1: read(rows ? probe_read_strips_kernel<1, true> : probe_read_strips_kernel<1, false>); break;
+      case 2: read(rows ? probe_read_strips_kernel<2, true> : probe_read_strips_kernel<2, false>); break;
+      case 3: read(rows ? probe_read_strips_kernel<3, true> : probe_read_strips_kernel<3, false>); break;
+      case 4: read(rows ? probe_read_strips_kernel<4, true> : probe_read_strips_kernel<4, false>); break;
+      case 5: read(probe_read_strips_kernel<5, true>); break;
+      case 6: read(probe_read_strips_kernel<6, true>); break;
+      case 8: read(probe_read_strips_kernel<8, true>); break;
+      default: e = hipErrorInvalidConfiguration;
+    }
   } else if (kind == 1) {
     GemmArgs a = {};
     a.B = B;
     a.M = 1;
     a.N = prob_n;
     a.K = prob_k;
-    a.gpb = plan[2];
-    a.wpt = plan[8];
+    a.gpb = split[4];
+    a.wpt = split[5];
     hipLaunchKernelGGL(probe_read_kernel, dim3(grid), dim3(256), 0, stream, a, (int*)nullptr);
   } else {
     // one workgroup of 8 waves per CU; n*k/8192 MFMAs per wave (a multiple of 32)
@@ -360,7 +398,7 @@ int marlin_amd_probe(int kind, const void* B, int prob_m, int prob_n, int prob_k
     hipLaunchKernelGGL(probe_mfma_kernel, dim3(cus), dim3(512), 0, stream,
                        (int)(per_wave / 32 > 0 ? per_wave / 32 : 1), (float*)nullptr);
   }
-  e = hipGetLastError();
+  if (e == hipSuccess) e = hipGetLastError();
   if (prev != dev) (void)hipSetDevice(prev);
   if (e != hipSuccess) {
     snprintf(g_probe_error, sizeof(g_probe_error), "probe launch: %s", hipGetErrorString(e));

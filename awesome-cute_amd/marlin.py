@@ -434,6 +434,8 @@ def _probes():
         lib = ctypes.CDLL(path)
         lib.marlin_amd_probe.restype = _I
         lib.marlin_amd_probe.argtypes = [_I, _P, _I, _I, _I, _I, _P]
+        lib.w4a16_probe_split.restype = _I
+        lib.w4a16_probe_split.argtypes = [_I, _I, _I, _I, _I, _P]
         lib.marlin_amd_probe_issue.restype = _I
         lib.marlin_amd_probe_issue.argtypes = [_I, _I, _I, _I, _I, _P]
         lib.marlin_amd_probe_pull.restype = _I
@@ -449,13 +451,26 @@ def _probe_check(rc, what):
                            f"{_probes().marlin_amd_probe_last_error().decode()}")
 
 
-def probe(kind, B, n, k, m=1):
+def probe(kind, B, n, k, m=1, groupsize=-1):
     """Measurement probe on the current stream: kind 0 = empty launch, 1 = plain read of the
-    packed weights B with the work split of the kernel planned for m rows of this shape, 2 = a
-    loop of nothing but MFMAs (n*k/8192 per wave, 8 waves per compute unit) (marlin_amd_probe)."""
+    packed weights B with the work split of the kernel that computes m rows of this shape with
+    these scales (probe_split), 2 = a loop of nothing but MFMAs (n*k/8192 per wave, 8 waves per
+    compute unit) (marlin_amd_probe)."""
     dev = B.get_device()
+    if groupsize == 128 and kind in (0, 1):
+        kind += 4
     _probe_check(_probes().marlin_amd_probe(kind, B.data_ptr(), m, n, k, dev, _raw_stream(dev)),
                  "marlin_amd_probe")
+
+
+def probe_split(m, n, k, groupsize=-1, cus=256):
+    """The split of probe kinds 0 and 1: that of the kernel that computes the problem (1 streaming,
+    3 column strips, 4 rows), or, where that is the prefill kernel, of the one for 16 rows (no GPU
+    touched)."""
+    out = (ctypes.c_int * 6)()
+    _probe_check(_probes().w4a16_probe_split(m, n, k, groupsize, cus, out), "w4a16_probe_split")
+    keys = ("kernel", "grid", "strips", "row_parts", "granules_per_wg", "wgs_per_tile")
+    return dict(zip(keys, out))
 
 
 def probe_issue(n_valu, n_lds=0, n_global=0, iters=2000, workgroups=256):

@@ -202,8 +202,8 @@ def time_shape(torch, marlin, O, name, steps, warmup, check=True, with_floor=Fal
     floor = None
     if with_floor and bound == "hbm":
         # what the launch alone and the weight stream alone cost, measured the same way
-        e_ms, _ = graph_ms(torch, side, lambda i: marlin.probe(0, dBs[0], N, K, M), steps, 1)
-        r_ms, r_spread = graph_ms(torch, side, lambda i: marlin.probe(1, dBs[i % nbuf], N, K, M),
+        e_ms, _ = graph_ms(torch, side, lambda i: marlin.probe(0, dBs[0], N, K, M, g), steps, 1)
+        r_ms, r_spread = graph_ms(torch, side, lambda i: marlin.probe(1, dBs[i % nbuf], N, K, M, g),
                                   steps, nbuf)
         floor = {"empty_kernel_us": e_ms * 1e3, "read_kernel_us": r_ms * 1e3,
                  "read_kernel_spread_us": [x * 1e3 for x in r_spread[:2]],

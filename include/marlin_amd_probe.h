@@ -17,11 +17,12 @@ extern "C" {
 
 /*
  * A probe launch on `stream` of device `dev`.  Kinds 0 and 1 use the grid and
- * the workgroup size marlin_gemm uses for prob_m rows of this shape (where
- * that is the prefill kernel's, for 16 rows): kind 0 = an empty kernel (what a
- * launch costs), kind 1 = a kernel that reads the packed weights B
+ * the workgroup size marlin_gemm uses for prob_m rows of this shape with one
+ * scale per column, kinds 4 and 5 with scales per group of 128 (where that is
+ * the prefill kernel's, for 16 rows): kind 0 (4) = an empty kernel (what a
+ * launch costs), kind 1 (5) = a kernel that reads the packed weights B
  * ((prob_k/16, 2*prob_n) int32) with the work split of the kernel planned for
- * the shape -- the streaming kernel's or the column-strip kernel's -- and
+ * the shape -- the streaming, the column-strip or the rows kernel's -- and
  * 128-bit loads and does nothing with them (what the weight stream alone
  * costs).  Kind 2 = a loop of nothing but v_mfma_f32_16x16x32_f16 on
  * pseudo-random operands, one workgroup of 8 waves per compute unit and

@@ -67,6 +67,23 @@ def test_not_where_it_was_slower(m, n, k, groupsize):
     assert marlin.rows_plan(m, n, k, groupsize) is None
 
 
+@pytest.mark.parametrize("m,n,k,groupsize", [(64, 28672, 8192, 128), (45, 12288, 4096, -1), (144, 2048, 1792, 128),
+                                             (491, 2048, 5760, 128)])
+def test_the_probes_follow_this_kernel(m, n, k, groupsize):
+    """The floor beside a problem is that of the launch that computes it."""
+    import marlin
+    strips, rows = marlin.rows_plan(m, n, k, groupsize)
+    parts = -(-m // rows)
+    assert marlin.probe_split(m, n, k, groupsize) == {
+        "kernel": 4, "grid": -(-(n // 16) // strips) * parts, "strips": strips, "row_parts": parts,
+        "granules_per_wg": 0, "wgs_per_tile": 0}
+    marlin.force_rows(-1)
+    try:
+        assert marlin.probe_split(m, n, k, groupsize)["kernel"] in (1, 3)
+    finally:
+        marlin.force_rows(0)
+
+
 def _gemm(A, B, s, n):
     import torch
     import marlin
@@ -117,6 +134,23 @@ def test_rows_return_dequantised_weights(pair, groupsize):
             assert np.array_equal(_gemm(A, B, sp, n).view(np.uint16), W[base:base + m].view(np.uint16)), base
     finally:
         marlin.force_rows(0)
+
+
+@pytest.mark.gpu
+def test_probes_of_every_pair_run():
+    import torch
+    import marlin
+    n, k = 1280, 1152
+    B = torch.randint(-2**31, 2**31 - 1, (k // 16, 2 * n), dtype=torch.int32, device="cuda:0")
+    for (strips, blocks), g in CASES:
+        marlin.force_rows(strips, blocks)
+        try:
+            assert marlin.probe_split(70, n, k, g)["kernel"] == 4
+            for kind in (0, 1):
+                marlin.probe(kind, B, n, k, 70, g)
+        finally:
+            marlin.force_rows(0)
+        torch.cuda.synchronize()
 
 
 @pytest.mark.gpu
