@@ -20,6 +20,7 @@
 #include <cstdio>
 
 #include "../../include/marlin_amd_convert.h"
+#include "../../include/marlin_amd_tools.h"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
@@ -484,19 +485,19 @@ bool grid_holds(long long x, int threads, long long y) {
 }
 long long pieces_of(long long a, int b) { return (a + b - 1) / b; }
 
-// Whether long groups are quantised in chunks.  In one launch, a workgroup per group
-// of 64 columns, a row takes a round of workgroups 14 to 30 ns, however few they
-// are; in chunks the chip is full whatever n is, but w is read twice and there are
-// three launches.  One scale per column, us in one launch and in chunks: n = 1024, k =
-// 1024 15.6 and 15.6, 2048 28.7 and 16.2, 8192 113.7 and 22.5; n = 4096 1024 17.1 and
-// 17.6, 4096 74.9 and 31.4, 8192 156 and 58; n = 8192 2048 40.4 and 30.3; n = 11008
-// 1024 23.9 and 24.2, 4096 100.8 and 82.0; n = 16384 2048 52.0 and 64.9, 4096 120.8
-// and 127.3; n = 28672 1024 46.6 and 49.7, 8192 556 and 454.
-bool in_chunks(int n, int k, int gs) {
-  constexpr double kUnits = 256;  // compute units of the chip
-  const double wgs = (double)pieces_of(n, 64) * (k / gs);
-  const double rounds = wgs <= kUnits ? 1.0 : (double)pieces_of((long long)wgs, (int)kUnits);
-  const double whole = gs * rounds * (0.0139 + 6.1e-5 * (wgs < kUnits ? wgs : kUnits));
+// Whether long groups are quantised in chunks, on a device of `cus` compute units.  In
+// one launch, a workgroup per group of 64 columns, a row takes a round of workgroups 14
+// to 30 ns, however few they are; in chunks the chip is full whatever n is, but w is
+// read twice and there are three launches.  One scale per column, 256 compute units, us
+// in one launch and in chunks: n = 1024, k = 1024 15.6 and 15.6, 2048 28.7 and 16.2, 8192
+// 113.7 and 22.5; n = 4096 1024 17.1 and 17.6, 4096 74.9 and 31.4, 8192 156 and 58; n =
+// 8192 2048 40.4 and 30.3; n = 11008 1024 23.9 and 24.2, 4096 100.8 and 82.0; n = 16384
+// 2048 52.0 and 64.9, 4096 120.8 and 127.3; n = 28672 1024 46.6 and 49.7, 8192 556 and
+// 454.
+bool in_chunks(int n, int k, int gs, int cus) {
+  const long long wgs = pieces_of(n, 64) * (k / gs);
+  const double rounds = (double)pieces_of(wgs, cus);
+  const double whole = gs * rounds * (0.0139 + 6.1e-5 * (wgs < cus ? wgs : cus));
   const double chunks = 16.0 + gs * wgs * 1.02e-4;
   return chunks < whole && pieces_of(gs, kChunkRows) * (k / gs) <= 65535;
 }
@@ -527,6 +528,9 @@ int marlin_amd_quantize(const void* w, int k, int n, int groupsize, int by_colum
                 : !grid_holds(pieces_of(n, small ? 256 : 64), kQThreads, k / gs))
     return MARLIN_ERR_PROB_SHAPE;
   OnDevice on(dev);
+  int cus = 0;
+  if (on.e == hipSuccess && !by_column && !small)
+    on.e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (on.e != hipSuccess) return on.done();
   const half_t* in = (const half_t*)w;
   const hipStream_t st = (hipStream_t)stream;
@@ -540,7 +544,7 @@ int marlin_amd_quantize(const void* w, int k, int n, int groupsize, int by_colum
   } else if (small) {
     hipLaunchKernelGGL(quantise_rows<64>, dim3((unsigned)pieces_of(n, 256), k / gs), dim3(kQThreads), 0, st, in,
                        n, gs, (half_t*)fake, (int*)q, (half_t*)s);
-  } else if (in_chunks(n, k, gs)) {
+  } else if (in_chunks(n, k, gs, cus)) {
     const int per_group = (int)pieces_of(gs, kChunkRows);
     const dim3 chunks((unsigned)pieces_of(n, 256), (unsigned)(k / gs) * per_group);
     hipLaunchKernelGGL(chunk_maxima, chunks, dim3(kQThreads), 0, st, in, n, gs, per_group, (unsigned short*)q);
@@ -553,6 +557,12 @@ int marlin_amd_quantize(const void* w, int k, int n, int groupsize, int by_colum
                        gs, (half_t*)fake, (int*)q, (half_t*)s);
   }
   return on.done();
+}
+
+int marlin_amd_quantize_launches(int k, int n, int groupsize, int by_column, int cus) {
+  const int gs = groupsize == -1 ? k : groupsize;
+  if (k <= 0 || n <= 0 || gs <= 0 || k % gs != 0 || cus <= 0) return 0;
+  return !by_column && gs > 128 && in_chunks(n, k, gs, cus) ? 3 : 1;
 }
 
 int marlin_amd_pack(const void* w, int k, int n, int groupsize, int by_column, const void* scales,

@@ -136,6 +136,13 @@ int marlin_amd_rows_plan(int prob_m, int prob_n, int prob_k, int groupsize, int 
 void marlin_amd_force_rows(int strips, int blocks);
 
 /*
+ * Launches of marlin_amd_quantize on a device of `cus` compute units: three where long
+ * groups are quantised in chunks of 128 rows, else one (0: no such problem).  No
+ * reference counterpart.
+ */
+int marlin_amd_quantize_launches(int k, int n, int groupsize, int by_column, int cus);
+
+/*
  * out[0..4] = compute units, shader clock (kHz), memory clock (kHz), memory
  * bus width (bits), L2 size (bytes) of device dev, as the HIP runtime reports
  * them.  Returns MARLIN_OK or MARLIN_ERR_RUNTIME.

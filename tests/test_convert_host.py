@@ -82,3 +82,14 @@ def test_what_the_kernels_do_not_take_is_left_to_the_tensor_operations():
         marlin.quantize(w, 2 ** 40)
     with pytest.raises(TypeError):
         marlin.quantize(w, 128.0)
+
+
+def test_the_devices_own_compute_units_decide_how_long_groups_are_quantised():
+    """A workgroup per 64 columns fills a small device sooner, and then takes rounds of them."""
+    import marlin
+    launches = marlin._lib.marlin_amd_quantize_launches
+    assert launches(4096, 4096, 128, 0, 256) == launches(4096, 4096, -1, 1, 256) == 1
+    assert launches(1024, 4096, -1, 0, 256) == 1 and launches(4096, 4096, -1, 0, 256) == 3
+    # 256 workgroups: one round of 256 compute units, four of 64
+    assert launches(2048, 16384, -1, 0, 256) == 1 and launches(2048, 16384, -1, 0, 64) == 3
+    assert launches(2048, 16384, -1, 0, 0) == 0
