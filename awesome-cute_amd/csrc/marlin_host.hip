@@ -760,9 +760,11 @@ RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& 
   return best;
 }
 
-// A thread's last plans, by everything that they are made from (no overrides among
-// it): planning takes the host up to a microsecond, a third of a launch, and a
-// decoder calls the same few sizes over and over.
+// A thread's last 32 plans, by everything that they are made from (no overrides among
+// it): planning takes the host 0.6 to 2.6 us, most for 17 to 300 rows, and a decoder calls
+// the same few sizes over and over.  The oldest makes room.  (One place for each size, by
+// a hash, was found sooner but given to another size of the same place at every call of
+// two such sizes: one set of four sizes in six.)
 struct Planned {
   int m = 0, n = 0, k = 0, sms = 0, cus = 0, counters = 0;
   size_t partial_limit = 0;
@@ -772,6 +774,7 @@ struct Planned {
 };
 constexpr int kPlansKept = 32;
 thread_local Planned t_plans[kPlansKept];
+thread_local int t_oldest_plan = 0;
 
 Planned make_plans(int m, int n, int k, int sms, const PlanCtx& cx) {
   Planned p;
@@ -788,14 +791,21 @@ Planned make_plans(int m, int n, int k, int sms, const PlanCtx& cx) {
   return p;
 }
 
+const Planned* kept_plans(int m, int n, int k, int sms, const PlanCtx& cx) {
+  for (const Planned& p : t_plans)
+    if (p.m == m && p.n == n && p.k == k && p.sms == sms && p.cus == cx.cus && p.counters == cx.counters &&
+        p.partial_limit == cx.partial_limit && p.grouped == cx.grouped)
+      return &p;
+  return nullptr;
+}
+
 Planned plans_for(int m, int n, int k, int sms, const PlanCtx& cx) {
   if (cx.force.any()) return make_plans(m, n, k, sms, cx);
-  const unsigned mix = (unsigned)m * 0x9e3779b1u ^ (unsigned)n * 0x85ebca6bu ^ (unsigned)k * 0xc2b2ae35u;
-  Planned& kept = t_plans[(mix >> 16) % kPlansKept];
-  if (kept.m != m || kept.n != n || kept.k != k || kept.sms != sms || kept.cus != cx.cus ||
-      kept.counters != cx.counters || kept.partial_limit != cx.partial_limit || kept.grouped != cx.grouped)
-    kept = make_plans(m, n, k, sms, cx);
-  return kept;
+  const Planned* kept = kept_plans(m, n, k, sms, cx);
+  if (kept) return *kept;
+  Planned& place = t_plans[t_oldest_plan];
+  t_oldest_plan = (t_oldest_plan + 1) % kPlansKept;
+  return place = make_plans(m, n, k, sms, cx);
 }
 
 // Enqueue the launches of plan pl with the scratch of `view` (null pointers
@@ -1100,6 +1110,16 @@ int marlin_amd_rows_plan(int prob_m, int prob_n, int prob_k, int groupsize, int 
   out[0] = rows.strips;
   out[1] = 16 * rows.blocks;
   return rc;
+}
+
+int marlin_amd_plan_kept(int prob_m, int prob_n, int prob_k, int groupsize, int cus) {
+  int thread_k = -1, thread_n = -1;
+  const int rc = check_shape(prob_m, prob_n, prob_k, groupsize, thread_k, thread_n);
+  if (rc != MARLIN_OK || prob_m == 0 || prob_n == 0 || prob_k == 0) return -1;
+  const PlanCtx cx = {cus, kPoolPartialLimit, t_force, groupsize != -1};
+  if (kept_plans(prob_m, prob_n, prob_k, -1, cx)) return 1;
+  plans_for(prob_m, prob_n, prob_k, -1, cx);
+  return 0;
 }
 
 int marlin_amd_plan_costs(int prob_m, int prob_n, int prob_k, int groupsize, int cus, double* out) {

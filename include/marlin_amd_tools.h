@@ -128,6 +128,14 @@ void marlin_amd_force_finish_polls(int polls);
 int marlin_amd_rows_plan(int prob_m, int prob_n, int prob_k, int groupsize, int cus, int *out);
 
 /*
+ * Whether the calling thread still has the plans of a marlin_gemm call of this shape on
+ * a device of `cus` compute units, without hints and with max_par >= 16: 1, or 0, and then
+ * it has them now, as after the call itself (it keeps the last 32; overrides are
+ * planned anew at every call).  -1: no such problem.  No reference counterpart.
+ */
+int marlin_amd_plan_kept(int prob_m, int prob_n, int prob_k, int groupsize, int cus);
+
+/*
  * That kernel with these strips (1 to 8) and row blocks of 16 (1 to 4) per
  * workgroup for every call of the calling thread without an `sms` hint, where the
  * pair exists; strips = 0: by cost (default; never beside another override),

@@ -616,3 +616,25 @@ int main(void) {
         run = subprocess.run([str(exe)], capture_output=True, text=True)
         assert run.returncode == 0, (run.returncode, run.stdout, run.stderr)
         assert "marlin_amd" in run.stdout
+
+
+def test_a_thread_keeps_its_last_32_plans(marlin):
+    """Whatever the sizes: none of 32 makes another's plan go, the 33rd the oldest."""
+    import threading
+
+    def run():
+        kept = marlin._lib.marlin_amd_plan_kept
+        sizes = [(m, n, k, g) for m in (1, 45) for n in (4096, 5120, 11008, 12288) for k in (4096, 11008) for g in (128, -1)]
+        assert [kept(*s, 256) for s in sizes] == [0] * 32
+        for _ in range(2):
+            assert [kept(*s, 256) for s in sizes] == [1] * 32
+        assert kept(*sizes[5], 64) == 0  # another device's
+        assert kept(*sizes[0], 256) == 0 and kept(*sizes[2], 256) == 1
+        assert kept(100, 1000, 64, 128, 256) == -1
+        seen.append(True)
+
+    seen = []
+    thread = threading.Thread(target=run)  # (a thread of its own: it has no plans yet)
+    thread.start()
+    thread.join()
+    assert seen
