@@ -31,6 +31,30 @@ def env():
     return torch, streamk
 
 
+@pytest.fixture(params=[0, -1], ids=["chosen", "planned"])
+def tiles(request, env):
+    """The tiles that are chosen by cost, and the plan's own launches."""
+    env[1].force_tile(request.param)
+    yield request.param
+    env[1].force_tile(0)
+
+
+@pytest.fixture(params=[(0,), (-1,), (32, 32, 2), (64, 128, 2), (64, 64, 4)], ids=str)
+def sliced(request, env):
+    """The same, and tiles in slices; whether a problem must run in slices that meet."""
+    streamk = env[1]
+    streamk.force_tile(*request.param)
+
+    def check(m, n, k):
+        tile = streamk.tile(m, n, k)
+        if request.param == (-1,):
+            assert tile is None and streamk.launches(m, n, k)[0]["slices"] > 1
+        elif request.param != (0,):
+            assert tile == request.param
+    yield check
+    streamk.force_tile(0)
+
+
 def inputs(m, n, k, seed, integers=False):
     rng = np.random.default_rng(seed)
     if integers:
@@ -68,13 +92,13 @@ SHAPES = [(256, 256, 64), (1, 256, 64), (16, 256, 192), (255, 256, 128), (257, 5
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
-def test_matches_oracle(env, m, n, k):
+def test_matches_oracle(env, m, n, k, tiles):
     A, B = inputs(m, n, k, m + n + k)
     close(gpu_gemm(env, A, B), O.dense_gemm_tn(A, B))
 
 
 @pytest.mark.parametrize("m,n,k", [(256, 256, 64), (300, 512, 320), (256, 512, 2048), (700, 768, 512)])
-def test_small_integers_are_exact(env, m, n, k):
+def test_small_integers_are_exact(env, m, n, k, tiles):
     """Sums of products of integers in [-3, 3] stay below 2048 in magnitude for these
     depths only in the typical case, so compare through the oracle where the value is
     exactly representable and demand bit equality there."""
@@ -86,7 +110,7 @@ def test_small_integers_are_exact(env, m, n, k):
     assert np.array_equal(C[exact], want[exact])
 
 
-def test_one_hot_rows_return_rows_of_b(env):
+def test_one_hot_rows_return_rows_of_b(env, tiles):
     """A one-hot row of A selects a row of B^T: C[i, :] = B[:, k_i], bit for bit; this
     pins the operand layout for every k position of two stages and every column."""
     m, n, k = 128, 512, 128
@@ -101,7 +125,7 @@ def test_one_hot_rows_return_rows_of_b(env):
 @pytest.mark.parametrize("m,n,k", [(4096, 4352, 4096), (1152, 4352, 4096), (4096, 4352, 10240),
                                    (4000, 4352, 512), (8100, 8192, 256), (2048, 2048, 2048),
                                    (1000, 4096, 4096)])
-def test_reference_examples(env, m, n, k):
+def test_reference_examples(env, m, n, k, tiles):
     """The reference's stream-K examples at full size (gemm/readme.md:27-31), and two
     shapes whose last row tile of 256 is partly empty: a sample of rows against the oracle, the whole result against torch's fp32 product by the
     reference's cosine criterion, and bit-identical results on a second run."""
@@ -122,12 +146,14 @@ def test_reference_examples(env, m, n, k):
     assert (C.float() - ref).abs().max().item() <= TOL * ref.abs().max().item()
 
 
-def test_back_to_back_calls_share_the_scratch(env):
+def test_back_to_back_calls_share_the_scratch(env, sliced):
     """Stream-K launches one after the other on a stream reuse the partial-sum buffer and
     hand the tile counters back zeroed: a different problem in between must not disturb
     either result."""
     torch, streamk = env
     dev = torch.device("cuda:0")
+    sliced(700, 768, 1024)
+    sliced(256, 512, 4096)
     A1, B1 = inputs(700, 768, 1024, 1)
     A2, B2 = inputs(256, 512, 4096, 2)
     d = [torch.from_numpy(x).to(dev) for x in (A1, B1, A2, B2)]
@@ -141,11 +167,13 @@ def test_back_to_back_calls_share_the_scratch(env):
     close(outs[0][1].cpu().numpy(), O.dense_gemm_tn(A2, B2))
 
 
-def test_two_streams_run_side_by_side(env):
+def test_two_streams_run_side_by_side(env, sliced):
     """Stream-K launches on two streams at once: each stream has its own partial-sum
     buffer and tile counters; every result equals the one the same call gives alone."""
     torch, streamk = env
     dev = torch.device("cuda:0")
+    sliced(700, 768, 1024)
+    sliced(256, 512, 4096)
     A1, B1 = inputs(700, 768, 1024, 3)
     A2, B2 = inputs(256, 512, 4096, 4)
     d = [torch.from_numpy(x).to(dev) for x in (A1, B1, A2, B2)]
@@ -163,13 +191,15 @@ def test_two_streams_run_side_by_side(env):
 
 
 @pytest.mark.parametrize("m,n,k", [(700, 768, 1024), (512, 256, 2048), (2048, 2048, 512)])
-def test_kernels_of_other_streams_beside_do_not_change_the_result(env, m, n, k):
+def test_kernels_of_other_streams_beside_do_not_change_the_result(env, m, n, k, sliced):
     """A launch must give the same bits whatever else runs on the GPU.  Kernels of another
     stream that keep the compute units' LDS and memory busy (softmax, sort) stretch the
     latencies inside the GEMM; once, operand reads still in flight when the main loop ended
     landed in registers that already held the addresses of the partial sums."""
     torch, streamk = env
     dev = torch.device("cuda:0")
+    if m < 2048:  # (2048 x 2048 runs in whole tiles)
+        sliced(m, n, k)
     A, B = inputs(m, n, k, 5)
     dA, dB = torch.from_numpy(A).to(dev), torch.from_numpy(B).to(dev)
     alone = streamk.gemm(dA, dB)
@@ -212,12 +242,14 @@ def test_degenerate_sizes_and_errors(env):
                      torch.zeros((256, 128), dtype=torch.half, device=dev))
 
 
-def test_graph_replays_match_eager(env):
+def test_graph_replays_match_eager(env, sliced):
     """A captured stream-K launch replayed several times, with eager launches and
     synchronisations in between, gives the eager result every time (the tile counters
     are handed back zeroed by the kernel itself, nothing in the launch is a memset)."""
     torch, streamk = env
     dev = torch.device("cuda:0")
+    sliced(700, 768, 1024)
+    sliced(256, 512, 2048)
     A, B = inputs(700, 768, 1024, 5)
     dA, dB = torch.from_numpy(A).to(dev), torch.from_numpy(B).to(dev)
     A2, B2 = inputs(256, 512, 2048, 6)
@@ -242,7 +274,7 @@ def test_graph_replays_match_eager(env):
 
 
 @pytest.mark.parametrize("tag", ["a", "b"])
-def test_frozen_known_answers(env, tag):
+def test_frozen_known_answers(env, tag, tiles):
     """The committed known answers (tests/golden/f16_gemm_known_answers.npz)."""
     z = np.load(os.path.join(ROOT, "tests", "golden", "f16_gemm_known_answers.npz"))
     A, B = z[f"{tag}_A"].view(np.float16), z[f"{tag}_B"].view(np.float16)

@@ -22,8 +22,17 @@ def env():
     return torch, streamk
 
 
+@pytest.fixture(autouse=True)
+def planned(env):
+    """The plan's own launches, also where tiles of other sizes would be taken."""
+    env[1].force_tile(-1)
+    yield
+    env[1].force_tile(0)
+
+
 def _check(env, m, n, k, top, tile):
     torch, streamk = env
+    assert streamk.tile(m, n, k) is None
     _, plan = streamk.plan(m, n, k)
     assert (plan["tile_rows"], plan["tile_cols"]) == tile
     gen = torch.Generator(device="cuda:0")
