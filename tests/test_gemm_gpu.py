@@ -30,6 +30,14 @@ def env():
     return torch, marlin
 
 
+@pytest.fixture(params=[0, -1], ids=["chosen", "planned"])
+def rows_choice(request, env):
+    """By cost, and without the kernel that keeps the rows of a strip set together: the plan's own."""
+    env[1].force_rows(request.param)
+    yield request.param
+    env[1].force_rows(0)
+
+
 @pytest.fixture
 def no_strips(env):
     """Up to 16 rows through the streaming kernel, as larger launches go: for
@@ -128,7 +136,7 @@ def test_closed_forms(env):
 
 
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 8, 12, 16, 24, 32, 48, 64, 118, 128, 152, 768, 1024])
-def test_tiles(env, m):
+def test_tiles(env, m, rows_choice):
     # marlin_test.py:78-84
     for thread_k, thread_n in [(64, 256), (128, 128)]:
         if m > 16 and thread_k == 128:
@@ -324,12 +332,19 @@ def test_two_host_threads_two_streams(env, no_strips):
 
 @pytest.mark.parametrize("m", [17, 31, 32, 33, 47, 48, 49, 63, 64])
 @pytest.mark.parametrize("groupsize", [128, -1])
-def test_lds_ring_row_counts(env, m, groupsize):
+@pytest.mark.parametrize("which", [0, 1])  # by cost, and the kernel with the ring
+def test_lds_ring_row_counts(env, which, m, groupsize):
     """2-4 row blocks take their activations through the LDS ring; ragged row
     counts, a deep k (many ring turns) and a shallow one (ring never full; one
     scale row would mean per-channel scales, so two groups at least)."""
-    check(env, m, 512, 4096, groupsize, seed=m)
-    check(env, m, 256, 256, groupsize, seed=m + 100)
+    torch, marlin = env
+    marlin.force_kernel(which)
+    try:
+        assert which == 0 or marlin.plan(m, 512, 4096, groupsize)[1]["kernel"] == which
+        check(env, m, 512, 4096, groupsize, seed=m)
+        check(env, m, 256, 256, groupsize, seed=m + 100)
+    finally:
+        marlin.force_kernel(0)
 
 
 @pytest.mark.parametrize("which", [1, 2])
@@ -913,7 +928,12 @@ def test_scratch_is_sized_by_the_plan_and_can_be_released(env, no_strips):
         # the dense GEMM's stream-K tiles use the same buffer of this stream
         a = torch.randn((256, 2048), dtype=torch.half, device=dev)
         b = torch.randn((512, 2048), dtype=torch.half, device=dev)
-        c = streamk.gemm(a, b)
+        streamk.force_tile(-1)
+        try:
+            assert streamk.launches(256, 512, 2048)[0]["slices"] > 1
+            c = streamk.gemm(a, b)
+        finally:
+            streamk.force_tile(0)
         streams[0].synchronize()
         assert marlin.scratch_bytes(0)[1] == 9
         assert torch.allclose(c.float(), a.float() @ b.float().t(), rtol=2e-2, atol=0.5)
@@ -1035,7 +1055,7 @@ def test_config4_prefill_rows_sample(env):
 
 
 @pytest.mark.parametrize("groupsize", [128, -1])
-def test_config5_large_uneven(env, groupsize):
+def test_config5_large_uneven(env, groupsize, rows_choice):
     """M=64, N=28672, K=8192.  Oracle on a column slice (columns are
     independent; a slice of the packed buffers on 128-column boundaries is a
     valid problem of its own), GPU on the full shape."""
@@ -1121,7 +1141,7 @@ def test_profiling_row(env, groupsize):
 
 
 @pytest.mark.parametrize("m,n,k,which", [(1, 4096, 4096, 4), (1, 4096, 4096, 3), (48, 1024, 4096, 0),
-                                         (200, 2048, 2048, 0)])
+                                         (200, 2048, 2048, 0), (48, 1024, 4096, 1), (200, 2048, 2048, 2)])
 def test_graph_replays_match_eager(env, m, n, k, which):
     """A captured launch (streaming kernel with shared tiles, column strips, LDS-ring
     variant, prefill kernel with k slices) replayed several times, with eager launches and
@@ -1131,6 +1151,9 @@ def test_graph_replays_match_eager(env, m, n, k, which):
     dev = torch.device("cuda:0")
     marlin.force_kernel(which)
     try:
+        plan = marlin.plan(m, n, k, 128)[1]
+        assert which in (0, 4) or plan["kernel"] == which
+        assert which != 2 or plan["k_slices"] > 1
         _graph_replays(torch, marlin, dev, m, n, k)
     finally:
         marlin.force_kernel(0)

@@ -99,11 +99,21 @@ def test_dequantised_weights_bit_exact(env, rows, groupsize):
 
 @pytest.mark.parametrize("m,n,k", [(690, 4608, 4096), (140, 11008, 4864), (565, 1792, 2816), (529, 768, 4992),
                                    (236, 3072, 4352)])
-def test_slices_captured_without_scratch(env, m, n, k):
+@pytest.mark.parametrize("rows", [0, -1])  # by cost (some of them in whole row blocks, without slices), and in slices
+def test_slices_captured_without_scratch(env, rows, m, n, k):
     """Problems that run in slices are captured on a stream that has no scratch, without any:
     nothing is allocated, and the replays are right whatever runs in between.  On a stream
     that has scratch the graph repeats the bits of the eager call."""
     torch, marlin = env
+    marlin.force_rows(rows)
+    try:
+        assert rows == 0 or marlin.rows_plan(m, n, k, 128) is None
+        _captured_without_scratch(torch, marlin, m, n, k)
+    finally:
+        marlin.force_rows(0)
+
+
+def _captured_without_scratch(torch, marlin, m, n, k):
     dev = torch.device("cuda:0")
     assert marlin.plan(m, n, k, 128)[1]["k_slices"] > 1
     A, _, _, B, sp = O.make_problem(m, n, k, 128, seed=m)
