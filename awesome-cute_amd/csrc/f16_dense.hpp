@@ -1,14 +1,14 @@
-// What the dense fp16 kernels share: their arguments, the numbering of tiles and
-// slices, and the loads that write LDS directly.
+// What the dense fp16 kernels share: their arguments and the numbering of tiles and
+// slices.
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
 
 constexpr int kDnStageK = 64;    // k depth of a stage (two MFMA k steps); k is a multiple
-constexpr int kDnOob = (int)0x80000000;
 constexpr int kDnMaxSlices = 4;
 constexpr int kDnCounterStride = 16;  // ints: a tile's slices meet in a cache line of their own
 
@@ -66,34 +66,6 @@ __host__ __device__ __forceinline__ void dn_slice_coord(int block, int tiles, in
   *tile = work / slices;
   *slice = work - *tile * slices;
 }
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t dn_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
-
-// 16 bytes per lane from a buffer straight into LDS: lane l's bytes land at
-// dst + 16*l (dst is wave-uniform).  The instruction's immediate offset stays
-// zero: the hardware would add it to the LDS address as well.  (Device pass
-// only; the host pass just needs the kernel's launch stub.)
-__device__ __forceinline__ void dn_dma16(__amdgpu_buffer_rsrc_t rsrc, char* dst, int voffset,
-                                         int soffset) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, voffset, soffset, 0, 0);
-#endif
-}
-
-// LDS reads of a main loop, outside the compiler's dependence tracking (it
-// would wait for every load in flight before each of them)
-template <int OFF>
-__device__ __forceinline__ void dn_read16(unsigned at, i4& v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF) : "memory");
-#endif
-}
-
-// s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
-constexpr int dn_vmcnt(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 
 __device__ __forceinline__ h4 dense_round(f4 v) {
   return (h4){(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};

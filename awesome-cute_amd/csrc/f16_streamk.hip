@@ -102,13 +102,6 @@ constexpr int kDnMaxSlots = 256;  // slices in flight per launch
 constexpr int kDnPairK = 7168;    // depth from which 128 x 256 tiles in two slices beat 128 x 128 ones
 constexpr int kDnRunsK = 6144;    // depth from which 128 x 256 tiles are not dealt out in runs, see there
 
-// the four words of a raw buffer resource: 48-bit base, stride 0, size in
-// bytes, data format flags
-__device__ __forceinline__ i4 dn_rsrc_words(const void* p, unsigned bytes) {
-  const unsigned long long a = (unsigned long long)p;
-  return (i4){(int)(unsigned)a, (int)(unsigned)((a >> 32) & 0xffffu), (int)bytes, 0x00020000};
-}
-
 // wait until at most PENDING later LDS reads are outstanding; `v` is the
 // operand the wait is for
 template <int PENDING>
@@ -230,10 +223,10 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
   const int last =
       SLICED ? (int)((unsigned)(ks + 1) * (unsigned)slabs_all / (unsigned)p.ksplit) : slabs_all;
   const int skip = first * (kDnStageK * 2);  // bytes of a row before them
-  i4 ra_words = dn_rsrc_words((const char*)p.A + (size_t)m0 * p.K * 2 + skip,
-                              (unsigned)rows * (unsigned)p.K * 2u - (unsigned)skip);
-  i4 rb_words = dn_rsrc_words((const char*)p.B + (size_t)n0 * p.K * 2 + skip,
-                              256u * (unsigned)p.K * 2u - (unsigned)skip);
+  i4 ra_words = rsrc_words((const char*)p.A + (size_t)m0 * p.K * 2 + skip,
+                           (unsigned)rows * (unsigned)p.K * 2u - (unsigned)skip);
+  i4 rb_words = rsrc_words((const char*)p.B + (size_t)n0 * p.K * 2 + skip,
+                           256u * (unsigned)p.K * 2u - (unsigned)skip);
 
   // wave w fetches the w-th quarter of the A rows and of the B rows of a slab,
   // eight rows per instruction: lane (r = lane/8, c = lane%8) lands at [r][c] and
@@ -319,7 +312,7 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
       // as in dense_small_kernel, with eight pieces of half the columns of a row
       // block (operands 4 (e % 2) ... + 3 of block e / 2 of every wave)
       __shared__ int s_shares;
-      const __amdgpu_buffer_rsrc_t rP = dn_rsrc(p.scratch, 0x7fffffffu);
+      const __amdgpu_buffer_rsrc_t rP = make_rsrc(p.scratch, 0x7fffffffu);
       int* const word = &p.locks[tile * kDnCounterStride];
       const int at = wave * (NF * 8 * 1024) + lane * 16;
       const auto part = [&](int k2) { return (tile * p.ksplit + k2) * Shape::kPartBytes; };
@@ -332,7 +325,7 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseArgs p) {
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, fin[e >> 1][o]), rP,
                                                    at + (8 * (e >> 1) + o) * 1024, part(ks), 16 /* sc1 */);
         }
-        __builtin_amdgcn_s_waitcnt(dn_vmcnt(0));  // my stores have been acknowledged
+        __builtin_amdgcn_s_waitcnt(vmcnt(0));  // my stores have been acknowledged
         __syncthreads();
       };
       const int my_share = finish_pieces(1 << ks, p.ksplit, 8);
@@ -420,9 +413,9 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   if (CUT && rows <= 0) return;  // a quarter below the last row, all its slices
 
   const __amdgpu_buffer_rsrc_t rA =
-      dn_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
+      make_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
   const __amdgpu_buffer_rsrc_t rB =
-      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)TN * (unsigned)p.K * 2u);
+      make_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)TN * (unsigned)p.K * 2u);
 
   // wave w fetches the w-th eighth of the A rows and of the B rows of a slab, as
   // dense_kernel does
@@ -445,14 +438,14 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   const int stages = st1 - st0;
 
   auto issue_slab = [&](int s, int slot) {
-    const int inv = s < stages ? 0 : kDnOob;  // a stage past the end fetches zeros
+    const int inv = s < stages ? 0 : kOob;  // a stage past the end fetches zeros
     const int at = (st0 + s) * (kDnStageK * 2);
     char* base = smem + slot * Sh::kSlab;
 #pragma unroll
-    for (int t = 0; t < TA; t++) dn_dma16(rA, base + (TA * wave + t) * 1024, a_src[t] | inv, at);
+    for (int t = 0; t < TA; t++) load_to_lds16(rA, base + (TA * wave + t) * 1024, a_src[t] | inv, at);
 #pragma unroll
     for (int t = 0; t < NJ; t++)
-      dn_dma16(rB, base + Sh::kSlabA + (NJ * wave + t) * 1024, b_src[t] | inv, at);
+      load_to_lds16(rB, base + Sh::kSlabA + (NJ * wave + t) * 1024, b_src[t] | inv, at);
   };
 
   f4 acc[RB][NJ];
@@ -479,11 +472,11 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
     b_rd[h] = (unsigned)(size_t)smem + Sh::kSlabA + (16 * NJ * wn + nu) * 128 + sw;
   }
   auto read_b = [&](unsigned at, i4 (&dst)[NJ]) {
-    dn_read16<0>(at, dst[0]);
-    dn_read16<2048>(at, dst[1]);
+    read_lds16<0>(at, dst[0]);
+    read_lds16<2048>(at, dst[1]);
     if constexpr (NJ == 4) {
-      dn_read16<2 * 2048>(at, dst[2]);
-      dn_read16<3 * 2048>(at, dst[3]);
+      read_lds16<2 * 2048>(at, dst[2]);
+      read_lds16<3 * 2048>(at, dst[3]);
     }
   };
 
@@ -491,12 +484,12 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   // first operands read
 #pragma unroll
   for (int r = 0; r < Sh::kRing; r++) issue_slab(r, r);
-  __builtin_amdgcn_s_waitcnt(dn_vmcnt((Sh::kRing - 1) * Sh::kLoads));
+  __builtin_amdgcn_s_waitcnt(vmcnt((Sh::kRing - 1) * Sh::kLoads));
   __builtin_amdgcn_s_barrier();
   read_b(b_rd[0], w[0]);
-  dn_read16<0>(a_rd[0], af[0]);
-  dn_read16<2048>(a_rd[0], af[1]);
-  dn_read16<4096>(a_rd[0], af[2]);
+  read_lds16<0>(a_rd[0], af[0]);
+  read_lds16<2048>(a_rd[0], af[1]);
+  read_lds16<4096>(a_rd[0], af[2]);
 
   // One k step (H) of the stage in slab `cur`.  LDS reads in issue order, with
   // Ai the operand of row block i and primes the prefetches for the step after:
@@ -531,7 +524,7 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
       // operand of row block i + 3: of this step, or of the step after
       auto read_a = [&](auto I) {
         constexpr int x = decltype(I)::value;
-        dn_read16<(x < RB ? x : x - RB) * 2048>(x < RB ? ac : an, af[x & 3]);
+        read_lds16<(x < RB ? x : x - RB) * 2048>(x < RB ? ac : an, af[x & 3]);
       };
       switch (i) {  // i is a constant after unrolling
         case 0: read_a(std::integral_constant<int, 3>{}); break;
@@ -613,7 +606,7 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
   // instruction), waits for the acknowledgement and arrives; the slices then
   // finish the tile together, each its share of the tile's eight pieces (one (i,
   // j) of every wave), all slices added in slice order.
-  const __amdgpu_buffer_rsrc_t rP = dn_rsrc(p.scratch, 0x7fffffffu);
+  const __amdgpu_buffer_rsrc_t rP = make_rsrc(p.scratch, 0x7fffffffu);
   int* const word = &p.locks[cut * kDnCounterStride];
   const int at = wave * (8 * 1024) + lane * 16;
   const auto write_out = [&](int which) {
@@ -623,7 +616,7 @@ __global__ __launch_bounds__(512) void dense_small_kernel(DenseArgs p) {
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, acc[e >> 1][e & 1]), rP,
                                                at + e * 1024, (cut * ksplit + ks) * Sh::kPartBytes,
                                                16 /* sc1 */);
-    __builtin_amdgcn_s_waitcnt(dn_vmcnt(0));  // my stores have been acknowledged
+    __builtin_amdgcn_s_waitcnt(vmcnt(0));  // my stores have been acknowledged
     __syncthreads();
   };
   const int my_share = finish_pieces(1 << ks, ksplit, 8);

@@ -68,7 +68,7 @@ template <int COUNT>
 __device__ __forceinline__ void dn_read_blocks(unsigned at, i4* v) {
   if constexpr (COUNT > 0) {
     dn_read_blocks<COUNT - 1>(at, v);
-    dn_read16<2048 * (COUNT - 1)>(at, v[COUNT - 1]);
+    read_lds16<2048 * (COUNT - 1)>(at, v[COUNT - 1]);
   }
 }
 
@@ -100,9 +100,9 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
   const int rows = min(TM, p.M - m0);
   const int cols = min(TN, p.N - n0);  // (192 columns: the last tile may have fewer)
   const __amdgpu_buffer_rsrc_t rA =
-      dn_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
+      make_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
   const __amdgpu_buffer_rsrc_t rB =
-      dn_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)cols * (unsigned)p.K * 2u);
+      make_rsrc((const char*)p.B + (size_t)n0 * p.K * 2, (unsigned)cols * (unsigned)p.K * 2u);
 
   // a wave fetches its share of the rows of A and of B, eight rows per
   // instruction; rows past the end of A repeat the last one (never stored)
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
 #pragma unroll
     for (int t = 0; t < TA; t++) {
       const int r = 8 * (TA * wave + t) + r8;
-      a_src[t] = r >= TM ? kDnOob : (r < rows ? r : rows - 1) * p.K * 2 + 16 * c;
+      a_src[t] = r >= TM ? kOob : (r < rows ? r : rows - 1) * p.K * 2 + 16 * c;
     }
 #pragma unroll
     for (int t = 0; t < TB; t++) b_src[t] = (8 * (TB * wave + t) + r8) * p.K * 2 + 16 * c;
@@ -124,14 +124,14 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
   const int stages = st1 - st0;
 
   auto issue_slab = [&](int s, int slot) {
-    const int inv = s < stages ? 0 : kDnOob;  // a stage past the end fetches zeros
+    const int inv = s < stages ? 0 : kOob;  // a stage past the end fetches zeros
     const int at = (st0 + s) * (kDnStageK * 2);
     char* const base = smem + slot * Sh::kSlab;
 #pragma unroll
-    for (int t = 0; t < TA; t++) dn_dma16(rA, base + (TA * wave + t) * 1024, a_src[t] | inv, at);
+    for (int t = 0; t < TA; t++) load_to_lds16(rA, base + (TA * wave + t) * 1024, a_src[t] | inv, at);
 #pragma unroll
     for (int t = 0; t < TB; t++)
-      dn_dma16(rB, base + Sh::kSlabA + (TB * wave + t) * 1024, b_src[t] | inv, at);
+      load_to_lds16(rB, base + Sh::kSlabA + (TB * wave + t) * 1024, b_src[t] | inv, at);
   };
 
   // operands of a stage, per k step B then A; where they sit in slab 0
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
   i4 even[Sh::kOps], odd[Sh::kOps];
 #pragma unroll
   for (int r = 0; r < RING; r++) issue_slab(r, r);
-  __builtin_amdgcn_s_waitcnt(dn_vmcnt((RING - 1) * Sh::kLoads));
+  __builtin_amdgcn_s_waitcnt(vmcnt((RING - 1) * Sh::kLoads));
   __builtin_amdgcn_s_barrier();
   read(even, 0);
   dn_landed(even);
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
   // this slab in registers), read the next stage's operands, request the slab
   // after the ring's last in this one's place, and multiply.
   auto stage = [&](int s, i4 (&cur)[Sh::kOps], i4 (&next)[Sh::kOps]) {
-    __builtin_amdgcn_s_waitcnt(dn_vmcnt((RING - 2) * Sh::kLoads));
+    __builtin_amdgcn_s_waitcnt(vmcnt((RING - 2) * Sh::kLoads));
     __builtin_amdgcn_s_barrier();
     const int slot_next = slot == RING - 1 ? 0 : slot + 1;
     __builtin_amdgcn_sched_barrier(0);
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
     store(-1);
   } else {
     // slices: as in dense_small_kernel, the pieces of a tile being its waves' parts
-    const __amdgpu_buffer_rsrc_t rP = dn_rsrc(p.scratch, 0x7fffffffu);
+    const __amdgpu_buffer_rsrc_t rP = make_rsrc(p.scratch, 0x7fffffffu);
     int* const word = &p.locks[tile * kDnCounterStride];
     const int at = wave * (RB * NJ * 1024) + lane * 16;
     const auto part = [&](int k2) { return (tile * p.ksplit + k2) * Sh::kPartBytes; };
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_tile_kernel(DenseArgs p) {
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, acc[e / NJ][e % NJ]), rP,
                                                  at + e * 1024, part(ks), 16 /* sc1 */);
       }
-      __builtin_amdgcn_s_waitcnt(dn_vmcnt(0));  // my stores have been acknowledged
+      __builtin_amdgcn_s_waitcnt(vmcnt(0));  // my stores have been acknowledged
       __syncthreads();
     };
     const int my_share = finish_pieces(1 << ks, p.ksplit, Sh::kWaves);

@@ -29,6 +29,7 @@
 // Per 32-deep k step a wave issues 4*RB MFMAs, RB + 2 LDS reads and the unpack
 // of 4 weight words (52 VALU instructions with group scales), software-
 // pipelined one step ahead and dealt out four behind every MFMA.
+#include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
@@ -39,7 +40,6 @@ constexpr int kPfTileN = 256;
 constexpr int kPfStageK = 64;
 constexpr int kPfSlabB = 4 * 2048;  // four 16-deep rows of packed weights
 constexpr int kPfRing = 3;          // slabs in LDS per k half
-constexpr int kOobPf = (int)0x80000000;
 
 // LDS geometry of a tile of RB row blocks
 template <int RB>
@@ -56,10 +56,6 @@ struct PfShape {
   // (64-row tiles: 8 KiB of bias sums sit behind the 64 KiB that the swap uses)
   static_assert(RB != 4 || 65536 + 8192 <= kLdsBytes, "");
 };
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t pf_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
 
 }  // namespace
 
@@ -137,11 +133,11 @@ __global__ __launch_bounds__(512) void prefill_kernel(GemmArgs p, int tiles_m, i
   const int m0 = tm * kPfTileM;
   const int rows = min(kPfTileM, p.M - m0);
 
-  const __amdgpu_buffer_rsrc_t rB = pf_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
+  const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   const __amdgpu_buffer_rsrc_t rS =
-      pf_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
+      make_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
   const __amdgpu_buffer_rsrc_t rA =
-      pf_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
+      make_rsrc((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
   const int b_row = p.N * 8;
 
   // Packed weights go through LDS too: the 256 threads of a half copy the
@@ -168,7 +164,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(GemmArgs p, int tiles_m, i
 #pragma unroll
   for (int i = 0; i < HB; i++) {
     const int r = (tid >> 3) + 32 * i;
-    a_lane[i] = r < rows ? r * p.K * 2 + 16 * ax : kOobPf;
+    a_lane[i] = r < rows ? r * p.K * 2 + 16 * ax : kOob;
   }
   // LDS slab: [step][k group][row][slot] dwords; chunk x -> step x/4, slot x%4
   const int a_wr = (ax >> 2) * kPfStepBytes + (tid >> 3) * 16 + (ax & 3) * 4;
@@ -195,14 +191,14 @@ __global__ __launch_bounds__(512) void prefill_kernel(GemmArgs p, int tiles_m, i
 
   auto issue_s = [&](int slot, int s) {
     const int sg = s_begin + s;  // stage in the whole k range
-    const int inv = sg < s_end ? 0 : kOobPf;
+    const int inv = sg < s_end ? 0 : kOob;
     if (GROUP)
       sreg[slot] = __builtin_amdgcn_raw_buffer_load_b64(rS, s_lane | inv,
                                                         (sg >> 1) * p.N * 2, 0);
   };
   auto issue_a = [&](int s) {
     const int sg = s_begin + s;
-    const int inv = sg < s_end ? 0 : kOobPf;
+    const int inv = sg < s_end ? 0 : kOob;
 #pragma unroll
     for (int i = 0; i < HB; i++)
       areg[i] = __builtin_amdgcn_raw_buffer_load_b128(rA, a_lane[i] | inv, sg * 128, 0);
@@ -354,7 +350,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(GemmArgs p, int tiles_m, i
     if (x < 0) return;
     char* base = smem + ring_next * kPfStageBytes;
     const int sg = s_begin + s_next2;
-    const int inv = sg < s_end ? 0 : kOobPf;
+    const int inv = sg < s_end ? 0 : kOob;
     if (x < HB * kPerA) {
       const int i = x / kPerA, g = x % kPerA;
       if (g < 2) {
@@ -462,7 +458,7 @@ __global__ __launch_bounds__(512) void prefill_kernel(GemmArgs p, int tiles_m, i
   // from registers at its place in that order) and carries on.  Nobody spins.
   if (ksplit > 1) {
     constexpr int part_bytes = kPfTileM * kPfTileN * 4;
-    const __amdgpu_buffer_rsrc_t rP = pf_rsrc(p.scratch, 0x7fffffffu);
+    const __amdgpu_buffer_rsrc_t rP = make_rsrc(p.scratch, 0x7fffffffu);
     const int at = ((kh * 4 + wave) * (HB * 4) * 64 + lane) * 16;
     const int mine = work * part_bytes;
 #pragma unroll

@@ -41,6 +41,7 @@
 // here computes what the statement takes in and finishes the tile.
 #include <type_traits>
 
+#include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
@@ -67,18 +68,6 @@ struct WdShape {
   static_assert(kTileM * kWdPitch <= kLdsBytes, "");
   static constexpr int kPartBytes = kSwapBytes;  // fp32 sums of a tile in scratch
 };
-constexpr int kOobWd = (int)0x80000000;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t wd_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
-
-// the four words of a raw buffer resource: 48-bit base, stride 0, size in
-// bytes, data format flags
-__device__ __forceinline__ i4 wd_rsrc_words(const void* p, unsigned bytes) {
-  const unsigned long long a = (unsigned long long)p;
-  return (i4){(int)(unsigned)a, (int)(unsigned)((a >> 32) & 0xffffu), (int)bytes, 0x00020000};
-}
 
 }  // namespace
 
@@ -143,10 +132,10 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
 
   // raw buffer resources (base, no stride, bytes, flags) as the words the
   // assembly takes; the A resource covers the rows of this tile only
-  const i4 rb_words = wd_rsrc_words(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
-  const i4 rs_words = wd_rsrc_words(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
+  const i4 rb_words = rsrc_words(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
+  const i4 rs_words = rsrc_words(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
   i4 ra_words =
-      wd_rsrc_words((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
+      rsrc_words((const char*)p.A + (size_t)m0 * p.K * 2, (unsigned)rows * (unsigned)p.K * 2u);
   const int b_row = p.N * 8;  // bytes per packed row (16 k of every column)
 
   // packed weights: piece of Marlin lane (t = kg, c = nu%8) of block 2nw + nu/8
@@ -167,7 +156,7 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   for (int i = 0; i < RB; i++) {
     const int at = i + HB * kh;
     const int r = (tid >> 3) + 16 * (at >= RB ? at - RB : at);
-    a_lane[i] = r < rows ? r * p.K * 2 + 16 * ax : kOobWd;
+    a_lane[i] = r < rows ? r * p.K * 2 + 16 * ax : kOob;
   }
   // LDS slab: [step][k group][row][slot] dwords; chunk x -> step x/4, slot x%4
   const int lds_wr =
@@ -239,7 +228,7 @@ __global__ __launch_bounds__(256) void prefill_wide_kernel(GemmArgs p, int tiles
   int pieces = (1 << NP) - 1;
   if constexpr (SLICED) {
     constexpr int part_bytes = Shape::kPartBytes;
-    const __amdgpu_buffer_rsrc_t rP = wd_rsrc(p.scratch, 0x7fffffffu);
+    const __amdgpu_buffer_rsrc_t rP = make_rsrc(p.scratch, 0x7fffffffu);
     int* const word = &p.locks[tile * p.lock_stride];
     const int at = (wave * (HB * 8) * 64 + lane) * 16;
     auto write_out = [&](int which) {

@@ -21,13 +21,13 @@
 
 #include "../../include/marlin_amd_probe.h"
 #include "../../include/marlin_amd_tools.h"
+#include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
 
 namespace {
 constexpr int kProbeDepth = 4;
-constexpr int kProbeOob = (int)0x80000000;
 }  // namespace
 
 __global__ __launch_bounds__(512) void probe_empty_kernel() {}
@@ -50,8 +50,7 @@ __global__ __launch_bounds__(256) void probe_read_kernel(GemmArgs p, int* sink) 
     u0 = wid * p.gpb;
     u1 = min(total, u0 + p.gpb);
   }
-  const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<void*>(p.B), 0, (int)((unsigned)p.K * (unsigned)(p.N / 2)), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   const int b_row = p.N * 8;
   const int b_lane = 64 * nu + 16 * kg;
   i4 acc = {0, 0, 0, 0};
@@ -59,7 +58,7 @@ __global__ __launch_bounds__(256) void probe_read_kernel(GemmArgs p, int* sink) 
   auto issue = [&](int slot, int u) {
     const bool valid = u < u1;
     const int t = u / KG, kq = u - t * KG;
-    const int vb = b_lane | (valid ? 0 : kProbeOob);
+    const int vb = b_lane | (valid ? 0 : kOob);
     const int sb = valid ? (4 * kq) * b_row + 1024 * t : 0;
 #pragma unroll
     for (int r = 0; r < 4; r++)
@@ -94,8 +93,7 @@ __global__ __launch_bounds__(512) void probe_read_strips_kernel(GemmArgs p, int*
   const int strip0 = (p.row_parts > 1 ? wid / p.row_parts : wid) * CS;
   const int n_chunks = ceil_div(p.K, 16 * kRows);
   const int c0 = (wave * n_chunks) / 8, c1 = ((wave + 1) * n_chunks) / 8;
-  const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<void*>(p.B), 0, (int)((unsigned)p.K * (unsigned)(p.N / 2)), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   const int b_row = p.N * 8;
   int b_lane[NL];
 #pragma unroll
@@ -106,12 +104,12 @@ __global__ __launch_bounds__(512) void probe_read_strips_kernel(GemmArgs p, int*
     // chunk's lines read nothing)
     b_lane[i] = strip < (p.N >> 4) && idx < 8 * CS * kRows
                     ? (idx / (8 * CS)) * b_row + 128 * strip + 16 * (idx % 8)
-                    : kProbeOob;
+                    : kOob;
   }
   i4 acc = {0, 0, 0, 0};
   i4 buf[kProbeDepth][NL];
   auto issue = [&](int slot, int c) {
-    const int inv = c < c1 ? 0 : kProbeOob;
+    const int inv = c < c1 ? 0 : kOob;
 #pragma unroll
     for (int i = 0; i < NL; i++)
       buf[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(

@@ -34,36 +34,16 @@
 // rows: two 6.6 us).
 #include <type_traits>
 
+#include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
 
 namespace {
 
-constexpr int kRowsOob = (int)0x80000000;  // offset past any buffer (sizes are < 2 GiB)
 constexpr int kRowsWaves = 8;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
-
-// 16 bytes per lane from a buffer straight into LDS, lane l's at dst + 16*l
-__device__ __forceinline__ void rows_dma16(__amdgpu_buffer_rsrc_t rsrc, char* dst, int voffset,
-                                           int soffset) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, voffset, soffset, 0, 0);
-#endif
-}
-
-// LDS accesses of the loop, outside the compiler's dependence tracking (it would
-// wait for every load in flight before each of them)
-template <int OFF>
-__device__ __forceinline__ void rows_read16(unsigned at, i4& v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF) : "memory");
-#endif
-}
+// LDS accesses of the loop, outside the compiler's dependence tracking as well
 template <int DW0, int DW1>  // offsets in dwords
 __device__ __forceinline__ void rows_read2(unsigned at, i2& v) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -75,8 +55,6 @@ __device__ __forceinline__ void rows_write16(unsigned at, i4 v) {
   asm volatile("ds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory");
 #endif
 }
-// s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
-constexpr int rows_vmcnt(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 
 template <int N, class F>
 __device__ __forceinline__ void rows_each(F f) {
@@ -131,10 +109,10 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   const int c0 = GROUP ? 2 * (wave * (chunks / 2) / kRowsWaves) : wave * chunks / kRowsWaves;
   const int c1 = GROUP ? 2 * ((wave + 1) * (chunks / 2) / kRowsWaves) : (wave + 1) * chunks / kRowsWaves;
 
-  const __amdgpu_buffer_rsrc_t rB = rows_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
-  const __amdgpu_buffer_rsrc_t rA = rows_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
+  const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
+  const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
   const __amdgpu_buffer_rsrc_t rS =
-      rows_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
+      make_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
   const int b_row = p.N * 8;  // bytes per row of B
 
   char* const stage = smem + wave * Sh::kStagePerWave;
@@ -150,7 +128,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
     for (int i = 0; i < NB; i++) {
       const int line = 8 * i + lane / 8, row = line / CS, strip = strip0 + line % CS;
       const bool on = line < 4 * CS;
-      b_src[i] = on && strip < n_strips ? row * b_row + 128 * strip + 16 * (lane % 8) : kRowsOob;
+      b_src[i] = on && strip < n_strips ? row * b_row + 128 * strip + 16 * (lane % 8) : kOob;
       b_wr[i] = lds_b + (on ? row * Sh::kBRow + 128 * (line % CS) + 16 * (lane % 8) : 3 * Sh::kBRow + CS * 128);
     }
   }
@@ -163,7 +141,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
 #pragma unroll
   for (int i = 0; i < NA; i++) {
     const int r = row0 + 8 * i + lane / 8;
-    a_src[i] = r < p.M ? r * p.K * 2 + 16 * ((lane % 8) ^ (lane / 8)) : kRowsOob;
+    a_src[i] = r < p.M ? r * p.K * 2 + 16 * ((lane % 8) ^ (lane / 8)) : kOob;
   }
   unsigned a_rd[2];
 #pragma unroll
@@ -181,7 +159,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   // chunk that is not mine is requested at an offset past everything.
   auto issue = [&](int d, int c, bool even) {
     __builtin_amdgcn_sched_barrier(0);
-    const int inv = c < c1 ? 0 : kRowsOob;
+    const int inv = c < c1 ? 0 : kOob;
     if (GROUP && even) {
       if constexpr (WIDE) {
         sq = __builtin_amdgcn_raw_buffer_load_b128(rS, s_src | inv, (c >> 1) * p.N * 2, 0);
@@ -196,7 +174,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
       bq[d][i] = __builtin_amdgcn_raw_buffer_load_b128(rB, b_src[WIDE ? 0 : i] | inv,
                                                        (WIDE ? 4 * c + i : 4 * c) * b_row, 2);
 #pragma unroll
-    for (int i = 0; i < NA; i++) rows_dma16(rA, stage + d * Sh::kSlot + 1024 * i, a_src[i] | inv, 128 * c);
+    for (int i = 0; i < NA; i++) load_to_lds16(rA, stage + d * Sh::kSlot + 1024 * i, a_src[i] | inv, 128 * c);
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -214,7 +192,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
     // chunk c has landed; the one after it may still be on its way
     constexpr int later = DEPTH == 1 ? 0 : NA + NB + (even ? 0 : NS);
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(rows_vmcnt(later));
+    __builtin_amdgcn_s_waitcnt(vmcnt(later));
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (!WIDE) {
 #pragma unroll
@@ -223,8 +201,8 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
     i4 av[MB][2];
     const unsigned slot = d * Sh::kSlot;
     rows_each<MB>([&](auto I) {
-      rows_read16<2048 * I.value>(a_rd[0] + slot, av[I.value][0]);
-      rows_read16<2048 * I.value>(a_rd[1] + slot, av[I.value][1]);
+      read_lds16<2048 * I.value>(a_rd[0] + slot, av[I.value][0]);
+      read_lds16<2048 * I.value>(a_rd[1] + slot, av[I.value][1]);
     });
     // the four words of row kg, t = 0 ... 3, for every strip (eight strips: for every j,
     // a word holding columns 16j + c and 16j + 8 + c)

@@ -22,17 +22,12 @@
 // offset, which returns zeros without touching memory.  Where a run crosses
 // tiles the ring keeps running: the first granules of the next tile are in
 // flight while the current tile is reduced and written.
+#include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
 
 namespace {
-
-constexpr int kOob = (int)0x80000000;  // offset past any buffer (sizes are < 2 GiB)
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
 
 // s_waitcnt vmcnt(0) with the other counters left alone (gfx9 encoding)
 constexpr int kWaitVm0 = 0x0F70;
@@ -79,19 +74,6 @@ struct StreamLds {
   static constexpr int kBytes =
       kOnePass ? MB * kReduceBytes : kReduceBytes + 4 * kRingBytesPerWave;
 };
-
-// 16 bytes per lane from a buffer straight into LDS: lane l's bytes land at
-// dst + 16*l (dst is wave-uniform).  The instruction's immediate offset is left
-// at zero: the hardware would add it to the LDS address as well.  (This and the
-// two helpers below are empty in the host pass, which only needs the kernels'
-// launch stubs.)
-__device__ __forceinline__ void ring_load(__amdgpu_buffer_rsrc_t rsrc, char* dst, int voffset,
-                                          int soffset) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, voffset, soffset, 0, 0);
-#endif
-}
 
 // The two halves of an MFMA activation operand from the LDS ring (dword kg of
 // chunks 0,1 and of chunks 2,3 of a row), and the wait for them.  Written as
@@ -250,8 +232,8 @@ __global__ __launch_bounds__(256) void stream_kernel(GemmArgs p) {
     for (int i = 0; i < MB; i++) {
       if constexpr (kDmaA) {
         char* dst = lds_a + (slot * MB + i) * 2048;
-        ring_load(rA, dst, a_lane[i] | inv, 128 * kq);
-        ring_load(rA, dst + 1024, a_lane[i] | inv, 128 * kq + 64);
+        load_to_lds16(rA, dst, a_lane[i] | inv, 128 * kq);
+        load_to_lds16(rA, dst + 1024, a_lane[i] | inv, 128 * kq + 64);
       } else {
         aq[slot][i][0] = __builtin_amdgcn_raw_buffer_load_b128(rA, a_lane[i] | inv, 128 * kq, 0);
         aq[slot][i][1] =

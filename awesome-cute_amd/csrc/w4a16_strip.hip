@@ -38,18 +38,14 @@
 // activations, and eight waves' rows of a chunk fill LDS.  M = 64: N = 2048,
 // K = 4096 12.9 us with four row blocks per workgroup, 7.0 in parts; N = 512,
 // K = 1024 5.4 / 3.6; N = K = 4096 13.1 / 9.5.)
+#include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
 namespace w4a16 {
 
 namespace {
 
-constexpr int kStripOob = (int)0x80000000;  // offset past any buffer (sizes are < 2 GiB)
 constexpr int kStripWaves = 8;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t strip_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
 
 }  // namespace
 
@@ -117,10 +113,10 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
   const int c0 = (wave * n_chunks) / kStripWaves;
   const int c1 = ((wave + 1) * n_chunks) / kStripWaves;
 
-  const __amdgpu_buffer_rsrc_t rB = strip_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
-  const __amdgpu_buffer_rsrc_t rA = strip_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
+  const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
+  const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
   const __amdgpu_buffer_rsrc_t rS =
-      strip_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
+      make_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
   const int b_row = p.N * 8;  // bytes per row of B
 
   // weights, fetched: the 128 (192) lanes of a chunk's loads take 16 bytes each
@@ -151,7 +147,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
 #pragma unroll
   for (int i = 0; i < Sh::kALoads; i++) {
     const int r = i * Sh::kRowsPerLoad + a_row;
-    a_lane[i] = row0 + r < p.M ? (row0 + r) * p.K * 2 + 16 * a_piece : kStripOob;
+    a_lane[i] = row0 + r < p.M ? (row0 + r) * p.K * 2 + 16 * a_piece : kOob;
   }
   char* stage = smem + wave * Sh::kStagePerWave;
   const int a_wr = a_row * Sh::kStride + 16 * a_piece;
@@ -190,15 +186,15 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
   // their own: past the end of a row lies the next row.)
   auto issue = [&](int slot, int c, bool valid) {
     __builtin_amdgcn_sched_barrier(0);
-    const int inv = valid ? 0 : kStripOob;
+    const int inv = valid ? 0 : kOob;
     const int k0 = c * Sh::kChunkK;
 #pragma unroll
     for (int i = 0; i < Sh::kALoads; i++) {
-      const int off = (k0 + 8 * a_piece < p.K) ? a_lane[i] : kStripOob;
+      const int off = (k0 + 8 * a_piece < p.K) ? a_lane[i] : kOob;
       aq[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rA, off | inv, 2 * k0, 0);
     }
     if constexpr (GROUP) {
-      int vs = s_lane + (valid ? (k0 >> 7) * p.N * 2 : kStripOob);
+      int vs = s_lane + (valid ? (k0 >> 7) * p.N * 2 : kOob);
 #pragma unroll
       for (int g = 0; g < NSC; g++) {
 #pragma unroll
@@ -211,11 +207,11 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
       }
     }
     // the weights last: what comes back first is small and near
-    const int b_chunk = valid ? c * (KC * 2) * b_row : kStripOob;
+    const int b_chunk = valid ? c * (KC * 2) * b_row : kOob;
 #pragma unroll
     for (int i = 0; i < NL; i++)
       bq[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(
-          rB, b_mine[i] ? b_lane[i] + b_chunk : kStripOob, 0, 2);
+          rB, b_mine[i] ? b_lane[i] + b_chunk : kOob, 0, 2);
     __builtin_amdgcn_sched_barrier(0);
   };
 
