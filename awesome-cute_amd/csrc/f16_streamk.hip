@@ -23,9 +23,12 @@
 //
 // dense_small_kernel: eight waves, two per SIMD, of half the tile's rows and a
 // quarter of its columns each.  128 x 128 tiles, whole or in slices: the problems
-// with few tiles (those with fewer still go to f16_tiles.hip), and the stream-K tiles of the others, every 256 x 256 tile of
-// the partial wave as four of its own.  And the large whole tiles over a shallow
-// k, where its shorter start and end count for more than dense_kernel's loop.
+// with few tiles, and the stream-K tiles of the others, every 256 x 256 tile of the
+// partial wave as four of its own.  And the large whole tiles over a shallow k, where
+// its shorter start and end count for more than dense_kernel's loop.
+//
+// Problems that take one launch of these go to f16_tiles.hip where tiles of another
+// size are cheaper (dn_tile there).
 //
 // In both, B is the first MFMA operand and A the second, so
 // v_mfma_f32_16x16x32_f16 yields D[n][m]; lane l = 16kg + nu of an operand holds

@@ -4,29 +4,32 @@
 // operands as the kernels there.
 //
 // Sizes between 64 x 128 and 128 x 256 are there for problems whose 128 x 256 tiles
-// leave a quarter to a half of the chip idle: 1514 x 3072 x 8576, 144 of those 115.7
-// us, 256 of 96 x 192 89.6; 701 x 5632 x 832 132 of them 13.8, 231 of 128 x 192 10.9;
-// 885 x 6912 x 1600 189 of them 25.8, 252 of 128 x 192 21.5.
+// leave a quarter to a half of the chip idle (us, operands from memory): 1514 x 3072 x
+// 8576, 144 of those 119.9, 256 of 96 x 192 90.8; 701 x 5632 x 832 132 of them 15.7, 240
+// of 96 x 192 12.3; 885 x 6912 x 1600 189 of them 27.3, 252 of 128 x 192 23.5.
 //
 // What bounds a problem of few small tiles is latency: the launch, the first loads, and per
-// stage a barrier and the trip of its operands from LDS, about 0.18 us whatever
-// the tile.  In slices of 128 x 128 tiles it also paid for the slices' meeting,
-// some 4 us of a launch of 9.  Small tiles fill the compute units without slices,
-// unless k is deep and C so small that even these leave most of the chip idle.
-// Measured, slices of 128 x 128 tiles against this kernel (us): 291 x 1280 x 896
-// 9.2 and 4.5, 1024^3 11.4 and 5.9, 777 x 2048 x 1024 11.1 and 7.9, 64 x 2048 x
-// 4096 13.8 and 8.6, 100 x 512 x 10240 22.7 and 9.3.
+// stage a barrier, the trip of its operands from LDS and, deeper than the ring, that
+// from memory: 0.10 us with 32 x 32 tiles, 0.21 with 64 x 64, 0.30 with 64 x 128, 0.04
+// to 0.10 more with the chip full (kDnFits).  In slices of 128 x 128 tiles it also paid
+// for the slices' meeting, some 4 us of a launch of 9.  Small tiles fill the compute
+// units without slices, unless k is deep and C so small that even these leave most of
+// the chip idle.  Measured, slices of 128 x 128 tiles against this kernel, operands from
+// memory (from the last-level cache), us: 291 x 1280 x 896 9.6 and 4.6 (9.0 and 4.2),
+// 1024^3 11.7 and 6.4 (10.3 and 5.4), 777 x 2048 x 1024 12.4 and 9.7 (10.9 and 7.5), 64 x
+// 2048 x 4096 14.7 and 10.2 (12.8 and 7.7), 100 x 512 x 10240 29.4 and 11.2 (22.2 and 8.6).
 //
 // A wave computes half the rows x a quarter (32 x 64 and less: half) of the columns.
 // Per 64-deep stage it reads
 // all operands of the next stage from LDS while the MFMAs of this one run, so a
 // slab is free again as soon as every wave has its operands, and one barrier per
-// stage does.  The ring holds as many slabs as leave room for a second workgroup
-// on the compute unit (64 x 128: one workgroup and six slabs, 48 KiB more in
-// flight: 777 x 2048 x 1024 7.9 us, with three slabs and room for a second one
-// 8.2).  Operands loaded straight from memory into registers, with the waves along
-// k and no barrier at all, took two to three times as long: sixteen rows of 64
-// bytes per load instruction.
+// stage does.  The rings of 32 x 32 to 64 x 64 hold as many slabs as leave room for a
+// second workgroup on the compute unit (64 to 72 KiB); from 64 x 128 on a workgroup
+// has the unit to itself, and three to six slabs of 24 to 48 KiB (64 x 128: six, 72 KiB
+// more in flight than the three that would leave room for a second workgroup: 777 x
+// 2048 x 1024 7.9 us, with three 8.2).  Operands loaded straight from memory into
+// registers, with the waves along k and no barrier at all, took two to three times as
+// long: sixteen rows of 64 bytes per load instruction.
 #include <hip/hip_runtime.h>
 
 #include "f16_dense.hpp"

@@ -23,9 +23,12 @@
 // Eight strips are two whole 64-column blocks: a lane then takes its 16-byte pieces
 // (t = kg, c = nu%8) of four rows of B straight into registers, and four lane swaps
 // per four words turn rows into lane groups -- no LDS for the weights.  That is
-// what many columns and 33 rows and more take (M = 64, N = 28672, K = 8192: 49.4 us
-// on 64-row prefill tiles, 41.6 so, 45.5 with seven strips through LDS; without
-// its loads it takes three quarters of that: unpacking and multiplying).
+// what many columns and 33 rows and more take (M = 64, N = 28672, K = 8192, in turn on
+// one box: 44.6 us on 64-row prefill tiles, 42.9 so; on others 42.6 and 41.7, 49.4 and
+// 41.6; with seven strips through LDS 45.5).  Neither the matrix units (busy 42 % of the
+// cycles) nor the issue of vector operations (57 %) is full there: a chunk's loads are
+// requested before the arithmetic of the one before it and waited for after it, and
+// the two take turns; without loads the launch takes two thirds of its time.
 //
 // The more chunks a wave has in flight the longer each takes to come: two where
 // strips and rows are few (a launch then waits for its first ones), else one, whose
