@@ -345,13 +345,15 @@ namespace {
 // Costs in us: a launch, a stage of the longest workgroup (dearer the fuller the chip)
 // and, whole, workgroups beyond one per compute unit and their stages; in slices the
 // launch holds their meeting.  Fitted to every tile on 2500 problems, m = 1 ... 8192, n =
-// 256 ... 16384, k = 64 ... 20480, 4 to 8 % rms where a tile is near the best.  Each
-// time is that with operands from memory, as a model's weights are, to 0.7 times that
-// with operands in the last-level cache to 0.3: the small tiles, which wait for
-// memory, take 1.2 to 1.5 times as long by the first as by the second, slices of 128 x
-// 128 1.1 times.  (Fitted to operands in the cache alone, 44 problems of 900 were given
-// tiles that took 2 to 19 % longer from memory than the plan's launch: 576 x 1536 x
-// 4544 23.0 us in 64 x 64, 19.4 in slices; 240 x 3328 x 4096 21.4 and 18.7.)
+// 256 ... 16384, k = 64 ... 20480; 5 % rms where a tile is within 1.2 times the best.
+// Each time is the geometric mean of that with operands from memory, as a model's
+// weights are, and of that with operands in the last-level cache: the small tiles, which
+// wait for memory, take 1.2 to 1.5 times as long by the first as by the second, slices of
+// 128 x 128 1.1 times.  (Fitted to the cache alone, 44 problems of 900 were given tiles
+// that took 2 to 19 % longer from memory than the plan's launch: 576 x 1536 x 4544 23.0
+// us in 64 x 64, 19.4 in slices; 240 x 3328 x 4096 21.4 and 18.7.  Fitted mostly to memory,
+// tiles were given up that were level there and 20 % faster from the cache: 665 x 1280 x
+// 3328 12.3 -> 15.6 us.)
 struct DnLine {
   double launch, stage, fill;
 };
@@ -359,17 +361,17 @@ constexpr struct DnFit {
   int rows, cols;
   DnLine whole;
   double more, more_stage;
-  DnLine by2, by4;  // (64 x 128: 1.04 times the fit, whose misses are there)
-} kDnFits[] = {{32, 32, {2.20, 0.096, 0.039}, 0.81, 0.083, {4.46, 0.099, 0.049}, {4.52, 0.092, 0.071}},
-               {32, 64, {2.31, 0.142, 0.055}, 0.86, 0.132, {4.92, 0.174, 0.044}, {5.27, 0.151, 0.108}},
-               {64, 64, {2.33, 0.209, 0.059}, 0.85, 0.182, {5.46, 0.221, 0.061}, {5.69, 0.214, 0.114}},
-               {64, 128, {3.06, 0.297, 0.095}, 2.30, 0.328, {7.09, 0.321, 0.118}, {7.65, 0.309, 0.203}},
-               {96, 128, {3.27, 0.389, 0.088}, 2.16, 0.438, {}, {}},
-               {64, 192, {3.16, 0.404, 0.118}, 2.23, 0.465, {}, {}},
-               {96, 192, {3.64, 0.499, 0.103}, 2.57, 0.612, {}, {}},
-               {128, 192, {4.11, 0.511, 0.170}, 3.05, 0.758, {}, {}},
-               {96, 256, {4.10, 0.574, 0.188}, 3.21, 0.849, {}, {}},
-               {128, 256, {4.53, 0.641, 0.265}, 4.42, 1.039, {}, {}}};
+  DnLine by2, by4;  // (64 x 128: 1.04 times the fit)
+} kDnFits[] = {{32, 32, {2.19, 0.093, 0.032}, 0.72, 0.079, {4.41, 0.096, 0.042}, {4.47, 0.090, 0.058}},
+               {32, 64, {2.29, 0.138, 0.043}, 0.84, 0.128, {4.84, 0.160, 0.047}, {5.18, 0.142, 0.099}},
+               {64, 64, {2.32, 0.191, 0.056}, 0.77, 0.179, {5.25, 0.204, 0.062}, {5.44, 0.192, 0.125}},
+               {64, 128, {3.05, 0.277, 0.088}, 2.18, 0.324, {7.08, 0.295, 0.116}, {7.45, 0.287, 0.206}},
+               {96, 128, {3.27, 0.359, 0.093}, 2.04, 0.436, {}, {}},
+               {64, 192, {3.17, 0.376, 0.109}, 2.17, 0.451, {}, {}},
+               {96, 192, {3.62, 0.471, 0.105}, 2.46, 0.611, {}, {}},
+               {128, 192, {4.03, 0.475, 0.196}, 2.92, 0.749, {}, {}},
+               {96, 256, {4.04, 0.531, 0.205}, 3.09, 0.828, {}, {}},
+               {128, 256, {4.46, 0.594, 0.294}, 4.30, 1.020, {}, {}}};
 
 // workgroups beyond one per compute unit: half way between the rounds they make and
 // their share of one
@@ -386,43 +388,43 @@ double dn_cost(const DnFit& f, int tiles, int stages, int slices, int cus) {
   return cost + more * (f.more + f.more_stage * stages);
 }
 
-// ... and of the launch that would compute the problem otherwise (3 to 4 % rms)
+// ... and of the launch that would compute the problem otherwise (3 % rms)
 double dn_plan_cost(const DnLaunch& l, int stages, int cus) {
   const double r = (double)l.tiles * l.slices / cus, fill = r < 1.0 ? r : 1.0;
   const double more = dn_more(l.tiles, cus);
   if (l.cols == 128) {
     const double each = (double)stages / l.slices;
-    return l.slices == 1   ? 3.12 + 0.58 * fill + stages * (0.464 + 0.075 * fill)
-           : l.slices == 2 ? 7.31 + each * (0.403 + 0.197 * fill)
-           : l.slices == 3 ? 8.05 + each * (0.288 + 0.347 * fill)
-                           : 7.90 + each * (0.404 + 0.251 * fill);
+    return l.slices == 1   ? 3.17 + 0.43 * fill + stages * (0.424 + 0.095 * fill)
+           : l.slices == 2 ? 7.23 + each * (0.367 + 0.213 * fill)
+           : l.slices == 3 ? 8.00 + each * (0.261 + 0.349 * fill)
+                           : 7.80 + each * (0.370 + 0.261 * fill);
   }
   if (l.rows == 128)
-    return l.waves == 4 ? 5.73 + stages * (0.635 + 0.216 * fill)
-                        : 3.93 + 0.80 * fill + stages * (0.644 + 0.223 * fill);
-  return l.waves == 4 ? 8.43 * fill + 1.87 * more + stages * (1.263 + 0.198 * fill + 1.92 * more)
-                      : 2.81 + 4.63 * fill + 6.70 * more + stages * (1.147 + 0.341 * fill + 1.74 * more);
+    return l.waves == 4 ? 5.52 + stages * (0.585 + 0.251 * fill)
+                        : 4.06 + 0.46 * fill + stages * (0.588 + 0.270 * fill);
+  return l.waves == 4 ? 0.13 + 8.17 * fill + 1.87 * more + stages * (1.186 + 0.248 * fill + 1.92 * more)
+                      : 2.59 + 4.68 * fill + 6.99 * more + stages * (1.102 + 0.379 * fill + 1.66 * more);
 }
 
 }  // namespace
 
-// The cheapest tile, if it is 3 % cheaper than the plan's slices, 5 % than its whole
+// The cheapest tile, if it is 1 % cheaper than the plan's slices, 3 % than its whole
 // tiles and 7 % than those of 256 x 256.  In 2 or 4 slices (waves share a tile unevenly
-// with 3) no more than the plan, at most one workgroup per compute unit.  2500 other
-// problems for which this or the line before it (one fit to operands in the cache)
-// takes a tile: operands from memory 1.48 times the speed of the plan's launches, 17
-// problems 2 to 9 % slower, most of them 10 to 20 % faster with operands in the cache;
-// by the line before 1.46 times, 131 slower, the worst by 20 %.  In the cache 1.59 times
-// and two slower; before 1.58 and 51.
+// with 3) no more than the plan, at most one workgroup per compute unit.  3000 other
+// problems for which this or the line before it (one fit, to operands in the cache)
+// takes a tile: operands from memory 1.47 times the speed of the plan's launches, 76
+// problems more than 2 % slower, the worst by 13 %; by the line before 1.45 times, 165
+// slower, the worst by 32 %.  In the cache 1.59 times and one slower; before 1.57 and 62.
 DnTile dn_tile(int m, int n, int k, int cus, const DnLaunch& plan) {
   const int stages = k / kDnStageK;
   DnTile best = {0, 0, 0};
-  double limit = dn_plan_cost(plan, stages, cus) / (plan.slices > 1 ? 1.03 : plan.rows == 256 ? 1.07 : 1.05);
+  double limit = dn_plan_cost(plan, stages, cus) / (plan.slices > 1 ? 1.01 : plan.rows == 256 ? 1.07 : 1.03);
   for (const DnFit& f : kDnFits) {
     const int tiles = ceil_div(m, f.rows) * ceil_div(n, f.cols);
     if (tiles > 4 * cus) continue;  // (never the best there)
     for (int s = 1; s <= (f.by2.launch > 0 ? plan.slices : 1); s *= 2) {
       if (s > 1 && (tiles * s > cus || tiles > kMaxCounters / kDnCounterStride)) break;
+      if (s > 1 && f.cols == 128 && 4 * tiles * s > 3 * cus) break;  // (0.9 to 1.3 times the fit there)
       const double c = dn_cost(f, tiles, stages, s, cus);
       if (c < limit) {
         best = {f.rows, f.cols, s};

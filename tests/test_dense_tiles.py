@@ -40,12 +40,16 @@ def test_tiles_stand_in_for_one_launch(cus):
     assert streamk.tile(4096, 4352, 4096) is None and streamk.tile(777, 4352, 10240) is None
 
 
-@pytest.mark.parametrize("m,n,k", [(576, 1536, 4544), (130, 7424, 3328), (240, 3328, 4096), (571, 1792, 5440), (265, 3840, 3072),
-                                   (172, 5376, 9920), (1486, 5376, 3008), (4798, 2048, 128)])
-def test_tiles_that_were_slower_are_not_taken(m, n, k):
-    """Sizes at which a tile took 1.05 to 1.19 times the plan's launch, operands from memory."""
+@pytest.mark.parametrize("m,n,k,slower", [
+    (576, 1536, 4544, (64, 64, 1)), (240, 3328, 4096, (64, 64, 1)),
+    (130, 7424, 3328, (64, 64, 1)), (265, 3840, 3072, (64, 64, 1)), (172, 5376, 9920, (64, 64, 1)),
+    (1486, 5376, 3008, (128, 256, 1)), (4798, 2048, 128, (96, 256, 1)), (1703, 10752, 128, (128, 256, 1)),
+    (586, 768, 16256, (64, 128, 4)), (449, 1024, 6208, (64, 128, 4))])
+def test_tiles_that_were_slower_are_not_taken(m, n, k, slower):
+    """Sizes at which a tile took 1.05 to 1.3 times the best one or the plan's launch, most of them by
+    a choice that knew only operands in the last-level cache."""
     import streamk
-    assert streamk.tile(m, n, k) is None
+    assert streamk.tile(m, n, k) != slower
 
 
 def _check(m, n, k, top):
