@@ -713,10 +713,11 @@ double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx)
 // low without (the factors below).  Not over k ranges below 640, nor, with 16 rows
 // per workgroup, below 2048: a wave has a chunk or two there, which the column strips
 // take in at once (M = 51, N = 11520, K = 512 5.7 us streaming, 6.6 by the fit's
-// choice; M = 123, N = 512, K = 1536 4.1 and 5.0).  Nine to twelve groups leave some
-// waves two of them and others one, which the fit does not hold: the line against a
-// streaming launch that shares no tile lies 5 % lower there (M = 123, N = 6912, K = 1280
-// 9.0 us streaming, 10.1; M = 64, N = 25600 13.5 and 14.7).  2500 other problems for
+// choice; M = 123, N = 512, K = 1536 4.1 and 5.0).  Ten and twelve groups leave some
+// waves two of them and others one, and take 1.06 to 1.18 times the fit (eleven 0.99 to
+// 1.03): the line against a streaming launch that shares no tile lies 5 % lower there (M
+// = 123, N = 6912, K = 1280 9.0 us streaming, 10.1; M = 64, N = 25600 13.5 and 14.7; K =
+// 1408, M = 248, N = 3584 the other way, 9.0 and 8.4).  2500 other problems for
 // which this or the line before it (neither that, nor the activations beyond an L2) takes
 // the kernel: 1.136 times the speed of the plans' launches, 37 problems more than 2 %
 // slower and 15 more than 5 %; by the line before 1.130, 107 and 60.  M = 46, N = 18432,
@@ -729,9 +730,9 @@ RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& 
   if (sms > 0 || m <= 16 || k < 640 || cx.force.any()) return {0, 0};
   double limit;
   if (pl.kernel == 1)
-    limit = stream_cost_as_planned(m, n, k, cx) * (!cx.grouped                             ? 0.99
-                                                   : pl.sp.wpt == 1 && k > 1024 && k <= 1536 ? 0.98
-                                                                                             : 1.03);
+    limit = stream_cost_as_planned(m, n, k, cx) * (!cx.grouped                                    ? 0.99
+                                                   : pl.sp.wpt == 1 && (k == 1280 || k == 1536) ? 0.98
+                                                                                                : 1.03);
   else if (pl.kernel == 2)
     limit = prefill_cost(m, n, k, cx) * (cx.grouped ? 1.03 : 1.04);
   else
