@@ -22,6 +22,7 @@ SOURCES = {
     "w4a16_stream.hip": [],
     "w4a16_strip.hip": [],
     "w4a16_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "w4a16_rows_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "w4a16_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "w4a16_prefill_wide.hip": [],
     "w4a16_convert.hip": [],

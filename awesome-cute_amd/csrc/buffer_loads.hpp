@@ -23,12 +23,14 @@ __device__ __forceinline__ i4 rsrc_words(const void* p, unsigned bytes) {
 // 16 bytes per lane from a buffer straight into LDS: lane l's bytes land at
 // dst + 16*l (dst is wave-uniform).  The instruction's immediate offset stays
 // zero: the hardware would add it to the LDS address as well.  (Device pass
-// only; the host pass just needs the kernel's launch stub.)
+// only; the host pass just needs the kernel's launch stub.)  AUX 2: read once, not to
+// stay in the caches.
+template <int AUX = 0>
 __device__ __forceinline__ void load_to_lds16(__amdgpu_buffer_rsrc_t rsrc, char* dst, int voffset,
                                               int soffset) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef __attribute__((address_space(3))) void* lds_ptr;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, voffset, soffset, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, voffset, soffset, 0, AUX);
 #endif
 }
 

@@ -64,7 +64,7 @@ bool configure_device(int dev) {
   if (g_dev[dev].configured) return true;
   if (configure_stream_kernels() != 0 || configure_prefill_kernels() != 0 ||
       configure_prefill_wide_kernels() != 0 || configure_strip_kernels() != 0 ||
-      configure_rows_kernels() != 0) {
+      configure_rows_kernels() != 0 || configure_rows_wide_kernels() != 0) {
     set_error(hipGetLastError(), "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
     return false;
   }

@@ -268,6 +268,10 @@ constexpr int kRowsMaxStrips = 8, kRowsMaxBlocks = 4;
 bool rows_exist(int strips, int blocks, bool group);
 int configure_rows_kernels();
 int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream_t stream);
+// ... of which eight strips are a kernel of their own (w4a16_rows_wide.hip)
+bool rows_wide_exist(int blocks);
+int configure_rows_wide_kernels();
+int launch_rows_wide(const GemmArgs& a, bool group, int blocks, hipStream_t stream);
 // ksplit >= 1 slices of the k range per tile; above 1 the launch needs
 // a.scratch (ksplit * tiles * tile bytes of fp32) and a.locks (one zeroed
 // counter per tile, zero again afterwards)

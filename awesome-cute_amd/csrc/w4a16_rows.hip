@@ -4,37 +4,34 @@
 // several times, and a column tile that shares its k range among workgroups pays
 // for their meeting (2 to 4 us of a launch of 10 to 15).
 //
-// What bounds it: what a compute unit takes in, 55 to 60 GB/s with all of them at
-// work -- 32 MB k bytes of activations from the L2s beside 8 CS k bytes of weights
-// -- and what its LDS takes in, 64 bytes per clock whatever the width of the stores
-// (reads come at 230).  So the activations go straight to LDS (buffer_load ... lds)
-// and are read once, as whole operands: sets of strips and rows are chosen to keep
-// both streams short (rows_plan in marlin_host.hip).  M = 45, N = 12288, K = 4096:
-// 15.1 us streaming, 12.7 so; M = 46, N = 18432, K = 4480 29.2 and 18.4.
+// What bounds it: what a compute unit takes in -- 32 MB k bytes of activations from the L2s
+// beside 8 CS k bytes of weights.  Loads come back in order, so activations that the L2
+// has (130 GB/s per compute unit by themselves) wait behind weights that it has not, and the
+// two together come at the 57 to 61 GB/s that a compute unit draws from beyond its L2: M = 45,
+// N = 12288, K = 4096 491 KB in 8 of 11.6 us.  Sets of strips and rows are chosen to keep
+// both streams short (rows_plan in marlin_host.hip).
 //
 // Eight waves split the k range into contiguous runs of chunks of 64 k-values and
-// meet once, at the end: no barrier in the loop, no scratch, no counters.  The
-// weights of a chunk are fetched 16 bytes per lane, four rows of B, and pass
-// through LDS into operand order.  MFMA lane (kg, nu) takes the sixteen k-values of
-// row kg of the four for column slot nu -- word j = (nu/2)%4 of the Marlin lanes
-// (t, c = 2s + e), t = 0 ... 3, e = nu/8 -- so that an activation operand is eight
-// neighbouring k-values of a row, 16 bytes.
+// meet once, at the end: no barrier in the loop, no scratch, no counters.  Activations
+// and weights go straight to LDS (buffer_load ... lds), eight rows or lines of 128 bytes
+// per load (four rows or fewer per load are 4 to 30 % slower), swizzled where they are
+// fetched, and are read once in operand order.  MFMA lane (kg, nu) takes the sixteen
+// k-values of row kg of four rows of B for column slot nu -- word j = (nu/2)%4 of the Marlin
+// lanes (t, c = 2s + e), t = 0 ... 3, e = nu/8 -- so that an activation operand is eight
+// neighbouring k-values of a row, 16 bytes.  (Weights
+// through registers into LDS, and the scales of columns fetched after the loop, took 1.05
+// times as long: 231 problems, 1.1 with three and four strips of 32 and 48 rows, 1.01 with
+// five and six; 45 x 12288 x 4096 13.0 us.)
 //
-// Eight strips are two whole 64-column blocks: a lane then takes its 16-byte pieces
-// (t = kg, c = nu%8) of four rows of B straight into registers, and four lane swaps
-// per four words turn rows into lane groups -- no LDS for the weights.  That is
-// what many columns and 33 rows and more take (M = 64, N = 28672, K = 8192, in turn on
-// one box: 44.6 us on 64-row prefill tiles, 42.9 so; on others 42.6 and 41.7, 49.4 and
-// 41.6; with seven strips through LDS 45.5).  Neither the matrix units (busy 42 % of the
-// cycles) nor the issue of vector operations (57 %) is full there: a chunk's loads are
-// requested before the arithmetic of the one before it and waited for after it, and
-// the two take turns; without loads the launch takes two thirds of its time.
+// The more a wave has in flight the longer each takes to come: two chunks where strips and
+// rows are few (a launch then waits for its first ones), else one, whose successor is
+// requested before its arithmetic (M = 45, N = 12288, K = 4096: all weights requested at
+// once 13.3 us, two units of 128 k-values 12.8, one 11.6; M = 18, N = 768, K = 2176, one
+// strip and 16 rows, one chunk 0.90, two 0.85 and two units as well 0.82 of the time with
+// weights through registers).  Weights that only one workgroup reads are requested as read
+// once: with several row parts that costs 4 to 15 % (one strip), without up to 3 % (six).
 //
-// The more chunks a wave has in flight the longer each takes to come: two where
-// strips and rows are few (a launch then waits for its first ones), else one, whose
-// successor is requested before its arithmetic (M = 45, N = 12288, K = 4096: one
-// 12.9 us, two 13.6; M = 111, N = 512, K = 4992, one strip and 16
-// rows: two 6.6 us).
+// Eight strips are a kernel of their own (w4a16_rows_wide.hip).
 #include <type_traits>
 
 #include "buffer_loads.hpp"
@@ -53,11 +50,6 @@ __device__ __forceinline__ void rows_read2(unsigned at, i2& v) {
   asm volatile("ds_read2_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(at), "n"(DW0), "n"(DW1) : "memory");
 #endif
 }
-__device__ __forceinline__ void rows_write16(unsigned at, i4 v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("ds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory");
-#endif
-}
 
 template <int N, class F>
 __device__ __forceinline__ void rows_each(F f) {
@@ -69,31 +61,30 @@ __device__ __forceinline__ void rows_each(F f) {
 
 }  // namespace
 
-template <int CS, int MB, int DEPTH>
+// DEPTH chunks of activations in LDS per wave and UNITS units of weights: a unit is a chunk's,
+// or with an odd number of strips those of two, which whole loads fetch
+template <int CS, int MB, int DEPTH, int UNITS>
 struct RowsShape {
-  static constexpr bool kWide = CS == 8;
-  static constexpr int kBLoads = (CS + 1) / 2;  // of 1 KiB per wave and chunk, eight lines of 128 bytes
-  static constexpr int kALoads = 2 * MB;        // ... eight rows
-  static constexpr int kSlot = 2048 * MB;       // activations of a chunk
-  static constexpr int kBRow = CS * 128 + 16;   // a row of B in LDS
-  static constexpr int kStagePerWave = DEPTH * kSlot + (kWide ? 0 : 4 * kBRow);
+  static constexpr int kALoads = 2 * MB;   // of 1 KiB per wave and chunk, eight rows
+  static constexpr int kSlot = 2048 * MB;  // activations of a chunk
+  static constexpr int kUnitChunks = CS % 2 == 0 ? 1 : 2;
+  static constexpr int kBLoads = CS * kUnitChunks / 2;  // of 1 KiB, eight lines of 128 bytes
+  static constexpr int kStagePerWave = DEPTH * kSlot + UNITS * 1024 * kBLoads;
+  static_assert(UNITS == 1 || (UNITS == 2 && DEPTH == 2), "");
   // the waves' sums meet through LDS in passes of at most 16 blocks of 16 x 16
   static constexpr int kBlocks = CS * MB;
   static constexpr int kPasses = (kBlocks + 15) / 16;
   static constexpr int kPass = (kBlocks + kPasses - 1) / kPasses;
+  static constexpr int kRounds = (kPass + kRowsWaves - 1) / kRowsWaves;  // blocks of a pass to a wave
   static constexpr int kReduce = kRowsWaves * kPass * 1024;
   static constexpr int kLds =
       kRowsWaves * kStagePerWave > kReduce ? kRowsWaves * kStagePerWave : kReduce;
-  static_assert(kLds <= 160 * 1024, "LDS of a compute unit");
-  static_assert(!kWide || DEPTH == 1, "its weights are taken from one slot");
 };
 
-template <int CS, int MB, bool GROUP, int DEPTH>
+template <int CS, int MB, bool GROUP, int DEPTH, int UNITS>
 __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
-  using Sh = RowsShape<CS, MB, DEPTH>;
-  constexpr int NA = Sh::kALoads, NB = Sh::kBLoads;
-  constexpr bool WIDE = Sh::kWide;
-  constexpr int NS = !GROUP ? 0 : WIDE ? 1 : CS;  // scale loads per group
+  using Sh = RowsShape<CS, MB, DEPTH, UNITS>;
+  constexpr int NA = Sh::kALoads, NB = Sh::kBLoads, NS = GROUP ? CS : 0;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // Sh::kLds
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -119,23 +110,21 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   const int b_row = p.N * 8;  // bytes per row of B
 
   char* const stage = smem + wave * Sh::kStagePerWave;
-  const unsigned lds_a = (unsigned)(size_t)stage, lds_b = lds_a + DEPTH * Sh::kSlot;
-  // weights: lines in the order [row][strip]; lanes past the last line fetch
-  // nothing and write to the padding.  Eight strips: pieces of one row per load.
-  int b_src[WIDE ? 1 : NB];
-  unsigned b_wr[NB];
-  if constexpr (WIDE) {
-    b_src[0] = 128 * strip0 + 512 * (nu >> 3) + 16 * (4 * (nu & 7) + kg);
-  } else {
+  char* const stage_w = stage + DEPTH * Sh::kSlot;
+  const unsigned lds_a = (unsigned)(size_t)stage, lds_w = lds_a + DEPTH * Sh::kSlot;
+  // weights of a unit: its lines in the order [row][strip], eight lines per load.  Piece p
+  // of a line sits at position p ^ (row % 4), which keeps the word reads (piece 4e + t of
+  // four rows) from meeting in a bank.  The row is part of the offset that the hardware
+  // checks: past the end of K there are zeros.
+  int b_src[NB];
 #pragma unroll
-    for (int i = 0; i < NB; i++) {
-      const int line = 8 * i + lane / 8, row = line / CS, strip = strip0 + line % CS;
-      const bool on = line < 4 * CS;
-      b_src[i] = on && strip < n_strips ? row * b_row + 128 * strip + 16 * (lane % 8) : kOob;
-      b_wr[i] = lds_b + (on ? row * Sh::kBRow + 128 * (line % CS) + 16 * (lane % 8) : 3 * Sh::kBRow + CS * 128);
-    }
+  for (int i = 0; i < NB; i++) {
+    const int line = 8 * i + lane / 8, row = line / CS, strip = strip0 + line % CS;
+    b_src[i] = strip < n_strips ? (4 * c0 + row) * b_row + 128 * strip + 16 * ((lane % 8) ^ (row & 3)) : kOob;
   }
-  const unsigned b_rd = lds_b + kg * Sh::kBRow + 64 * (nu >> 3) + 4 * ((nu >> 1) & 3);
+  unsigned b_rd[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) b_rd[t] = lds_w + kg * CS * 128 + 64 * (nu >> 3) + 16 * (t ^ kg) + 4 * ((nu >> 1) & 3);
   const int shift = 8 * (nu & 1);  // h = nu%2 picks the low or the high byte pairs
   // activations: 128 bytes of eight rows per load; piece p of row r sits at position
   // p ^ (r % 8), so that the operand reads (piece 2 kg + q of row nu) meet no bank
@@ -149,36 +138,54 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   unsigned a_rd[2];
 #pragma unroll
   for (int q = 0; q < 2; q++) a_rd[q] = lds_a + nu * 128 + 16 * ((2 * kg + q) ^ (nu & 7));
-  // a group's scale of slot nu, 32 bytes per strip; eight strips: those of columns
-  // 16j + 8h + c of my block, in one 16-byte piece
-  const int s_src = WIDE ? 32 * strip0 + 128 * (nu >> 3) + 16 * (nu & 7) : 2 * (16 * strip0 + nu);
+  const int s_src = 2 * (16 * strip0 + nu);  // a group's scale of slot nu, 32 bytes per strip
+
+  // One scale per column: those of the blocks that this wave writes in the end, in the
+  // order of the passes (register r of lane (row, kg) holds slot 4 kg + r, column 16j +
+  // 8h + 2s + e of the strip's block, e = kg / 2, j = 2 (kg % 2) + r / 2, h = r % 2)
+  const int slot_col = 32 * (kg & 1) + (kg >> 1);
+  unsigned short chan[Sh::kPasses][Sh::kRounds][4];
+  if constexpr (!GROUP) {
+#pragma unroll
+    for (int ps = 0; ps < Sh::kPasses; ps++)
+#pragma unroll
+      for (int i = 0; i < Sh::kRounds; i++) {
+        const int strip = strip0 + (ps * Sh::kPass + i * kRowsWaves + wave) / MB;
+        const int col = 64 * (strip >> 2) + 2 * (strip & 3) + slot_col;
+#pragma unroll
+        for (int r = 0; r < 4; r++)  // (past the last column: zeros, and not used)
+          chan[ps][i][r] = __builtin_amdgcn_raw_buffer_load_b16(
+              rS, 2 * scale_index_single(col + 16 * (r >> 1) + 8 * (r & 1)), 0, 0);
+      }
+  }
 
   const DequantConsts dc;
-  i4 bq[DEPTH][NB];
-  using Scales = std::conditional_t<WIDE, i4, unsigned short[CS]>;
-  Scales sq = {}, sc = {};
+  unsigned short sq[CS] = {}, sc[CS] = {};
 
-  // Request chunk c into slot d, and with an even one the scales of its group; a
-  // chunk that is not mine is requested at an offset past everything.
-  auto issue = [&](int d, int c, bool even) {
-    __builtin_amdgcn_sched_barrier(0);
+  // What is not mine is requested at an offset past everything.
+  auto issue_scales = [&](int c) {
     const int inv = c < c1 ? 0 : kOob;
-    if (GROUP && even) {
-      if constexpr (WIDE) {
-        sq = __builtin_amdgcn_raw_buffer_load_b128(rS, s_src | inv, (c >> 1) * p.N * 2, 0);
-      } else {
 #pragma unroll
-        for (int s = 0; s < CS; s++)
-          sq[s] = __builtin_amdgcn_raw_buffer_load_b16(rS, (s_src + 32 * s) | inv, (c >> 1) * p.N * 2, 0);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < NB; i++)
-      bq[d][i] = __builtin_amdgcn_raw_buffer_load_b128(rB, b_src[WIDE ? 0 : i] | inv,
-                                                       (WIDE ? 4 * c + i : 4 * c) * b_row, 2);
+    for (int s = 0; s < CS; s++)
+      sq[s] = __builtin_amdgcn_raw_buffer_load_b16(rS, (s_src + 32 * s) | inv, (c >> 1) * p.N * 2, 0);
+  };
+  auto issue_rows = [&](int d, int c) {
+    const int inv = c < c1 ? 0 : kOob;
 #pragma unroll
     for (int i = 0; i < NA; i++) load_to_lds16(rA, stage + d * Sh::kSlot + 1024 * i, a_src[i] | inv, 128 * c);
-    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the unit that starts with chunk c, to place `at`; read once only where the rows are in one part
+  auto issue_weights = [&](int at, int c) {
+    const bool mine = c < c1;
+    const int off = 4 * (c - c0) * b_row;
+    char* const dst = stage_w + at * (1024 * NB);
+    if (p.row_parts == 1) {
+#pragma unroll
+      for (int i = 0; i < NB; i++) load_to_lds16<2>(rB, dst + 1024 * i, mine ? b_src[i] + off : kOob, 0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NB; i++) load_to_lds16(rB, dst + 1024 * i, mine ? b_src[i] + off : kOob, 0);
+    }
   };
 
   f4 acc[CS][MB];
@@ -190,106 +197,98 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   const h2 sub = {(half_t)1032.f, (half_t)1032.f};
   const h2 mul = {(half_t)0.0625f, (half_t)0.0625f};
   const h2 add = {(half_t)-72.f, (half_t)-72.f};
-  auto step = [&](int d, int c, auto EVEN) {
+  int w_at = 0;  // place of the unit in use
+  auto step = [&](int c, auto EVEN) {
     constexpr bool even = decltype(EVEN)::value;
-    // chunk c has landed; the one after it may still be on its way
-    constexpr int later = DEPTH == 1 ? 0 : NA + NB + (even ? 0 : NS);
+    constexpr bool first = even || Sh::kUnitChunks == 1;                   // a unit of weights starts here
+    constexpr bool last = !even || Sh::kUnitChunks == 1;                   // ... ends
+    constexpr int d = DEPTH == 2 && !even ? 1 : 0;                         // this chunk's activations
+    // chunk c has landed; what was requested after it may still be on its way
+    constexpr int later = DEPTH == 1 ? 0 : UNITS == 2 ? NA + NB + (even ? 0 : NS) : first ? NA : NS + NA;
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(vmcnt(later));
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (!WIDE) {
-#pragma unroll
-      for (int i = 0; i < NB; i++) rows_write16(b_wr[i], bq[d][i]);
-    }
     i4 av[MB][2];
-    const unsigned slot = d * Sh::kSlot;
     rows_each<MB>([&](auto I) {
-      read_lds16<2048 * I.value>(a_rd[0] + slot, av[I.value][0]);
-      read_lds16<2048 * I.value>(a_rd[1] + slot, av[I.value][1]);
+      read_lds16<2048 * I.value>(a_rd[0] + d * Sh::kSlot, av[I.value][0]);
+      read_lds16<2048 * I.value>(a_rd[1] + d * Sh::kSlot, av[I.value][1]);
     });
-    // the four words of row kg, t = 0 ... 3, for every strip (eight strips: for every j,
-    // a word holding columns 16j + c and 16j + 8 + c)
-    constexpr int NW = WIDE ? 4 : CS;
-    i2 wv[NW][2];
-    if constexpr (!WIDE)
-      rows_each<CS>([&](auto I) {
-        rows_read2<32 * I.value, 32 * I.value + 4>(b_rd, wv[I.value][0]);
-        rows_read2<32 * I.value + 8, 32 * I.value + 12>(b_rd, wv[I.value][1]);
+    // the four words of row kg, t = 0 ... 3, for every strip, two strips at a time
+    constexpr int NP = (CS + 1) / 2;
+    i2 wv[4][NP];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const unsigned at = b_rd[t] + w_at * (1024 * NB) + (first ? 0 : 512 * CS);
+      rows_each<NP>([&](auto I) {
+        rows_read2<64 * I.value, 64 * I.value + (2 * I.value + 1 < CS ? 32 : 0)>(at, wv[t][I.value]);
       });
+    }
     // every operand has come back: nothing stands between the reads and this, and
     // the registers are named so that they count as in use up to here
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(av[0][0]), "+v"(av[0][1]));
 #pragma unroll
     for (int m = 1; m < MB; m++) asm volatile("" : "+v"(av[m][0]), "+v"(av[m][1]));
-    if constexpr (!WIDE) {
 #pragma unroll
-      for (int s = 0; s < CS; s++) asm volatile("" : "+v"(wv[s][0]), "+v"(wv[s][1]));
-    } else {
-      // lane group t of register i holds row i: a 4 x 4 transpose over the two
+    for (int t = 0; t < 4; t++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const auto x = __builtin_amdgcn_permlane32_swap(bq[d][0][j], bq[d][2][j], false, false);
-        const auto y = __builtin_amdgcn_permlane32_swap(bq[d][1][j], bq[d][3][j], false, false);
-        const auto u = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
-        const auto v = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
-        wv[j][0] = (i2){(int)u[0], (int)u[1]};
-        wv[j][1] = (i2){(int)v[0], (int)v[1]};
-      }
-    }
+      for (int i = 0; i < NP; i++) asm volatile("" : "+v"(wv[t][i]));
 #endif
     if (GROUP && even) {
-      if constexpr (WIDE) {
-        sc = sq;
-      } else {
 #pragma unroll
-        for (int s = 0; s < CS; s++) sc[s] = sq[s];
-      }
+      for (int s = 0; s < CS; s++) sc[s] = sq[s];
     }
-    issue(d, c + DEPTH, DEPTH == 1 ? !even : even);
+    __builtin_amdgcn_sched_barrier(0);
+    if (GROUP && even) issue_scales(c + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    // (two units: the rows first, so that a chunk's do not wait for later weights)
+    if (UNITS == 2) issue_rows(d, c + DEPTH);
+    __builtin_amdgcn_sched_barrier(0);
+    if (last) {
+      issue_weights(w_at, c + 1 + (UNITS - 1) * Sh::kUnitChunks);
+      if (UNITS == 2) w_at ^= 1;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (UNITS == 1) issue_rows(d, c + DEPTH);
+    __builtin_amdgcn_sched_barrier(0);
     // a block of 16 slots: k-values 2t, 2t + 1 and 2t + 8, 2t + 9 of the lane's sixteen
-    const auto multiply = [&](const h2(&lo)[4], const h2(&hi)[4], f4(&sum)[MB]) {
+#pragma unroll
+    for (int s = 0; s < CS; s++) {
+      h2 lo[4], hi[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const int w = (int)((unsigned)wv[t][s >> 1][s & 1] >> shift);
+        lo[t] = as_h2((w & dc.lo_mask) | dc.ex) - sub;
+        hi[t] = __builtin_elementwise_fma(as_h2((w & dc.hi_mask) | dc.ex), mul, add);
+        if constexpr (GROUP) {
+          const half_t x = __builtin_bit_cast(half_t, sc[s]);
+          const h2 s2 = {x, x};
+          lo[t] *= s2;
+          hi[t] *= s2;
+        }
+      }
       const h8 w0 = make_h8(lo[0], lo[1], lo[2], lo[3]), w1 = make_h8(hi[0], hi[1], hi[2], hi[3]);
 #pragma unroll
       for (int m = 0; m < MB; m++)
-        sum[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, __builtin_bit_cast(h8, av[m][0]), sum[m], 0, 0, 0);
+        acc[s][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, __builtin_bit_cast(h8, av[m][0]), acc[s][m], 0, 0, 0);
 #pragma unroll
       for (int m = 0; m < MB; m++)
-        sum[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, __builtin_bit_cast(h8, av[m][1]), sum[m], 0, 0, 0);
-    };
-#pragma unroll
-    for (int s = 0; s < NW; s++) {
-      h2 lo[4], hi[4];
-      if constexpr (WIDE) {
-        h2 lo8[4], hi8[4];  // of column c + 8
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-          dequant_word<GROUP>(wv[s][t >> 1][t & 1], as_h2(sc[s]), dc, lo[t], hi[t], lo8[t], hi8[t]);
-        multiply(lo, hi, acc[2 * s]);
-        multiply(lo8, hi8, acc[2 * s + 1]);
-      } else {
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const int w = (int)((unsigned)wv[s][t >> 1][t & 1] >> shift);
-          lo[t] = as_h2((w & dc.lo_mask) | dc.ex) - sub;
-          hi[t] = __builtin_elementwise_fma(as_h2((w & dc.hi_mask) | dc.ex), mul, add);
-          if constexpr (GROUP) {
-            const half_t x = __builtin_bit_cast(half_t, sc[s]);
-            const h2 s2 = {x, x};
-            lo[t] *= s2;
-            hi[t] *= s2;
-          }
-        }
-        multiply(lo, hi, acc[s]);
-      }
+        acc[s][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, __builtin_bit_cast(h8, av[m][1]), acc[s][m], 0, 0, 0);
     }
   };
 
-#pragma unroll
-  for (int d = 0; d < DEPTH; d++) issue(d, c0 + d, d == 0);
+  if (GROUP) issue_scales(c0);
+  __builtin_amdgcn_sched_barrier(0);
+  issue_rows(0, c0);
+  __builtin_amdgcn_sched_barrier(0);
+  issue_weights(0, c0);
+  __builtin_amdgcn_sched_barrier(0);
+  if (DEPTH == 2) issue_rows(1, c0 + 1);
+  __builtin_amdgcn_sched_barrier(0);
+  if (UNITS == 2) issue_weights(1, c0 + Sh::kUnitChunks);
   for (int c = c0; c < c1; c += 2) {
-    step(0, c, std::true_type{});
-    if (c + 1 < c1) step(DEPTH - 1, c + 1, std::false_type{});
+    step(c, std::true_type{});
+    if (c + 1 < c1) step(c + 1, std::false_type{});
   }
   // nothing may still be on its way into LDS when it is reused
   __builtin_amdgcn_s_waitcnt(0);
@@ -297,52 +296,38 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   // ---- sum the eight waves, a block of 16 slots x 16 rows to a wave
   f4* const red = (f4*)smem;
 #pragma unroll
-  for (int b0 = 0; b0 < Sh::kBlocks; b0 += Sh::kPass) {
+  for (int ps = 0; ps < Sh::kPasses; ps++) {
+    const int b0 = ps * Sh::kPass;
     __syncthreads();
 #pragma unroll
     for (int b = b0; b < b0 + Sh::kPass && b < Sh::kBlocks; b++)
       red[(wave * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < (Sh::kPass + kRowsWaves - 1) / kRowsWaves; i++) {
+    for (int i = 0; i < Sh::kRounds; i++) {
       const int b = b0 + i * kRowsWaves + wave;
       if (b >= b0 + Sh::kPass || b >= Sh::kBlocks) continue;
       f4 v = red[(b - b0) * 64 + lane];
 #pragma unroll
       for (int w = 1; w < kRowsWaves; w++) v += red[(w * Sh::kPass + b - b0) * 64 + lane];
       const int row = row0 + 16 * (b % MB) + nu;
-      if constexpr (WIDE) {
-        // register r of lane (row, kg) holds column slot nu' = 4 kg + r, column 16j +
-        // 8h + nu' % 8 of block nu' / 8, b / MB = 2j + h: four neighbouring columns
-        const int s = b / MB;
-        const int col = 16 * strip0 + 64 * (kg >> 1) + 16 * (s >> 1) + 8 * (s & 1) + 4 * (kg & 1);
-        h4 o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-        if constexpr (!GROUP) {
+      const int strip = strip0 + b / MB;
+      if (strip >= n_strips) continue;
+      // The lanes of both e, 32 apart, exchange halves and store two columns at a time.
+      const int col = 64 * (strip >> 2) + 2 * (strip & 3) + 32 * (kg & 1);
+      const int e = kg >> 1;
+      unsigned o[4];
 #pragma unroll
-          for (int r = 0; r < 4; r++) o[r] *= ((const half_t*)p.S)[scale_index_single(col + r)];
-        }
-        if (row < p.M) *(h4*)((half_t*)p.C + (size_t)row * p.N + col) = o;
-      } else {
-        const int strip = strip0 + b / MB;
-        if (strip >= n_strips) continue;
-        // Register r of lane (row, kg) holds slot 4 kg + r, column 16j + 8h + 2s + e
-        // of the strip's block, e = kg / 2, j = 2 (kg % 2) + r / 2, h = r % 2.  The
-        // lanes of both e, 32 apart, exchange halves and store two columns at a time.
-        const int col = 64 * (strip >> 2) + 2 * (strip & 3) + 32 * (kg & 1);
-        const int e = kg >> 1;
-        unsigned o[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          half_t x = (half_t)v[r];
-          if constexpr (!GROUP) x *= ((const half_t*)p.S)[scale_index_single(col + e + 16 * (r >> 1) + 8 * (r & 1))];
-          o[r] = __builtin_bit_cast(unsigned short, x);
-        }
-        const unsigned got = __shfl_xor((int)(e ? o[0] | (o[1] << 16) : o[2] | (o[3] << 16)), 32);
-        if (row < p.M) {
-          unsigned* const out = (unsigned*)((half_t*)p.C + (size_t)row * p.N + col + 16 * e);
-          out[0] = e ? (got & 0xffffu) | (o[2] << 16) : o[0] | (got << 16);
-          out[4] = e ? (got >> 16) | (o[3] << 16) : o[1] | (got & 0xffff0000u);
-        }
+      for (int r = 0; r < 4; r++) {
+        half_t x = (half_t)v[r];
+        if constexpr (!GROUP) x *= __builtin_bit_cast(half_t, chan[ps][i][r]);
+        o[r] = __builtin_bit_cast(unsigned short, x);
+      }
+      const unsigned got = __shfl_xor((int)(e ? o[0] | (o[1] << 16) : o[2] | (o[3] << 16)), 32);
+      if (row < p.M) {
+        unsigned* const out = (unsigned*)((half_t*)p.C + (size_t)row * p.N + col + 16 * e);
+        out[0] = e ? (got & 0xffffu) | (o[2] << 16) : o[0] | (got << 16);
+        out[4] = e ? (got >> 16) | (o[3] << 16) : o[1] | (got & 0xffff0000u);
       }
     }
   }
@@ -353,30 +338,29 @@ namespace {
 // calls f(kernel, LDS bytes) for a set of strips and rows that exists
 template <class F>
 bool with_rows_kernel(int strips, int blocks, bool group, F f) {
-#define ROWS(CS, MB, DEPTH, GROUP)                                               \
-  if (strips == CS && blocks == MB && group == GROUP) {                         \
-    f(rows_kernel<CS, MB, GROUP, DEPTH>, RowsShape<CS, MB, DEPTH>::kLds);       \
-    return true;                                                                \
+#define ROWS(CS, MB, DEPTH, UNITS, GROUP)                                               \
+  if (strips == CS && blocks == MB && group == GROUP) {                               \
+    using Sh = RowsShape<CS, MB, DEPTH, UNITS>;                                       \
+    static_assert(Sh::kLds <= 160 * 1024, "LDS of a compute unit");                   \
+    f(rows_kernel<CS, MB, GROUP, DEPTH, UNITS>, Sh::kLds);                            \
+    return true;                                                                      \
   }
-#define ROWS_OF_BOTH(CS, MB, DEPTH) ROWS(CS, MB, DEPTH, true) ROWS(CS, MB, DEPTH, false)
-  ROWS_OF_BOTH(1, 1, 2)
-  ROWS_OF_BOTH(2, 1, 2)
-  ROWS_OF_BOTH(3, 1, 2)
-  ROWS_OF_BOTH(2, 2, 2)
-  ROWS_OF_BOTH(3, 2, 1)
-  ROWS_OF_BOTH(4, 2, 1)
-  ROWS_OF_BOTH(6, 2, 1)
-  ROWS_OF_BOTH(2, 3, 1)
-  ROWS_OF_BOTH(3, 3, 1)
-  ROWS_OF_BOTH(4, 3, 1)
-  ROWS_OF_BOTH(5, 3, 1)
-  ROWS_OF_BOTH(6, 3, 1)
-  ROWS(4, 4, 1, true)  // (never the cheapest with one scale per column)
-  ROWS_OF_BOTH(5, 4, 1)
-  ROWS_OF_BOTH(6, 4, 1)
-  ROWS_OF_BOTH(8, 2, 1)
-  ROWS_OF_BOTH(8, 3, 1)
-  ROWS_OF_BOTH(8, 4, 1)
+#define ROWS_OF_BOTH(CS, MB, DEPTH, UNITS) ROWS(CS, MB, DEPTH, UNITS, true) ROWS(CS, MB, DEPTH, UNITS, false)
+  ROWS_OF_BOTH(1, 1, 2, 2)
+  ROWS_OF_BOTH(2, 1, 2, 2)
+  ROWS_OF_BOTH(3, 1, 2, 1)
+  ROWS_OF_BOTH(2, 2, 2, 2)
+  ROWS_OF_BOTH(3, 2, 1, 1)
+  ROWS_OF_BOTH(4, 2, 1, 1)
+  ROWS_OF_BOTH(6, 2, 1, 1)
+  ROWS_OF_BOTH(2, 3, 1, 1)
+  ROWS_OF_BOTH(3, 3, 1, 1)
+  ROWS_OF_BOTH(4, 3, 1, 1)
+  ROWS_OF_BOTH(5, 3, 1, 1)
+  ROWS_OF_BOTH(6, 3, 1, 1)
+  ROWS(4, 4, 1, 1, true)
+  ROWS_OF_BOTH(5, 4, 1, 1)
+  ROWS_OF_BOTH(6, 4, 1, 1)
 #undef ROWS_OF_BOTH
 #undef ROWS
   return false;
@@ -385,7 +369,7 @@ bool with_rows_kernel(int strips, int blocks, bool group, F f) {
 }  // namespace
 
 bool rows_exist(int strips, int blocks, bool group) {
-  return with_rows_kernel(strips, blocks, group, [](auto, int) {});
+  return strips == 8 ? rows_wide_exist(blocks) : with_rows_kernel(strips, blocks, group, [](auto, int) {});
 }
 
 int configure_rows_kernels() {
@@ -401,10 +385,10 @@ int configure_rows_kernels() {
 }
 
 int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream_t stream) {
+  if (strips == 8) return launch_rows_wide(a, group, blocks, stream);
   GemmArgs b = a;
   b.row_parts = ceil_div(a.M, 16 * blocks);
   b.gpb = ceil_div(a.N / 16, strips) * b.row_parts;
-  if (strips == 8 && a.N % 128 != 0) return 2;  // (whole blocks of 64 columns only)
   const bool found = with_rows_kernel(strips, blocks, group, [&](auto kernel, int lds) {
     hipLaunchKernelGGL(kernel, dim3(b.gpb), dim3(64 * kRowsWaves), lds, stream, b);
   });
