@@ -680,10 +680,11 @@ struct RowsPlan {
 // fuller the chip, the same again for workgroups beyond one per compute unit (half
 // way between the rounds they make and their share of one), and the weights'
 // way from memory.  2800 launches over 320 problems, M = 17 ... 1500, N = 512 ...
-// 28672, K = 512 ... 13824; 6 % rms.
+// 28672, K = 512 ... 13824; 6 % rms, of a kernel whose weights went through registers; by
+// how much less each pair takes since is in the factors of rows_plan.
 // And where the rows that an XCD's workgroups read outgrow its L2 -- an eighth of the
 // strip sets each, with fewer than eight an eighth of (set, row part) pairs -- 0.24 us
-// per MB beyond 3.5: over n of 256 to 1024 with a thousand rows the kernel was taken
+// per MB beyond 3.5, 0.4 with one scale per column: over n of 256 to 1024 with a thousand rows the kernel was taken
 // for faster where it took up to 1.46 times the plan's time (M = 1015, N = 256, K = 7296
 // 13.6 us in column strips, 19.9; M = 1531, N = 512, K = 8448 25.7 on prefill tiles,
 // 33.7).
@@ -696,7 +697,7 @@ double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx)
   const double K = k / 1000.0, sums = strips * blocks;
   const double memory = 0.5e-7 * n * k;
   const double beyond = 2e-6 * m * k * (sets < 8 ? sets / 8.0 : 1.0) - 3.5;
-  const double rows = beyond > 0.0 ? 0.24 * beyond : 0.0;
+  const double rows = beyond > 0.0 ? (cx.grouped ? 0.24 : 0.4) * beyond : 0.0;
   if (cx.grouped)
     return rows + 2.88 + 0.167 * sums +
            K * (0.335 * blocks + 0.239 * strips + fill * (0.075 * blocks + 0.033 * strips) +
@@ -717,12 +718,13 @@ double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx)
 // waves two of them and others one, and take 1.06 to 1.18 times the fit (eleven 0.99 to
 // 1.03): the line against a streaming launch that shares no tile lies 5 % lower there (M
 // = 123, N = 6912, K = 1280 9.0 us streaming, 10.1; M = 64, N = 25600 13.5 and 14.7; K =
-// 1408, M = 248, N = 3584 the other way, 9.0 and 8.4).  2500 other problems for
-// which this or the line before it (neither that, nor the activations beyond an L2) takes
-// the kernel: 1.136 times the speed of the plans' launches, 37 problems more than 2 %
-// slower and 15 more than 5 %; by the line before 1.130, 107 and 60.  M = 46, N = 18432,
-// K = 4480 29.2 -> 18.4 us, 45 x 12288 x 4096 15.1 -> 12.9, 144 x 2048 x 1792 9.0 -> 6.6,
-// 501 x 1024 x 2176 11.1 -> 8.5.
+// 1408, M = 248, N = 3584 the other way, 9.0 and 8.4).  With the factors
+// below 820 problems of 7200 changed pair or kernel by them: 0.918 of the time that the former
+// choice took with the same kernels, 63 more than 2 % slower and 28 more than 5 % (1490 x
+// 512 x 3456 13.0 -> 15.2, 47 x 7168 x 9472 18.4 -> 20.7).  (A fit of every coefficient to
+// 11100 launches over 2000 problems chose no better: 1100 others 0.941, 78 more than 5 %
+// slower.)  M = 46, N = 18432, K = 4480 29.2 -> 17.9 us, 45 x 12288 x 4096 15.1 -> 11.6, 144
+// x 2048 x 1792 9.0 -> 6.0.
 RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& cx) {
   if (cx.force.rows_strips > 0 && sms <= 0 && (cx.force.rows_strips < 8 || n % 128 == 0) &&
       rows_exist(cx.force.rows_strips, cx.force.rows_blocks, cx.grouped))
@@ -731,28 +733,29 @@ RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& 
   double limit;
   if (pl.kernel == 1)
     limit = stream_cost_as_planned(m, n, k, cx) * (!cx.grouped                                    ? 0.99
-                                                   : pl.sp.wpt == 1 && (k == 1280 || k == 1536) ? 0.98
+                                                   : pl.sp.wpt == 1 && (k == 1280 || k == 1536) ? 0.92
                                                                                                 : 1.03);
   else if (pl.kernel == 2)
     limit = prefill_cost(m, n, k, cx) * (cx.grouped ? 1.03 : 1.04);
   else
     limit = strip_cost(m, n, k, pl.strips, cx.cus) * (cx.grouped ? 1.07 : 1.0);
   limit /= 1.04;
-  // the pairs, and how much longer than the fit each takes
+  // the pairs, and how much longer than the fit each takes, with group scales and without
   static const struct {
     int strips, blocks;
-    double by;
-  } pairs[] = {{1, 1, 1.06}, {2, 1, 0.97}, {3, 1, 1.03}, {2, 2, 0.96}, {3, 2, 1.08}, {4, 2, 1.00},
-               {6, 2, 0.97}, {2, 3, 0.99}, {3, 3, 1.03}, {4, 3, 0.97}, {5, 3, 0.98}, {6, 3, 0.98},
-               {4, 4, 0.98}, {5, 4, 1.00}, {6, 4, 0.98},
-               {8, 2, 0.92}, {8, 3, 0.93}, {8, 4, 0.94}};
+    double by[2];
+  } pairs[] = {{1, 1, {0.95, 0.89}}, {2, 1, {0.97, 0.93}}, {3, 1, {0.99, 0.98}}, {2, 2, {0.94, 0.91}},
+               {3, 2, {0.99, 0.97}}, {4, 2, {0.94, 0.91}}, {6, 2, {0.96, 0.92}}, {2, 3, {0.90, 0.87}},
+               {3, 3, {0.95, 0.92}}, {4, 3, {0.93, 0.87}}, {5, 3, {0.96, 0.96}}, {6, 3, {0.97, 0.93}},
+               {4, 4, {0.95, 0.98}}, {5, 4, {1.00, 0.98}}, {6, 4, {0.96, 0.94}}, {8, 2, {0.92, 0.92}},
+               {8, 3, {0.93, 0.93}}, {8, 4, {0.94, 0.94}}};
   RowsPlan best = {0, 0};
   for (const auto& p : pairs) {
     if (m <= 16 * (p.blocks - 1) || (p.blocks == 1 && k < 2048)) continue;  // (fewer blocks hold all rows)
     if (p.strips == 4 && p.blocks == 4 && !cx.grouped) continue;            // (does not exist)
     // (beyond what was fitted, and never the best there)
     if (ceil_div(n / 16, p.strips) * ceil_div(m, 16 * p.blocks) > 2.7 * cx.cus) continue;
-    const double c = rows_cost(m, n, k, p.strips, p.blocks, cx) * p.by;
+    const double c = rows_cost(m, n, k, p.strips, p.blocks, cx) * p.by[cx.grouped ? 0 : 1];
     if (c < limit) {
       best = {p.strips, p.blocks};
       limit = c;
