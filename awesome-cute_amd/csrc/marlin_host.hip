@@ -451,16 +451,15 @@ bool prefer_prefill(int m, int n, int k, const PlanCtx& cx) {
 }
 
 // Fitted time (us) of the column-strip kernel with `cs` strips per workgroup.
-// Up to 16 rows a launch costs 2.7 us.  A workgroup takes in its 8 cs k bytes
-// of weights at about 23 GB/s, what its eight waves unpack and multiply, and
-// workgroups beyond one per compute unit queue up behind each other, 0.3 us
-// each; all together they draw 4.8 TB/s from memory at most.  Every workgroup
+// Up to 8 rows a launch costs 2.9 us.  A workgroup takes in its 8 cs k bytes
+// of weights at about 28 GB/s, what its eight waves unpack and multiply, and
+// workgroups beyond one per compute unit queue up behind each other, 0.4 us
+// each; all together they draw 5.9 TB/s from memory at most.  Every workgroup
 // also reads all rows of activations, which a compute unit takes from the L2s
-// at about 87 GB/s.  Measured (M = 1, one strip): N = K = 2048 3.2 us, 4096 x
+// at about 73 GB/s.  Measured (M = 1, one strip): N = K = 2048 3.2 us, 4096 x
 // 4096 4.3, N = 11008, K = 4096 7.8, N = 1024, K = 8192 5.5, N = 4096, K =
 // 11008 7.5, 8192 x 8192 10.4 (two strips 9.1), N = 13824, K = 5120 11.4 (four
-// strips 10.0); M = 16: 4096 x 4096 5.8, N = 11008, K = 4096 15.0 (four strips
-// 9.4), N = 4096, K = 11008 11.8.
+// strips 10.0); M = 16: 4096 x 4096 5.7, N = 11008, K = 4096 8.4, N = 4096, K = 11008 11.3.
 // More rows are cut into parts of 16, a workgroup per strip set and part, and
 // fitted on their own: 1.8 us, and per round of workgroups over the compute
 // units 1.27 us, the weights at 32.7 GB/s and the part's 16 rows at 67.8 GB/s,
@@ -469,12 +468,8 @@ bool prefer_prefill(int m, int n, int k, const PlanCtx& cx) {
 // K = 1024 3.6, N = 2048, K = 4096 7.7, 4096 x 4096 9.7; M = 128: N = 256, K =
 // 512 3.4, 2048 x 2048 6.8; M = 512: N = 256, K = 1024 3.7; M = 1024: N =
 // 256, K = 512 3.8.
-double strip_cost(int m, int n, int k, int cs, int cus) {
-  // a wave's chunk is 256 / cs k-values (128 with three strips): a k range of
-  // fewer than eight chunks leaves waves idle (K = 1024: one strip 0.2 to 0.3
-  // us behind two at every N from 8 rows on; fewer rows are no slower for it)
-  const int chunks = ceil_div(k, cs == 3 ? 128 : 256 / cs);
-  const double idle = m >= 8 && chunks < 8 ? 0.7 * (1.0 - chunks / 8.0) : 0.0;
+double strip_cost(int m, int n, int k, int cs, const PlanCtx& cx) {
+  const int cus = cx.cus;
   if (m > 16) {
     // rows in parts of 16, a workgroup each: fitted to 17...128 rows over N =
     // 256...28672, K = 512...11008 (8 % rms where the strips are within 1.6
@@ -484,26 +479,45 @@ double strip_cost(int m, int n, int k, int cs, int cus) {
     const double per_wg = 1.27 + 8.0 * cs * k / 32.7e3 + 32.0 * k / 67.8e3;
     const double by_cu = rounds * per_wg * (1.0 - 0.24 * (1.0 - 1.0 / rounds));
     const double by_memory = 0.5 * k * n / 4.8e6;
-    return 1.8 + (by_cu > by_memory ? by_cu : by_memory) + idle;
+    // (two strips stay the choice where one would fill the compute units over a short k
+    // range: M = 100, N = 512, K = 1024 3.6 us, with one strip 3.2)
+    const double full = cs == 1 && k < 2048 && 8 * wgs >= 7 * cus ? 0.7 * (1.0 - k / 2048.0) : 0.0;
+    return 1.8 + (by_cu > by_memory ? by_cu : by_memory) + full;
   }
-  // Up to 8 rows the group scales go to the sums, not to the weights, and the
-  // constants are fitted on their own (M = 1, 4, 8: 7 % rms): the launch, the
+  const int wgs = ceil_div(n / 16, cs);
+  if (m > 8) {
+    // 9 to 16 rows, on the rows kernel: a launch, the strips' sums, what a workgroup takes in
+    // and computes, dearer the fuller the chip, and workgroups beyond one per compute unit
+    // (half way between the rounds they make and their share of one).  6400 launches over 2100
+    // problems of 1 to 16 rows, 4 % rms; against the streaming kernel's fit, which does not
+    // tell the kinds of scales apart, 0.98 of it with group scales and 1.09 without
+    const double K = k / 1000.0, r = (double)wgs / cus, fill = r < 1.0 ? r : 1.0;
+    const double more = r > 1.0 ? 0.5 * (ceil_div(wgs, cus) + r) - 1.0 : 0.0;
+    if (cx.grouped)
+      return 0.98 * (cs == 3 ? 1.05 : 1.02) *
+             (2.46 + 0.25 * cs + K * (0.40 + 0.158 * cs + 0.099 * fill * cs + more * (0.134 + 0.367 * cs)) +
+              0.71 * more + 0.0093 * m * K);
+    return 1.09 * (cs == 3 ? 1.05 : 1.01) *
+           (2.49 + 0.191 * cs + K * (0.303 + 0.128 * cs + 0.102 * fill * cs + more * (0.265 + 0.267 * cs)) +
+            0.84 * more + 0.0124 * m * K);
+  }
+  // Up to 8 rows the constants are fitted on their own (M = 1, 4, 8: 7 % rms): the launch, the
   // rate a compute unit unpacks at, the rate it reads rows at, a queued
   // workgroup, and memory -- 5.85 TB/s while every round of workgroups fills
   // the compute units.
-  const bool few = m <= 8;
-  const int wgs = ceil_div(n / 16, cs);
   const int per_cu = ceil_div(wgs, cus);
   const double last_round = wgs > cus ? (double)wgs / (per_cu * cus) : 1.0;
-  const double by_cu = per_cu * 8.0 * cs * k / (few ? 28.0e3 : 23e3);
-  const double by_memory = 0.5 * k * n / (few ? 5.85e6 * last_round : 4.8e6);
-  // (with 172 of 256 compute units reading 16 rows the rows came in a third
-  // sooner than this: N = 11008, K = 4096 with four strips)
-  const double rows =
-      per_cu * 2.0 * m * k / (few ? 72.5e3 : 87e3) * (wgs < cus ? (0.5 + 0.5 * wgs / cus) : 1.0);
+  const double by_cu = per_cu * 8.0 * cs * k / 28.0e3;
+  const double by_memory = 0.5 * k * n / (5.85e6 * last_round);
+  // (with fewer workgroups than compute units the rows come in sooner than this)
+  const double rows = per_cu * 2.0 * m * k / 72.5e3 * (wgs < cus ? (0.5 + 0.5 * wgs / cus) : 1.0);
+  // a wave's chunk is 256 / cs k-values (128 with three strips): a k range of
+  // fewer than eight chunks leaves waves idle (K = 1024: one strip 0.2 to 0.3
+  // us behind two at every N with 8 rows; fewer rows are no slower for it)
+  const int chunks = ceil_div(k, cs == 3 ? 128 : 256 / cs);
+  const double idle = m == 8 && chunks < 8 ? 0.7 * (1.0 - chunks / 8.0) : 0.0;
   // (a little of by_cu always: it decides between widths that memory bounds alike)
-  return (few ? 2.88 : 2.7) + (by_cu > by_memory ? by_cu : by_memory) + rows +
-         (few ? 0.43 : 0.3) * (per_cu - 1) + 0.02 * by_cu + idle;
+  return 2.88 + (by_cu > by_memory ? by_cu : by_memory) + rows + 0.43 * (per_cu - 1) + 0.02 * by_cu + idle;
 }
 
 // 16-column strips per workgroup of the column-strip kernel: the cheapest of
@@ -529,7 +543,9 @@ int strips_per_workgroup(int m, int n, int k, const PlanCtx& cx) {
     // 13.5 against 11.2)
     if (m > 16 && !forced && ceil_div(n / 16, cs) * ceil_div(m, 16) > 2 * cx.cus) continue;
     if (cx.force.strips != 0 && cx.force.strips != cs && best != 0) continue;
-    const double c = strip_cost(m, n, k, cs, cx.cus);
+    // (in parts, fitted to a kernel whose weights went through registers: one strip and two
+    // take 0.87 to 0.95 of it on the rows kernel, four 0.97)
+    const double c = strip_cost(m, n, k, cs, cx) * (m <= 16 ? 1.0 : cs == 1 ? 0.94 : cs == 2 ? 0.96 : 1.0);
     if (best == 0 || cx.force.strips == cs || c < best_cost) {
       best = cs;
       best_cost = c;
@@ -561,7 +577,7 @@ bool prefer_strips(int m, int n, int k, const PlanCtx& cx) {
   // (beyond one row block the fits are looser, the streaming kernel's above all
   // over short k ranges: the strips have to win by a margin)
   if (cs == 0) return false;
-  const double strips = strip_cost(m, n, k, cs, cx.cus) * (m > 16 ? 1.05 : 1.0);
+  const double strips = strip_cost(m, n, k, cs, cx) * (m > 16 ? 1.05 : 1.0);
   if (strips >= stream_cost_as_planned(m, n, k, cx)) return false;
   return !(n % 256 == 0 && m > 48 && prefill_cost(m, n, k, cx) <= strips);
 }
@@ -724,7 +740,7 @@ double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx)
 // 512 x 3456 13.0 -> 15.2, 47 x 7168 x 9472 18.4 -> 20.7).  (A fit of every coefficient to
 // 11100 launches over 2000 problems chose no better: 1100 others 0.941, 78 more than 5 %
 // slower.)  M = 46, N = 18432, K = 4480 29.2 -> 17.9 us, 45 x 12288 x 4096 15.1 -> 11.6, 144
-// x 2048 x 1792 9.0 -> 6.0.
+// x 2048 x 1792 9.0 -> 6.2.
 RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& cx) {
   if (cx.force.rows_strips > 0 && sms <= 0 && (cx.force.rows_strips < 8 || n % 128 == 0) &&
       rows_exist(cx.force.rows_strips, cx.force.rows_blocks, cx.grouped))
@@ -738,7 +754,7 @@ RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& 
   else if (pl.kernel == 2)
     limit = prefill_cost(m, n, k, cx) * (cx.grouped ? 1.03 : 1.04);
   else
-    limit = strip_cost(m, n, k, pl.strips, cx.cus) * (cx.grouped ? 1.07 : 1.0);
+    limit = strip_cost(m, n, k, pl.strips, cx) * (cx.grouped ? 1.07 : 1.0);
   limit /= 1.04;
   // the pairs, and how much longer than the fit each takes, with group scales and without
   static const struct {
@@ -1136,7 +1152,7 @@ int marlin_amd_plan_costs(int prob_m, int prob_n, int prob_k, int groupsize, int
   if (prob_n % 256 == 0) out[1] = prefill_cost(prob_m, prob_n, prob_k, cx);
   if (prob_m <= kStripMaxRows) {
     const int cs = strips_per_workgroup(prob_m, prob_n, prob_k, cx);
-    if (cs > 0) out[2] = strip_cost(prob_m, prob_n, prob_k, cs, cx.cus);
+    if (cs > 0) out[2] = strip_cost(prob_m, prob_n, prob_k, cs, cx);
     out[3] = cs;
   }
   return rc;

@@ -98,10 +98,12 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   const int strip0 = set * CS;
   const int n_strips = p.N >> 4;  // (the last set may have fewer strips than CS)
 
-  // my chunks [c0, c1): whole groups where there are groups
+  // my chunks [c0, c1): whole groups where there are groups, but no more than one chunk as long
+  // as that keeps waves busy (16 rows, K = 512, four strips: four waves of two 1.14 times as long)
   const int chunks = p.K / 64;
-  const int c0 = GROUP ? 2 * (wave * (chunks / 2) / kRowsWaves) : wave * chunks / kRowsWaves;
-  const int c1 = GROUP ? 2 * ((wave + 1) * (chunks / 2) / kRowsWaves) : (wave + 1) * chunks / kRowsWaves;
+  const bool pairs = GROUP && chunks > kRowsWaves;
+  const int c0 = pairs ? 2 * (wave * (chunks / 2) / kRowsWaves) : wave * chunks / kRowsWaves;
+  const int c1 = pairs ? 2 * ((wave + 1) * (chunks / 2) / kRowsWaves) : (wave + 1) * chunks / kRowsWaves;
 
   const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
@@ -349,6 +351,7 @@ bool with_rows_kernel(int strips, int blocks, bool group, F f) {
   ROWS_OF_BOTH(1, 1, 2, 2)
   ROWS_OF_BOTH(2, 1, 2, 2)
   ROWS_OF_BOTH(3, 1, 2, 1)
+  ROWS_OF_BOTH(4, 1, 2, 1)
   ROWS_OF_BOTH(2, 2, 2, 2)
   ROWS_OF_BOTH(3, 2, 1, 1)
   ROWS_OF_BOTH(4, 2, 1, 1)

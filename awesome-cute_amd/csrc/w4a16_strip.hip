@@ -1,6 +1,5 @@
-// Column-strip W4A16 kernel, 16 activation rows per workgroup (decode, small
-// batches, and more rows over small weights): a workgroup owns 16*CS columns
-// over the whole k range, so no two workgroups ever meet -- no partial sums in
+// Column-strip W4A16 kernel, up to 8 activation rows (decode, small batches): a workgroup
+// owns 16*CS columns over the whole k range, so no two workgroups ever meet -- no partial sums in
 // global memory, no counters, no last arrival.  What that exchange costs a launch of a few microseconds
 // (store, acknowledge, ticket, read back: four trips to memory one after the
 // other) is more than what narrow strips cost the weight stream.
@@ -27,17 +26,12 @@
 // computes, M*K*2 bytes against 8*CS*K bytes of weights, so narrow strips pay
 // off for few rows.
 //
-// More than 16 rows are cut into parts of 16, each a workgroup of its own over
-// the same strips: grid = strip sets x parts.  The parts of a strip set have
-// neighbouring work indices (one L2), so the weights come from memory once and
-// mostly from the L2 for the other parts (M = 64, N = K = 4096: 13.5 MB of
-// memory traffic per launch, 9.7 MB algorithmic); every part unpacks them again, which a
-// launch of a few microseconds over small weights can afford.  (Several row
-// blocks inside one workgroup, sharing every unpacked weight, were slower
-// wherever they were tried: a workgroup then reads 16 x row blocks rows of
-// activations, and eight waves' rows of a chunk fill LDS.  M = 64: N = 2048,
-// K = 4096 12.9 us with four row blocks per workgroup, 7.0 in parts; N = 512,
-// K = 1024 5.4 / 3.6; N = K = 4096 13.1 / 9.5.)
+// More rows are the rows kernel's (w4a16_rows.hip), 16 to a workgroup: the parts of a
+// strip set have neighbouring work indices (one L2), so the weights come from memory once
+// and mostly from the L2 for the other parts, and every part unpacks them again, which a
+// launch of a few microseconds over small weights can afford.  (With 16 rows staged
+// through registers this kernel took 1.1 times as long over 1325 problems of 9 to 16 rows,
+// 1.02 to 1.16 over 348 with rows in parts: 16 x 12288 x 4096 10.4 us, 8.4 there.)
 #include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
@@ -51,7 +45,7 @@ constexpr int kStripWaves = 8;
 
 // CS: 16-column strips per workgroup (1 to 4; three where N's strips fill the
 // compute units better in threes, the last workgroup then with fewer).
-// MR: activation rows staged (2, 4, 8 or 16; rows past M are read as zeros).
+// MR: activation rows staged (2, 4 or 8; rows past M are read as zeros).
 template <int CS, int MR>
 struct StripShape {
   // a chunk is two weight loads of 1 KiB per wave (three for three strips): 16
@@ -79,20 +73,13 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
   constexpr int KC = Sh::kSteps;
   constexpr int NL = Sh::kLoads;
   constexpr int NSC = GROUP ? (CS == 1 ? 2 : 1) : 0;  // scale rows a chunk touches
-  // Group scales, up to 8 rows: applied to the sums of a group instead of to
-  // its weights (below).  With 16 rows staged the two forms are within 1.5 %
-  // of each other either way (M = 16: N = 11008, K = 4096 9.3 us against 9.2,
-  // N = K = 4096 5.85 / 5.83, N = 8192, K = 2048 5.0 / 5.1) and the weights
-  // keep their scales.
-  constexpr bool kScaleSums = GROUP && MR <= 8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   {
     // all kernel arguments in one trip to memory, ahead of the first load
     const void *a_ = p.A, *b_ = p.B, *s_ = p.S;
     void* c_ = p.C;
-    asm volatile("" ::"s"(a_), "s"(b_), "s"(s_), "s"(c_), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.gpb),
-                 "s"(p.row_parts));
+    asm volatile("" ::"s"(a_), "s"(b_), "s"(s_), "s"(c_), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.gpb));
   }
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -100,11 +87,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
   const int kg = lane >> 4;
   const int nu = lane & 15;
   // (p.gpb carries the grid: the launch's own record of it is a second trip to memory)
-  const int wid = xcd_work_index((int)blockIdx.x, p.gpb);
-  // rows in parts (p.row_parts > 1): work index w computes rows [16 part, 16
-  // part + 16) of strip set w / row_parts, part = w % row_parts
-  const int set = p.row_parts > 1 ? wid / p.row_parts : wid;
-  const int row0 = p.row_parts > 1 ? 16 * (wid - set * p.row_parts) : 0;
+  const int set = xcd_work_index((int)blockIdx.x, p.gpb);
   const int strip0 = set * CS;  // my first strip; strip S holds bytes [128 S, 128 S + 128) of a row of B
   const int n_strips = p.N >> 4;  // (three strips per workgroup: the last one may hold fewer)
 
@@ -136,10 +119,9 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
   // group scales: a group's row holds the column of slot nu of strip S at
   // position 16S + 8e + 2j + h = 16S + nu (the 64-column permutation of
   // reference marlin.py:50-51 puts the 8 columns of a Marlin lane side by side).
-  // Applied to the weights, MFMA lane (kg, nu) needs the scale of slot nu;
-  // applied to the sums, result lane (row, kg) needs those of the slots 4 kg
+  // Applied to the sums, result lane (row, kg) needs those of the slots 4 kg
   // ... 4 kg + 3, four scales in 8 bytes.
-  const int s_lane = 2 * (16 * strip0 + (kScaleSums ? 4 * kg : nu));
+  const int s_lane = 2 * (16 * strip0 + 4 * kg);
   // activations: lane (row, piece) fetches 16 bytes (8 k-values)
   const int a_row = lane / Sh::kLanesPerRow;
   const int a_piece = lane % Sh::kLanesPerRow;
@@ -147,7 +129,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
 #pragma unroll
   for (int i = 0; i < Sh::kALoads; i++) {
     const int r = i * Sh::kRowsPerLoad + a_row;
-    a_lane[i] = row0 + r < p.M ? (row0 + r) * p.K * 2 + 16 * a_piece : kOob;
+    a_lane[i] = r < p.M ? r * p.K * 2 + 16 * a_piece : kOob;
   }
   char* stage = smem + wave * Sh::kStagePerWave;
   const int a_wr = a_row * Sh::kStride + 16 * a_piece;
@@ -199,10 +181,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
       for (int g = 0; g < NSC; g++) {
 #pragma unroll
         for (int s = 0; s < CS; s++)
-          if constexpr (kScaleSums)
-            sq[slot][g * CS + s] = __builtin_amdgcn_raw_buffer_load_b64(rS, vs + 32 * s, 0, 0);
-          else
-            sq[slot][g * CS + s][0] = __builtin_amdgcn_raw_buffer_load_b16(rS, vs + 32 * s, 0, 0);
+          sq[slot][g * CS + s] = __builtin_amdgcn_raw_buffer_load_b64(rS, vs + 32 * s, 0, 0);
         vs += p.N * 2;
       }
     }
@@ -279,16 +258,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
           h2 ha = __builtin_elementwise_fma(as_h2((wa & dc.hi_mask) | dc.ex), mul, add);
           h2 lb = as_h2((wb & dc.lo_mask) | dc.ex) - sub;
           h2 hb = __builtin_elementwise_fma(as_h2((wb & dc.hi_mask) | dc.ex), mul, add);
-          if constexpr (GROUP && !kScaleSums) {
-            const int g = CS == 1 ? q / 4 : 0;
-            const half_t sc = __builtin_bit_cast(half_t, (unsigned short)sq[slot][g * CS + s][0]);
-            const h2 s2 = {sc, sc};
-            la *= s2;
-            ha *= s2;
-            lb *= s2;
-            hb *= s2;
-          }
-          if constexpr (kScaleSums) {
+          if constexpr (GROUP) {
             const bool first = CS == 1 ? u == 0 : q == 0;
             const f4 from = first ? (f4){0.f, 0.f, 0.f, 0.f} : part[s];
             part[s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(make_h8(la, ha, lb, hb), af, from, 0, 0, 0);
@@ -299,7 +269,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
         }
       }
       // (a group ends with every half chunk of one strip, else with the chunk)
-      if (kScaleSums && (CS == 1 || half == 1)) {
+      if (GROUP && (CS == 1 || half == 1)) {
 #pragma unroll
         for (int s = 0; s < CS; s++) {
           const h4 sc = __builtin_bit_cast(h4, sq[slot][(CS == 1 ? half : 0) * CS + s]);
@@ -331,7 +301,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void strip_kernel(GemmArgs p) {
     f4 v = red[s * 64 + lane];
 #pragma unroll
     for (int w = 1; w < kStripWaves; w++) v += red[(w * CS + s) * 64 + lane];
-    const int m = row0 + nu;
+    const int m = nu;
     if (m < p.M) {
       half_t* crow = (half_t*)p.C + (size_t)m * p.N + res_col;
 #pragma unroll
@@ -359,8 +329,7 @@ template <int CS>
 static int configure_strip_width() {
   return configure_strip_variant<CS, 2, false>() | configure_strip_variant<CS, 2, true>() |
          configure_strip_variant<CS, 4, false>() | configure_strip_variant<CS, 4, true>() |
-         configure_strip_variant<CS, 8, false>() | configure_strip_variant<CS, 8, true>() |
-         configure_strip_variant<CS, 16, false>() | configure_strip_variant<CS, 16, true>();
+         configure_strip_variant<CS, 8, false>() | configure_strip_variant<CS, 8, true>();
 }
 
 int configure_strip_kernels() {
@@ -373,8 +342,7 @@ int configure_strip_kernels() {
 template <int CS, int MR, bool GROUP>
 static int launch_strip_variant(const GemmArgs& a, hipStream_t stream) {
   constexpr int lds = StripShape<CS, MR>::kBytes;
-  const dim3 grid(ceil_div(a.N / 16, CS) * (a.row_parts > 1 ? a.row_parts : 1)),
-      block(64 * kStripWaves);
+  const dim3 grid(ceil_div(a.N / 16, CS)), block(64 * kStripWaves);
   GemmArgs b = a;
   b.gpb = (int)grid.x;
   // Chunks in flight per wave: one where a wave has two at most, else two.
@@ -392,11 +360,9 @@ static int launch_strip_variant(const GemmArgs& a, hipStream_t stream) {
 }
 template <int CS, bool GROUP>
 static int launch_strip_rows(const GemmArgs& a, hipStream_t stream) {
-  if (a.row_parts > 1) return launch_strip_variant<CS, 16, GROUP>(a, stream);  // parts of 16 rows
   if (a.M <= 2) return launch_strip_variant<CS, 2, GROUP>(a, stream);
   if (a.M <= 4) return launch_strip_variant<CS, 4, GROUP>(a, stream);
-  if (a.M <= 8) return launch_strip_variant<CS, 8, GROUP>(a, stream);
-  return launch_strip_variant<CS, 16, GROUP>(a, stream);
+  return launch_strip_variant<CS, 8, GROUP>(a, stream);
 }
 
 // strips: 16-column strips per workgroup (1, 2 or 4 with N a multiple of
@@ -405,6 +371,7 @@ int launch_strip(const GemmArgs& a, bool group, int strips, hipStream_t stream) 
   const int parts = a.row_parts > 1 ? a.row_parts : 1;
   if (a.M > 16 * parts || a.M > kStripMaxRows || (strips != 3 && a.N % (16 * strips) != 0))
     return 2;
+  if (a.M > 8) return launch_rows(a, group, strips, 1, stream);  // (parts of 16 rows)
   switch (strips * 2 + (group ? 1 : 0)) {
     case 2: return launch_strip_rows<1, false>(a, stream);
     case 3: return launch_strip_rows<1, true>(a, stream);
