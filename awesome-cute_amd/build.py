@@ -70,10 +70,10 @@ def _run(cmd, verbose):
 def build_library(verbose=False):
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
-    # the assembly statements of the four-wave kernels (prologue, main loop and
-    # accumulator hand-over with fixed registers) are written by generators;
-    # w4a16_prefill_wide.hip and f16_streamk.hip include them from the build directory
-    for gen in ("gen_prefill_wide.py", "gen_dense.py"):
+    # the assembly statements of the four-wave kernels and of the rows kernel over 128
+    # columns (prologue, main loop and accumulator hand-over with fixed registers) are
+    # written by generators; the sources include them from the build directory
+    for gen in ("gen_prefill_wide.py", "gen_rows_wide.py", "gen_dense.py"):
         _run([sys.executable, os.path.join(CSRC, gen), objdir], verbose)
     objs = [os.path.join(objdir, src.replace(".hip", ".o")) for src in SOURCES]
     with ThreadPoolExecutor(4) as pool:

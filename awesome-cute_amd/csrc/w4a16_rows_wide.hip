@@ -11,9 +11,14 @@
 // thirds of them activations, in 27 us: 57 GB/s, as much as a compute unit draws from
 // beyond its L2.  Its loads come back in order, so activations that the L2 has wait behind
 // weights that it has not: the loads of the launch alone take 28 us, the weights' alone
-// 15, the activations' alone 10, the arithmetic alone 23 (weights requested two chunks
-// ahead and the unpack dealt out behind the MFMAs, in assembly, took 39.6 us instead of
-// 41.0, and 3 to 5 % longer over short k ranges).
+// 15, the activations' alone 10, the arithmetic alone 23.
+//
+// rows_deep_kernel, for 33 rows and more over a deep k: weights requested three chunks ahead,
+// activations two, and the unpack dealt out behind the MFMAs of the operand before
+// (gen_rows_wide.py).  Its start and its code are longer.  Time by it over the time
+// without, 64 x 16384: k = 1024 1.04, 2048 1.03, 3072 0.97, 4096 0.97, 8192 0.95; 256 x 8192:
+// 1.05, 1.01, 0.99, 1.01, 0.94, k = 11008 0.93; 64 x 28672 x 8192 42.1 -> 41.2 us; with three
+// row blocks 192 x 8192 1.06, 1.03, 1.00, 0.97, 0.96; 40 x 24576 x 4096 1.00, 8192 0.99.
 #include <type_traits>
 
 #include "buffer_loads.hpp"
@@ -24,6 +29,7 @@ namespace w4a16 {
 namespace {
 
 constexpr int kWaves = 8;
+constexpr int kDeepLds = kWaves * 2 * 8192;  // rows_deep_kernel: two slots per wave
 
 template <int MB>
 struct WideShape {
@@ -40,6 +46,53 @@ __device__ __forceinline__ void wide_each(F f) {
   if constexpr (N > 0) {
     wide_each<N - 1>(f);
     f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+// the waves' sums meet, a block of 16 slots x 16 rows to a wave, and C is written
+template <int MB, bool GROUP>
+__device__ __forceinline__ void wide_finish(const GemmArgs& p, char* smem, const f4 (&acc)[8][MB],
+                                            const __amdgpu_buffer_rsrc_t rS, int set, int row0, int wave, int lane) {
+  using Sh = WideShape<MB>;
+  const int kg = lane >> 4, nu = lane & 15;
+  f4* const red = (f4*)smem;
+#pragma unroll
+  for (int ps = 0; ps < Sh::kPasses; ps++) {
+    const int b0 = ps * Sh::kPass;
+    // (one scale per column: on their way while the sums meet)
+    h4 chan[Sh::kRounds];
+    const int col0 = 128 * set + 64 * (kg >> 1) + 4 * (kg & 1);
+    if constexpr (!GROUP) {
+#pragma unroll
+      for (int i = 0; i < Sh::kRounds; i++) {
+        const int s = (b0 + i * kWaves + wave) / MB;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          chan[i][r] = __builtin_bit_cast(
+              half_t, __builtin_amdgcn_raw_buffer_load_b16(
+                          rS, 2 * scale_index_single(col0 + 16 * (s >> 1) + 8 * (s & 1) + r), 0, 0));
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = b0; b < b0 + Sh::kPass; b++) red[(wave * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < Sh::kRounds; i++) {
+      const int b = b0 + i * kWaves + wave;
+      if (b >= b0 + Sh::kPass) continue;
+      f4 v = red[(b - b0) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < kWaves; w++) v += red[(w * Sh::kPass + b - b0) * 64 + lane];
+      const int row = row0 + 16 * (b % MB) + nu;
+      // register r of lane (row, kg) holds column slot nu' = 4 kg + r, column 16j +
+      // 8h + nu' % 8 of block nu' / 8, b / MB = 2j + h: four neighbouring columns
+      const int s = b / MB;
+      const int col = col0 + 16 * (s >> 1) + 8 * (s & 1);
+      h4 o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+      if constexpr (!GROUP) o *= chan[i];
+      if (row < p.M) *(h4*)((half_t*)p.C + (size_t)row * p.N + col) = o;
+    }
   }
 }
 
@@ -174,53 +227,85 @@ __global__ __launch_bounds__(64 * kWaves) void rows_wide_kernel(GemmArgs p) {
   // nothing may still be on its way into LDS when it is reused
   __builtin_amdgcn_s_waitcnt(0);
 
-  // ---- sum the eight waves, a block of 16 slots x 16 rows to a wave
-  f4* const red = (f4*)smem;
+  wide_finish<MB, GROUP>(p, smem, acc, rS, set, row0, wave, lane);
+}
+
+// The same over a deep k range, with the loop that gen_rows_wide.py writes: weights requested
+// three chunks ahead, activations two.
+template <int MB, bool GROUP>
+__global__ __launch_bounds__(64 * kWaves) void rows_deep_kernel(GemmArgs p) {
+  constexpr int kSlot = 8192;  // activations of a chunk, slots swapped by an exclusive or
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // kDeepLds
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int kg = lane >> 4;
+  const int nu = lane & 15;
+  // the parts of a strip set are neighbours behind one L2 (p.gpb carries the grid)
+  const int wid = xcd_work_index((int)blockIdx.x, p.gpb);
+  const int set = wid / p.row_parts;
+  const int row0 = 16 * MB * (wid - set * p.row_parts);
+
+  // my chunks [c0, c1) of 64 k-values: whole groups where there are groups
+  const int chunks = p.K / 64;
+  const int c0 = GROUP ? 2 * (wave * (chunks / 2) / kWaves) : wave * chunks / kWaves;
+  const int c1 = GROUP ? 2 * ((wave + 1) * (chunks / 2) / kWaves) : (wave + 1) * chunks / kWaves;
+
+  i4 rb_words = rsrc_words(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
+  i4 ra_words = rsrc_words(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
+  i4 rs_words = rsrc_words(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
+  const int b_row = p.N * 8;  // bytes per row of B
+  const int s_row = p.N * 2;
+  // this lane's 16-byte pieces of B (Marlin lane t = kg, c = nu%8 of block nu/8), and the
+  // scales of columns 16j + 8h + c of that block
+  const int b_src = 1024 * set + 512 * (nu >> 3) + 16 * (4 * (nu & 7) + kg);
+  const int s_src = 256 * set + 128 * (nu >> 3) + 16 * (nu & 7);
+  // activations: 128 bytes of eight rows per load; piece p of row r sits at position
+  // p ^ (r % 8), so that the operand reads (piece 2 kg + q of row nu) meet no bank
+  // twice.  Rows past M are zeros.
+  int a_src[2 * MB];
 #pragma unroll
-  for (int ps = 0; ps < Sh::kPasses; ps++) {
-    const int b0 = ps * Sh::kPass;
-    // (one scale per column: on their way while the sums meet)
-    h4 chan[Sh::kRounds];
-    const int col0 = 128 * set + 64 * (kg >> 1) + 4 * (kg & 1);
-    if constexpr (!GROUP) {
-#pragma unroll
-      for (int i = 0; i < Sh::kRounds; i++) {
-        const int s = (b0 + i * kWaves + wave) / MB;
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          chan[i][r] = __builtin_bit_cast(
-              half_t, __builtin_amdgcn_raw_buffer_load_b16(
-                          rS, 2 * scale_index_single(col0 + 16 * (s >> 1) + 8 * (s & 1) + r), 0, 0));
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = b0; b < b0 + Sh::kPass; b++) red[(wave * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < Sh::kRounds; i++) {
-      const int b = b0 + i * kWaves + wave;
-      if (b >= b0 + Sh::kPass) continue;
-      f4 v = red[(b - b0) * 64 + lane];
-#pragma unroll
-      for (int w = 1; w < kWaves; w++) v += red[(w * Sh::kPass + b - b0) * 64 + lane];
-      const int row = row0 + 16 * (b % MB) + nu;
-      // register r of lane (row, kg) holds column slot nu' = 4 kg + r, column 16j +
-      // 8h + nu' % 8 of block nu' / 8, b / MB = 2j + h: four neighbouring columns
-      const int s = b / MB;
-      const int col = col0 + 16 * (s >> 1) + 8 * (s & 1);
-      h4 o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-      if constexpr (!GROUP) o *= chan[i];
-      if (row < p.M) *(h4*)((half_t*)p.C + (size_t)row * p.N + col) = o;
-    }
+  for (int i = 0; i < 2 * MB; i++) {
+    const int r = row0 + 8 * i + lane / 8;
+    a_src[i] = r < p.M ? r * p.K * 2 + 16 * ((lane % 8) ^ (lane / 8)) : kOob;
   }
+  unsigned lds_slot = (unsigned)(size_t)smem + wave * 2 * kSlot;  // (the only LDS of the kernel: at 0)
+  unsigned a_rd[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) a_rd[q] = lds_slot + nu * 128 + 16 * ((2 * kg + q) ^ (nu & 7));
+
+  f4 acc[8][MB];
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(MB == 3 || MB == 4, "");
+  if constexpr (GROUP && MB == 4) {
+#include "w4a16_rows_wide_group64.inc"
+  } else if constexpr (GROUP && MB == 3) {
+#include "w4a16_rows_wide_group48.inc"
+  } else if constexpr (MB == 4) {
+#include "w4a16_rows_wide_chan64.inc"
+  } else {
+#include "w4a16_rows_wide_chan48.inc"
+  }
+#else  // the host pass only needs the launch stub
+  (void)rb_words, (void)ra_words, (void)rs_words, (void)b_row, (void)s_row, (void)b_src, (void)s_src;
+  (void)a_src, (void)a_rd, (void)lds_slot, (void)c0, (void)c1;
+  for (auto& r : acc)
+    for (auto& v : r) v = (f4){0.f, 0.f, 0.f, 0.f};
+#endif
+
+  __amdgpu_buffer_rsrc_t rS = make_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
+  wide_finish<MB, GROUP>(p, smem, acc, rS, set, row0, wave, lane);
 }
 
 namespace {
 
 template <class F>
-bool with_wide_kernel(int blocks, bool group, F f) {
-  switch (2 * blocks + (group ? 1 : 0)) {
+bool with_wide_kernel(int blocks, bool group, bool deep, F f) {
+  switch ((deep ? 100 : 0) + 2 * blocks + (group ? 1 : 0)) {
+    case 106: f(rows_deep_kernel<3, false>, kDeepLds); return true;
+    case 107: f(rows_deep_kernel<3, true>, kDeepLds); return true;
+    case 108: f(rows_deep_kernel<4, false>, kDeepLds); return true;
+    case 109: f(rows_deep_kernel<4, true>, kDeepLds); return true;
     case 4: f(rows_wide_kernel<2, false>, WideShape<2>::kLds); return true;
     case 5: f(rows_wide_kernel<2, true>, WideShape<2>::kLds); return true;
     case 6: f(rows_wide_kernel<3, false>, WideShape<3>::kLds); return true;
@@ -234,17 +319,18 @@ bool with_wide_kernel(int blocks, bool group, F f) {
 }  // namespace
 
 bool rows_wide_exist(int blocks) {
-  return with_wide_kernel(blocks, true, [](auto, int) {});
+  return with_wide_kernel(blocks, true, false, [](auto, int) {});
 }
 
 int configure_rows_wide_kernels() {
   bool ok = true;
   for (int blocks = 1; blocks <= kRowsMaxBlocks; blocks++)
     for (const bool group : {false, true})
-      with_wide_kernel(blocks, group, [&](auto kernel, int lds) {
-        ok = ok && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       lds) == hipSuccess;
-      });
+      for (const bool deep : {false, true})
+        with_wide_kernel(blocks, group, deep, [&](auto kernel, int lds) {
+          ok = ok && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         lds) == hipSuccess;
+        });
   return ok ? 0 : 3;
 }
 
@@ -253,7 +339,8 @@ int launch_rows_wide(const GemmArgs& a, bool group, int blocks, hipStream_t stre
   GemmArgs b = a;
   b.row_parts = ceil_div(a.M, 16 * blocks);
   b.gpb = a.N / 128 * b.row_parts;
-  const bool found = with_wide_kernel(blocks, group, [&](auto kernel, int lds) {
+  const bool deep = (blocks == 4 && a.K >= 4096) || (blocks == 3 && a.K >= 5120);
+  const bool found = with_wide_kernel(blocks, group, deep, [&](auto kernel, int lds) {
     hipLaunchKernelGGL(kernel, dim3(b.gpb), dim3(64 * kWaves), lds, stream, b);
   });
   return found ? launch_status() : 2;

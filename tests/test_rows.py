@@ -137,6 +137,33 @@ def test_rows_return_dequantised_weights(pair, groupsize):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("pair,k", [((8, 3), 5120), ((8, 3), 5888), ((8, 4), 4096), ((8, 4), 4736), ((8, 4), 8192)])
+@pytest.mark.parametrize("groupsize", [128, -1])
+def test_rows_over_a_deep_k(pair, k, groupsize):
+    """From where weights are requested three chunks ahead: chunks per wave that the ring of
+    three does and does not divide and that differ between waves, ragged rows, one-hot rows."""
+    import marlin
+    n = 512
+    if groupsize == -1 and k % 1024:
+        k -= 64  # an odd number of chunks
+    marlin.force_rows(*pair)
+    try:
+        for m in (33, 16 * pair[1], 100):
+            A, q, s, B, sp = O.make_problem(m, n, k, groupsize, seed=m + k)
+            r = O.compare(_gemm(A, B, sp, n), O.gemm(A, B, sp, n, groupsize))
+            assert r.max_abs_err <= 1e-2 * r.max_abs_ref and r.rel_mean_abs_err <= 1e-3, (m, r)
+        W = O.dequant(B, sp, k, n, groupsize)
+        if groupsize == -1:
+            W = W * O.unpack_scales(sp, False)  # fp16(q-8) * s, one rounding
+        rows = np.random.default_rng(k).permutation(k)[:200]
+        one = np.zeros((len(rows), k), np.float16)
+        one[np.arange(len(rows)), rows] = 1.0
+        assert np.array_equal(_gemm(one, B, sp, n).view(np.uint16), W[rows].view(np.uint16))
+    finally:
+        marlin.force_rows(0)
+
+
+@pytest.mark.gpu
 def test_probes_of_every_pair_run():
     import torch
     import marlin
