@@ -294,7 +294,9 @@ __global__ __launch_bounds__(64 * kWaves) void rows_deep_kernel(GemmArgs p) {
 #endif
 
   __amdgpu_buffer_rsrc_t rS = make_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
-  wide_finish<MB, GROUP>(p, smem, acc, rS, set, row0, wave, lane);
+  // (the lane once more, so that no register is held through the statement, which leaves six)
+  const int again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  wide_finish<MB, GROUP>(p, smem, acc, rS, set, row0, wave, again);
 }
 
 namespace {
