@@ -1017,6 +1017,12 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
           pl = make_plan(m, n, k, sms, cx);
         }
         ok = pl.partial_bytes == 0;
+      } else if (!ok && pl.kernel == 1 && m > 8 && m <= 16 && sms <= 0 && !cx.force.any()) {
+        // and 9 to 16 rows, where the line between the two is a matter of a tenth, by
+        // column strips (10 x 768 x 7296 is one that was always captured without scratch)
+        cx.force.kernel = 3;
+        pl = make_plan(m, n, k, sms, cx);
+        ok = pl.partial_bytes == 0;
       }
     }
     // (with the plan's scratch in hand: what a stream must have seen before it can be

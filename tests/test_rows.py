@@ -214,3 +214,34 @@ def test_chosen_and_captured(m, n, k, g):
         marlin.mul(A, B, C, sp, ws)
         torch.cuda.synchronize()
         assert torch.equal(C, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,g", [(10, 768, 7296, 128), (16, 4096, 11008, 128), (9, 512, 8192, -1)])
+def test_few_rows_captured_without_scratch(m, n, k, g):
+    """Problems that the streaming kernel shares out are captured on a stream that has no
+    scratch, as column strips, replayed between eager calls."""
+    import torch
+    import marlin
+    assert marlin.plan(m, n, k, g)[1]["partial_kib"] > 0
+    dev = torch.device("cuda:0")
+    A, q, s, B, sp = O.make_problem(m, n, k, g, seed=m + n)
+    want = O.gemm(A, B, sp, n, g)
+    dA, dB, dS = (torch.from_numpy(x).to(dev) for x in (A, B, sp))
+    C = torch.empty((m, n), dtype=torch.half, device=dev)
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int, device=dev)
+    marlin.mul(dA, dB, C, dS, ws)
+    torch.cuda.synchronize()
+    marlin.release()  # (a new stream may have the handle of one that had scratch)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        marlin.mul(dA, dB, C, dS, ws)
+    for _ in range(3):
+        C.fill_(7.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        r = O.compare(C.cpu().numpy(), want)
+        assert r.max_abs_err <= 1e-2 * r.max_abs_ref and r.rel_mean_abs_err <= 1e-3, r
+        r = O.compare(_gemm(A, B, sp, n), want)
+        assert r.max_abs_err <= 1e-2 * r.max_abs_ref, r
