@@ -28,8 +28,13 @@
 // requested before its arithmetic (M = 45, N = 12288, K = 4096: all weights requested at
 // once 13.3 us, two units of 128 k-values 12.8, one 11.6; M = 18, N = 768, K = 2176, one
 // strip and 16 rows, one chunk 0.90, two 0.85 and two units as well 0.82 of the time with
-// weights through registers).  Weights that only one workgroup reads are requested as read
-// once: with several row parts that costs 4 to 15 % (one strip), without up to 3 % (six).
+// weights through registers).
+//
+// Weights that only one workgroup reads are requested as read once, those of several row
+// parts are not: two kernels.  (A branch on it in the loop cost 1 % on average and 4 % with
+// two strips, 16 rows and group scales: 41 x 2304 x 2048 4.92 us, 4.6 without.  As read once
+// whatever the parts: 0.94 to 1.18 of the time over weights from memory, 2 to 12 % longer
+// where a cache has them.)
 //
 // Eight strips are a kernel of their own (w4a16_rows_wide.hip).
 #include <type_traits>
@@ -81,7 +86,8 @@ struct RowsShape {
       kRowsWaves * kStagePerWave > kReduce ? kRowsWaves * kStagePerWave : kReduce;
 };
 
-template <int CS, int MB, bool GROUP, int DEPTH, int UNITS>
+// ONCE: the weights are requested as read once, where one workgroup reads them (launch_rows)
+template <int CS, int MB, bool GROUP, int DEPTH, int UNITS, bool ONCE>
 __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   using Sh = RowsShape<CS, MB, DEPTH, UNITS>;
   constexpr int NA = Sh::kALoads, NB = Sh::kBLoads, NS = GROUP ? CS : 0;
@@ -176,18 +182,13 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
 #pragma unroll
     for (int i = 0; i < NA; i++) load_to_lds16(rA, stage + d * Sh::kSlot + 1024 * i, a_src[i] | inv, 128 * c);
   };
-  // the unit that starts with chunk c, to place `at`; read once only where the rows are in one part
+  // the unit that starts with chunk c, to place `at`
   auto issue_weights = [&](int at, int c) {
     const bool mine = c < c1;
     const int off = 4 * (c - c0) * b_row;
     char* const dst = stage_w + at * (1024 * NB);
-    if (p.row_parts == 1) {
 #pragma unroll
-      for (int i = 0; i < NB; i++) load_to_lds16<2>(rB, dst + 1024 * i, mine ? b_src[i] + off : kOob, 0);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NB; i++) load_to_lds16(rB, dst + 1024 * i, mine ? b_src[i] + off : kOob, 0);
-    }
+    for (int i = 0; i < NB; i++) load_to_lds16<ONCE ? 2 : 0>(rB, dst + 1024 * i, mine ? b_src[i] + off : kOob, 0);
   };
 
   f4 acc[CS][MB];
@@ -339,12 +340,15 @@ namespace {
 
 // calls f(kernel, LDS bytes) for a set of strips and rows that exists
 template <class F>
-bool with_rows_kernel(int strips, int blocks, bool group, F f) {
+bool with_rows_kernel(int strips, int blocks, bool group, bool once, F f) {
 #define ROWS(CS, MB, DEPTH, UNITS, GROUP)                                               \
   if (strips == CS && blocks == MB && group == GROUP) {                               \
     using Sh = RowsShape<CS, MB, DEPTH, UNITS>;                                       \
     static_assert(Sh::kLds <= 160 * 1024, "LDS of a compute unit");                   \
-    f(rows_kernel<CS, MB, GROUP, DEPTH, UNITS>, Sh::kLds);                            \
+    if (once)                                                                         \
+      f(rows_kernel<CS, MB, GROUP, DEPTH, UNITS, true>, Sh::kLds);                    \
+    else                                                                              \
+      f(rows_kernel<CS, MB, GROUP, DEPTH, UNITS, false>, Sh::kLds);                   \
     return true;                                                                      \
   }
 #define ROWS_OF_BOTH(CS, MB, DEPTH, UNITS) ROWS(CS, MB, DEPTH, UNITS, true) ROWS(CS, MB, DEPTH, UNITS, false)
@@ -372,7 +376,7 @@ bool with_rows_kernel(int strips, int blocks, bool group, F f) {
 }  // namespace
 
 bool rows_exist(int strips, int blocks, bool group) {
-  return strips == 8 ? rows_wide_exist(blocks) : with_rows_kernel(strips, blocks, group, [](auto, int) {});
+  return strips == 8 ? rows_wide_exist(blocks) : with_rows_kernel(strips, blocks, group, true, [](auto, int) {});
 }
 
 int configure_rows_kernels() {
@@ -380,10 +384,11 @@ int configure_rows_kernels() {
   for (int strips = 1; strips <= kRowsMaxStrips; strips++)
     for (int blocks = 1; blocks <= kRowsMaxBlocks; blocks++)
       for (const bool group : {false, true})
-        with_rows_kernel(strips, blocks, group, [&](auto kernel, int lds) {
-          ok = ok && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         lds) == hipSuccess;
-        });
+        for (const bool once : {false, true})
+          with_rows_kernel(strips, blocks, group, once, [&](auto kernel, int lds) {
+            ok = ok && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           lds) == hipSuccess;
+          });
   return ok ? 0 : 3;
 }
 
@@ -392,7 +397,7 @@ int launch_rows(const GemmArgs& a, bool group, int strips, int blocks, hipStream
   GemmArgs b = a;
   b.row_parts = ceil_div(a.M, 16 * blocks);
   b.gpb = ceil_div(a.N / 16, strips) * b.row_parts;
-  const bool found = with_rows_kernel(strips, blocks, group, [&](auto kernel, int lds) {
+  const bool found = with_rows_kernel(strips, blocks, group, b.row_parts == 1, [&](auto kernel, int lds) {
     hipLaunchKernelGGL(kernel, dim3(b.gpb), dim3(64 * kRowsWaves), lds, stream, b);
   });
   return found ? launch_status() : 2;
