@@ -18,23 +18,26 @@
 // fetched, and are read once in operand order.  MFMA lane (kg, nu) takes the sixteen
 // k-values of row kg of four rows of B for column slot nu -- word j = (nu/2)%4 of the Marlin
 // lanes (t, c = 2s + e), t = 0 ... 3, e = nu/8 -- so that an activation operand is eight
-// neighbouring k-values of a row, 16 bytes.  (Weights
-// through registers into LDS, and the scales of columns fetched after the loop, took 1.05
-// times as long: 231 problems, 1.1 with three and four strips of 32 and 48 rows, 1.01 with
-// five and six; 45 x 12288 x 4096 13.0 us.)
+// neighbouring k-values of a row, 16 bytes.  (Weights through registers into LDS, and the
+// scales of columns fetched after the loop, took 1.10 times as long: 528 problems over every
+// pair but eight strips, 1.05 with five strips, 1.07 with six, 1.11 with two to four; 45 x 12288
+// x 4096 13.0 us.)
 //
 // The more a wave has in flight the longer each takes to come: two chunks where strips and
 // rows are few (a launch then waits for its first ones), else one, whose successor is
 // requested before its arithmetic (M = 45, N = 12288, K = 4096: all weights requested at
 // once 13.3 us, two units of 128 k-values 12.8, one 11.6; M = 18, N = 768, K = 2176, one
 // strip and 16 rows, one chunk 0.90, two 0.85 and two units as well 0.82 of the time with
-// weights through registers).
+// weights through registers).  The last two chunks are steps of their own, which request
+// nothing more.  (Requests past the end, dropped by the hardware's check, took as long as
+// others: without them 0.97 of the time over 1128 problems, none more than 1.012, 0.93 where k
+// is a chunk or two per wave.  11 x 16640 x 512 took 4.5 us with weights through registers, 5.15
+// with requests past the end, 4.45 now.)
 //
 // Weights that only one workgroup reads are requested as read once, those of several row
-// parts are not: two kernels.  (A branch on it in the loop cost 1 % on average and 4 % with
-// two strips, 16 rows and group scales: 41 x 2304 x 2048 4.92 us, 4.6 without.  As read once
-// whatever the parts: 0.94 to 1.18 of the time over weights from memory, 2 to 12 % longer
-// where a cache has them.)
+// parts are not: two kernels.  (A branch on it in the loop took 1 % on average and 4 % with two
+// strips, 16 rows and group scales.  As read once whatever the parts: 0.94 to 1.18 of the time
+// over weights from memory, 2 to 12 % longer where a cache has them.)
 //
 // Eight strips are a kernel of their own (w4a16_rows_wide.hip).
 #include <type_traits>
@@ -201,15 +204,24 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   const h2 mul = {(half_t)0.0625f, (half_t)0.0625f};
   const h2 add = {(half_t)-72.f, (half_t)-72.f};
   int w_at = 0;  // place of the unit in use
-  auto step = [&](int c, auto EVEN) {
-    constexpr bool even = decltype(EVEN)::value;
+  // MORE: chunks follow c + 1.  Else c is the last or the last but one, and nothing is requested
+  // that no step reads: the hardware takes as long over a request past the end as over another.
+  auto step = [&](int c, auto EVEN, auto MORE) {
+    constexpr bool even = decltype(EVEN)::value, more = decltype(MORE)::value;
     constexpr bool first = even || Sh::kUnitChunks == 1;                   // a unit of weights starts here
     constexpr bool last = !even || Sh::kUnitChunks == 1;                   // ... ends
     constexpr int d = DEPTH == 2 && !even ? 1 : 0;                         // this chunk's activations
-    // chunk c has landed; what was requested after it may still be on its way
+    // chunk c has landed; what was requested after it may still be on its way (of the last two
+    // chunks the second one's; the first of them may have come from before the loop)
     constexpr int later = DEPTH == 1 ? 0 : UNITS == 2 ? NA + NB + (even ? 0 : NS) : first ? NA : NS + NA;
+    constexpr int later_of_two = DEPTH == 1 ? 0 : UNITS == 2 && Sh::kUnitChunks == 1 ? NA + NB : NA;
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(vmcnt(later));
+    if (more)
+      __builtin_amdgcn_s_waitcnt(vmcnt(later));
+    else if (even && later_of_two > 0 && c + 1 < c1)
+      __builtin_amdgcn_s_waitcnt(vmcnt(later_of_two));
+    else
+      __builtin_amdgcn_s_waitcnt(vmcnt(0));
     __builtin_amdgcn_sched_barrier(0);
     i4 av[MB][2];
     rows_each<MB>([&](auto I) {
@@ -242,17 +254,21 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
       for (int s = 0; s < CS; s++) sc[s] = sq[s];
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (GROUP && even) issue_scales(c + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    // (two units: the rows first, so that a chunk's do not wait for later weights)
-    if (UNITS == 2) issue_rows(d, c + DEPTH);
-    __builtin_amdgcn_sched_barrier(0);
-    if (last) {
-      issue_weights(w_at, c + 1 + (UNITS - 1) * Sh::kUnitChunks);
-      if (UNITS == 2) w_at ^= 1;
+    if constexpr (more) {
+      if (GROUP && even) issue_scales(c + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      // (two units: the rows first, so that a chunk's do not wait for later weights)
+      if (UNITS == 2) issue_rows(d, c + DEPTH);
+      __builtin_amdgcn_sched_barrier(0);
+      if (last) issue_weights(w_at, c + 1 + (UNITS - 1) * Sh::kUnitChunks);
+      __builtin_amdgcn_sched_barrier(0);
+      if (UNITS == 1) issue_rows(d, c + DEPTH);
+    } else if (even && UNITS == 1 && c + 1 < c1) {
+      if (last) issue_weights(w_at, c + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (DEPTH == 1) issue_rows(d, c + 1);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    if (UNITS == 1) issue_rows(d, c + DEPTH);
+    if (UNITS == 2 && last) w_at ^= 1;
     __builtin_amdgcn_sched_barrier(0);
     // a block of 16 slots: k-values 2t, 2t + 1 and 2t + 8, 2t + 9 of the lane's sixteen
 #pragma unroll
@@ -286,13 +302,16 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   __builtin_amdgcn_sched_barrier(0);
   issue_weights(0, c0);
   __builtin_amdgcn_sched_barrier(0);
-  if (DEPTH == 2) issue_rows(1, c0 + 1);
+  if (DEPTH == 2 && c0 + 1 < c1) issue_rows(1, c0 + 1);
   __builtin_amdgcn_sched_barrier(0);
-  if (UNITS == 2) issue_weights(1, c0 + Sh::kUnitChunks);
-  for (int c = c0; c < c1; c += 2) {
-    step(c, std::true_type{});
-    if (c + 1 < c1) step(c + 1, std::false_type{});
+  if (UNITS == 2 && c0 + Sh::kUnitChunks < c1) issue_weights(1, c0 + Sh::kUnitChunks);
+  int c = c0;
+  for (; c + 2 < c1; c += 2) {
+    step(c, std::true_type{}, std::true_type{});
+    step(c + 1, std::false_type{}, std::true_type{});
   }
+  if (c < c1) step(c, std::true_type{}, std::false_type{});
+  if (c + 1 < c1) step(c + 1, std::false_type{}, std::false_type{});
   // nothing may still be on its way into LDS when it is reused
   __builtin_amdgcn_s_waitcnt(0);
 

@@ -137,6 +137,23 @@ def test_rows_return_dequantised_weights(pair, groupsize):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("pair,groupsize", CASES)
+def test_rows_of_few_chunks(pair, groupsize):
+    """From no chunk of 64 k-values in most waves to two, three and four in each: the last two
+    are steps of their own.  One row part and several."""
+    import marlin
+    marlin.force_rows(*pair)
+    try:
+        for k in (256, 384, 512, 1024, 1408, 1536, 2048) + (() if groupsize == 128 else (128, 192, 576, 1088, 1600)):
+            for m in (17, 16 * pair[1] + 3):
+                A, q, s, B, sp = O.make_problem(m, 256, k, groupsize, seed=m + k)
+                r = O.compare(_gemm(A, B, sp, 256), O.gemm(A, B, sp, 256, groupsize))
+                assert r.max_abs_err <= 1e-2 * r.max_abs_ref and r.cosine >= 0.9999, (m, k, r)
+    finally:
+        marlin.force_rows(0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("pair,k", [((8, 3), 5120), ((8, 3), 5888), ((8, 4), 4096), ((8, 4), 4736), ((8, 4), 8192)])
 @pytest.mark.parametrize("groupsize", [128, -1])
 def test_rows_over_a_deep_k(pair, k, groupsize):
