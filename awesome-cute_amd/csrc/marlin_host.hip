@@ -6,6 +6,7 @@
 // partition are this library's own.
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -834,6 +835,35 @@ Planned plans_for(int m, int n, int k, int sms, const PlanCtx& cx) {
   return place = make_plans(m, n, k, sms, cx);
 }
 
+// Operands that 16-byte loads straight into LDS may fetch.  A tensor may start anywhere in its
+// storage; loads to registers take any address, and that a load into LDS does is documented
+// nowhere.
+bool whole_lines(const void* A, const void* B) {
+  return (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
+}
+
+// The plan of a call whose operands do not start on 16 bytes, in place of one on the rows
+// kernel: 9 to 16 rows stay column strips (enqueue launches them 8 at a time), more take
+// 64-row prefill tiles, which load through registers, whole: nothing that a capture or a full
+// pool could refuse.
+Planned plans_off_lines(Planned p, PlanCtx cx) {
+  const bool rows_kernel = p.rows.strips > 0 || (p.plan.kernel == 3 && p.m > 8);
+  if (!rows_kernel) return p;
+  p.rows = {0, 0};
+  if (p.m > 16) {
+    cx.partial_limit = 0;
+    cx.force = Force();
+    cx.force.kernel = 2;
+    cx.force.tile_rows = 64;
+    p.plan = make_plan(p.m, p.n, p.k, -1, cx);
+  } else if (p.plan.kernel != 3) {
+    cx.force = Force();
+    cx.force.kernel = 3;
+    p.plan = make_plan(p.m, p.n, p.k, -1, cx);
+  }
+  return p;
+}
+
 // Enqueue the launches of plan pl with the scratch of `view` (null pointers
 // when the plan exchanges nothing through scratch).
 int enqueue(const Plan& pl, const ScratchView& view, const void* A, const void* B, void* C,
@@ -848,23 +878,22 @@ int enqueue(const Plan& pl, const ScratchView& view, const void* A, const void* 
   (void)hipGetLastError();  // an earlier call's error is not this launch's
   int rc = MARLIN_OK;
   if (pl.kernel == 3) {
-    GemmArgs a;
-    const int strip_parts = pl.row_parts;
-    a.A = A;
-    a.B = B;
-    a.C = C;
-    a.S = s;
-    a.M = m;
-    a.N = n;
-    a.K = k;
-    a.locks = nullptr;
-    a.lock_stride = 1;
-    a.scratch = nullptr;
-    a.gpb = 0;
-    a.wpt = 0;
-    a.row_parts = strip_parts;
-    a.part_rows = strip_parts > 1 ? 16 : 0;
-    rc = launch_strip(a, groupsize != -1, pl.strips, stream);
+    // (off 16 bytes: up to 8 rows a launch, through registers)
+    const int rows_per_launch = whole_lines(A, B) ? m : 8;
+    for (int m0 = 0; m0 < m && rc == MARLIN_OK; m0 += rows_per_launch) {
+      GemmArgs a = {};
+      a.A = (const char*)A + (size_t)m0 * k * 2;
+      a.B = B;
+      a.C = (char*)C + (size_t)m0 * n * 2;
+      a.S = s;
+      a.M = m - m0 < rows_per_launch ? m - m0 : rows_per_launch;
+      a.N = n;
+      a.K = k;
+      a.lock_stride = 1;
+      a.row_parts = pl.row_parts;
+      a.part_rows = pl.row_parts > 1 ? 16 : 0;
+      rc = launch_strip(a, groupsize != -1, pl.strips, stream);
+    }
   } else if (pl.kernel == 2) {
     GemmArgs a;
     a.A = A;
@@ -984,7 +1013,8 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
   if (cus > 0 && configure_device(dev)) {
     PlanCtx cx = {cus, use_static ? kStaticPartialBytes : kPoolPartialLimit, t_force, groupsize != -1};
     cx.counters = max_par > 16 ? 16 : max_par;  // the counters of a tile sit that many ints apart
-    const Planned planned = plans_for(m, n, k, sms, cx);
+    Planned planned = plans_for(m, n, k, sms, cx);
+    if (!whole_lines(A, B)) planned = plans_off_lines(planned, cx);
     Plan pl = planned.plan;
     ScratchView view = {nullptr, nullptr};
     bool ok = true;

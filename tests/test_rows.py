@@ -262,3 +262,31 @@ def test_few_rows_captured_without_scratch(m, n, k, g):
         assert r.max_abs_err <= 1e-2 * r.max_abs_ref and r.rel_mean_abs_err <= 1e-3, r
         r = O.compare(_gemm(A, B, sp, n), want)
         assert r.max_abs_err <= 1e-2 * r.max_abs_ref, r
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,g", [(9, 512, 1024, 128), (16, 256, 512, -1), (13, 768, 1152, 128), (40, 256, 512, 128),
+                                     (300, 512, 1152, -1), (41, 2304, 2048, 128), (64, 1024, 4096, -1)])
+def test_operands_that_start_anywhere(m, n, k, g):
+    """Views into larger storage: A off by one half, B by one word, or both.  Loads straight into
+    LDS are for operands that start on 16 bytes; these take kernels that load to registers."""
+    import torch
+    import marlin
+    assert m > 8 and (marlin.plan(m, n, k, g)[1]["kernel"] == 3 or marlin.rows_plan(m, n, k, g) is not None)
+    dev = torch.device("cuda:0")
+    A, q, s, B, sp = O.make_problem(m, n, k, g, seed=m + k)
+    want = O.gemm(A, B, sp, n, g)
+    store_a = torch.zeros(m * k + 8, dtype=torch.half, device=dev)
+    store_b = torch.zeros(B.size + 4, dtype=torch.int32, device=dev)
+    dS = torch.from_numpy(sp).to(dev)
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int, device=dev)
+    for off_a, off_b in ((1, 0), (0, 1), (3, 2), (4, 0)):
+        dA, dB = store_a[off_a:off_a + m * k].view(m, k), store_b[off_b:off_b + B.size].view(B.shape)
+        dA.copy_(torch.from_numpy(A))
+        dB.copy_(torch.from_numpy(B))
+        C = torch.full((m + 1, n), 7.0, dtype=torch.half, device=dev)
+        marlin.mul(dA, dB, C[:m], dS, ws)
+        torch.cuda.synchronize()
+        assert (C[m] == 7.0).all() and not ws.any().item()
+        r = O.compare(C[:m].cpu().numpy(), want)
+        assert r.max_abs_err <= 1e-2 * r.max_abs_ref and r.rel_mean_abs_err <= 1e-3, (off_a, off_b, r)
