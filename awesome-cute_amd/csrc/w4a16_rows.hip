@@ -111,8 +111,9 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
   // as that keeps waves busy (16 rows, K = 512, four strips: four waves of two 1.14 times as long)
   const int chunks = p.K / 64;
   const bool pairs = GROUP && chunks > kRowsWaves;
-  const int c0 = pairs ? 2 * (wave * (chunks / 2) / kRowsWaves) : wave * chunks / kRowsWaves;
-  const int c1 = pairs ? 2 * ((wave + 1) * (chunks / 2) / kRowsWaves) : (wave + 1) * chunks / kRowsWaves;
+  const int run = rows_run(wave);
+  const int c0 = pairs ? 2 * (run * (chunks / 2) / kRowsWaves) : run * chunks / kRowsWaves;
+  const int c1 = pairs ? 2 * ((run + 1) * (chunks / 2) / kRowsWaves) : (run + 1) * chunks / kRowsWaves;
 
   const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
@@ -323,7 +324,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
     __syncthreads();
 #pragma unroll
     for (int b = b0; b < b0 + Sh::kPass && b < Sh::kBlocks; b++)
-      red[(wave * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
+      red[(run * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < Sh::kRounds; i++) {

@@ -75,7 +75,7 @@ __device__ __forceinline__ void wide_finish(const GemmArgs& p, char* smem, const
     }
     __syncthreads();
 #pragma unroll
-    for (int b = b0; b < b0 + Sh::kPass; b++) red[(wave * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
+    for (int b = b0; b < b0 + Sh::kPass; b++) red[(rows_run(wave) * Sh::kPass + b - b0) * 64 + lane] = acc[b / MB][b % MB];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < Sh::kRounds; i++) {
@@ -115,8 +115,9 @@ __global__ __launch_bounds__(64 * kWaves) void rows_wide_kernel(GemmArgs p) {
 
   // my chunks [c0, c1) of 64 k-values: whole groups where there are groups
   const int chunks = p.K / 64;
-  const int c0 = GROUP ? 2 * (wave * (chunks / 2) / kWaves) : wave * chunks / kWaves;
-  const int c1 = GROUP ? 2 * ((wave + 1) * (chunks / 2) / kWaves) : (wave + 1) * chunks / kWaves;
+  const int run = rows_run(wave);
+  const int c0 = GROUP ? 2 * (run * (chunks / 2) / kWaves) : run * chunks / kWaves;
+  const int c1 = GROUP ? 2 * ((run + 1) * (chunks / 2) / kWaves) : (run + 1) * chunks / kWaves;
 
   const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
@@ -248,8 +249,9 @@ __global__ __launch_bounds__(64 * kWaves) void rows_deep_kernel(GemmArgs p) {
 
   // my chunks [c0, c1) of 64 k-values: whole groups where there are groups
   const int chunks = p.K / 64;
-  const int c0 = GROUP ? 2 * (wave * (chunks / 2) / kWaves) : wave * chunks / kWaves;
-  const int c1 = GROUP ? 2 * ((wave + 1) * (chunks / 2) / kWaves) : (wave + 1) * chunks / kWaves;
+  const int run = rows_run(wave);
+  const int c0 = GROUP ? 2 * (run * (chunks / 2) / kWaves) : run * chunks / kWaves;
+  const int c1 = GROUP ? 2 * ((run + 1) * (chunks / 2) / kWaves) : (run + 1) * chunks / kWaves;
 
   i4 rb_words = rsrc_words(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   i4 ra_words = rsrc_words(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
