@@ -480,10 +480,7 @@ double strip_cost(int m, int n, int k, int cs, const PlanCtx& cx) {
     const double per_wg = 1.27 + 8.0 * cs * k / 32.7e3 + 32.0 * k / 67.8e3;
     const double by_cu = rounds * per_wg * (1.0 - 0.24 * (1.0 - 1.0 / rounds));
     const double by_memory = 0.5 * k * n / 4.8e6;
-    // (two strips stay the choice where one would nearly fill the compute units over a short k
-    // range: M = 100, N = 512, K = 1024 3.6 us, with one strip 3.2)
-    const double full = cs == 1 && k < 2048 && 8 * wgs >= 7 * cus && wgs < cus ? 0.7 * (1.0 - k / 2048.0) : 0.0;
-    return 1.8 + (by_cu > by_memory ? by_cu : by_memory) + full;
+    return 1.8 + (by_cu > by_memory ? by_cu : by_memory);
   }
   const int wgs = ceil_div(n / 16, cs);
   if (m > 8) {
