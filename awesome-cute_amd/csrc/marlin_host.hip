@@ -403,9 +403,27 @@ double stream_parts_cost(int m, int n, int k, const PlanCtx& cx, int* parts, int
   return 0.65 * (11.3 + 0.28 * *gpb) - (w == 1 ? 2.0 : 0.0);
 }
 
+// 9 to 16 rows, one launch, by kind of scales: a launch that shares its tiles and one that does
+// not, the granules of the longest workgroup, the weights' way from memory, runs that straddle
+// tiles, sharers beyond eight.  1490 launches over N = 256 ... 28672, K = 512 ... 16384, 4 % rms.
+// (By the fit above, without the weights and of group scales alone, one scale per column read 0.88
+// of it where a tile has one workgroup and 1.05 with nine and more: 15 x 18176 x 4608 took 14.5 us
+// as strips, 12.3 streaming, 14 x 2048 x 5504 7.0 streaming, 6.3 as strips.)
+double stream_cost_few(int n, int k, const PlanCtx& cx) {
+  const StreamSplit s = choose_stream_split(1, n, k, cx.cus);
+  const int sharers = s.wpt > 0 ? s.wpt : ceil_div(k / kGranuleK, s.gpb);
+  const bool alone = sharers == 1 && !s.straddle;
+  const int beyond = sharers > 8 ? sharers - 8 : 0;
+  const double MB = 0.5e-6 * n * k;
+  if (cx.grouped)
+    return (alone ? 3.77 : 5.08) + 0.108 * s.gpb + 0.073 * MB + (s.straddle ? 4.5 : 0.0) + 0.24 * beyond;
+  return (alone ? 3.87 : 5.24) + 0.074 * s.gpb + 0.075 * MB + (s.straddle ? 4.4 : 0.0) + 0.24 * beyond;
+}
+
 // The streaming kernel's cost as make_plan would launch it: with the rows cut
 // in two or into parts of 32 where that is cheaper.
 double stream_cost_as_planned(int m, int n, int k, const PlanCtx& cx) {
+  if (m > 8 && m <= 16) return stream_cost_few(n, k, cx);
   double stream = stream_cost(m, n, k, cx.cus);
   if (m <= kStreamMaxRows && cx.force.row_halves != 1 && cx.counters >= 2) {
     // what the launch gains where make_plan cuts its rows in two
@@ -486,18 +504,16 @@ double strip_cost(int m, int n, int k, int cs, const PlanCtx& cx) {
   if (m > 8) {
     // 9 to 16 rows, on the rows kernel: a launch, the strips' sums, what a workgroup takes in
     // and computes, dearer the fuller the chip, and workgroups beyond one per compute unit
-    // (half way between the rounds they make and their share of one).  6400 launches over 2100
-    // problems of 1 to 16 rows, 4 % rms; against the streaming kernel's fit, which does not
-    // tell the kinds of scales apart, 0.98 of it with group scales and 1.09 without
+    // (half way between the rounds they make and their share of one).  4981 launches over 1850
+    // problems, 4 % rms
     const double K = k / 1000.0, r = (double)wgs / cus, fill = r < 1.0 ? r : 1.0;
     const double more = r > 1.0 ? 0.5 * (ceil_div(wgs, cus) + r) - 1.0 : 0.0;
+    const double by = cs == 3 ? 1.055 : cs == 2 ? 1.0 : 1.03;
     if (cx.grouped)
-      return 0.98 * (cs == 3 ? 1.05 : 1.02) *
-             (2.46 + 0.25 * cs + K * (0.40 + 0.158 * cs + 0.099 * fill * cs + more * (0.134 + 0.367 * cs)) +
-              0.71 * more + 0.0093 * m * K);
-    return 1.09 * (cs == 3 ? 1.05 : 1.01) *
-           (2.49 + 0.191 * cs + K * (0.303 + 0.128 * cs + 0.102 * fill * cs + more * (0.265 + 0.267 * cs)) +
-            0.84 * more + 0.0124 * m * K);
+      return by * (2.25 + 0.278 * cs + K * (0.168 + 0.119 * cs + 0.145 * fill * cs + more * (0.211 + 0.355 * cs)) +
+                   0.32 * more + 0.0239 * m * K);
+    return by * (2.23 + 0.252 * cs + K * (0.127 + 0.109 * cs + 0.130 * fill * cs + more * (0.257 + 0.327 * cs)) +
+                 0.27 * more + 0.0266 * m * K);
   }
   // Up to 8 rows the constants are fitted on their own (M = 1, 4, 8: 7 % rms): the launch, the
   // rate a compute unit unpacks at, the rate it reads rows at, a queued
@@ -521,10 +537,9 @@ double strip_cost(int m, int n, int k, int cs, const PlanCtx& cx) {
 // 16-column strips per workgroup of the column-strip kernel: the cheapest of
 // 1, 2 and 4 where they divide n's strips, and for up to 16 rows of 3, which
 // leaves the last workgroup with fewer (N = 11008, K = 4096, 230 workgroups
-// of three strips against 172 of four: M = 16 9.2 against 9.3 us, M = 8 8.2 /
-// 8.5, M = 1 7.5 / 7.7 with one strip; K = 8192: M = 1 12.3 against 13.6, M =
-// 4 11.7 / 13.6, M = 16 14.4 / 15.2; N = 5120, K = 5120: 10.3 against 8.4 with
-// two)
+// of three strips against 172 of four: M = 8 8.2 against 8.5 us, M = 1 7.5 / 7.7
+// with one strip; K = 8192: M = 1 12.3 against 13.6, M = 4 11.7 / 13.6; N = 5120,
+// K = 5120: 10.3 against 8.4 with two)
 // (0 where the planner's own rules leave none; a forced launch takes any)
 int strips_per_workgroup(int m, int n, int k, const PlanCtx& cx) {
   const bool forced = cx.force.kernel == 3 || cx.force.strips != 0;
@@ -560,8 +575,10 @@ int strips_per_workgroup(int m, int n, int k, const PlanCtx& cx) {
 // strips win while the weights are a few MiB per launch (M = 1: 4096 x 4096
 // 4.3 against 6.3 us, N = 11008, K = 4096 8.5 against 9.7, N = 4096, K = 11008
 // 7.5 against 9.1, 8192 x 8192 9.1 against 10.4, N = 28672, K = 8192 27.6
-// against 23.9 -- there no more; M = 16: 4096 x 4096 5.8 against 6.6, N =
-// 11008, K = 4096 9.4 against 9.9, N = 4096, K = 11008 11.8 against 9.6), and
+// against 23.9 -- there no more), 9 to 16 rows the same with a fit of its own for either kernel
+// (over 3694 problems the choice takes 1.005 of the better of the two, 8 of them more than 10 %
+// longer; by the fits of a kernel whose requests past the end made short ranges slow 1.018 and
+// 210), and
 // with more rows, in parts, while the parts fill the compute units at most
 // twice (M = 32: N = K = 1024 3.9 against 5.6, 4096 x 4096 7.6 against 8.5, N =
 // 8192, K = 4096 9.5 against 10.3, N = 4096, K = 8192 11.0 against 10.7; M =
