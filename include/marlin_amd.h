@@ -46,6 +46,8 @@ extern "C" {
  *   sms        number of workgroups of the streaming kernel, -1 = automatic
  *   max_par    at least 1 (else MARLIN_ERR_WORKSPACE); sizes the workspace
  *       contract, and the tile counters sit min(max_par, 16) ints apart in it
+ * A and B that do not start on 16 bytes are accepted; such calls stay off the
+ * kernel whose 16-byte loads write LDS directly, and may take longer for it.
  * Not re-entrant over the same workspace or the same C concurrently.
  * Partial sums of output tiles that several workgroups share live in a
  * library-owned buffer per (device, stream), sized by the call's plan and
@@ -53,9 +55,12 @@ extern "C" {
  * counters + whole MiB of partial sums, 4 MiB for N = K = 4096 at one row).  Nothing
  * is allocated while `stream` is being captured into a graph, and no more than
  * 256 buffers per device.  A call that cannot have its scratch for that runs
- * without if it has the rows for the prefill kernel: its tiles are computed whole
- * instead of in slices of the k range, which may take longer and may round the
- * last bit of an element the other way.  Other calls return
+ * without in two cases: planned for the prefill kernels, its tiles are computed
+ * whole instead of in slices of the k range; of 9 to 16 rows (no `sms` hint), it
+ * is computed by column strips over the whole k range instead of streaming.
+ * Either may take longer and sums in another order, so that the last bit of an
+ * element may be rounded the other way than by the same call with its scratch --
+ * by a graph captured so and an eager call, for instance.  Other calls return
  * MARLIN_ERR_RUNTIME.  Run the call once on that stream before the capture, or use
  * marlin_gemm_static.
  */
