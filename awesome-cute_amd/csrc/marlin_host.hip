@@ -469,6 +469,59 @@ bool prefer_prefill(int m, int n, int k, const PlanCtx& cx) {
   return prefill_cost(m, n, k, cx) <= stream_cost_as_planned(m, n, k, cx) * (cx.grouped ? 1.0 : 0.9);
 }
 
+// Fitted time (us) of the rows kernel (w4a16_rows.hip, w4a16_rows_wide.hip) with more than 16
+// rows, also where it computes column strips in parts: a launch, the meeting of the waves' sums,
+// the activations and weights a workgroup takes in and what it computes, dearer the fuller the
+// chip, much the same again for workgroups beyond one per compute unit (by the rounds they make,
+// and half way between these and their share of one), the weights' way from memory, and by how much
+// the longest of the eight waves, and of the four SIMDs, is longer than the others where k does not
+// divide evenly (ten groups: two for two of the waves, one for six).  And where the rows that an
+// XCD's workgroups read outgrow its L2 -- an eighth of the strip sets each, with fewer than eight
+// an eighth of (set, row part) pairs -- 0.4 us per MB beyond 3.5.  17600 launches over 3211
+// problems, M = 17 ... 1500, N = 512 ... 28672, K = 640 ... 13824, 5 % rms.  The factors are those
+// of the pairs, with group scales and without.
+struct RowsPair {
+  int strips, blocks;
+  double by[2];
+};
+constexpr RowsPair kRowsPairs[] = {
+    {1, 1, {1.060, 1.103}}, {2, 1, {0.999, 1.003}}, {3, 1, {1.045, 1.053}}, {2, 2, {1.000, 1.000}},
+    {3, 2, {1.000, 0.993}}, {4, 2, {0.963, 0.927}}, {6, 2, {1.014, 0.952}}, {2, 3, {1.010, 0.976}},
+    {3, 3, {0.982, 0.957}}, {4, 3, {1.008, 0.951}}, {5, 3, {1.036, 0.989}}, {6, 3, {1.037, 0.963}},
+    {4, 4, {1.010, 1.000}}, {5, 4, {1.046, 1.008}}, {6, 4, {1.020, 0.950}}, {8, 2, {0.989, 0.940}},
+    {8, 3, {0.999, 0.949}}, {8, 4, {1.004, 0.946}}, {4, 1, {1.016, 1.007}},
+};
+const RowsPair& rows_pair(int strips, int blocks) {
+  const RowsPair* p = kRowsPairs;
+  while (p->strips != strips || p->blocks != blocks) p++;  // (a pair of the table)
+  return *p;
+}
+double rows_cost(int m, int n, int k, const RowsPair& p, const PlanCtx& cx) {
+  const int sets = ceil_div(n / 16, p.strips);
+  const int wgs = sets * ceil_div(m, 16 * p.blocks);
+  const double r = (double)wgs / cx.cus;
+  const double fill = r < 1.0 ? r : 1.0;
+  const double more = r > 1.0 ? 0.5 * (ceil_div(wgs, cx.cus) + r) - 1.0 : 0.0;
+  const int whole = ceil_div(wgs, cx.cus) - 1;
+  const double K = k / 1000.0, b = p.blocks, s = p.strips, sums = b * s;
+  const double memory = 0.5e-7 * n * k;
+  const double out = 2e-6 * m * k * (sets < 8 ? sets / 8.0 : 1.0) - 3.5;
+  const double beyond = out > 0.0 ? out : 0.0;
+  // (the kernel deals out whole groups where there are more than four)
+  const int unit = cx.grouped && k > 512 ? 128 : 64;
+  const double wave = 8e-3 * unit * ceil_div(k / unit, 8) - K, simd = 4e-3 * unit * ceil_div(k / unit, 4) - K;
+  double by = p.by[cx.grouped ? 0 : 1];
+  // (six and eight strips with all rows in one workgroup take less)
+  if (p.strips >= 6 && wgs == sets && p.blocks < 4) by *= p.blocks == 2 ? 0.93 : 0.96;
+  if (cx.grouped)
+    return by * (2.29 + 0.154 * sums + K * (0.259 * b + 0.218 * s + fill * (0.045 * b + 0.009 * s) +
+                 whole * (0.160 * b + 0.139 * s) + more * 0.079 * sums) +
+                 0.231 * more * sums + 0.52 * memory + 0.40 * beyond + wave * (0.062 * b + 0.134 * s) + 0.100 * simd * s);
+  return by * (2.10 + 0.189 * sums + K * (0.309 * b + 0.177 * s + fill * (0.018 * b + 0.005 * s) +
+                 whole * (0.203 * b + 0.085 * s) + more * 0.071 * sums) +
+                 0.250 * more * sums + 0.71 * memory + 0.40 * beyond + (0.116 * wave + 0.067 * simd) * s);
+}
+
 // Fitted time (us) of the column-strip kernel with `cs` strips per workgroup.
 // Up to 8 rows a launch costs 2.9 us.  A workgroup takes in its 8 cs k bytes
 // of weights at about 28 GB/s, what its eight waves unpack and multiply, and
@@ -479,27 +532,10 @@ bool prefer_prefill(int m, int n, int k, const PlanCtx& cx) {
 // 4096 4.3, N = 11008, K = 4096 7.8, N = 1024, K = 8192 5.5, N = 4096, K =
 // 11008 7.5, 8192 x 8192 10.4 (two strips 9.1), N = 13824, K = 5120 11.4 (four
 // strips 10.0); M = 16: 4096 x 4096 5.7, N = 11008, K = 4096 8.4, N = 4096, K = 11008 11.3.
-// More rows are cut into parts of 16, a workgroup per strip set and part, and
-// fitted on their own: 1.8 us, and per round of workgroups over the compute
-// units 1.27 us, the weights at 32.7 GB/s and the part's 16 rows at 67.8 GB/s,
-// a quarter of which later rounds hide behind the one before.  Measured: M =
-// 32, N = K = 1024 3.9 us, 2048 x 2048 4.6, 4096 x 4096 7.6; M = 64: N = 512,
-// K = 1024 3.6, N = 2048, K = 4096 7.7, 4096 x 4096 9.7; M = 128: N = 256, K =
-// 512 3.4, 2048 x 2048 6.8; M = 512: N = 256, K = 1024 3.7; M = 1024: N =
-// 256, K = 512 3.8.
+// More rows are cut into parts of 16, a workgroup of the rows kernel per strip set and part.
 double strip_cost(int m, int n, int k, int cs, const PlanCtx& cx) {
   const int cus = cx.cus;
-  if (m > 16) {
-    // rows in parts of 16, a workgroup each: fitted to 17...128 rows over N =
-    // 256...28672, K = 512...11008 (8 % rms where the strips are within 1.6
-    // times the other kernels' time)
-    const int wgs = ceil_div(n / 16, cs) * ceil_div(m, 16);
-    const int rounds = ceil_div(wgs, cus);
-    const double per_wg = 1.27 + 8.0 * cs * k / 32.7e3 + 32.0 * k / 67.8e3;
-    const double by_cu = rounds * per_wg * (1.0 - 0.24 * (1.0 - 1.0 / rounds));
-    const double by_memory = 0.5 * k * n / 4.8e6;
-    return 1.8 + (by_cu > by_memory ? by_cu : by_memory);
-  }
+  if (m > 16) return rows_cost(m, n, k, rows_pair(cs, 1), cx);
   const int wgs = ceil_div(n / 16, cs);
   if (m > 8) {
     // 9 to 16 rows, on the rows kernel: a launch, the strips' sums, what a workgroup takes in
@@ -556,9 +592,7 @@ int strips_per_workgroup(int m, int n, int k, const PlanCtx& cx) {
     // 13.5 against 11.2)
     if (m > 16 && !forced && ceil_div(n / 16, cs) * ceil_div(m, 16) > 2 * cx.cus) continue;
     if (cx.force.strips != 0 && cx.force.strips != cs && best != 0) continue;
-    // (in parts, fitted to a kernel whose weights went through registers: one strip and two
-    // take 0.87 to 0.95 of it on the rows kernel, four 0.97)
-    const double c = strip_cost(m, n, k, cs, cx) * (m <= 16 ? 1.0 : cs == 1 ? 0.94 : cs == 2 ? 0.96 : 1.0);
+    const double c = strip_cost(m, n, k, cs, cx);
     if (best == 0 || cx.force.strips == cs || c < best_cost) {
       best = cs;
       best_cost = c;
@@ -578,21 +612,15 @@ int strips_per_workgroup(int m, int n, int k, const PlanCtx& cx) {
 // against 23.9 -- there no more), 9 to 16 rows the same with a fit of its own for either kernel
 // (over 3694 problems the choice takes 1.005 of the better of the two, 8 of them more than 10 %
 // longer; by the fits of a kernel whose requests past the end made short ranges slow 1.018 and
-// 210), and
-// with more rows, in parts, while the parts fill the compute units at most
-// twice (M = 32: N = K = 1024 3.9 against 5.6, 4096 x 4096 7.6 against 8.5, N =
-// 8192, K = 4096 9.5 against 10.3, N = 4096, K = 8192 11.0 against 10.7; M =
-// 64: N = 512, K = 1024 3.6 against 6.9, N = 2048, K = 4096 7.7 against 8.7,
-// 4096 x 4096 9.7 against 10.5, N = 8192, K = 4096 15.0 against 13.3; M =
-// 128: N = 256, K = 512 3.4 against 7.0, 2048 x 2048 6.8 against 8.1, 4096 x
-// 4096 14.6 against 12.9; M = 1024: N = 256, K = 512 3.8 against 7.7, N = 512,
-// K = 1024 6.6 against 11.4).
+// 210), and with more rows, in parts, while the parts fill the compute units at most twice (M =
+// 100, N = 512, K = 1024 3.0 us; M = 41, N = 2304, K = 2048 4.6; M = 96, N = K = 4096 11.7 against
+// 12.5 streaming, M = 1000, N = 256, K = 12416 17.8 against 22.7 on prefill tiles).
 bool prefer_strips(int m, int n, int k, const PlanCtx& cx) {
   const int cs = strips_per_workgroup(m, n, k, cx);
-  // (beyond one row block the fits are looser, the streaming kernel's above all
-  // over short k ranges: the strips have to win by a margin)
+  // (more rows over a deep k: what the rows kernel takes in the plan's place it takes for a pair
+  // of its own, and the plan leaves strips by a margin)
   if (cs == 0) return false;
-  const double strips = strip_cost(m, n, k, cs, cx) * (m > 16 ? 1.05 : 1.0);
+  const double strips = strip_cost(m, n, k, cs, cx) * (m > 16 && k >= 4096 ? 1.05 : 1.0);
   // Up to 8 rows with group scales over runs that straddle tiles the line lay here where it
   // cost least: over 74 such problems what it leaves takes 1.002 of the better of the two, by
   // equal costs 1.05 (4 x 21504 x 8192 22.8 us streaming, 19.5).  (Without group scales, and for
@@ -600,7 +628,17 @@ bool prefer_strips(int m, int n, int k, const PlanCtx& cx) {
   const double line =
       m <= 8 && cx.grouped && cs > 1 && choose_stream_split(1, n, k, cx.cus).straddle ? 1.2 : 1.0;
   if (strips >= stream_cost_as_planned(m, n, k, cx) * line) return false;
-  return !(n % 256 == 0 && m > 48 && prefill_cost(m, n, k, cx) <= strips);
+  // (near prefill tiles the plan keeps those: the rows kernel, of which strips are a part, takes
+  // their place where it is cheaper)
+  return !(n % 256 == 0 && m > 48 && prefill_cost(m, n, k, cx) <= 1.03 * strips);
+}
+
+// Whether column strips may take the place of a streaming launch whose scratch cannot be had.
+bool strips_instead(int m, int n, int k, const PlanCtx& cx) {
+  if (m <= 8 || m > kStripMaxRows) return false;
+  if (m <= 16) return true;
+  const int cs = strips_per_workgroup(m, n, k, cx);
+  return cs > 0 && strip_cost(m, n, k, cs, cx) <= 1.1 * stream_cost_as_planned(m, n, k, cx);
 }
 
 Plan make_plan(int m, int n, int k, int sms, const PlanCtx& cx) {
@@ -712,87 +750,56 @@ struct RowsPlan {
   int strips, blocks;
 };
 
-// Fitted time (us) of that kernel: a launch, the meeting of the waves' sums, the
-// activations and weights a workgroup takes in and what it computes, dearer the
-// fuller the chip, the same again for workgroups beyond one per compute unit (half
-// way between the rounds they make and their share of one), and the weights'
-// way from memory.  2800 launches over 320 problems, M = 17 ... 1500, N = 512 ...
-// 28672, K = 512 ... 13824; 6 % rms, of a kernel whose weights went through registers; by
-// how much less each pair takes since is in the factors of rows_plan.
-// And where the rows that an XCD's workgroups read outgrow its L2 -- an eighth of the
-// strip sets each, with fewer than eight an eighth of (set, row part) pairs -- 0.24 us
-// per MB beyond 3.5, 0.4 with one scale per column: over n of 256 to 1024 with a thousand rows the kernel was taken
-// for faster where it took up to 1.46 times the plan's time (M = 1015, N = 256, K = 7296
-// 13.6 us in column strips, 19.9; M = 1531, N = 512, K = 8448 25.7 on prefill tiles,
-// 33.7).
-double rows_cost(int m, int n, int k, int strips, int blocks, const PlanCtx& cx) {
-  const int sets = ceil_div(n / 16, strips);
-  const int wgs = sets * ceil_div(m, 16 * blocks);
-  const double r = (double)wgs / cx.cus;
-  const double fill = r < 1.0 ? r : 1.0;
-  const double more = r > 1.0 ? 0.5 * (ceil_div(wgs, cx.cus) + r) - 1.0 : 0.0;
-  const double K = k / 1000.0, sums = strips * blocks;
-  const double memory = 0.5e-7 * n * k;
-  const double beyond = 2e-6 * m * k * (sets < 8 ? sets / 8.0 : 1.0) - 3.5;
-  const double rows = beyond > 0.0 ? (cx.grouped ? 0.24 : 0.4) * beyond : 0.0;
-  if (cx.grouped)
-    return rows + 2.88 + 0.167 * sums +
-           K * (0.335 * blocks + 0.239 * strips + fill * (0.075 * blocks + 0.033 * strips) +
-                more * (0.297 * blocks + 0.202 * strips + 0.080 * sums)) +
-           0.240 * more * sums + 0.180 * memory;
-  return rows + 2.71 + 0.174 * sums +
-         K * (0.363 * blocks + 0.186 * strips + fill * (0.086 * blocks + 0.032 * strips) +
-              more * (0.285 * blocks + 0.188 * strips + 0.039 * sums)) +
-         0.294 * more * sums + 0.149 * memory;
+// What the fit of streaming launches of 17 to 64 rows over k of 2048 and more is off by: it does
+// not tell the kinds of scales apart, and knows little of how many workgroups share a tile (1108
+// launches, by row blocks, cut in halves or not, and sharers: 2 to 4 % rms; 64 x 2048 x 8192,
+// sixteen, 1.25 of the fit, 47 x 7168 x 9472, four, 0.93).  And a line between these launches
+// and the rows kernel costs least 2 % above, with three row blocks uncut 2 % below.
+double stream_off(int m, const Plan& pl, bool grouped) {
+  const int sharers = pl.sp.wpt, blocks = ceil_div(m, 16);
+  if (sharers == 0) return grouped ? 1.17 : 1.23;  // (runs that straddle tiles)
+  double off;
+  if (sharers == 1)
+    off = pl.row_parts > 1 ? 0.94 : blocks == 2 ? 0.91 : 0.81;
+  else if (pl.row_parts == 1)
+    off = (blocks == 2 ? 1.02 : 0.907) + 0.006 * (sharers - 2);
+  else if (sharers <= 8)
+    off = 0.984 + 0.0133 * (sharers - 2);
+  else  // (fetched in two rounds)
+    off = blocks == 2 ? 1.07 : 1.173 + 0.0133 * (sharers - 9);
+  return off * (grouped ? 1.0 : sharers > 8 ? 0.98 : 0.935);
 }
 
-// For 17 rows and more, where it is 4 % cheaper than the plan -- by the plan's own
-// fits, which on these problems read 3 to 7 % low with group scales, 1 % high to 4 %
-// low without (the factors below).  Not over k ranges below 640, nor, with 16 rows
-// per workgroup, below 2048: a wave has a chunk or two there, which the column strips
-// take in at once (M = 51, N = 11520, K = 512 5.7 us streaming, 6.6 by the fit's
-// choice; M = 123, N = 512, K = 1536 4.1 and 5.0).  Ten and twelve groups leave some
-// waves two of them and others one, and take 1.06 to 1.18 times the fit (eleven 0.99 to
-// 1.03): the line against a streaming launch that shares no tile lies 5 % lower there (M
-// = 123, N = 6912, K = 1280 9.0 us streaming, 10.1; M = 64, N = 25600 13.5 and 14.7; K =
-// 1408, M = 248, N = 3584 the other way, 9.0 and 8.4).  With the factors
-// below 820 problems of 7200 changed pair or kernel by them: 0.918 of the time that the former
-// choice took with the same kernels, 63 more than 2 % slower and 28 more than 5 % (1490 x
-// 512 x 3456 13.0 -> 15.2, 47 x 7168 x 9472 18.4 -> 20.7).  (A fit of every coefficient to
-// 11100 launches over 2000 problems chose no better: 1100 others 0.941, 78 more than 5 %
-// slower.)  M = 46, N = 18432, K = 4480 29.2 -> 17.9 us, 45 x 12288 x 4096 15.1 -> 11.6, 144
-// x 2048 x 1792 9.0 -> 6.2.
+// For 17 rows and more, where it is cheaper than the plan.  Not over k ranges below 640, nor,
+// with 16 rows per workgroup, below 2048, where the plan's column strips are that launch.  Over
+// 6262 problems the choice takes 1.006 of the best launch measured, 42 of them more than 10 %
+// longer (by a fit of a kernel whose weights went through registers, with factors: 1.016 and
+// 355).  What the plans' own fits are off by near the line is in the limits; 0.03 to either side
+// costs less than 0.001 of the time.
 RowsPlan rows_plan(int m, int n, int k, int sms, const Plan& pl, const PlanCtx& cx) {
   if (cx.force.rows_strips > 0 && sms <= 0 && (cx.force.rows_strips < 8 || n % 128 == 0) &&
       rows_exist(cx.force.rows_strips, cx.force.rows_blocks, cx.grouped))
     return {cx.force.rows_strips, cx.force.rows_blocks};
   if (sms > 0 || m <= 16 || k < 640 || cx.force.any()) return {0, 0};
   double limit;
-  if (pl.kernel == 1)
-    limit = stream_cost_as_planned(m, n, k, cx) * (!cx.grouped                                    ? 0.99
-                                                   : pl.sp.wpt == 1 && (k == 1280 || k == 1536) ? 0.92
-                                                                                                : 1.03);
-  else if (pl.kernel == 2)
-    limit = prefill_cost(m, n, k, cx) * (cx.grouped ? 1.03 : 1.04);
-  else
-    limit = strip_cost(m, n, k, pl.strips, cx) * (cx.grouped ? 1.07 : 1.0);
-  limit /= 1.04;
-  // the pairs, and how much longer than the fit each takes, with group scales and without
-  static const struct {
-    int strips, blocks;
-    double by[2];
-  } pairs[] = {{1, 1, {0.95, 0.89}}, {2, 1, {0.97, 0.93}}, {3, 1, {0.99, 0.98}}, {2, 2, {0.94, 0.91}},
-               {3, 2, {0.99, 0.97}}, {4, 2, {0.94, 0.91}}, {6, 2, {0.96, 0.92}}, {2, 3, {0.90, 0.87}},
-               {3, 3, {0.95, 0.92}}, {4, 3, {0.93, 0.87}}, {5, 3, {0.96, 0.96}}, {6, 3, {0.97, 0.93}},
-               {4, 4, {0.95, 0.98}}, {5, 4, {1.00, 0.98}}, {6, 4, {0.96, 0.94}}, {8, 2, {0.92, 0.92}},
-               {8, 3, {0.93, 0.93}}, {8, 4, {0.94, 0.94}}};
+  if (pl.kernel == 1) {
+    const double off = m > kStreamMaxRows ? (pl.sp.wpt == 1 ? 0.93 : cx.grouped ? 1.02 : 0.98)
+                       : k < 2048         ? 1.03
+                                          : stream_off(m, pl, cx.grouped);
+    limit = stream_cost_as_planned(m, n, k, cx) * off;
+  } else if (pl.kernel == 2) {
+    // (rows far beyond an XCD's L2: 1316 x 512 x 5504 17.6 us, 18.3 on the rows kernel)
+    limit = prefill_cost(m, n, k, cx) * (2e-6 * m * k > 8.0 ? 0.91 : 0.99);
+  } else {
+    limit = strip_cost(m, n, k, pl.strips, cx) * 1.0001;  // (up to three strips in parts are a pair of the list)
+  }
   RowsPlan best = {0, 0};
-  for (const auto& p : pairs) {
+  for (const RowsPair& p : kRowsPairs) {
     if (m <= 16 * (p.blocks - 1) || (p.blocks == 1 && k < 2048)) continue;  // (fewer blocks hold all rows)
-    if (p.strips == 4 && p.blocks == 4 && !cx.grouped) continue;            // (does not exist)
+    if (p.strips == 4 && (p.blocks == 1 || (p.blocks == 4 && !cx.grouped))) continue;  // (strips alone; does not exist)
     // (beyond what was fitted, and never the best there)
     if (ceil_div(n / 16, p.strips) * ceil_div(m, 16 * p.blocks) > 2.7 * cx.cus) continue;
-    const double c = rows_cost(m, n, k, p.strips, p.blocks, cx) * p.by[cx.grouped ? 0 : 1];
+    const double c = rows_cost(m, n, k, p, cx);
     if (c < limit) {
       best = {p.strips, p.blocks};
       limit = c;
@@ -1061,9 +1068,9 @@ int run(const void* A, const void* B, void* C, const void* s, int m, int n, int 
           pl = make_plan(m, n, k, sms, cx);
         }
         ok = pl.partial_bytes == 0;
-      } else if (!ok && pl.kernel == 1 && m > 8 && m <= 16 && sms <= 0 && !cx.force.any()) {
-        // and 9 to 16 rows, where the line between the two is a matter of a tenth, by
-        // column strips (10 x 768 x 7296 is one that was always captured without scratch)
+      } else if (!ok && pl.kernel == 1 && sms <= 0 && !cx.force.any() && strips_instead(m, n, k, cx)) {
+        // and streaming launches of 9 to 16 rows, or of more where the line between the two is
+        // a matter of a tenth, by column strips: where it lies moves with either kernel's speed
         cx.force.kernel = 3;
         pl = make_plan(m, n, k, sms, cx);
         ok = pl.partial_bytes == 0;

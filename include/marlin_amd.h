@@ -56,8 +56,9 @@ extern "C" {
  * is allocated while `stream` is being captured into a graph, and no more than
  * 256 buffers per device.  A call that cannot have its scratch for that runs
  * without in two cases: planned for the prefill kernels, its tiles are computed
- * whole instead of in slices of the k range; of 9 to 16 rows (no `sms` hint), it
- * is computed by column strips over the whole k range instead of streaming.
+ * whole instead of in slices of the k range; planned to stream, of 9 to 16 rows, or
+ * of more where column strips over the whole k range take about as long (no `sms`
+ * hint), it is computed by those.
  * Either may take longer and sums in another order, so that the last bit of an
  * element may be rounded the other way than by the same call with its scratch --
  * by a graph captured so and an eager call, for instance.  Other calls return

@@ -76,6 +76,24 @@ def test_few_rows_take_the_faster_kernel(m, n, k, groupsize, kernel):
     assert marlin.plan(m, n, k, groupsize)[1]["kernel"] == kernel
 
 
+@pytest.mark.parametrize("m,n,k,groupsize", [(47, 7168, 9472, 128), (48, 7168, 9984, 128), (46, 7424, 11776, -1),
+                                              (46, 7936, 11008, 128), (44, 7168, 11648, 128), (1342, 512, 6400, 128)])
+def test_a_deep_k_streams(m, n, k, groupsize):
+    """Sizes at which the kernel took 1.10 to 1.21 times the plan's launch: 33 to 48 rows over a
+    deep k, where the streaming kernel's fit reads high, and rows far beyond an XCD's L2."""
+    import marlin
+    assert marlin.rows_plan(m, n, k, groupsize) is None
+
+
+@pytest.mark.parametrize("m,n,k,groupsize", [(96, 4096, 4096, 128), (128, 4096, 4096, 128), (64, 8192, 4096, 128),
+                                              (141, 3840, 1536, 128), (179, 3072, 1536, 128), (36, 12288, 1280, 128)])
+def test_where_the_plan_was_slower(m, n, k, groupsize):
+    """Sizes at which the plan's launch took 1.2 times the kernel's time and more, three of them
+    of ten and twelve groups."""
+    import marlin
+    assert marlin.rows_plan(m, n, k, groupsize) is not None
+
+
 @pytest.mark.parametrize("m,n,k,groupsize", [(64, 28672, 8192, 128), (45, 12288, 4096, -1), (144, 2048, 1792, 128),
                                              (491, 2048, 5760, 128)])
 def test_the_probes_follow_this_kernel(m, n, k, groupsize):
@@ -243,7 +261,7 @@ def test_chosen_and_captured(m, n, k, g):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k,g", [(10, 768, 11392, 128), (16, 4096, 11008, 128), (9, 512, 12288, -1)])
+@pytest.mark.parametrize("m,n,k,g", [(10, 768, 11392, 128), (16, 4096, 11008, 128), (9, 512, 12288, -1), (17, 16128, 2176, 128)])
 def test_few_rows_captured_without_scratch(m, n, k, g):
     """Problems that the streaming kernel shares out are captured on a stream that has no
     scratch, as column strips, to the bits of an eager call on that kernel, and replayed between
