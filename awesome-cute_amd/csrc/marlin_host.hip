@@ -753,26 +753,27 @@ struct RowsPlan {
 // What the fit of streaming launches of 17 to 64 rows over k of 2048 and more is off by: it does
 // not tell the kinds of scales apart, and knows little of how many workgroups share a tile (1108
 // launches, by row blocks, cut in halves or not, and sharers: 2 to 4 % rms; 64 x 2048 x 8192,
-// sixteen, 1.25 of the fit, 47 x 7168 x 9472, four, 0.93).  And a line between these launches
-// and the rows kernel costs least 2 % above, with three row blocks uncut 2 % below.
+// sixteen, 1.25 of the fit, 47 x 7168 x 9472, four, 0.93; tiles that are not shared by their depth:
+// 17 x 28672 x 8192 1.03, a quarter of that 0.86).  And a line between these launches
+// and the rows kernel costs least 2 % above, with three row blocks uncut at it.
 double stream_off(int m, const Plan& pl, bool grouped) {
   const int sharers = pl.sp.wpt, blocks = ceil_div(m, 16);
   if (sharers == 0) return grouped ? 1.17 : 1.23;  // (runs that straddle tiles)
   double off;
   if (sharers == 1)
-    off = pl.row_parts > 1 ? 0.94 : blocks == 2 ? 0.91 : 0.81;
+    off = pl.row_parts > 1 ? 0.94 : blocks == 2 ? 0.82 + 0.0017 * pl.sp.gpb : 0.80 + 0.001 * pl.sp.gpb;
   else if (pl.row_parts == 1)
-    off = (blocks == 2 ? 1.02 : 0.907) + 0.006 * (sharers - 2);
+    off = (blocks == 2 ? 1.02 : 0.925) + 0.006 * (sharers - 2);
   else if (sharers <= 8)
     off = 0.984 + 0.0133 * (sharers - 2);
   else  // (fetched in two rounds)
     off = blocks == 2 ? 1.07 : 1.173 + 0.0133 * (sharers - 9);
-  return off * (grouped ? 1.0 : sharers > 8 ? 0.98 : 0.935);
+  return off * (grouped ? 1.0 : sharers > 8 ? 0.98 : pl.row_parts == 1 ? 0.955 : 0.935);
 }
 
 // For 17 rows and more, where it is cheaper than the plan.  Not over k ranges below 640, nor,
 // with 16 rows per workgroup, below 2048, where the plan's column strips are that launch.  Over
-// 6262 problems the choice takes 1.006 of the best launch measured, 42 of them more than 10 %
+// 6262 problems the choice takes 1.005 of the best launch measured, 37 of them more than 10 %
 // longer (by a fit of a kernel whose weights went through registers, with factors: 1.016 and
 // 355).  What the plans' own fits are off by near the line is in the limits; 0.03 to either side
 // costs less than 0.001 of the time.
