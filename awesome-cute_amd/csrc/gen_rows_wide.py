@@ -2,8 +2,8 @@
 """Writes the loop of the rows kernel over 128 columns (w4a16_rows_wide.hip) as one
 inline-assembly statement with fixed registers.
 
-Why assembly: a wave keeps weights requested two chunks ahead and activations more
-than one, next to 128 accumulators and the operands in use, in 256 registers.  The
+Why assembly: a wave keeps weights requested three chunks ahead and activations
+two, next to 128 accumulators and the operands in use, in 256 registers.  The
 compiler moves registers that are still being loaded from one turn of the loop to
 the next, which waits for everything in flight, and puts twelve vector operations
 in a row before the MFMAs that need them.  Here every wait lets exactly the later
@@ -36,9 +36,9 @@ Register map (v = VGPR, a = AGPR, s = SGPR):
 import sys
 
 RING = 3
+SLOT = 8192  # a chunk's activations in LDS (a power of two)
 W0, S0, OP0, A0, WT0, AL0 = 0, 48, 60, 72, 104, 108
 VB, VS, VRD, VEX, VNEG72 = 116, 117, (118, 119), 120, 121
-N_VGPR = 122
 RA, RB, RS = 40, 44, 48
 S_BEGIN, S_END, S_BROW, S_N2, S_LDS = 52, 53, 54, 55, 56
 (S_C, S_T, S_SA, S_SB, S_SS, S_FULLA, S_FULLB, S_FULLS, S_LOMASK, S_HIMASK, S_NEG1032,
@@ -46,10 +46,9 @@ S_BEGIN, S_END, S_BROW, S_N2, S_LDS = 52, 53, 54, 55, 56
 
 
 def set_blocks(mb):
-    """row blocks of 16, and what follows from them"""
-    global MB, SLOT
+    """row blocks of 16"""
+    global MB
     MB = mb
-    SLOT = 8192  # a chunk's activations in LDS (a power of two)
 
 
 def W(r, i): return W0 + 16 * r + 4 * i

@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace w4a16 {
 
 typedef _Float16 half_t;
@@ -237,6 +239,15 @@ __device__ __forceinline__ int finish_pieces(int shares, int slices, int pieces)
     mask |= (1 << (pieces * (r + 1) / slices)) - (1 << (pieces * r / slices));
   }
   return mask;
+}
+
+// f(0) ... f(N - 1) with constants
+template <int N, class F>
+__device__ __forceinline__ void for_each(F f) {
+  if constexpr (N > 0) {
+    for_each<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
 }
 
 // Which of the eight runs of a k range the rows kernels' wave computes.  Waves w and w + 4 share a

@@ -40,8 +40,6 @@
 // over weights from memory, 2 to 12 % longer where a cache has them.)
 //
 // Eight strips are a kernel of their own (w4a16_rows_wide.hip).
-#include <type_traits>
-
 #include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
@@ -57,14 +55,6 @@ __device__ __forceinline__ void rows_read2(unsigned at, i2& v) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("ds_read2_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(at), "n"(DW0), "n"(DW1) : "memory");
 #endif
-}
-
-template <int N, class F>
-__device__ __forceinline__ void rows_each(F f) {
-  if constexpr (N > 0) {
-    rows_each<N - 1>(f);
-    f(std::integral_constant<int, N - 1>{});
-  }
 }
 
 }  // namespace
@@ -225,7 +215,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
       __builtin_amdgcn_s_waitcnt(vmcnt(0));
     __builtin_amdgcn_sched_barrier(0);
     i4 av[MB][2];
-    rows_each<MB>([&](auto I) {
+    for_each<MB>([&](auto I) {
       read_lds16<2048 * I.value>(a_rd[0] + d * Sh::kSlot, av[I.value][0]);
       read_lds16<2048 * I.value>(a_rd[1] + d * Sh::kSlot, av[I.value][1]);
     });
@@ -235,7 +225,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void rows_kernel(GemmArgs p) {
 #pragma unroll
     for (int t = 0; t < 4; t++) {
       const unsigned at = b_rd[t] + w_at * (1024 * NB) + (first ? 0 : 512 * CS);
-      rows_each<NP>([&](auto I) {
+      for_each<NP>([&](auto I) {
         rows_read2<64 * I.value, 64 * I.value + (2 * I.value + 1 < CS ? 32 : 0)>(at, wv[t][I.value]);
       });
     }

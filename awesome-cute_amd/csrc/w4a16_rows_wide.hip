@@ -8,10 +8,11 @@
 // 41.7, 49.4 and 41.6; with seven strips through LDS 45.5).
 //
 // Bound: what the compute unit takes in.  1.5 MB each at M = 64, N = 28672, K = 8192, two
-// thirds of them activations, in 27 us: 57 GB/s, as much as a compute unit draws from
-// beyond its L2.  Its loads come back in order, so activations that the L2 has wait behind
-// weights that it has not: the loads of the launch alone take 28 us, the weights' alone
-// 15, the activations' alone 10, the arithmetic alone 23.
+// thirds of them activations, in a loop of 27 us: 57 GB/s, as much as a compute unit draws
+// from beyond its L2.  Its loads come back in order, so activations that the L2 has wait
+// behind weights that it has not: in builds without the rest the loop takes 28 us for the
+// loads alone, 15 for the weights', 10 for the activations', 23 for the arithmetic (whole
+// launches 35.4, 23.7, 16.3 and 29.5).
 //
 // rows_deep_kernel, for 33 rows and more over a deep k: weights requested three chunks ahead,
 // activations two, and the unpack dealt out behind the MFMAs of the operand before
@@ -19,8 +20,6 @@
 // without, 64 x 16384: k = 1024 1.04, 2048 1.03, 3072 0.97, 4096 0.97, 8192 0.95; 256 x 8192:
 // 1.05, 1.01, 0.99, 1.01, 0.94, k = 11008 0.93; 64 x 28672 x 8192 42.1 -> 41.2 us; with three
 // row blocks 192 x 8192 1.06, 1.03, 1.00, 0.97, 0.96; 40 x 24576 x 4096 1.00, 8192 0.99.
-#include <type_traits>
-
 #include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
@@ -40,14 +39,6 @@ struct WideShape {
   static constexpr int kReduce = kWaves * kPass * 1024;
   static constexpr int kLds = kWaves * kSlot > kReduce ? kWaves * kSlot : kReduce;
 };
-
-template <int N, class F>
-__device__ __forceinline__ void wide_each(F f) {
-  if constexpr (N > 0) {
-    wide_each<N - 1>(f);
-    f(std::integral_constant<int, N - 1>{});
-  }
-}
 
 // the waves' sums meet, a block of 16 slots x 16 rows to a wave, and C is written
 template <int MB, bool GROUP>
@@ -96,6 +87,45 @@ __device__ __forceinline__ void wide_finish(const GemmArgs& p, char* smem, const
   }
 }
 
+// what a lane of either kernel computes and where its pieces lie
+template <int MB, bool GROUP>
+struct WideLane {
+  int wave, lane, kg, nu;
+  int set, row0;  // my strip set, my first row
+  int c0, c1;     // my chunks of 64 k-values: whole groups where there are groups
+  // this lane's 16-byte pieces of B (Marlin lane t = kg, c = nu%8 of block nu/8) and, of a
+  // group, the scales of columns 16j + 8h + c of that block
+  int b_src, s_src;
+  // activations: 128 bytes of eight rows per load; piece p of row r sits at position p ^ (r % 8),
+  // so that the operand reads (piece 2 kg + q of row nu) meet no bank twice.  Rows past M are
+  // zeros.
+  int a_src[2 * MB];
+
+  __device__ __forceinline__ explicit WideLane(const GemmArgs& p) {
+    const int tid = threadIdx.x;
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    lane = tid & 63;
+    kg = lane >> 4;
+    nu = lane & 15;
+    // the parts of a strip set are neighbours behind one L2 (p.gpb carries the grid)
+    const int wid = xcd_work_index((int)blockIdx.x, p.gpb);
+    set = wid / p.row_parts;
+    row0 = 16 * MB * (wid - set * p.row_parts);
+    const int chunks = p.K / 64;
+    const int run = rows_run(wave);
+    c0 = GROUP ? 2 * (run * (chunks / 2) / kWaves) : run * chunks / kWaves;
+    c1 = GROUP ? 2 * ((run + 1) * (chunks / 2) / kWaves) : (run + 1) * chunks / kWaves;
+    b_src = 1024 * set + 512 * (nu >> 3) + 16 * (4 * (nu & 7) + kg);
+    s_src = 256 * set + 128 * (nu >> 3) + 16 * (nu & 7);
+#pragma unroll
+    for (int i = 0; i < 2 * MB; i++) {
+      const int r = row0 + 8 * i + lane / 8;
+      a_src[i] = r < p.M ? r * p.K * 2 + 16 * ((lane % 8) ^ (lane / 8)) : kOob;
+    }
+  }
+  __device__ __forceinline__ unsigned a_rd(int q) const { return nu * 128 + 16 * ((2 * kg + q) ^ (nu & 7)); }
+};
+
 }  // namespace
 
 template <int MB, bool GROUP>
@@ -103,21 +133,7 @@ __global__ __launch_bounds__(64 * kWaves) void rows_wide_kernel(GemmArgs p) {
   using Sh = WideShape<MB>;
   constexpr int NA = 2 * MB;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // Sh::kLds
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int kg = lane >> 4;
-  const int nu = lane & 15;
-  // the parts of a strip set are neighbours behind one L2 (p.gpb carries the grid)
-  const int wid = xcd_work_index((int)blockIdx.x, p.gpb);
-  const int set = wid / p.row_parts;
-  const int row0 = 16 * MB * (wid - set * p.row_parts);
-
-  // my chunks [c0, c1) of 64 k-values: whole groups where there are groups
-  const int chunks = p.K / 64;
-  const int run = rows_run(wave);
-  const int c0 = GROUP ? 2 * (run * (chunks / 2) / kWaves) : run * chunks / kWaves;
-  const int c1 = GROUP ? 2 * ((run + 1) * (chunks / 2) / kWaves) : (run + 1) * chunks / kWaves;
+  const WideLane<MB, GROUP> me(p);
 
   const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
@@ -125,23 +141,9 @@ __global__ __launch_bounds__(64 * kWaves) void rows_wide_kernel(GemmArgs p) {
       make_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
   const int b_row = p.N * 8;  // bytes per row of B
 
-  char* const stage = smem + wave * Sh::kSlot;
+  char* const stage = smem + me.wave * Sh::kSlot;
   const unsigned lds_a = (unsigned)(size_t)stage;
-  // this lane's pieces of B and, of a group, the scales of columns 16j + 8h + c of its block
-  const int b_src = 1024 * set + 512 * (nu >> 3) + 16 * (4 * (nu & 7) + kg);
-  const int s_src = 256 * set + 128 * (nu >> 3) + 16 * (nu & 7);
-  // activations: 128 bytes of eight rows per load; piece p of row r sits at position
-  // p ^ (r % 8), so that the operand reads (piece 2 kg + q of row nu) meet no bank
-  // twice.  Rows past M are zeros.
-  int a_src[NA];
-#pragma unroll
-  for (int i = 0; i < NA; i++) {
-    const int r = row0 + 8 * i + lane / 8;
-    a_src[i] = r < p.M ? r * p.K * 2 + 16 * ((lane % 8) ^ (lane / 8)) : kOob;
-  }
-  unsigned a_rd[2];
-#pragma unroll
-  for (int q = 0; q < 2; q++) a_rd[q] = lds_a + nu * 128 + 16 * ((2 * kg + q) ^ (nu & 7));
+  const unsigned a_rd[2] = {lds_a + me.a_rd(0), lds_a + me.a_rd(1)};
 
   const DequantConsts dc;
   i4 bq[4];
@@ -151,13 +153,13 @@ __global__ __launch_bounds__(64 * kWaves) void rows_wide_kernel(GemmArgs p) {
   // mine is requested at an offset past everything.
   auto issue = [&](int c, bool even) {
     __builtin_amdgcn_sched_barrier(0);
-    const int inv = c < c1 ? 0 : kOob;
-    if (GROUP && even) sq = __builtin_amdgcn_raw_buffer_load_b128(rS, s_src | inv, (c >> 1) * p.N * 2, 0);
+    const int inv = c < me.c1 ? 0 : kOob;
+    if (GROUP && even) sq = __builtin_amdgcn_raw_buffer_load_b128(rS, me.s_src | inv, (c >> 1) * p.N * 2, 0);
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      bq[i] = __builtin_amdgcn_raw_buffer_load_b128(rB, b_src | inv, (4 * c + i) * b_row, 2);
+      bq[i] = __builtin_amdgcn_raw_buffer_load_b128(rB, me.b_src | inv, (4 * c + i) * b_row, 2);
 #pragma unroll
-    for (int i = 0; i < NA; i++) load_to_lds16(rA, stage + 1024 * i, a_src[i] | inv, 128 * c);
+    for (int i = 0; i < NA; i++) load_to_lds16(rA, stage + 1024 * i, me.a_src[i] | inv, 128 * c);
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(64 * kWaves) void rows_wide_kernel(GemmArgs p) {
     __builtin_amdgcn_s_waitcnt(vmcnt(0));  // chunk c has landed
     __builtin_amdgcn_sched_barrier(0);
     i4 av[MB][2];
-    wide_each<MB>([&](auto I) {
+    for_each<MB>([&](auto I) {
       read_lds16<2048 * I.value>(a_rd[0], av[I.value][0]);
       read_lds16<2048 * I.value>(a_rd[1], av[I.value][1]);
     });
@@ -220,15 +222,15 @@ __global__ __launch_bounds__(64 * kWaves) void rows_wide_kernel(GemmArgs p) {
     }
   };
 
-  issue(c0, true);
-  for (int c = c0; c < c1; c += 2) {
+  issue(me.c0, true);
+  for (int c = me.c0; c < me.c1; c += 2) {
     step(c, std::true_type{});
-    if (c + 1 < c1) step(c + 1, std::false_type{});
+    if (c + 1 < me.c1) step(c + 1, std::false_type{});
   }
   // nothing may still be on its way into LDS when it is reused
   __builtin_amdgcn_s_waitcnt(0);
 
-  wide_finish<MB, GROUP>(p, smem, acc, rS, set, row0, wave, lane);
+  wide_finish<MB, GROUP>(p, smem, acc, rS, me.set, me.row0, me.wave, me.lane);
 }
 
 // The same over a deep k range, with the loop that gen_rows_wide.py writes: weights requested
@@ -237,44 +239,17 @@ template <int MB, bool GROUP>
 __global__ __launch_bounds__(64 * kWaves) void rows_deep_kernel(GemmArgs p) {
   constexpr int kSlot = 8192;  // activations of a chunk, slots swapped by an exclusive or
   extern __shared__ __attribute__((aligned(16))) char smem[];  // kDeepLds
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int kg = lane >> 4;
-  const int nu = lane & 15;
-  // the parts of a strip set are neighbours behind one L2 (p.gpb carries the grid)
-  const int wid = xcd_work_index((int)blockIdx.x, p.gpb);
-  const int set = wid / p.row_parts;
-  const int row0 = 16 * MB * (wid - set * p.row_parts);
-
-  // my chunks [c0, c1) of 64 k-values: whole groups where there are groups
-  const int chunks = p.K / 64;
-  const int run = rows_run(wave);
-  const int c0 = GROUP ? 2 * (run * (chunks / 2) / kWaves) : run * chunks / kWaves;
-  const int c1 = GROUP ? 2 * ((run + 1) * (chunks / 2) / kWaves) : (run + 1) * chunks / kWaves;
+  const WideLane<MB, GROUP> me(p);
 
   i4 rb_words = rsrc_words(p.B, (unsigned)p.K * (unsigned)(p.N / 2));
   i4 ra_words = rsrc_words(p.A, (unsigned)p.M * (unsigned)p.K * 2u);
   i4 rs_words = rsrc_words(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
   const int b_row = p.N * 8;  // bytes per row of B
   const int s_row = p.N * 2;
-  // this lane's 16-byte pieces of B (Marlin lane t = kg, c = nu%8 of block nu/8), and the
-  // scales of columns 16j + 8h + c of that block
-  const int b_src = 1024 * set + 512 * (nu >> 3) + 16 * (4 * (nu & 7) + kg);
-  const int s_src = 256 * set + 128 * (nu >> 3) + 16 * (nu & 7);
-  // activations: 128 bytes of eight rows per load; piece p of row r sits at position
-  // p ^ (r % 8), so that the operand reads (piece 2 kg + q of row nu) meet no bank
-  // twice.  Rows past M are zeros.
-  int a_src[2 * MB];
-#pragma unroll
-  for (int i = 0; i < 2 * MB; i++) {
-    const int r = row0 + 8 * i + lane / 8;
-    a_src[i] = r < p.M ? r * p.K * 2 + 16 * ((lane % 8) ^ (lane / 8)) : kOob;
-  }
-  unsigned lds_slot = (unsigned)(size_t)smem + wave * 2 * kSlot;  // (the only LDS of the kernel: at 0)
-  unsigned a_rd[2];
-#pragma unroll
-  for (int q = 0; q < 2; q++) a_rd[q] = lds_slot + nu * 128 + 16 * ((2 * kg + q) ^ (nu & 7));
+  const int b_src = me.b_src, s_src = me.s_src, c0 = me.c0, c1 = me.c1;
+  const int(&a_src)[2 * MB] = me.a_src;
+  unsigned lds_slot = (unsigned)(size_t)smem + me.wave * 2 * kSlot;  // (the only LDS of the kernel: at 0)
+  unsigned a_rd[2] = {lds_slot + me.a_rd(0), lds_slot + me.a_rd(1)};
 
   f4 acc[8][MB];
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -298,7 +273,7 @@ __global__ __launch_bounds__(64 * kWaves) void rows_deep_kernel(GemmArgs p) {
   __amdgpu_buffer_rsrc_t rS = make_rsrc(p.S, (unsigned)(GROUP ? p.K / 128 : 1) * (unsigned)p.N * 2u);
   // (the lane once more, so that no register is held through the statement, which leaves six)
   const int again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
-  wide_finish<MB, GROUP>(p, smem, acc, rS, set, row0, wave, again);
+  wide_finish<MB, GROUP>(p, smem, acc, rS, me.set, me.row0, me.wave, again);
 }
 
 namespace {
