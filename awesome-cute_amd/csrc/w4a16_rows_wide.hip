@@ -17,9 +17,10 @@
 // rows_deep_kernel, for 33 rows and more over a deep k: weights requested three chunks ahead,
 // activations two, and the unpack dealt out behind the MFMAs of the operand before
 // (gen_rows_wide.py).  Its start and its code are longer.  Time by it over the time
-// without, 64 x 16384: k = 1024 1.04, 2048 1.03, 3072 0.97, 4096 0.97, 8192 0.95; 256 x 8192:
-// 1.05, 1.01, 0.99, 1.01, 0.94, k = 11008 0.93; 64 x 28672 x 8192 42.1 -> 41.2 us; with three
-// row blocks 192 x 8192 1.06, 1.03, 1.00, 0.97, 0.96; 40 x 24576 x 4096 1.00, 8192 0.99.
+// without, means over 1435 problems of one to four row parts by k in steps of 512, four row
+// blocks: from k = 2560 0.996, 3072 0.989, 3584 0.985, 4096 0.978, 5120 0.967, 6656 0.964;
+// three: 1.029, 1.018, 1.010, 1.005, from 4608 0.999, 5120 0.994, 6656 0.989; 64 x 28672 x
+// 8192 42.1 -> 41.2 us.
 #include "buffer_loads.hpp"
 #include "w4a16_common.hpp"
 
@@ -318,7 +319,8 @@ int launch_rows_wide(const GemmArgs& a, bool group, int blocks, hipStream_t stre
   GemmArgs b = a;
   b.row_parts = ceil_div(a.M, 16 * blocks);
   b.gpb = a.N / 128 * b.row_parts;
-  const bool deep = (blocks == 4 && a.K >= 4096) || (blocks == 3 && a.K >= 5120);
+  // (from where it is a hundredth faster with four row blocks, half that with three)
+  const bool deep = (blocks == 4 && a.K >= 3072) || (blocks == 3 && a.K >= 5120);
   const bool found = with_wide_kernel(blocks, group, deep, [&](auto kernel, int lds) {
     hipLaunchKernelGGL(kernel, dim3(b.gpb), dim3(64 * kWaves), lds, stream, b);
   });

@@ -181,7 +181,7 @@ def test_rows_of_few_chunks(pair, groupsize):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("pair,k", [((8, 3), 5120), ((8, 3), 5888), ((8, 4), 4096), ((8, 4), 4736), ((8, 4), 8192)])
+@pytest.mark.parametrize("pair,k", [((8, 3), 5120), ((8, 3), 5888), ((8, 4), 3072), ((8, 4), 3200), ((8, 4), 4096), ((8, 4), 4736), ((8, 4), 8192)])
 @pytest.mark.parametrize("groupsize", [128, -1])
 def test_rows_over_a_deep_k(pair, k, groupsize):
     """From where weights are requested three chunks ahead: chunks per wave that the ring of
